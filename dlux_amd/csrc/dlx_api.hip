@@ -6,6 +6,7 @@
 #include <mutex>
 #include <vector>
 
+#include "dlx_fold.h"
 #include "dlx_internal.h"
 #include "dlx_split.h"
 
@@ -598,14 +599,63 @@ int dlx_intensity(int64_t npix, int32_t batch, const void* field, int32_t sum_ov
 namespace dlx {
 namespace {
 
-// Bytes of the psf chain's buffers for a chunk of c wavelengths: the pupils P,
-// the transfer matrices (used when they are not taken from the cache), the
-// stage-1 intermediate U^T and the per-wavelength |E|^2 planes.
+// The psf chain's buffers for a chunk of c wavelengths: the tables (used when
+// they are not taken from the cache), the stage-1 result, the per-wavelength
+// |E|^2 planes and, when `bytes` leaves room for it, the folded pupil.
+struct PsfLayout {
+  size_t T, U, I, P, total;   // total without P
+};
+PsfLayout psf_layout(const dlx_mft_geom& g, int c) {
+  PsfLayout L;
+  L.T = align_up((size_t)c * fold_table_bytes(g.n_in, g.n_out));
+  L.U = align_up((size_t)c * fold_mid_bytes(g.n_in, g.n_out));
+  L.I = align_up((size_t)c * g.n_out * g.n_out * sizeof(float));
+  L.P = align_up((size_t)c * fold_field_bytes(g.n_in));
+  L.total = L.T + L.U + L.I;
+  return L;
+}
+
+// Workspace of the psf chain: a complex pupil, two complex matrices and the
+// planes per wavelength -- which the folded buffers fit in on all but the
+// smallest grids -- so that the limits a caller meets do not depend on how the
+// chain lays its buffers out.
 size_t psf_poly_bytes(const dlx_mft_geom& g, int c, bool split) {
   const size_t P = align_up((size_t)c * mat_bytes(g.n_in, g.n_in, split));
   const size_t W = align_up((size_t)c * mat_bytes(g.n_out, g.n_in, split));
   const size_t I = align_up((size_t)c * g.n_out * g.n_out * sizeof(float));
-  return P + 2 * W + I;
+  const size_t plain = P + 2 * W + I, fold = psf_layout(g, c).total;
+  return plain > fold ? plain : fold;
+}
+
+// The cosine / sine tables of nb wavelengths (and, with `adjoint`, of the
+// transposed contraction), from the device cache -- an entry holds both -- or
+// generated into `ws` when the cache is bypassed.
+struct FoldTables {
+  const uint8_t *fwd, *adj;
+  long stride;
+};
+int fold_tables(const dlx_mft_geom& g, int nb, const double* wl, double dx, double p_out, bool split,
+                bool adjoint, bool use_cache, uint8_t* ws, hipStream_t s, FoldTables* out,
+                CacheLease* lease) {
+  const long tf = fold_table_bytes(g.n_in, g.n_out), ta = fold_table_bytes(g.n_out, g.n_in);
+  std::vector<double> key = {2001.0, (double)g.n_in, (double)g.n_out, split ? 1.0 : 0.0};
+  for (int i = 0; i < nb; ++i) key.push_back(fold_step(g, wl[i], dx, p_out));
+  const double* step = key.data() + 4;
+  void* mem = nullptr;
+  bool fresh = true;
+  if (use_cache)
+    if (int st = cache_acquire_raw(key, (size_t)nb * (tf + ta), s, &mem, &lease->h, &fresh, true))
+      return st;
+  uint8_t* base = mem ? (uint8_t*)mem : ws;
+  out->stride = mem || adjoint ? tf + ta : tf;
+  out->fwd = base;
+  out->adj = base + tf;
+  if (fresh) {
+    DLX_HIP(launch_fold_tables(step, nb, g.n_in, g.n_out, split, mem || adjoint, base, out->stride,
+                               s));
+    if (int st = cache_ready(lease->h, s)) return st;
+  }
+  return DLX_OK;
 }
 
 int check_psf_poly_args(const dlx_mft_geom* geom, int32_t nwl, const double* wavelength,
@@ -630,86 +680,78 @@ int check_psf_poly_args(const dlx_mft_geom* geom, int32_t nwl, const double* wav
 }
 
 // The psf chain over chunks of at most c wavelengths in `ws` (psf_poly_bytes(c)
-// bytes): pupils, matrices (from the device cache when `use_cache`, else
-// generated into ws), the two contractions with the |E|^2 epilogue, and the
-// running sum over wavelengths in wavelength order (so the result does not
-// depend on c).  With `planes` set, every wavelength's w_l |E_l|^2 plane is
-// written there instead (planes + l N_out^2) and nothing is summed.  `prof`
-// records the contractions' live timing.
+// bytes): tables (from the device cache when `use_cache`, else generated into
+// ws), the two folded contractions with the |E|^2 epilogue, and the running
+// sum over wavelengths in wavelength order (so the result does not depend on
+// c).  With `planes` set, every wavelength's w_l |E_l|^2 plane is written there
+// instead (planes + l N_out^2) and nothing is summed.  `prof` records the
+// contractions' live timing.
 int psf_poly_run(const dlx_mft_geom& g, int32_t nwl, const double* wavelength,
                  const double* weight, double pixel_scale_in, double pixel_scale_out,
                  double center, double tilt_x, double tilt_y, const float* amp,
                  const float* opd, const float* phase, double scale, float* psf, bool split,
                  uint8_t* ws, int c, bool use_cache, bool prof, hipStream_t s,
                  float* planes = nullptr) {
-  const size_t Pb = align_up((size_t)c * mat_bytes(g.n_in, g.n_in, split));
-  const size_t Wb = align_up((size_t)c * mat_bytes(g.n_out, g.n_in, split));
-  uint8_t* P = ws;
-  uint8_t* W_ws = P + Pb;
-  uint8_t* Ut = P + Pb + Wb;
-  float* I = (float*)(P + Pb + 2 * Wb);
+  const PsfLayout L = psf_layout(g, c);
+  uint8_t* T_ws = ws;
+  uint8_t* U = T_ws + L.T;
+  float* I = (float*)(U + L.U);
+  uint8_t* P = (uint8_t*)I + L.I;
+  const bool room = L.total + L.P <= psf_poly_bytes(g, c, split);
   const long nout2 = (long)g.n_out * g.n_out;
-  const double x0 = center - (g.n_in - 1) / 2.0 * pixel_scale_in;
-
-  std::vector<double> dx(c, pixel_scale_in), pout(c, pixel_scale_out), alpha(c);
+  FoldStage1 f1{};
+  f1.n = g.n_in;
+  f1.m = g.n_out;
+  f1.out = U;
+  f1.out_stride = fold_mid_bytes(g.n_in, g.n_out);
+  f1.pupil = {opd, amp, phase, pixel_scale_in, center - (g.n_in - 1) / 2.0 * pixel_scale_in, tilt_x,
+              tilt_y, (float)scale};
+  // the pupil formed in stage 1's loader (no pupil array in HBM), or written
+  // first where many column tiles would each form it again
+  const bool in_loader = !room || (!phase && pupil_prologue_enabled() && fold_pupil_in_loader(g.n_out));
   for (int l0 = 0; l0 < nwl; l0 += c) {
     const int nb = nwl - l0 < c ? nwl - l0 : c;
-    float* Ic = planes ? planes + (long)l0 * nout2 : I;
-    // |E_l|^2 = (c_l sqrt(w_l))^2 |Y^T P X|^2: the scale is applied in the
-    // stage-2 epilogue, so the matrices depend on the geometry only.
-    for (int i = 0; i < nb; ++i)
-      alpha[i] = mft_norm(g, wavelength[l0 + i], pixel_scale_in, pixel_scale_out) *
-                 std::sqrt(weight[l0 + i]);
-    void* W = nullptr;
+    // one wavelength is its own sum
+    float* Ic = planes ? planes + (long)l0 * nout2 : nwl == 1 ? psf : I;
     CacheLease h(s);
-    if (use_cache) {
-      if (int st = get_matrices(g, nb, wavelength + l0, dx.data(), pout.data(), nullptr, split,
-                                W_ws, s, &W, &h.h))
-        return st;
-    } else {
-      W = W_ws;
-      if (int st = gen_dft(g, nb, wavelength + l0, dx.data(), pout.data(), nullptr, nullptr,
-                           W_ws, split, s))
-        return st;
+    FoldTables tab;
+    if (int st = fold_tables(g, nb, wavelength + l0, pixel_scale_in, pixel_scale_out, split, false,
+                             use_cache, T_ws, s, &tab, &h))
+      return st;
+    f1.batch = nb;
+    f1.table = tab.fwd;
+    f1.table_stride = tab.stride;
+    for (int i = 0; i < nb; ++i) f1.inv_wl[i] = 1.0 / wavelength[l0 + i];
+    if (!in_loader) {
+      f1.src = P;
+      f1.src_stride = fold_field_bytes(g.n_in);
+      DLX_HIP(launch_fold_pupil(f1.pupil, f1.inv_wl, nb, g.n_in, split, P, f1.src_stride, s));
     }
-    if (split) {
-      // the pupil generated in stage 1's loader from the amplitude and OPD
-      // planes where the shape allows (no pupil array in HBM), else written
-      // by the pupil kernel
-      PupilGen pg{};
-      pg.opd = opd;
-      pg.amp = amp;
-      pg.dx = pixel_scale_in;
-      pg.x0 = x0;
-      pg.tx = tilt_x;
-      pg.ty = tilt_y;
-      pg.scale = (float)scale;
-      pg.n = g.n_in;
-      for (int i = 0; i < nb; ++i) pg.inv_wl[i] = 1.0 / wavelength[l0 + i];
-      const bool fuse = !phase && pupil_prologue_enabled() &&
-                        cgemm_pupil_supported(stage1_split(g, 0, nb, nullptr,
-                                                           (const uint8_t*)W, Ut), pg);
-      if (!fuse) {
-        PupilChunk pc;
-        for (int i = 0; i < nb; ++i) pc.inv_wl[i] = pg.inv_wl[i];
-        DLX_HIP(launch_pupil_split4(pc, nb, g.n_in, pixel_scale_in, x0, tilt_x, tilt_y, amp,
-                                    opd, phase, (float)scale, P,
-                                    (long)mat_bytes(g.n_in, g.n_in, true), s));
-      }
-      if (int st = mft_split4(g, nb, P, (const uint8_t*)W, (const uint8_t*)W, Ut, alpha.data(),
-                              Ic, EPI_INTENSITY, s, prof ? prof_begin : nullptr,
-                              prof ? prof_end : nullptr, fuse ? &pg : nullptr))
-        return st;
-    } else {
-      if (int st = dlx_pupil_field(g.n_in, nb, wavelength + l0, pixel_scale_in, center, tilt_x,
-                                   tilt_y, amp, opd, phase, scale, nullptr, P, s))
-        return st;
-      if (int st = mft_fp32(g, nb, (const float2*)P, (const float2*)W, (const float2*)W,
-                            (float2*)Ut, alpha.data(), Ic, EPI_INTENSITY, s, prof))
-        return st;
-    }
+    int slot = -1;
+    if (prof) { if (int st = prof_begin(1, s, &slot)) return st; }
+    DLX_HIP(launch_fold_stage1(f1, in_loader ? FOLD_PUPIL : FOLD_MEM, split, s));
+    if (prof) { if (int st = prof_end(slot, s)) return st; }
+    // |E_l|^2 = (c_l sqrt(w_l))^2 |W_y P W_x^T|^2: the scale is applied in the
+    // stage-2 epilogue, so the tables depend on the geometry only.
+    FoldStage2 f2{};
+    f2.n = g.n_in;
+    f2.m = g.n_out;
+    f2.batch = nb;
+    f2.inverse = g.inverse;
+    f2.table = tab.fwd;
+    f2.table_stride = tab.stride;
+    f2.mid = U;
+    f2.mid_stride = f1.out_stride;
+    f2.out = Ic;
+    f2.out_stride = nout2;
+    for (int i = 0; i < nb; ++i)
+      f2.alpha[i] = (float)(mft_norm(g, wavelength[l0 + i], pixel_scale_in, pixel_scale_out) *
+                            std::sqrt(weight[l0 + i]));
+    if (prof) { if (int st = prof_begin(2, s, &slot)) return st; }
+    DLX_HIP(launch_fold_stage2(f2, FOLD_INTENSITY, split, s));
+    if (prof) { if (int st = prof_end(slot, s)) return st; }
     if (int st = h.release()) return st;
-    if (!planes) DLX_HIP(launch_sum_planes(nout2, nb, I, l0 > 0, psf, s));
+    if (!planes && nwl > 1) DLX_HIP(launch_sum_planes(nout2, nb, I, l0 > 0, psf, s));
   }
   return DLX_OK;
 }

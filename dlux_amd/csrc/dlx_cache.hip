@@ -271,7 +271,7 @@ uint64_t hash_key(const std::vector<double>& key) {
 }
 
 int cache_acquire_raw(const std::vector<double>& key_in, size_t bytes, hipStream_t s,
-                      void** ptr, void** handle, bool* fresh) {
+                      void** ptr, void** handle, bool* fresh, bool eager) {
   *ptr = nullptr;
   *handle = nullptr;
   *fresh = true;   // bypass and miss: the caller generates the contents
@@ -308,10 +308,11 @@ int cache_acquire_raw(const std::vector<double>& key_in, size_t bytes, hipStream
   ++c.misses;
   const size_t need = align_up(bytes);
   if (need > c.budget) return DLX_OK;
-  const uint64_t h = hash_key(key);
-  bool again = false;
-  for (auto& kv : c.seen)
-    if (kv.first == h) { again = true; kv.second = ++c.tick; break; }
+  bool again = eager;
+  const uint64_t h = eager ? 0 : hash_key(key);
+  if (!eager)
+    for (auto& kv : c.seen)
+      if (kv.first == h) { again = true; kv.second = ++c.tick; break; }
   if (!again) {
     if (c.seen.size() >= 256) {
       size_t old = 0;

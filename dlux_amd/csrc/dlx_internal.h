@@ -258,8 +258,10 @@ int cache_release(void* handle, hipStream_t s);
 // for work on s; on a miss (*fresh true) the caller fills it on s and then
 // calls cache_ready.  *ptr == NULL (and *fresh true) when bypassed (capture,
 // budget, memory): the caller generates into its own buffer.
+// The block is allocated on a key's second sighting, or on the first with
+// `eager`.
 int cache_acquire_raw(const std::vector<double>& key, size_t bytes, hipStream_t s,
-                      void** ptr, void** handle, bool* fresh);
+                      void** ptr, void** handle, bool* fresh, bool eager = false);
 int cache_ready(void* handle, hipStream_t s);
 
 // The detector chain (dlx_detector.hip) on one image that is the in-order sum
