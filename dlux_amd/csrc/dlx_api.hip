@@ -241,26 +241,131 @@ int mft_split4(const dlx_mft_geom& g, int batch, const uint8_t* P, const uint8_t
   return DLX_OK;
 }
 
-// Workspace of the VJP for one chunk of c wavelengths: pupils P, forward and
-// adjoint matrices (used when the cache is bypassed), the stage-1 intermediate
-// (U^T, later V^T), Ebar, and the per-wavelength gradient planes.
-struct VjpLayout {
-  size_t P, U, Wf, Wa, T, Eb, H, H2, total;
+// The psf chain's buffers for a chunk of c wavelengths: the tables (used when
+// they are not taken from the cache), the stage-1 result, the per-wavelength
+// |E|^2 planes and, when `bytes` leaves room for it, the folded pupil.
+struct PsfLayout {
+  size_t T, U, I, P, total;   // total without P
 };
-VjpLayout vjp_layout(const dlx_mft_geom& g, int c, bool split) {
+PsfLayout psf_layout(const dlx_mft_geom& g, int c) {
+  PsfLayout L;
+  L.T = align_up((size_t)c * fold_table_bytes(g.n_in, g.n_out));
+  L.U = align_up((size_t)c * fold_mid_bytes(g.n_in, g.n_out));
+  L.I = align_up((size_t)c * g.n_out * g.n_out * sizeof(float));
+  L.P = align_up((size_t)c * fold_field_bytes(g.n_in));
+  L.total = L.T + L.U + L.I;
+  return L;
+}
+
+// Workspace of the psf chain: a complex pupil, two complex matrices and the
+// planes per wavelength -- which the folded buffers fit in on all but the
+// smallest grids -- so that the limits a caller meets do not depend on how the
+// chain lays its buffers out.
+size_t psf_poly_bytes(const dlx_mft_geom& g, int c, bool split) {
+  const size_t P = align_up((size_t)c * mat_bytes(g.n_in, g.n_in, split));
+  const size_t W = align_up((size_t)c * mat_bytes(g.n_out, g.n_in, split));
+  const size_t I = align_up((size_t)c * g.n_out * g.n_out * sizeof(float));
+  const size_t plain = P + 2 * W + I, fold = psf_layout(g, c).total;
+  return plain > fold ? plain : fold;
+}
+
+// The cosine / sine tables of nb phase steps contracting side n into side m
+// (and, with `adjoint`, of the transposed contraction), from the device cache
+// -- an entry holds both -- or generated into `ws` when the cache is bypassed.
+// Equal steps share one table (stride 0).
+struct FoldTables {
+  const uint8_t *fwd, *adj;
+  long stride;
+};
+int fold_tables(int n, int m, const std::vector<double>& steps, bool split, bool adjoint,
+                bool use_cache, uint8_t* ws, hipStream_t s, FoldTables* out, CacheLease* lease) {
+  const long tf = fold_table_bytes(n, m), ta = fold_table_bytes(m, n);
+  bool one = true;
+  for (double v : steps) one = one && v == steps[0];
+  const int nb = one ? 1 : (int)steps.size();
+  void* mem = nullptr;
+  bool fresh = true;
+  if (use_cache) {
+    std::vector<double> key = {2001.0, (double)n, (double)m, split ? 1.0 : 0.0};
+    key.insert(key.end(), steps.begin(), steps.begin() + nb);
+    if (int st = cache_acquire_raw(key, (size_t)nb * (tf + ta), s, &mem, &lease->h, &fresh, true))
+      return st;
+  }
+  uint8_t* base = mem ? (uint8_t*)mem : ws;
+  const long stride = mem || adjoint ? tf + ta : tf;
+  out->stride = one ? 0 : stride;
+  out->fwd = base;
+  out->adj = base + tf;
+  if (fresh) {
+    DLX_HIP(launch_fold_tables(steps.data(), nb, n, m, split, mem || adjoint, base, stride, s));
+    if (int st = cache_ready(lease->h, s)) return st;
+  }
+  return DLX_OK;
+}
+
+std::vector<double> psf_steps(const dlx_mft_geom& g, int nb, const double* wl, double dx,
+                              double p_out) {
+  std::vector<double> st(nb);
+  for (int i = 0; i < nb; ++i) st[i] = fold_step(g, wl[i], dx, p_out);
+  return st;
+}
+
+// The transform of `batch` complex64 fields with per-instance phase steps,
+// input and output phases (either may be NULL) and scales: folded stage 1
+// loading the fields, stage 2 storing complex64.  `ws`: tables of the batch,
+// then the stage-1 results of a chunk (field_transform_bytes).
+constexpr int kFieldChunk = FoldStage1::kMaxBatch;
+size_t field_transform_bytes(int n, int m, int batch) {
+  const int c = batch < kFieldChunk ? batch : kFieldChunk;
+  return align_up((size_t)batch * fold_table_bytes(n, m)) +
+         align_up((size_t)c * fold_mid_bytes(n, m));
+}
+int field_transform(int n, int m, int batch, bool inverse, const std::vector<double>& steps,
+                    const FoldPhase* pin, const FoldPhase* pout, const double* alpha,
+                    const void* in, void* out, bool split, uint8_t* ws, hipStream_t s) {
+  CacheLease h(s);
+  FoldTables tab;
+  if (int st = fold_tables(n, m, steps, split, false, true, ws, s, &tab, &h)) return st;
+  uint8_t* U = ws + align_up((size_t)batch * fold_table_bytes(n, m));
+  for (int b0 = 0; b0 < batch; b0 += kFieldChunk) {
+    const int nb = batch - b0 < kFieldChunk ? batch - b0 : kFieldChunk;
+    FoldStage1 f{};
+    f.n = n; f.m = m; f.batch = nb;
+    f.src_stride = 8L * n * n;
+    f.src = (const uint8_t*)in + b0 * f.src_stride;
+    f.table = tab.fwd + b0 * tab.stride; f.table_stride = tab.stride;
+    f.out = U; f.out_stride = fold_mid_bytes(n, m);
+    FoldStage2 e{};
+    e.n = n; e.m = m; e.batch = nb; e.inverse = inverse;
+    e.table = f.table; e.table_stride = tab.stride;
+    e.mid = U; e.mid_stride = f.out_stride;
+    e.out_stride = (long)m * m;
+    e.out = (float2*)out + b0 * e.out_stride;
+    for (int i = 0; i < nb; ++i) {
+      if (pin) f.phase[i] = pin[b0 + i];
+      if (pout) e.phase[i] = pout[b0 + i];
+      e.alpha[i] = (float)alpha[b0 + i];
+    }
+    DLX_HIP(launch_fold_stage1(f, FOLD_FIELD, split, s));
+    DLX_HIP(launch_fold_stage2(e, FOLD_STORE, split, s));
+  }
+  return h.release();
+}
+
+// Workspace of the VJP for one chunk of c wavelengths: the tables of both
+// directions (used when the cache is bypassed), the stage-1 intermediate of
+// either direction, Ebar, and the per-wavelength gradient planes.
+struct VjpLayout {
+  size_t T, U, Eb, H, total;
+};
+VjpLayout vjp_layout(const dlx_mft_geom& g, int c, bool amp) {
   VjpLayout L;
-  L.P = align_up((size_t)c * mat_bytes(g.n_in, g.n_in, split));
-  L.Wf = align_up((size_t)c * mat_bytes(g.n_out, g.n_in, split));
-  L.Wa = align_up((size_t)c * mat_bytes(g.n_in, g.n_out, split));
-  const size_t t1 = mat_bytes(g.n_out, g.n_in, split), t2 = mat_bytes(g.n_in, g.n_out, split);
-  L.T = align_up((size_t)c * (t1 > t2 ? t1 : t2));
-  L.Eb = align_up((size_t)c * mat_bytes(g.n_out, g.n_out, split));
+  L.T = align_up((size_t)c * (fold_table_bytes(g.n_in, g.n_out) + fold_table_bytes(g.n_out, g.n_in)));
+  const long u = fold_mid_bytes(g.n_in, g.n_out), v = fold_mid_bytes(g.n_out, g.n_in);
+  L.U = align_up((size_t)c * (u > v ? u : v));
+  L.Eb = align_up((size_t)c * fold_field_bytes(g.n_out));
   L.H = align_up((size_t)c * g.n_in * g.n_in * sizeof(float));
-  // the amplitude cotangent: phasors U = P / A (P at unit amplitude) and the
-  // Re(conj(U) Pbar) planes
-  L.U = L.P;
-  L.H2 = L.H;
-  L.total = L.P + L.U + L.Wf + L.Wa + L.T + L.Eb + L.H + L.H2;
+  L.total = L.T + L.U + L.Eb + (amp ? 2 : 1) * L.H;
   return L;
 }
 
@@ -292,9 +397,12 @@ size_t dlx_mft_workspace_size(const dlx_mft_geom* geom, int32_t batch, int32_t p
   if (!geom || batch <= 0) return 0;
   const bool split = precision == DLX_PREC_BF16X3;
   const size_t mat = align_up((size_t)batch * mat_bytes(geom->n_out, geom->n_in, split));
-  size_t total = 3 * mat;  // W_x, W_y, U^T
+  // three complex matrices per instance (and a converted field), which the
+  // folded tables and intermediate fit in on all but the smallest grids
+  size_t total = 3 * mat;
   if (split) total += align_up((size_t)batch * mat_bytes(geom->n_in, geom->n_in, true));
-  return total;
+  const size_t fold = field_transform_bytes(geom->n_in, geom->n_out, batch);
+  return total > fold ? total : fold;
 }
 
 int dlx_mft(const dlx_mft_geom* geom, int32_t batch, const void* in, void* out,
@@ -317,55 +425,40 @@ int dlx_mft(const dlx_mft_geom* geom, int32_t batch, const void* in, void* out,
   }
   const dlx_mft_geom& g = *geom;
   hipStream_t s = (hipStream_t)stream;
-  const bool split = precision == DLX_PREC_BF16X3;
-  const size_t mat = align_up((size_t)batch * mat_bytes(g.n_out, g.n_in, split));
-  uint8_t* Wx_ws = (uint8_t*)workspace;
-  uint8_t* Wy_ws = Wx_ws + mat;
-  uint8_t* Ut = Wx_ws + 2 * mat;
-
-  bool same = true;
-  for (int b = 0; b < batch && same; ++b) {
+  // Per axis W = exp(-2 pi i s a_k b_l) with a_k = (u_k - sh) / N and
+  // b_l = (u_l - sh) b: the product splits into the centred kernel and the
+  // phases step sh u_k on the input and step (sh u_l - sh^2) on the output,
+  // step = b / N; the tables depend on neither shift nor scale.
+  std::vector<double> steps(batch), c(batch);
+  std::vector<FoldPhase> pin(batch), pout(batch);
+  const double sg = g.inverse ? -1.0 : 1.0;
+  bool shifted = false;
+  for (int b = 0; b < batch; ++b) {
+    DLX_CHECK_ARG(std::isfinite(wavelength[b]) && wavelength[b] > 0, "wavelength[%d] must be > 0",
+                  b);
+    DLX_CHECK_ARG(std::isfinite(pixel_scale_in[b]) && pixel_scale_in[b] != 0,
+                  "pixel_scale_in[%d] must be non-zero", b);
+    DLX_CHECK_ARG(std::isfinite(pixel_scale_out[b]), "pixel_scale_out[%d] must be finite", b);
+    const double st = fold_step(g, wavelength[b], pixel_scale_in[b], pixel_scale_out[b]);
     const double sx = shift_x ? shift_x[b] : 0.0, sy = shift_y ? shift_y[b] : 0.0;
-    same = (sx == sy);
-  }
-  // c_b * field_scale_b is applied in the stage-2 epilogue: the matrices are
-  // unscaled and therefore cacheable.
-  std::vector<double> c(batch);
-  for (int b = 0; b < batch; ++b)
+    steps[b] = st;
+    pin[b] = {0.0, sg * st * sx, sg * st * sy, 0.0};
+    pout[b] = {0.0, sg * st * sx, sg * st * sy, -sg * st * (sx * sx + sy * sy)};
+    shifted = shifted || sx != 0.0 || sy != 0.0;
     c[b] = mft_norm(g, wavelength[b], pixel_scale_in[b], pixel_scale_out[b]) *
            (field_scale ? field_scale[b] : 1.0);
-
-  void *Wx = nullptr, *Wy = nullptr;
-  CacheLease hx(s), hy(s);
-  if (int st = get_matrices(g, batch, wavelength, pixel_scale_in, pixel_scale_out, shift_x,
-                            split, Wx_ws, s, &Wx, &hx.h))
-    return st;
-  if (same) {
-    Wy = Wx;
-  } else if (int st = get_matrices(g, batch, wavelength, pixel_scale_in, pixel_scale_out,
-                                   shift_y, split, Wy_ws, s, &Wy, &hy.h)) {
-    return st;
   }
-  int st;
-  if (split) {
-    uint8_t* X = Wx_ws + 3 * mat;
-    DLX_HIP(launch_to_split4((const float2*)in, batch, g.n_in, g.n_in, (long)g.n_in * g.n_in,
-                             X, (long)mat_bytes(g.n_in, g.n_in, true), s));
-    st = mft_split4(g, batch, X, (const uint8_t*)Wx, (const uint8_t*)Wy, Ut, c.data(), out,
-                    EPI_STORE, s, nullptr, nullptr);
-  } else {
-    st = mft_fp32(g, batch, (const float2*)in, (const float2*)Wx, (const float2*)Wy,
-                  (float2*)Ut, c.data(), out, EPI_STORE, s, false);
-  }
-  if (st) return st;
-  if (int r = hx.release()) return r;
-  return hy.release();
+  return field_transform(g.n_in, g.n_out, batch, g.inverse != 0, steps,
+                         shifted ? pin.data() : nullptr, shifted ? pout.data() : nullptr, c.data(),
+                         in, out, precision == DLX_PREC_BF16X3, (uint8_t*)workspace, s);
 }
 
 size_t dlx_lct_workspace_size(int32_t n_in, int32_t n_out, int32_t batch, int32_t precision) {
   if (n_in <= 0 || n_out <= 0 || batch <= 0) return 0;
   const bool split = precision == DLX_PREC_BF16X3;
-  size_t total = 2 * align_up((size_t)batch * mat_bytes(n_out, n_in, split));  // K, U^T
+  size_t total = 2 * align_up((size_t)batch * mat_bytes(n_out, n_in, split));
+  const size_t fold = field_transform_bytes(n_in, n_out, batch);
+  if (fold > total) total = fold;
   if (split) total += align_up((size_t)batch * mat_bytes(n_in, n_in, true));
   return total;
 }
@@ -398,64 +491,25 @@ int dlx_lct(int32_t n_in, int32_t n_out, int32_t batch, const double* abcd,
     return DLX_ERR_WORKSPACE;
   }
   hipStream_t s = (hipStream_t)stream;
-  const bool split = precision == DLX_PREC_BF16X3;
-  const size_t mat = align_up((size_t)batch * mat_bytes(n_out, n_in, split));
-  uint8_t* K_ws = (uint8_t*)workspace;
-  uint8_t* Ut = K_ws + mat;
-  const long kst = (long)n_out * n_in;
-  const long kbytes = (long)mat_bytes(n_out, n_in, split);
-  const double x0i = center_in - (n_in - 1) / 2.0 * pixel_scale_in;
-  const double x0o = center_out - (n_out - 1) / 2.0 * pixel_scale_out;
-  std::vector<double> alpha(batch);
-  for (int b = 0; b < batch; ++b)
-    alpha[b] = pixel_scale_in * pixel_scale_out / (wavelength[b] * std::fabs(B));
-  // the kernels depend only on the grids, the ABCD matrix and lambda: keep them
-  // resident in the device cache across calls (generated on a miss)
-  std::vector<double> key = {1001.0, (double)n_in, (double)n_out, (double)batch,
-                             split ? 1.0 : 0.0, A, B, D, pixel_scale_in, center_in,
-                             pixel_scale_out, center_out};
-  key.insert(key.end(), wavelength, wavelength + batch);
-  void* cached = nullptr;
-  CacheLease lease(s);
-  bool fresh = true;
-  if (int st = cache_acquire_raw(key, (size_t)batch * kbytes, s, &cached, &lease.h, &fresh))
-    return st;
-  uint8_t* Kp = cached ? (uint8_t*)cached : K_ws;
-  if (fresh) {
-    for (int b0 = 0; b0 < batch; b0 += LctMatChunk::kMax) {
-      const int nb = batch - b0 < LctMatChunk::kMax ? batch - b0 : LctMatChunk::kMax;
-      LctMatChunk c;
-      for (int i = 0; i < nb; ++i) {
-        const double lb = wavelength[b0 + i] * B;
-        c.ci2[i] = A / (2.0 * lb);
-        c.co2[i] = D / (2.0 * lb);
-        c.cx[i] = -1.0 / lb;
-        c.c0[i] = B > 0 ? -0.125 : 0.125;   // the phase of 1 / sqrt(i B), per axis
-      }
-      if (split)
-        DLX_HIP(launch_lct_matrix_split4(c, nb, n_in, n_out, x0i, pixel_scale_in, x0o,
-                                         pixel_scale_out, Kp + (long)b0 * kbytes, kbytes, s));
-      else
-        DLX_HIP(launch_lct_matrix(c, nb, n_in, n_out, x0i, pixel_scale_in, x0o,
-                                  pixel_scale_out, (float2*)Kp + (long)b0 * kst, kst, s));
-    }
-    if (int st = cache_ready(lease.h, s)) return st;
+  // Per axis the Collins kernel exp(2 pi i (A x^2 - 2 x x' + D x'^2) / (2 lambda B)
+  // -+ i pi / 4), x = xc + u dx, x' = xc' + v dx', is the centred kernel of
+  // step dx dx' / (lambda |B|) between the chirps of u and of v.
+  const double xc = center_in, xo = center_out, dx = pixel_scale_in, dxo = pixel_scale_out;
+  std::vector<double> steps(batch), alpha(batch);
+  std::vector<FoldPhase> pin(batch), pout(batch);
+  for (int b = 0; b < batch; ++b) {
+    const double lb = wavelength[b] * B;
+    steps[b] = dx * dxo / std::fabs(lb);
+    alpha[b] = dx * dxo / (wavelength[b] * std::fabs(B));
+    const double li = (A * xc - xo) / lb * dx, lo = (D * xo - xc) / lb * dxo;
+    pin[b] = {A * dx * dx / (2.0 * lb), li, li, 0.0};
+    // the constants of both axes: chirps at the centres, the cross term, 1 / (i B)
+    pout[b] = {D * dxo * dxo / (2.0 * lb), lo, lo,
+               2.0 * ((A * xc * xc - 2.0 * xc * xo + D * xo * xo) / (2.0 * lb)) +
+                   (B > 0 ? -0.25 : 0.25)};
   }
-  dlx_mft_geom g{};
-  g.n_in = n_in;
-  g.n_out = n_out;
-  int st;
-  if (split) {
-    uint8_t* X = K_ws + 2 * mat;
-    DLX_HIP(launch_to_split4((const float2*)in, batch, n_in, n_in, (long)n_in * n_in, X,
-                             (long)mat_bytes(n_in, n_in, true), s));
-    st = mft_split4(g, batch, X, Kp, Kp, Ut, alpha.data(), out, EPI_STORE, s, nullptr, nullptr);
-  } else {
-    st = mft_fp32(g, batch, (const float2*)in, (const float2*)Kp, (const float2*)Kp,
-                  (float2*)Ut, alpha.data(), out, EPI_STORE, s, false);
-  }
-  if (int r = lease.release()) return r;
-  return st;
+  return field_transform(n_in, n_out, batch, B < 0, steps, pin.data(), pout.data(), alpha.data(),
+                         in, out, precision == DLX_PREC_BF16X3, (uint8_t*)workspace, s);
 }
 
 size_t dlx_lct_fft_workspace_size(int32_t n, int32_t m, int32_t batch) {
@@ -599,65 +653,6 @@ int dlx_intensity(int64_t npix, int32_t batch, const void* field, int32_t sum_ov
 namespace dlx {
 namespace {
 
-// The psf chain's buffers for a chunk of c wavelengths: the tables (used when
-// they are not taken from the cache), the stage-1 result, the per-wavelength
-// |E|^2 planes and, when `bytes` leaves room for it, the folded pupil.
-struct PsfLayout {
-  size_t T, U, I, P, total;   // total without P
-};
-PsfLayout psf_layout(const dlx_mft_geom& g, int c) {
-  PsfLayout L;
-  L.T = align_up((size_t)c * fold_table_bytes(g.n_in, g.n_out));
-  L.U = align_up((size_t)c * fold_mid_bytes(g.n_in, g.n_out));
-  L.I = align_up((size_t)c * g.n_out * g.n_out * sizeof(float));
-  L.P = align_up((size_t)c * fold_field_bytes(g.n_in));
-  L.total = L.T + L.U + L.I;
-  return L;
-}
-
-// Workspace of the psf chain: a complex pupil, two complex matrices and the
-// planes per wavelength -- which the folded buffers fit in on all but the
-// smallest grids -- so that the limits a caller meets do not depend on how the
-// chain lays its buffers out.
-size_t psf_poly_bytes(const dlx_mft_geom& g, int c, bool split) {
-  const size_t P = align_up((size_t)c * mat_bytes(g.n_in, g.n_in, split));
-  const size_t W = align_up((size_t)c * mat_bytes(g.n_out, g.n_in, split));
-  const size_t I = align_up((size_t)c * g.n_out * g.n_out * sizeof(float));
-  const size_t plain = P + 2 * W + I, fold = psf_layout(g, c).total;
-  return plain > fold ? plain : fold;
-}
-
-// The cosine / sine tables of nb wavelengths (and, with `adjoint`, of the
-// transposed contraction), from the device cache -- an entry holds both -- or
-// generated into `ws` when the cache is bypassed.
-struct FoldTables {
-  const uint8_t *fwd, *adj;
-  long stride;
-};
-int fold_tables(const dlx_mft_geom& g, int nb, const double* wl, double dx, double p_out, bool split,
-                bool adjoint, bool use_cache, uint8_t* ws, hipStream_t s, FoldTables* out,
-                CacheLease* lease) {
-  const long tf = fold_table_bytes(g.n_in, g.n_out), ta = fold_table_bytes(g.n_out, g.n_in);
-  std::vector<double> key = {2001.0, (double)g.n_in, (double)g.n_out, split ? 1.0 : 0.0};
-  for (int i = 0; i < nb; ++i) key.push_back(fold_step(g, wl[i], dx, p_out));
-  const double* step = key.data() + 4;
-  void* mem = nullptr;
-  bool fresh = true;
-  if (use_cache)
-    if (int st = cache_acquire_raw(key, (size_t)nb * (tf + ta), s, &mem, &lease->h, &fresh, true))
-      return st;
-  uint8_t* base = mem ? (uint8_t*)mem : ws;
-  out->stride = mem || adjoint ? tf + ta : tf;
-  out->fwd = base;
-  out->adj = base + tf;
-  if (fresh) {
-    DLX_HIP(launch_fold_tables(step, nb, g.n_in, g.n_out, split, mem || adjoint, base, out->stride,
-                               s));
-    if (int st = cache_ready(lease->h, s)) return st;
-  }
-  return DLX_OK;
-}
-
 int check_psf_poly_args(const dlx_mft_geom* geom, int32_t nwl, const double* wavelength,
                         const double* weight, double pixel_scale_in, double pixel_scale_out,
                         double center, double tilt_x, double tilt_y, double scale, float* psf,
@@ -715,8 +710,9 @@ int psf_poly_run(const dlx_mft_geom& g, int32_t nwl, const double* wavelength,
     float* Ic = planes ? planes + (long)l0 * nout2 : nwl == 1 ? psf : I;
     CacheLease h(s);
     FoldTables tab;
-    if (int st = fold_tables(g, nb, wavelength + l0, pixel_scale_in, pixel_scale_out, split, false,
-                             use_cache, T_ws, s, &tab, &h))
+    if (int st = fold_tables(g.n_in, g.n_out,
+                             psf_steps(g, nb, wavelength + l0, pixel_scale_in, pixel_scale_out),
+                             split, false, use_cache, T_ws, s, &tab, &h))
       return st;
     f1.batch = nb;
     f1.table = tab.fwd;
@@ -840,7 +836,11 @@ size_t dlx_psf_poly_vjp_workspace_size(const dlx_mft_geom* geom, int32_t nwl,
                                        int32_t precision) {
   if (!geom || nwl <= 0) return 0;
   const int c = nwl < kWlChunk ? nwl : kWlChunk;
-  return vjp_layout(*geom, c, precision == DLX_PREC_BF16X3).total;
+  // more than the PSF's own workspace: one buffer serves a step's forward and
+  // backward calls
+  const size_t psf = psf_poly_bytes(*geom, c, precision == DLX_PREC_BF16X3);
+  const VjpLayout L = vjp_layout(*geom, c, true);
+  return (L.total > psf ? L.total : psf) + 256;
 }
 
 int dlx_psf_poly_vjp(const dlx_mft_geom* geom, int32_t nwl, const double* wavelength,
@@ -876,132 +876,61 @@ int dlx_psf_poly_vjp(const dlx_mft_geom* geom, int32_t nwl, const double* wavele
   hipStream_t s = (hipStream_t)stream;
   const bool split = precision == DLX_PREC_BF16X3;
   const int c = nwl < kWlChunk ? nwl : kWlChunk;
-  const VjpLayout L = vjp_layout(g, c, split);
-  uint8_t* P = (uint8_t*)workspace;
-  uint8_t* Wf_ws = P + L.P;
-  uint8_t* Wa_ws = Wf_ws + L.Wf;
-  uint8_t* T = Wa_ws + L.Wa;
-  uint8_t* Eb = T + L.T;
+  const VjpLayout L = vjp_layout(g, c, true);
+  uint8_t* T_ws = (uint8_t*)workspace;
+  uint8_t* U = T_ws + L.T;
+  uint8_t* Eb = U + L.U;
   float* H = (float*)(Eb + L.Eb);
   float* H2 = grad_amp ? (float*)((uint8_t*)H + L.H) : nullptr;
-  uint8_t* U = (uint8_t*)H + L.H + L.H2;
-  const long nin = g.n_in, nout = g.n_out;
-  const double x0 = center - (g.n_in - 1) / 2.0 * pixel_scale_in;
-
-  std::vector<double> dx(c, pixel_scale_in), pout(c, pixel_scale_out);
+  const long nin = g.n_in;
+  const FoldPupil pup = {opd, amp, phase, pixel_scale_in,
+                         center - (g.n_in - 1) / 2.0 * pixel_scale_in, tilt_x, tilt_y, (float)scale};
   for (int l0 = 0; l0 < nwl; l0 += c) {
     const int nb = nwl - l0 < c ? nwl - l0 : c;
-    float alpha[kWlChunk];
     GradChunk gc;
+    CacheLease h(s);
+    FoldTables tab;
+    if (int st = fold_tables(g.n_in, g.n_out,
+                             psf_steps(g, nb, wavelength + l0, pixel_scale_in, pixel_scale_out),
+                             split, true, true, T_ws, s, &tab, &h))
+      return st;
+    FoldStage2 e{}, b{};
     for (int i = 0; i < nb; ++i) {
-      alpha[i] = (float)(mft_norm(g, wavelength[l0 + i], pixel_scale_in, pixel_scale_out) *
-                         std::sqrt(weight[l0 + i]));
+      e.alpha[i] = b.alpha[i] =
+          (float)(mft_norm(g, wavelength[l0 + i], pixel_scale_in, pixel_scale_out) *
+                  std::sqrt(weight[l0 + i]));
       gc.kw[i] = (float)(2.0 * M_PI / wavelength[l0 + i]);
+      b.inv_wl[i] = 1.0 / wavelength[l0 + i];
     }
-    void *Wf = nullptr, *Wa = nullptr;
-    CacheLease hf(s), ha(s);
-    if (int st = get_matrices(g, nb, wavelength + l0, dx.data(), pout.data(), nullptr, split,
-                              Wf_ws, s, &Wf, &hf.h))
-      return st;
-    if (int st = get_matrices(g, nb, wavelength + l0, dx.data(), pout.data(), nullptr, split,
-                              Wa_ws, s, &Wa, &ha.h, true))
-      return st;
-    if (split) {
-      const long rb_in = split4_row_bytes(g.n_in), rb_out = split4_row_bytes(g.n_out);
-      const long pb = (long)mat_bytes(nin, nin, true), wfb = (long)mat_bytes(nout, nin, true);
-      const long wab = (long)mat_bytes(nin, nout, true), eb = (long)mat_bytes(nout, nout, true);
-      PupilChunk pc;
-      for (int i = 0; i < nb; ++i) pc.inv_wl[i] = 1.0 / wavelength[l0 + i];
-      DLX_HIP(launch_pupil_split4(pc, nb, g.n_in, pixel_scale_in, x0, tilt_x, tilt_y, amp, opd,
-                                  phase, (float)scale, P, pb, s));
-      if (grad_amp)
-        DLX_HIP(launch_pupil_split4(pc, nb, g.n_in, pixel_scale_in, x0, tilt_x, tilt_y, nullptr,
-                                    opd, phase, (float)scale, U, pb, s));
-      // forward stage 1: U^T = (P W^T)^T, split4 rows n_out
-      GemmSplit g1{};
-      g1.A = P; g1.a_row_bytes = rb_in; g1.a_batch_bytes = pb;
-      g1.B = (const uint8_t*)Wf; g1.b_row_bytes = rb_in; g1.b_batch_bytes = wfb;
-      g1.C = T; g1.ldc = rb_in; g1.c_batch = wfb;
-      g1.M = g.n_in; g1.N = g.n_out; g1.K = g.n_in; g1.batch = nb; g1.epilogue = EPI_SPLIT_T;
-      for (int i = 0; i < nb; ++i) g1.alpha[i] = 1.0f;
-      DLX_HIP(launch_cgemm_split4(g1, s));
-      // forward stage 2 in transposed order, E^T = U^T W^T, so that the split4
-      // epilogue writes rows of Ebar = 2 G E (rows n_out, k = n_out)
-      GemmSplit g2{};
-      g2.A = T; g2.a_row_bytes = rb_in; g2.a_batch_bytes = wfb;
-      g2.B = (const uint8_t*)Wf; g2.b_row_bytes = rb_in; g2.b_batch_bytes = wfb;
-      g2.C = Eb; g2.ldc = rb_out; g2.c_batch = eb;
-      g2.M = g.n_out; g2.N = g.n_out; g2.K = g.n_in; g2.batch = nb;
-      g2.epilogue = EPI_VJP_SPLIT_T;
-      for (int i = 0; i < nb; ++i) g2.alpha[i] = alpha[i];
-      g2.G = dpsf; g2.ldg = g.n_out; g2.g_batch = 0;
-      DLX_HIP(launch_cgemm_split4(g2, s));
-      // adjoint stage 1: V = Ebar conj(W), stored V^T (rows n_in, k = n_out)
-      GemmSplit g3{};
-      g3.A = Eb; g3.a_row_bytes = rb_out; g3.a_batch_bytes = eb;
-      g3.B = (const uint8_t*)Wa; g3.b_row_bytes = rb_out; g3.b_batch_bytes = wab;
-      g3.C = T; g3.ldc = rb_out; g3.c_batch = wab;
-      g3.M = g.n_out; g3.N = g.n_in; g3.K = g.n_out; g3.batch = nb; g3.epilogue = EPI_SPLIT_T;
-      for (int i = 0; i < nb; ++i) g3.alpha[i] = 1.0f;
-      DLX_HIP(launch_cgemm_split4(g3, s));
-      // adjoint stage 2: Pbar = alpha W^H V, epilogue Im(conj(P) Pbar)
-      GemmSplit g4{};
-      g4.A = (const uint8_t*)Wa; g4.a_row_bytes = rb_out; g4.a_batch_bytes = wab;
-      g4.B = T; g4.b_row_bytes = rb_out; g4.b_batch_bytes = wab;
-      g4.C = H; g4.ldc = nin; g4.c_batch = nin * nin;
-      g4.M = g.n_in; g4.N = g.n_in; g4.K = g.n_out; g4.batch = nb; g4.epilogue = EPI_GRAD;
-      for (int i = 0; i < nb; ++i) g4.alpha[i] = alpha[i];
-      g4.P = P; g4.p_ld = rb_in; g4.p_batch = pb;
-      g4.C2 = H2; g4.U = U;
-      DLX_HIP(launch_cgemm_split4(g4, s));
-    } else {
-      const long pst = nin * nin, wst = nout * nin, est = nout * nout;
-      if (int st = dlx_pupil_field(g.n_in, nb, wavelength + l0, pixel_scale_in, center, tilt_x,
-                                   tilt_y, amp, opd, phase, scale, nullptr, P, stream))
-        return st;
-      if (grad_amp)
-        if (int st = dlx_pupil_field(g.n_in, nb, wavelength + l0, pixel_scale_in, center,
-                                     tilt_x, tilt_y, nullptr, opd, phase, scale, nullptr, U,
-                                     stream))
-          return st;
-      GemmBatch g1{};
-      g1.A = (const float2*)P; g1.lda = nin; g1.sA = pst;
-      g1.B = (const float2*)Wf; g1.ldb = nin; g1.sB = wst;
-      g1.C = T; g1.ldc = nin; g1.sC = wst;
-      g1.M = g.n_in; g1.N = g.n_out; g1.K = g.n_in; g1.batch = nb;
-      g1.epilogue = EPI_STORE_T; g1.precision = DLX_PREC_FP32;
-      for (int i = 0; i < nb; ++i) g1.alpha[i] = 1.0f;
-      DLX_HIP(launch_cgemm_nt(g1, s));
-      GemmBatch g2{};
-      g2.A = (const float2*)Wf; g2.lda = nin; g2.sA = wst;
-      g2.B = (const float2*)T; g2.ldb = nin; g2.sB = wst;
-      g2.C = Eb; g2.ldc = nout; g2.sC = est;
-      g2.M = g.n_out; g2.N = g.n_out; g2.K = g.n_in; g2.batch = nb;
-      g2.epilogue = EPI_VJP; g2.precision = DLX_PREC_FP32;
-      for (int i = 0; i < nb; ++i) g2.alpha[i] = alpha[i];
-      g2.G = dpsf; g2.ldg = nout; g2.g_batch = 0;
-      DLX_HIP(launch_cgemm_nt(g2, s));
-      GemmBatch g3{};
-      g3.A = (const float2*)Eb; g3.lda = nout; g3.sA = est;
-      g3.B = (const float2*)Wa; g3.ldb = nout; g3.sB = wst;
-      g3.C = T; g3.ldc = nout; g3.sC = wst;
-      g3.M = g.n_out; g3.N = g.n_in; g3.K = g.n_out; g3.batch = nb;
-      g3.epilogue = EPI_STORE_T; g3.precision = DLX_PREC_FP32;
-      for (int i = 0; i < nb; ++i) g3.alpha[i] = 1.0f;
-      DLX_HIP(launch_cgemm_nt(g3, s));
-      GemmBatch g4{};
-      g4.A = (const float2*)Wa; g4.lda = nout; g4.sA = wst;
-      g4.B = (const float2*)T; g4.ldb = nout; g4.sB = wst;
-      g4.C = H; g4.ldc = nin; g4.sC = pst;
-      g4.M = g.n_in; g4.N = g.n_in; g4.K = g.n_out; g4.batch = nb;
-      g4.epilogue = EPI_GRAD; g4.precision = DLX_PREC_FP32;
-      for (int i = 0; i < nb; ++i) g4.alpha[i] = alpha[i];
-      g4.P = P; g4.p_ld = nin; g4.p_batch = pst;
-      g4.C2 = H2; g4.U = U;
-      DLX_HIP(launch_cgemm_nt(g4, s));
-    }
-    if (int st = hf.release()) return st;
-    if (int st = ha.release()) return st;
+    // forward: the pupil through stage 1, then Ebar = 2 G E folded for the way back
+    FoldStage1 f{};
+    f.n = g.n_in; f.m = g.n_out; f.batch = nb;
+    f.table = tab.fwd; f.table_stride = tab.stride;
+    f.out = U; f.out_stride = fold_mid_bytes(g.n_in, g.n_out);
+    f.pupil = pup;
+    for (int i = 0; i < nb; ++i) f.inv_wl[i] = b.inv_wl[i];
+    DLX_HIP(launch_fold_stage1(f, FOLD_PUPIL, split, s));
+    e.n = g.n_in; e.m = g.n_out; e.batch = nb; e.inverse = g.inverse;
+    e.table = tab.fwd; e.table_stride = tab.stride;
+    e.mid = U; e.mid_stride = f.out_stride;
+    e.out = Eb; e.out_stride = fold_field_bytes(g.n_out);
+    e.G = dpsf;
+    DLX_HIP(launch_fold_stage2(e, FOLD_VJP, split, s));
+    // adjoint: the same transform with the sides exchanged and the sign
+    // flipped; its epilogue multiplies by the pupil's phasor
+    FoldStage1 v{};
+    v.n = g.n_out; v.m = g.n_in; v.batch = nb;
+    v.src = Eb; v.src_stride = e.out_stride;
+    v.table = tab.adj; v.table_stride = tab.stride;
+    v.out = U; v.out_stride = fold_mid_bytes(g.n_out, g.n_in);
+    DLX_HIP(launch_fold_stage1(v, FOLD_MEM, split, s));
+    b.n = g.n_out; b.m = g.n_in; b.batch = nb; b.inverse = !g.inverse;
+    b.table = tab.adj; b.table_stride = tab.stride;
+    b.mid = U; b.mid_stride = v.out_stride;
+    b.out = H; b.out_stride = nin * nin; b.out2 = H2;
+    b.pupil = pup;
+    DLX_HIP(launch_fold_stage2(b, FOLD_GRAD, split, s));
+    if (int st = h.release()) return st;
     if (grad_opd || grad_phase)
       DLX_HIP(launch_grad_reduce(gc, nb, nin * nin, H, l0 > 0, grad_opd, grad_phase, s));
     if (grad_amp)   // sum over wavelengths of Re(conj(U) Pbar) = dL/dA

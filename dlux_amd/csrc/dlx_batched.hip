@@ -2,15 +2,16 @@
 // pupil and output sizes, computed by grouped persistent launches (gfx950).
 //
 // One call of dlx_mft_batched_psf runs, whatever the mix of shapes:
-//   1. one launch that converts every distinct complex64 input field to split4;
-//   2. one launch that generates every instance's transfer matrices W_x, W_y
-//      (split4, FP64 phase arguments);
-//   3. one grouped GEMM launch for all stage-1 products U_i^T = (P_i W_x,i^T)^T;
-//   4. one grouped GEMM launch for all stage-2 products with the |E|^2
-//      epilogue, I_i = |alpha_i W_y,i U_i|^2 (alpha_i = c_i sqrt(weight_i));
-//   5. one launch that sums the planes of each output image, in a fixed order.
-// Per-job descriptors live in the caller's workspace; the host fills them in
-// a pinned staging slot and copies them with the launches (stream-ordered).
+//   1. one launch that generates the distinct cosine / sine tables (instances
+//      of equal sides and phase step share one);
+//   2. one grouped launch per tile width (output sides to 64, to 128, above)
+//      of the folded stage 1, which loads the complex64 fields directly and
+//      applies each instance's shift as a phase (dlx_fold.h);
+//   3. one grouped launch of stage 2 with the |E|^2 epilogue,
+//      I_i = |alpha_i W_y,i U_i|^2 (alpha_i = c_i sqrt(weight_i));
+//   4. one launch that sums the planes of each output image, in a fixed order.
+// Per-instance descriptors live in the caller's workspace; the host fills them
+// in a pinned staging slot and copies them with the launches (stream-ordered).
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -18,31 +19,14 @@
 #include <map>
 #include <mutex>
 #include <numeric>
+#include <unordered_map>
 #include <vector>
 
+#include "dlx_fold.h"
 #include "dlx_internal.h"
-#include "dlx_split.h"
 
 namespace dlx {
 namespace {
-
-// ---------------------------------------------------------------------------
-// device job descriptors
-// ---------------------------------------------------------------------------
-struct CvtJob {              // complex64 rows x k -> split4
-  const float2* in;
-  uint8_t* out;
-  long row_start;            // first row of this job in the launch's row list
-  int rows, k;
-};
-
-struct MatJob {              // split4 rows x cols of exp(sign 2 pi i u_r v_c)
-  uint8_t* out;
-  long row_start;
-  int rows, cols, sign_inv, pad_;
-  double c_scale, c_off;     // column coordinate v_c = c * c_scale + c_off
-  double r_scale, r_off;     // row coordinate    u_r = r * r_scale + r_off
-};
 
 struct SumJob {              // out[p] = sum_{q < count} planes[q * npix + p]
   float* out;
@@ -51,73 +35,23 @@ struct SumJob {              // out[p] = sum_{q < count} planes[q * npix + p]
   int count, pad_;
 };
 
-// Workgroup-per-row kernels: a workgroup takes whole rows (grid-stride over the
-// launch's row list), finds the row's job once with a workgroup-uniform binary
-// search on scalar loads, and its lanes cover the row's chunks, a quad of
-// lanes per chunk with quad-cooperative 16-byte stores.  Chunk counts times 4
-// and the workgroup size are multiples of 4, so whole quads take each chunk.
-template <typename Job>
-__device__ __forceinline__ int find_row_job(const Job* jobs, int njobs, long row) {
-  int lo = 0, hi = njobs - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (jobs[mid].row_start <= row) lo = mid; else hi = mid - 1;
-  }
-  return lo;
-}
-
-__global__ void __launch_bounds__(256)
-group_to_split4_kernel(const CvtJob* __restrict__ jobs, int njobs, long total_rows) {
-  for (long row = blockIdx.x; row < total_rows; row += gridDim.x) {
-    const CvtJob& j = jobs[find_row_job(jobs, njobs, row)];
-    const long r = row - j.row_start;
-    const int kc = (int)split4_chunks(j.k);
-    const float2* src = j.in + r * j.k;
-    for (int item = threadIdx.x; item < 4 * kc; item += blockDim.x) {
-      const int q = item & 3, ch = item >> 2;
-      const int x = ch * 8 + 2 * q;
-      const float2 v0 = x < j.k ? src[x] : make_float2(0.f, 0.f);
-      const float2 v1 = x + 1 < j.k ? src[x + 1] : make_float2(0.f, 0.f);
-      store_chunk_quad(j.out, r, split4_row_bytes(j.k), ch, q, v0, v1);
-    }
-  }
-}
-
-__global__ void __launch_bounds__(256)
-group_dft_split4_kernel(const MatJob* __restrict__ jobs, int njobs, long total_rows) {
-  for (long row = blockIdx.x; row < total_rows; row += gridDim.x) {
-    const MatJob& j = jobs[find_row_job(jobs, njobs, row)];
-    const long r = row - j.row_start;
-    const int kc = (int)split4_chunks(j.cols);
-    const double u = (double)r * j.r_scale + j.r_off;
-    for (int item = threadIdx.x; item < 4 * kc; item += blockDim.x) {
-      const int q = item & 3, ch = item >> 2;
-      float2 v[2];
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const int c = ch * 8 + 2 * q + e;
-        if (c < j.cols) {
-          double t = u * ((double)c * j.c_scale + j.c_off);
-          t -= rint(t);
-          // hardware sin/cos take turns; max abs error 1.3e-7 on [-1/2, 1/2]
-          const float sn = __builtin_amdgcn_sinf((float)t), cs = __builtin_amdgcn_cosf((float)t);
-          v[e] = make_float2(cs, j.sign_inv ? sn : -sn);
-        } else {
-          v[e] = make_float2(0.f, 0.f);
-        }
-      }
-      store_chunk_quad(j.out, r, split4_row_bytes(j.cols), ch, q, v[0], v[1]);
-    }
-  }
-}
-
+// One pixel per lane (a wave reads 256 contiguous bytes of a plane), 16 planes
+// in flight per lane before the in-order additions.
 __global__ void __launch_bounds__(256)
 group_sum_kernel(const SumJob* __restrict__ jobs) {
   const SumJob& j = jobs[blockIdx.y];
   for (long p = (long)blockIdx.x * blockDim.x + threadIdx.x; p < j.npix;
        p += (long)gridDim.x * blockDim.x) {
     float acc = 0.f;
-    for (int q = 0; q < j.count; ++q) acc += j.planes[(long)q * j.npix + p];
+    int q = 0;
+    for (; q + 16 <= j.count; q += 16) {
+      float v[16];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) v[e] = j.planes[(long)(q + e) * j.npix + p];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc += v[e];
+    }
+    for (; q < j.count; ++q) acc += j.planes[(long)q * j.npix + p];
     j.out[p] = acc;
   }
 }
@@ -173,19 +107,21 @@ int upload(const void* src, size_t bytes, void* dst, hipStream_t s) {
 // ---------------------------------------------------------------------------
 // planning
 // ---------------------------------------------------------------------------
+constexpr int kLists = 6;       // stage-1 lists: tile width (32, 64, 128) x (scalar, 16-byte loads)
+
 struct Plan {
-  // workspace offsets (bytes)
-  size_t off_cvt, off_mat, off_g1, off_g2, off_sum, off_P, off_W, off_U, off_I, total;
-  std::vector<CvtJob> cvt;
-  std::vector<MatJob> mat;
-  std::vector<GroupProblem> g1, g2, g1n, g2n;   // n: problems with N <= 64 (128 x 64 tiles)
+  // workspace offsets (bytes); descriptors first
+  size_t off_tab, off_prob, off_map1[kLists], off_map2, off_sum, desc, off_T, off_U, off_I, total;
+  size_t tab_bytes = 0;
+  std::vector<FoldTableJob> tab;
+  std::vector<size_t> tab_off;       // of each distinct table, from off_T
+  std::vector<int> tab_of;           // instance -> table
+  long tab_most = 0;                 // threads of the largest table
+  std::vector<FoldProblem> prob;     // in launch order
+  std::vector<uint32_t> map1[kLists], map2;
+  int xcd1[kLists][9], xcd2[9];
   std::vector<SumJob> sum;
-  int g1_xcd[9], g2_xcd[9], g1n_xcd[9], g2n_xcd[9];
-  long cvt_work = 0, mat_work = 0;   // rows of the conversion / matrix launches
-  std::vector<int> field_of;       // instance -> distinct-field index
-  std::vector<const void*> fields;
-  std::vector<int> field_n;
-  std::vector<size_t> P_off, Wx_off, Wy_off, U_off, I_off;
+  std::vector<size_t> U_off, I_off;  // per instance
 };
 
 int validate(int n, const dlx_mft_instance* inst, int n_outputs) {
@@ -235,185 +171,198 @@ dlx_mft_geom geom_of(const dlx_mft_instance& d) {
   return g;
 }
 
-// Deal problems (largest first) round-robin to the 8 XCD ranges, then lay the
-// ranges out contiguously and number their tiles.
-void order_problems(std::vector<GroupProblem>& probs, int (&xcd)[9]) {
-  std::vector<size_t> idx(probs.size());
-  std::iota(idx.begin(), idx.end(), 0);
-  auto cost = [&](const GroupProblem& p) {
-    return (double)p.tiles_m * p.tiles_n * (double)split4_chunks(p.K);
+struct TableKey {
+  int n, m;
+  double step;
+  bool operator==(const TableKey& o) const {
+    return n == o.n && m == o.m && std::memcmp(&step, &o.step, sizeof(double)) == 0;
+  }
+};
+struct TableHash {
+  size_t operator()(const TableKey& k) const {
+    uint64_t b;
+    std::memcpy(&b, &k.step, sizeof(b));
+    b ^= ((uint64_t)(uint32_t)k.n << 32 | (uint32_t)k.m) * 0x9E3779B97F4A7C15ull;
+    b *= 0xBF58476D1CE4E5B9ull;
+    return (size_t)(b ^ (b >> 31));
+  }
+};
+
+int tiles1(int n, int m) {
+  const int w = fold_group_width(m);
+  return ((fold_half(n) + kFoldTilePy - 1) / kFoldTilePy) * ((fold_half(m) + w - 1) / w);
+}
+int tiles2(int m) {
+  const int mh = fold_half(m);
+  return ((mh + kFoldTileQy - 1) / kFoldTileQy) * ((mh + kFoldTileQx - 1) / kFoldTileQx);
+}
+
+// Sizes and offsets of the batch's buffers.
+int plan_sizes(int n, const dlx_mft_instance* inst, int n_outputs, Plan& P) {
+  std::unordered_map<const void*, int> field_n;
+  size_t plain = 0;      // the unfolded layout's buffers: never asked for less
+  const void* last = nullptr;
+  for (int i = 0; i < n; ++i) {
+    const dlx_mft_instance& d = inst[i];
+    if (d.field != last || i == 0) {
+      auto it = field_n.emplace(d.field, d.n_in);
+      if (it.second) plain += align_up(mat_bytes(d.n_in, d.n_in, true));
+      last = d.field;
+    }
+    if (field_n[d.field] != d.n_in) {
+      set_error("instance %d: the same field pointer is used with n_in %d and %d", i,
+                field_n[d.field], d.n_in);
+      return DLX_ERR_INVALID;
+    }
+  }
+  // distinct tables
+  std::unordered_map<TableKey, int, TableHash> tables;
+  P.tab_of.resize(n);
+  for (int i = 0; i < n; ++i) {
+    const dlx_mft_instance& d = inst[i];
+    const TableKey k = {d.n_in, d.n_out,
+                        fold_step(geom_of(d), d.wavelength, d.pixel_scale_in, d.pixel_scale_out)};
+    auto it = tables.emplace(k, (int)P.tab.size());
+    if (it.second) {
+      P.tab.push_back({nullptr, k.step, k.n, k.m});
+      P.tab_off.push_back(P.tab_bytes);
+      P.tab_bytes += fold_table_bytes(k.n, k.m);
+      const long work = (long)fold_pad(fold_half(k.m)) * fold_pad(fold_half(k.n)) / 4;
+      P.tab_most = std::max(P.tab_most, work);
+    }
+    P.tab_of[i] = it.first->second;
+  }
+  size_t off = 0;
+  auto take = [&](size_t bytes) { const size_t o = off; off += align_up(bytes); return o; };
+  P.off_tab = take(P.tab.size() * sizeof(FoldTableJob));
+  P.off_prob = take((size_t)n * sizeof(FoldProblem));
+  size_t n1[kLists] = {}, n2 = 0;
+  auto list_of = [&](int i) {
+    const int w = fold_group_width(inst[i].n_out);
+    const bool vec = inst[i].n_in % 8 == 0 && ((uintptr_t)inst[i].field & 15) == 0;
+    return (w == 128 ? 2 : w == 64 ? 1 : 0) * 2 + (vec ? 1 : 0);
   };
-  std::stable_sort(idx.begin(), idx.end(),
-                   [&](size_t a, size_t b) { return cost(probs[a]) > cost(probs[b]); });
-  std::vector<std::vector<GroupProblem>> lists(8);
-  std::vector<double> load(8, 0.0);
-  for (size_t q : idx) {
-    // greedy: the XCD with the least work so far
+  for (int i = 0; i < n; ++i) {
+    n1[list_of(i)] += tiles1(inst[i].n_in, inst[i].n_out);
+    n2 += tiles2(inst[i].n_out);
+  }
+  for (int l = 0; l < kLists; ++l) P.off_map1[l] = take(n1[l] * sizeof(uint32_t));
+  P.off_map2 = take(n2 * sizeof(uint32_t));
+  P.off_sum = take((size_t)n_outputs * sizeof(SumJob));
+  P.desc = off;
+  P.off_T = take(P.tab_bytes);
+  P.off_U = off;
+  P.U_off.resize(n);
+  for (int i = 0; i < n; ++i) {
+    P.U_off[i] = take(fold_mid_bytes(inst[i].n_in, inst[i].n_out));
+    plain += align_up(mat_bytes(inst[i].n_out, inst[i].n_in, true)) *
+             (inst[i].shift_x == inst[i].shift_y ? 2 : 3);
+  }
+  // planes grouped by output, in instance order within an output
+  std::vector<int> count(n_outputs, 0), seen(n_outputs, 0);
+  std::vector<size_t> base(n_outputs, 0);
+  for (int i = 0; i < n; ++i) ++count[inst[i].out_index];
+  P.off_I = off;
+  P.I_off.resize(n);
+  for (int i = 0; i < n; ++i) {
+    const int o = inst[i].out_index;
+    const size_t plane = (size_t)inst[i].n_out * inst[i].n_out * sizeof(float);
+    if (seen[o] == 0) {
+      base[o] = take(count[o] * plane);
+      plain += align_up(count[o] * plane);
+    }
+    P.I_off[i] = base[o] + (size_t)seen[o]++ * plane;
+  }
+  P.total = std::max(off, P.desc + plain);
+  return DLX_OK;
+}
+
+// The descriptors.  Instances that share a field go to one XCD (its L2 then
+// holds the field while their stage-1 tiles read it), fields dealt largest
+// first to the XCD with the least work; with few fields the instances are
+// dealt one by one.  Stage 2 keeps stage 1's XCDs: it reads what they wrote.
+void plan_fill(int n, const dlx_mft_instance* inst, int n_outputs, float* const* outs, uint8_t* ws,
+               Plan& P) {
+  for (size_t q = 0; q < P.tab.size(); ++q) P.tab[q].out = ws + P.off_T + P.tab_off[q];
+  // stage 1's stages and a tile's fixed part, plus stage 2
+  auto cost = [&](int i) {
+    const int st = (fold_half(inst[i].n_in) + 15) / 16;
+    const int w = fold_group_width(inst[i].n_out);
+    return (double)tiles1(inst[i].n_in, inst[i].n_out) * (st + 6) * (w + 64) / 192.0 +
+           (double)tiles2(inst[i].n_out) * (st + 8) * 0.5;
+  };
+  std::unordered_map<const void*, int> unit_of;
+  std::vector<std::vector<int>> units;
+  std::vector<double> ucost;
+  for (int i = 0; i < n; ++i) {
+    auto it = unit_of.emplace(inst[i].field, (int)units.size());
+    if (it.second) { units.emplace_back(); ucost.push_back(0.0); }
+    units[it.first->second].push_back(i);
+    ucost[it.first->second] += cost(i);
+  }
+  if (units.size() < 32) {
+    std::vector<std::vector<int>> one;
+    std::vector<double> c;
+    for (auto& u : units)
+      for (int i : u) { one.push_back({i}); c.push_back(cost(i)); }
+    units.swap(one);
+    ucost.swap(c);
+  }
+  std::vector<int> idx(units.size());
+  std::iota(idx.begin(), idx.end(), 0);
+  std::stable_sort(idx.begin(), idx.end(), [&](int a, int b) { return ucost[a] > ucost[b]; });
+  std::vector<int> on[8];
+  double load[8] = {};
+  for (int u : idx) {
     int best = 0;
     for (int x = 1; x < 8; ++x)
       if (load[x] < load[best]) best = x;
-    lists[best].push_back(probs[q]);
-    load[best] += cost(probs[q]);
+    on[best].insert(on[best].end(), units[u].begin(), units[u].end());
+    load[best] += ucost[u];
   }
-  probs.clear();
-  int t = 0;
+  P.prob.reserve(n);
   for (int x = 0; x < 8; ++x) {
-    xcd[x] = t;
-    for (GroupProblem& p : lists[x]) {
-      p.tile_start = t;
-      t += p.tiles_m * p.tiles_n;
-      probs.push_back(p);
+    for (int l = 0; l < kLists; ++l) P.xcd1[l][x] = (int)P.map1[l].size();
+    P.xcd2[x] = (int)P.map2.size();
+    for (int i : on[x]) {
+      const dlx_mft_instance& d = inst[i];
+      const FoldTableJob& t = P.tab[P.tab_of[i]];
+      const double sg = d.inverse ? -1.0 : 1.0;
+      const double c = mft_norm(geom_of(d), d.wavelength, d.pixel_scale_in, d.pixel_scale_out);
+      FoldProblem p{};
+      p.src = (const uint8_t*)d.field;
+      p.table = t.out;
+      p.mid = ws + P.U_off[i];
+      p.out = (float*)(ws + P.I_off[i]);
+      // the input half of the shift (the output half is a phase: no intensity)
+      p.cx = sg * t.step * d.shift_x;
+      p.cy = sg * t.step * d.shift_y;
+      p.alpha = (float)(c * std::sqrt(d.weight));
+      p.n = d.n_in;
+      p.m = d.n_out;
+      p.inverse = d.inverse ? 1 : 0;
+      const int w = fold_group_width(d.n_out);
+      const bool vec = d.n_in % 8 == 0 && ((uintptr_t)d.field & 15) == 0;
+      std::vector<uint32_t>& m1 = P.map1[(w == 128 ? 2 : w == 64 ? 1 : 0) * 2 + (vec ? 1 : 0)];
+      p.tile1 = (int)m1.size();
+      p.tile2 = (int)P.map2.size();
+      m1.insert(m1.end(), tiles1(p.n, p.m), (uint32_t)P.prob.size());
+      P.map2.insert(P.map2.end(), tiles2(p.m), (uint32_t)P.prob.size());
+      P.prob.push_back(p);
     }
   }
-  xcd[8] = t;
-}
-
-GroupProblem make_problem(const uint8_t* A, long arb, const uint8_t* B, long brb, void* C,
-                          long ldc, int M, int N, int K, float alpha) {
-  GroupProblem p{};
-  p.A = A; p.a_row_bytes = arb;
-  p.B = B; p.b_row_bytes = brb;
-  p.C = C; p.ldc = ldc;
-  p.M = M; p.N = N; p.K = K;
-  const int tile_n = N <= 64 ? 64 : 128;
-  p.tiles_m = (M + 127) / 128;
-  p.tiles_n = (N + tile_n - 1) / tile_n;
-  p.alpha = alpha;
-  return p;
-}
-
-// Problems with N <= 64 go to a launch with 128 x 64 tiles (no half-empty tiles).
-void split_narrow(std::vector<GroupProblem>& all, std::vector<GroupProblem>& narrow) {
-  std::vector<GroupProblem> wide;
-  for (const GroupProblem& p : all) (p.N <= 64 ? narrow : wide).push_back(p);
-  all.swap(wide);
-}
-
-// Sizes and offsets; with ws != nullptr also the device pointers in the jobs.
-int plan_batched(int n, const dlx_mft_instance* inst, int n_outputs, float* const* outs,
-                 uint8_t* ws, Plan& P) {
-  // distinct input fields (instances of one source share its pupil field)
-  P.field_of.assign(n, -1);
+  for (int l = 0; l < kLists; ++l) P.xcd1[l][8] = (int)P.map1[l].size();
+  P.xcd2[8] = (int)P.map2.size();
+  std::vector<int> job(n_outputs, -1);
   for (int i = 0; i < n; ++i) {
-    int f = -1;
-    for (size_t q = 0; q < P.fields.size(); ++q)
-      if (P.fields[q] == inst[i].field) { f = (int)q; break; }
-    if (f < 0) {
-      f = (int)P.fields.size();
-      P.fields.push_back(inst[i].field);
-      P.field_n.push_back(inst[i].n_in);
+    int& j = job[inst[i].out_index];
+    if (j < 0) {
+      j = (int)P.sum.size();
+      P.sum.push_back({outs[inst[i].out_index], (const float*)(ws + P.I_off[i]),
+                       (long)inst[i].n_out * inst[i].n_out, 0, 0});
     }
-    if (P.field_n[f] != inst[i].n_in) {
-      set_error("instance %d: the same field pointer is used with n_in %d and %d", i,
-                P.field_n[f], inst[i].n_in);
-      return DLX_ERR_INVALID;
-    }
-    P.field_of[i] = f;
+    ++P.sum[j].count;
   }
-  // output planes grouped by output, in instance order within an output
-  std::vector<std::vector<int>> members(n_outputs);
-  for (int i = 0; i < n; ++i) members[inst[i].out_index].push_back(i);
-
-  size_t off = 0;
-  auto take = [&](size_t bytes) { const size_t o = off; off += align_up(bytes); return o; };
-  const size_t nf = P.fields.size();
-  P.off_cvt = take(nf * sizeof(CvtJob));
-  P.off_mat = take(2 * (size_t)n * sizeof(MatJob));
-  // each stage's problems: wide list then narrow list (n in total)
-  P.off_g1 = take((size_t)n * sizeof(GroupProblem));
-  P.off_g2 = take((size_t)n * sizeof(GroupProblem));
-  P.off_sum = take((size_t)n_outputs * sizeof(SumJob));
-  P.P_off.resize(nf);
-  P.off_P = off;
-  for (size_t f = 0; f < nf; ++f) P.P_off[f] = take(mat_bytes(P.field_n[f], P.field_n[f], true));
-  P.Wx_off.resize(n);
-  P.Wy_off.resize(n);
-  P.off_W = off;
-  for (int i = 0; i < n; ++i) {
-    P.Wx_off[i] = take(mat_bytes(inst[i].n_out, inst[i].n_in, true));
-    P.Wy_off[i] = inst[i].shift_x == inst[i].shift_y
-                      ? P.Wx_off[i]
-                      : take(mat_bytes(inst[i].n_out, inst[i].n_in, true));
-  }
-  P.U_off.resize(n);
-  P.off_U = off;
-  for (int i = 0; i < n; ++i) P.U_off[i] = take(mat_bytes(inst[i].n_out, inst[i].n_in, true));
-  P.I_off.resize(n);
-  P.off_I = off;
-  for (int o = 0; o < n_outputs; ++o) {
-    if (members[o].empty()) continue;
-    const size_t npix = (size_t)inst[members[o][0]].n_out * inst[members[o][0]].n_out;
-    const size_t base = take(members[o].size() * npix * sizeof(float));
-    for (size_t q = 0; q < members[o].size(); ++q)
-      P.I_off[members[o][q]] = base + q * npix * sizeof(float);
-  }
-  P.total = off;
-  if (!ws) return DLX_OK;
-
-  // conversion jobs
-  long w = 0;
-  for (size_t f = 0; f < nf; ++f) {
-    CvtJob j{};
-    j.in = (const float2*)P.fields[f];
-    j.out = ws + P.P_off[f];
-    j.rows = P.field_n[f];
-    j.k = P.field_n[f];
-    j.row_start = w;
-    w += j.rows;
-    P.cvt.push_back(j);
-  }
-  P.cvt_work = w;
-  // matrix jobs
-  w = 0;
-  for (int i = 0; i < n; ++i) {
-    const dlx_mft_geom g = geom_of(inst[i]);
-    for (int axis = 0; axis < 2; ++axis) {
-      if (axis == 1 && P.Wy_off[i] == P.Wx_off[i]) continue;
-      const double sh = axis == 0 ? inst[i].shift_x : inst[i].shift_y;
-      const MftInst p = make_inst(g, inst[i].wavelength, inst[i].pixel_scale_in,
-                                  inst[i].pixel_scale_out, sh);
-      MatJob j{};
-      j.out = ws + (axis == 0 ? P.Wx_off[i] : P.Wy_off[i]);
-      j.rows = inst[i].n_out;
-      j.cols = inst[i].n_in;
-      j.sign_inv = inst[i].inverse ? 1 : 0;
-      j.c_scale = p.a_scale; j.c_off = p.a_off;
-      j.r_scale = p.b_scale; j.r_off = p.b_off;
-      j.row_start = w;
-      w += j.rows;
-      P.mat.push_back(j);
-    }
-  }
-  P.mat_work = w;
-  // GEMM problems
-  for (int i = 0; i < n; ++i) {
-    const int ni = inst[i].n_in, no = inst[i].n_out;
-    const long rbi = split4_row_bytes(ni);
-    const double c = mft_norm(geom_of(inst[i]), inst[i].wavelength, inst[i].pixel_scale_in,
-                              inst[i].pixel_scale_out);
-    P.g1.push_back(make_problem(ws + P.P_off[P.field_of[i]], rbi, ws + P.Wx_off[i], rbi,
-                                ws + P.U_off[i], rbi, ni, no, ni, 1.0f));
-    P.g2.push_back(make_problem(ws + P.Wy_off[i], rbi, ws + P.U_off[i], rbi,
-                                ws + P.I_off[i], no, no, no, ni,
-                                (float)(c * std::sqrt(inst[i].weight))));
-  }
-  split_narrow(P.g1, P.g1n);
-  split_narrow(P.g2, P.g2n);
-  order_problems(P.g1, P.g1_xcd);
-  order_problems(P.g2, P.g2_xcd);
-  order_problems(P.g1n, P.g1n_xcd);
-  order_problems(P.g2n, P.g2n_xcd);
-  // sums
-  for (int o = 0; o < n_outputs; ++o) {
-    if (members[o].empty()) continue;
-    SumJob j{};
-    j.out = outs[o];
-    j.planes = (const float*)(ws + P.I_off[members[o][0]]);
-    j.npix = (long)inst[members[o][0]].n_out * inst[members[o][0]].n_out;
-    j.count = (int)members[o].size();
-    P.sum.push_back(j);
-  }
-  return DLX_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -425,33 +374,21 @@ int plan_batched(int n, const dlx_mft_instance* inst, int n_outputs, float* cons
 // the same shape, whatever the fields, wavelengths, weights, shifts, outputs
 // and matrix addresses (all uploaded before the launch).
 int launch_plan(const Plan& Q, uint8_t* ws, bool with_matrices, hipStream_t s) {
-  auto blocks = [](long rows) { return (unsigned)(rows < 16384 ? rows : 16384); };
-  if (Q.cvt_work > 0) {
-    hipLaunchKernelGGL(group_to_split4_kernel, dim3(blocks(Q.cvt_work)), dim3(256), 0, s,
-                       (const CvtJob*)(ws + Q.off_cvt), (int)Q.cvt.size(), Q.cvt_work);
-    if (int st = launch_status("group_to_split4_kernel")) return st;
+  if (with_matrices)
+    DLX_HIP(launch_fold_group_tables((const FoldTableJob*)(ws + Q.off_tab), (int)Q.tab.size(),
+                                     Q.tab_most, s));
+  FoldGroup g{};
+  g.probs = (const FoldProblem*)(ws + Q.off_prob);
+  const int width[3] = {32, 64, 128};
+  for (int l = kLists - 1; l >= 0; --l) {   // the largest outputs first
+    if (Q.map1[l].empty()) continue;
+    g.map = (const uint32_t*)(ws + Q.off_map1[l]);
+    std::memcpy(g.xcd, Q.xcd1[l], sizeof(g.xcd));
+    DLX_HIP(launch_fold_group_stage1(g, width[l / 2], l % 2 != 0, s));
   }
-  if (with_matrices && Q.mat_work > 0) {
-    hipLaunchKernelGGL(group_dft_split4_kernel, dim3(blocks(Q.mat_work)), dim3(256), 0, s,
-                       (const MatJob*)(ws + Q.off_mat), (int)Q.mat.size(), Q.mat_work);
-    if (int st = launch_status("group_dft_split4_kernel")) return st;
-  }
-  auto grouped = [&](size_t off, const std::vector<GroupProblem>& probs, const int (&xcd)[9],
-                     int tile_n, int epi) -> int {
-    if (probs.empty()) return DLX_OK;
-    GroupLaunch l{};
-    l.probs = (const GroupProblem*)(ws + off);
-    l.nprobs = (int)probs.size();
-    l.tile_n = tile_n;
-    std::memcpy(l.xcd_start, xcd, sizeof(l.xcd_start));
-    DLX_HIP(launch_cgemm_split4_group(l, epi, s));
-    return DLX_OK;
-  };
-  const size_t n1 = Q.g1.size() * sizeof(GroupProblem), n2 = Q.g2.size() * sizeof(GroupProblem);
-  if (int st = grouped(Q.off_g1, Q.g1, Q.g1_xcd, 128, EPI_SPLIT_T)) return st;
-  if (int st = grouped(Q.off_g1 + n1, Q.g1n, Q.g1n_xcd, 64, EPI_SPLIT_T)) return st;
-  if (int st = grouped(Q.off_g2, Q.g2, Q.g2_xcd, 128, EPI_INTENSITY)) return st;
-  if (int st = grouped(Q.off_g2 + n2, Q.g2n, Q.g2n_xcd, 64, EPI_INTENSITY)) return st;
+  g.map = (const uint32_t*)(ws + Q.off_map2);
+  std::memcpy(g.xcd, Q.xcd2, sizeof(g.xcd));
+  DLX_HIP(launch_fold_group_stage2(g, s));
   if (Q.sum.empty()) return DLX_OK;
   long most = 0;
   for (const SumJob& j : Q.sum) most = j.npix > most ? j.npix : most;
@@ -463,13 +400,14 @@ int launch_plan(const Plan& Q, uint8_t* ws, bool with_matrices, hipStream_t s) {
 
 // Everything launch_plan's grids and by-value arguments depend on.
 std::vector<long> plan_shape(const Plan& Q, const uint8_t* ws, bool fresh, int dev) {
-  std::vector<long> k = {(long)dev, (long)(uintptr_t)ws, (long)fresh, (long)Q.off_mat,
-                         (long)Q.mat.size(), Q.mat_work, (long)Q.off_cvt, (long)Q.cvt.size(),
-                         Q.cvt_work,
-                         (long)Q.off_g1, (long)Q.off_g2, (long)Q.g1.size(), (long)Q.g1n.size(),
-                         (long)Q.g2.size(), (long)Q.g2n.size(), (long)Q.off_sum,
-                         (long)Q.sum.size()};
-  for (const int* x : {Q.g1_xcd, Q.g1n_xcd, Q.g2_xcd, Q.g2n_xcd}) k.insert(k.end(), x, x + 9);
+  std::vector<long> k = {(long)dev, (long)(uintptr_t)ws, (long)fresh, (long)Q.off_tab,
+                         (long)Q.tab.size(), Q.tab_most, (long)Q.off_prob, (long)Q.off_map2,
+                         (long)Q.off_sum, (long)Q.sum.size()};
+  for (int l = 0; l < kLists; ++l) {
+    k.push_back((long)Q.off_map1[l]);
+    k.insert(k.end(), Q.xcd1[l], Q.xcd1[l] + 9);
+  }
+  k.insert(k.end(), Q.xcd2, Q.xcd2 + 9);
   for (const SumJob& j : Q.sum) k.push_back(j.npix);
   return k;
 }
@@ -588,7 +526,7 @@ size_t dlx_mft_batched_workspace_size(int32_t n, const dlx_mft_instance* instanc
         instances[i].n_in <= 0 || instances[i].n_out <= 0)
       return 0;
   Plan P;
-  if (plan_batched(n, instances, n_outputs, nullptr, nullptr, P) != DLX_OK) return 0;
+  if (plan_sizes(n, instances, n_outputs, P) != DLX_OK) return 0;
   return P.total;
 }
 
@@ -603,10 +541,10 @@ int dlx_mft_batched_psf(int32_t n, const dlx_mft_instance* instances, int32_t n_
     DLX_CHECK_ARG(outputs[instances[i].out_index] != nullptr, "outputs[%d] is NULL",
                   instances[i].out_index);
   hipStream_t s = (hipStream_t)stream;
-  Plan P;
-  if (int st = plan_batched(n, instances, n_outputs, nullptr, nullptr, P)) return st;
-  if (!workspace || workspace_bytes < P.total) {
-    set_error("dlx_mft_batched_psf workspace too small: need %zu bytes, got %zu", P.total,
+  Plan Q;
+  if (int st = plan_sizes(n, instances, n_outputs, Q)) return st;
+  if (!workspace || workspace_bytes < Q.total) {
+    set_error("dlx_mft_batched_psf workspace too small: need %zu bytes, got %zu", Q.total,
               workspace_bytes);
     return DLX_ERR_WORKSPACE;
   }
@@ -616,42 +554,30 @@ int dlx_mft_batched_psf(int32_t n, const dlx_mft_instance* instances, int32_t n_
     set_error("dlx_mft_batched_psf uploads per-call descriptors and cannot be captured");
     return DLX_ERR_UNSUPPORTED;
   }
-  Plan Q;
   uint8_t* ws = (uint8_t*)workspace;
-  if (int st = plan_batched(n, instances, n_outputs, outputs, ws, Q)) return st;
 
-  // Transfer matrices depend only on the instances' geometry, wavelengths,
-  // scales and shifts: keep the whole set resident in the device cache, keyed
-  // by every matrix's parameters, and regenerate only on a miss.
+  // The tables depend only on the instances' sides and phase steps: keep the
+  // whole set resident in the device cache and regenerate only on a miss.
   std::vector<double> key;
-  key.reserve(Q.mat.size() * 7);
-  for (const MatJob& j : Q.mat)
-    key.insert(key.end(), {(double)j.rows, (double)j.cols, (double)j.sign_inv, j.c_scale,
-                           j.c_off, j.r_scale, j.r_off});
-  const size_t wbytes = Q.off_U - Q.off_W;
-  void* wcache = nullptr;
-  CacheLease whandle(s);
+  key.reserve(1 + Q.tab.size() * 3);
+  key.push_back(2002.0);
+  for (const FoldTableJob& j : Q.tab) key.insert(key.end(), {(double)j.n, (double)j.m, j.step});
+  void* tcache = nullptr;
+  CacheLease lease(s);
   bool fresh = true;
-  if (int st = cache_acquire_raw(key, wbytes, s, &wcache, &whandle.h, &fresh)) return st;
-  if (wcache) {
-    uint8_t* w0 = ws + Q.off_W;
-    auto rebase = [&](const uint8_t* p) -> uint8_t* {
-      return (p >= w0 && p < w0 + wbytes) ? (uint8_t*)wcache + (p - w0) : (uint8_t*)p;
-    };
-    for (MatJob& j : Q.mat) j.out = rebase(j.out);
-    for (GroupProblem& g : Q.g1) g.B = rebase(g.B);
-    for (GroupProblem& g : Q.g2) g.A = rebase(g.A);
-    for (GroupProblem& g : Q.g1n) g.B = rebase(g.B);
-    for (GroupProblem& g : Q.g2n) g.A = rebase(g.A);
+  if (int st = cache_acquire_raw(key, Q.tab_bytes, s, &tcache, &lease.h, &fresh)) return st;
+  plan_fill(n, instances, n_outputs, outputs, ws, Q);
+  if (tcache) {
+    const uint8_t* t0 = ws + Q.off_T;
+    for (FoldTableJob& j : Q.tab) j.out = (uint8_t*)tcache + (j.out - t0);
+    for (FoldProblem& p : Q.prob) p.table = (const uint8_t*)tcache + (p.table - t0);
   }
   // all descriptors sit at the front of the workspace: one upload
-  std::vector<uint8_t> host(Q.off_P, 0);
-  put(host, Q.off_cvt, Q.cvt);
-  put(host, Q.off_mat, Q.mat);
-  put(host, Q.off_g1, Q.g1);
-  put(host, Q.off_g1 + Q.g1.size() * sizeof(GroupProblem), Q.g1n);
-  put(host, Q.off_g2, Q.g2);
-  put(host, Q.off_g2 + Q.g2.size() * sizeof(GroupProblem), Q.g2n);
+  std::vector<uint8_t> host(Q.desc, 0);
+  put(host, Q.off_tab, Q.tab);
+  put(host, Q.off_prob, Q.prob);
+  for (int l = 0; l < kLists; ++l) put(host, Q.off_map1[l], Q.map1[l]);
+  put(host, Q.off_map2, Q.map2);
   put(host, Q.off_sum, Q.sum);
   if (int st = upload(host.data(), host.size(), ws, s)) return st;
 
@@ -662,8 +588,8 @@ int dlx_mft_batched_psf(int32_t n, const dlx_mft_instance* instances, int32_t n_
   if (eager)
     if (int st = launch_plan(Q, ws, fresh, s)) return st;
   if (fresh)
-    if (int st = cache_ready(whandle.h, s)) return st;
-  return whandle.release();
+    if (int st = cache_ready(lease.h, s)) return st;
+  return lease.release();
 }
 
 int dlx_batched_graph_stats(uint64_t* captures, uint64_t* launches, int32_t* entries) {

@@ -68,7 +68,14 @@ hipError_t launch_fold_tables(const double* step, int nb, int n, int m, bool spl
 enum FoldLoad {
   FOLD_MEM = 0,     // folded rows in memory
   FOLD_PUPIL = 1,   // phasors of amplitude and OPD planes, formed in the loader
-  FOLD_FIELD = 2,   // a complex64 field (optionally times a phase ramp per axis)
+  FOLD_FIELD = 2,   // a complex64 field (optionally times a separable phase)
+};
+
+// A separable phase over a grid's centred indices u = k - (side - 1) / 2, in turns:
+// c2 (ux^2 + uy^2) + cx ux + cy uy + c0.  An output or input shift of the MFT
+// is the linear part, the Collins kernel's chirps the quadratic one.
+struct FoldPhase {
+  double c2, cx, cy, c0;
 };
 
 // The pupil of instance b: a(y, x) exp(2 pi i path(y, x) inv_wl[b]),
@@ -83,17 +90,16 @@ struct FoldStage1 {
   static constexpr int kMaxBatch = 64;
   int n, m, batch;                     // field side, output side
   const uint8_t* src; long src_stride; // FOLD_MEM / FOLD_FIELD, bytes per instance
-  const float2* ramp; long ramp_stride;   // FOLD_FIELD: x then y ramps of ceil(n/2) values at
-                                          // the positive half (the other half is conjugate)
   const uint8_t* table; long table_stride;
   uint8_t* out; long out_stride;
   FoldPupil pupil;                     // FOLD_PUPIL
   double inv_wl[kMaxBatch];
+  FoldPhase phase[kMaxBatch];          // FOLD_FIELD: multiplies the field
 };
 
 enum FoldEpilogue {
   FOLD_INTENSITY = 0,   // out[b](ly, lx) = |alpha E|^2, float
-  FOLD_STORE = 1,       // out[b](ly, lx) = alpha E [ox(lx) oy(ly)], complex64
+  FOLD_STORE = 1,       // out[b](ly, lx) = alpha E exp(2 pi i phase(ly, lx)), complex64
   FOLD_VJP = 2,         // folded rows ((alpha, beta, c), qy), k = qx, of 2 G alpha E
   FOLD_GRAD = 3,        // out[b](y, x) = Im(conj(P) alpha E), out2 (optional) = Re(conj(U) alpha E)
 };
@@ -106,15 +112,48 @@ struct FoldStage2 {
   const uint8_t* mid; long mid_stride; // stage-1 result
   void* out; long out_stride;          // elements (INTENSITY, STORE, GRAD) or bytes (VJP)
   float alpha[kMaxBatch];
-  const float2* ramp; long ramp_stride;   // STORE: ox then oy, m values each (or null)
   const float* G;                      // VJP: dL/dPSF, m x m
   float* out2;                         // GRAD
   FoldPupil pupil;                     // GRAD: P, U = P / a at amplitude scale
   double inv_wl[kMaxBatch];
+  FoldPhase phase[kMaxBatch];          // STORE: multiplies the result
 };
 
 hipError_t launch_fold_stage1(const FoldStage1& a, FoldLoad load, bool split, hipStream_t s);
 hipError_t launch_fold_stage2(const FoldStage2& a, FoldEpilogue epi, bool split, hipStream_t s);
+
+// One transform of an uneven batch, in device memory: |alpha W_y P W_x^T|^2 of
+// a complex64 field (times the linear phase cx ux + cy uy) into a float plane.
+// Its stage-1 tiles are [tile1, ...) of its width's list, its stage-2 tiles
+// [tile2, ...), each numbered column-fastest as in the uniform launches.
+struct FoldProblem {
+  const uint8_t* src;
+  const uint8_t* table;
+  uint8_t* mid;
+  float* out;
+  double cx, cy;
+  float alpha;
+  int n, m, inverse, tile1, tile2;
+};
+// A launch over the tiles of many problems: map[t] is the problem of tile t;
+// XCD x runs [xcd[x], xcd[x + 1]).
+struct FoldGroup {
+  const FoldProblem* probs;
+  const uint32_t* map;
+  int xcd[9];
+};
+struct FoldTableJob {
+  uint8_t* out;
+  double step;
+  int n, m;
+};
+// Output columns per stage-1 tile for an output side m (32, 64 or 128), and
+// the rows and columns of a stage-2 tile.
+int fold_group_width(int m);
+constexpr int kFoldTileQy = 64, kFoldTileQx = 32, kFoldTilePy = 32;
+hipError_t launch_fold_group_tables(const FoldTableJob* jobs, int njobs, long most, hipStream_t s);
+hipError_t launch_fold_group_stage1(const FoldGroup& g, int width, bool vec, hipStream_t s);
+hipError_t launch_fold_group_stage2(const FoldGroup& g, hipStream_t s);
 
 // The folded pupil written to memory (FOLD_MEM rows), bit for bit what
 // FOLD_PUPIL forms.
