@@ -356,16 +356,17 @@ int field_transform(int n, int m, int batch, bool inverse, const std::vector<dou
 // directions (used when the cache is bypassed), the stage-1 intermediate of
 // either direction, Ebar, and the per-wavelength gradient planes.
 struct VjpLayout {
-  size_t T, U, Eb, H, total;
+  size_t T, U, Eb, H, P, total;   // P: the folded pupil, where the loader does not form it
 };
-VjpLayout vjp_layout(const dlx_mft_geom& g, int c, bool amp) {
+VjpLayout vjp_layout(const dlx_mft_geom& g, int c) {
   VjpLayout L;
   L.T = align_up((size_t)c * (fold_table_bytes(g.n_in, g.n_out) + fold_table_bytes(g.n_out, g.n_in)));
   const long u = fold_mid_bytes(g.n_in, g.n_out), v = fold_mid_bytes(g.n_out, g.n_in);
   L.U = align_up((size_t)c * (u > v ? u : v));
   L.Eb = align_up((size_t)c * fold_field_bytes(g.n_out));
   L.H = align_up((size_t)c * g.n_in * g.n_in * sizeof(float));
-  L.total = L.T + L.U + L.Eb + (amp ? 2 : 1) * L.H;
+  L.P = align_up((size_t)c * fold_field_bytes(g.n_in));
+  L.total = L.T + L.U + L.Eb + 2 * L.H + L.P;
   return L;
 }
 
@@ -703,7 +704,8 @@ int psf_poly_run(const dlx_mft_geom& g, int32_t nwl, const double* wavelength,
               tilt_y, (float)scale};
   // the pupil formed in stage 1's loader (no pupil array in HBM), or written
   // first where many column tiles would each form it again
-  const bool in_loader = !room || (!phase && pupil_prologue_enabled() && fold_pupil_in_loader(g.n_out));
+  const bool in_loader =
+      !room || (pupil_prologue_enabled() && fold_pupil_in_loader(f1.pupil, g.n_out));
   for (int l0 = 0; l0 < nwl; l0 += c) {
     const int nb = nwl - l0 < c ? nwl - l0 : c;
     // one wavelength is its own sum
@@ -839,7 +841,7 @@ size_t dlx_psf_poly_vjp_workspace_size(const dlx_mft_geom* geom, int32_t nwl,
   // more than the PSF's own workspace: one buffer serves a step's forward and
   // backward calls
   const size_t psf = psf_poly_bytes(*geom, c, precision == DLX_PREC_BF16X3);
-  const VjpLayout L = vjp_layout(*geom, c, true);
+  const VjpLayout L = vjp_layout(*geom, c);
   return (L.total > psf ? L.total : psf) + 256;
 }
 
@@ -876,12 +878,13 @@ int dlx_psf_poly_vjp(const dlx_mft_geom* geom, int32_t nwl, const double* wavele
   hipStream_t s = (hipStream_t)stream;
   const bool split = precision == DLX_PREC_BF16X3;
   const int c = nwl < kWlChunk ? nwl : kWlChunk;
-  const VjpLayout L = vjp_layout(g, c, true);
+  const VjpLayout L = vjp_layout(g, c);
   uint8_t* T_ws = (uint8_t*)workspace;
   uint8_t* U = T_ws + L.T;
   uint8_t* Eb = U + L.U;
   float* H = (float*)(Eb + L.Eb);
   float* H2 = grad_amp ? (float*)((uint8_t*)H + L.H) : nullptr;
+  uint8_t* P = (uint8_t*)H + 2 * L.H;
   const long nin = g.n_in;
   const FoldPupil pup = {opd, amp, phase, pixel_scale_in,
                          center - (g.n_in - 1) / 2.0 * pixel_scale_in, tilt_x, tilt_y, (float)scale};
@@ -909,7 +912,13 @@ int dlx_psf_poly_vjp(const dlx_mft_geom* geom, int32_t nwl, const double* wavele
     f.out = U; f.out_stride = fold_mid_bytes(g.n_in, g.n_out);
     f.pupil = pup;
     for (int i = 0; i < nb; ++i) f.inv_wl[i] = b.inv_wl[i];
-    DLX_HIP(launch_fold_stage1(f, FOLD_PUPIL, split, s));
+    const bool in_loader = fold_pupil_in_loader(pup, g.n_out);
+    if (!in_loader) {
+      f.src = P;
+      f.src_stride = fold_field_bytes(g.n_in);
+      DLX_HIP(launch_fold_pupil(pup, f.inv_wl, nb, g.n_in, split, P, f.src_stride, s));
+    }
+    DLX_HIP(launch_fold_stage1(f, in_loader ? FOLD_PUPIL : FOLD_MEM, split, s));
     e.n = g.n_in; e.m = g.n_out; e.batch = nb; e.inverse = g.inverse;
     e.table = tab.fwd; e.table_stride = tab.stride;
     e.mid = U; e.mid_stride = f.out_stride;

@@ -3,10 +3,11 @@
 //
 // One call of dlx_mft_batched_psf runs, whatever the mix of shapes:
 //   1. one launch that generates the distinct cosine / sine tables (instances
-//      of equal sides and phase step share one);
+//      of equal sides and phase step share one), and one that folds each
+//      distinct complex64 field;
 //   2. one grouped launch per tile width (output sides to 64, to 128, above)
-//      of the folded stage 1, which loads the complex64 fields directly and
-//      applies each instance's shift as a phase (dlx_fold.h);
+//      of the folded stage 1, whose workgroups take several instances of one
+//      field and apply each one's shift as a phase (dlx_fold.h);
 //   3. one grouped launch of stage 2 with the |E|^2 epilogue,
 //      I_i = |alpha_i W_y,i U_i|^2 (alpha_i = c_i sqrt(weight_i));
 //   4. one launch that sums the planes of each output image, in a fixed order.
@@ -107,17 +108,25 @@ int upload(const void* src, size_t bytes, void* dst, hipStream_t s) {
 // ---------------------------------------------------------------------------
 // planning
 // ---------------------------------------------------------------------------
-constexpr int kLists = 6;       // stage-1 lists: tile width (32, 64, 128) x (scalar, 16-byte loads)
+constexpr int kLists = 3;                   // stage-1 lists by tile width
+constexpr int kWidth[kLists] = {32, 64, 128};
+int list_of(int m) { return fold_group_width(m) == 128 ? 2 : fold_group_width(m) == 64 ? 1 : 0; }
 
 struct Plan {
   // workspace offsets (bytes); descriptors first
-  size_t off_tab, off_prob, off_map1[kLists], off_map2, off_sum, desc, off_T, off_U, off_I, total;
+  size_t off_tab, off_fld, off_prob, off_cols, off_map1[kLists], off_map2, off_sum, desc;
+  size_t off_T, off_P, off_U, off_I, total;
   size_t tab_bytes = 0;
   std::vector<FoldTableJob> tab;
   std::vector<size_t> tab_off;       // of each distinct table, from off_T
   std::vector<int> tab_of;           // instance -> table
   long tab_most = 0;                 // threads of the largest table
+  std::vector<FoldFieldJob> fld;     // distinct fields
+  std::vector<size_t> fld_off;
+  std::vector<int> fld_of;           // instance -> field
+  int fld_most = 0;                  // side of the largest field
   std::vector<FoldProblem> prob;     // in launch order
+  std::vector<FoldColumns> cols;
   std::vector<uint32_t> map1[kLists], map2;
   int xcd1[kLists][9], xcd2[9];
   std::vector<SumJob> sum;
@@ -188,10 +197,8 @@ struct TableHash {
   }
 };
 
-int tiles1(int n, int m) {
-  const int w = fold_group_width(m);
-  return ((fold_half(n) + kFoldTilePy - 1) / kFoldTilePy) * ((fold_half(m) + w - 1) / w);
-}
+int rows1(int n) { return (fold_half(n) + kFoldTilePy - 1) / kFoldTilePy; }
+int cols1(int m) { return (fold_half(m) + fold_group_width(m) - 1) / fold_group_width(m); }
 int tiles2(int m) {
   const int mh = fold_half(m);
   return ((mh + kFoldTileQy - 1) / kFoldTileQy) * ((mh + kFoldTileQx - 1) / kFoldTileQx);
@@ -199,19 +206,28 @@ int tiles2(int m) {
 
 // Sizes and offsets of the batch's buffers.
 int plan_sizes(int n, const dlx_mft_instance* inst, int n_outputs, Plan& P) {
-  std::unordered_map<const void*, int> field_n;
+  std::unordered_map<const void*, int> fields;
   size_t plain = 0;      // the unfolded layout's buffers: never asked for less
-  const void* last = nullptr;
+  size_t fbytes = 0;
+  P.fld_of.resize(n);
   for (int i = 0; i < n; ++i) {
     const dlx_mft_instance& d = inst[i];
-    if (d.field != last || i == 0) {
-      auto it = field_n.emplace(d.field, d.n_in);
-      if (it.second) plain += align_up(mat_bytes(d.n_in, d.n_in, true));
-      last = d.field;
+    if (i > 0 && d.field == inst[i - 1].field) {
+      P.fld_of[i] = P.fld_of[i - 1];
+    } else {
+      auto it = fields.emplace(d.field, (int)P.fld.size());
+      P.fld_of[i] = it.first->second;
+      if (it.second) {
+        P.fld.push_back({(const float2*)d.field, nullptr, d.n_in, 0});
+        P.fld_off.push_back(fbytes);
+        fbytes += align_up(fold_field_bytes(d.n_in));
+        P.fld_most = std::max(P.fld_most, (int)d.n_in);
+        plain += align_up(mat_bytes(d.n_in, d.n_in, true));
+      }
     }
-    if (field_n[d.field] != d.n_in) {
+    if (P.fld[P.fld_of[i]].n != d.n_in) {
       set_error("instance %d: the same field pointer is used with n_in %d and %d", i,
-                field_n[d.field], d.n_in);
+                P.fld[P.fld_of[i]].n, d.n_in);
       return DLX_ERR_INVALID;
     }
   }
@@ -235,22 +251,23 @@ int plan_sizes(int n, const dlx_mft_instance* inst, int n_outputs, Plan& P) {
   size_t off = 0;
   auto take = [&](size_t bytes) { const size_t o = off; off += align_up(bytes); return o; };
   P.off_tab = take(P.tab.size() * sizeof(FoldTableJob));
+  P.off_fld = take(P.fld.size() * sizeof(FoldFieldJob));
   P.off_prob = take((size_t)n * sizeof(FoldProblem));
-  size_t n1[kLists] = {}, n2 = 0;
-  auto list_of = [&](int i) {
-    const int w = fold_group_width(inst[i].n_out);
-    const bool vec = inst[i].n_in % 8 == 0 && ((uintptr_t)inst[i].field & 15) == 0;
-    return (w == 128 ? 2 : w == 64 ? 1 : 0) * 2 + (vec ? 1 : 0);
-  };
+  // bounds: a column group per column tile
+  size_t n1[kLists] = {}, n2 = 0, nc = 0;
   for (int i = 0; i < n; ++i) {
-    n1[list_of(i)] += tiles1(inst[i].n_in, inst[i].n_out);
+    const int c = cols1(inst[i].n_out);
+    n1[list_of(inst[i].n_out)] += (size_t)rows1(inst[i].n_in) * c;
     n2 += tiles2(inst[i].n_out);
+    nc += c;
   }
+  P.off_cols = take(nc * sizeof(FoldColumns));
   for (int l = 0; l < kLists; ++l) P.off_map1[l] = take(n1[l] * sizeof(uint32_t));
   P.off_map2 = take(n2 * sizeof(uint32_t));
   P.off_sum = take((size_t)n_outputs * sizeof(SumJob));
   P.desc = off;
   P.off_T = take(P.tab_bytes);
+  P.off_P = take(fbytes);
   P.off_U = off;
   P.U_off.resize(n);
   for (int i = 0; i < n; ++i) {
@@ -277,78 +294,106 @@ int plan_sizes(int n, const dlx_mft_instance* inst, int n_outputs, Plan& P) {
   return DLX_OK;
 }
 
-// The descriptors.  Instances that share a field go to one XCD (its L2 then
-// holds the field while their stage-1 tiles read it), fields dealt largest
-// first to the XCD with the least work; with few fields the instances are
-// dealt one by one.  Stage 2 keeps stage 1's XCDs: it reads what they wrote.
+// The descriptors.  The instances of one field go to one XCD, their stage-1
+// workgroups for the same rows next to each other (its L2 then serves the
+// field to all of them), fields dealt largest first to the XCD with the least
+// work; with few fields (a scene's shared pupil) the instances are dealt in
+// sets of a column group each.  Stage 2 keeps stage 1's XCDs: it reads what
+// they wrote.
 void plan_fill(int n, const dlx_mft_instance* inst, int n_outputs, float* const* outs, uint8_t* ws,
                Plan& P) {
   for (size_t q = 0; q < P.tab.size(); ++q) P.tab[q].out = ws + P.off_T + P.tab_off[q];
-  // stage 1's stages and a tile's fixed part, plus stage 2
+  for (size_t f = 0; f < P.fld.size(); ++f) P.fld[f].out = ws + P.off_P + P.fld_off[f];
+  // stage 1's column blocks over the field's rows and stages, a tile's fixed
+  // part, and stage 2's tiles
   auto cost = [&](int i) {
     const int st = (fold_half(inst[i].n_in) + 15) / 16;
     const int w = fold_group_width(inst[i].n_out);
-    return (double)tiles1(inst[i].n_in, inst[i].n_out) * (st + 6) * (w + 64) / 192.0 +
+    return (double)rows1(inst[i].n_in) * cols1(inst[i].n_out) * (st + 4) * (w + 32) / 160.0 +
            (double)tiles2(inst[i].n_out) * (st + 8) * 0.5;
   };
-  std::unordered_map<const void*, int> unit_of;
-  std::vector<std::vector<int>> units;
-  std::vector<double> ucost;
-  for (int i = 0; i < n; ++i) {
-    auto it = unit_of.emplace(inst[i].field, (int)units.size());
-    if (it.second) { units.emplace_back(); ucost.push_back(0.0); }
-    units[it.first->second].push_back(i);
-    ucost[it.first->second] += cost(i);
-  }
+  std::vector<std::vector<int>> units(P.fld.size());
+  for (int i = 0; i < n; ++i) units[P.fld_of[i]].push_back(i);
   if (units.size() < 32) {
-    std::vector<std::vector<int>> one;
-    std::vector<double> c;
-    for (auto& u : units)
-      for (int i : u) { one.push_back({i}); c.push_back(cost(i)); }
-    units.swap(one);
-    ucost.swap(c);
+    std::vector<std::vector<int>> cut;
+    for (auto& u : units) {
+      std::stable_sort(u.begin(), u.end(),
+                       [&](int a, int b) { return inst[a].n_out > inst[b].n_out; });
+      for (size_t i = 0; i < u.size();) {
+        const size_t k = 128 / fold_group_width(inst[u[i]].n_out);
+        const size_t e = std::min(u.size(), i + k);
+        cut.emplace_back(u.begin() + i, u.begin() + e);
+        i = e;
+      }
+    }
+    units.swap(cut);
   }
+  std::vector<double> ucost(units.size(), 0.0);
+  for (size_t u = 0; u < units.size(); ++u)
+    for (int i : units[u]) ucost[u] += cost(i);
   std::vector<int> idx(units.size());
   std::iota(idx.begin(), idx.end(), 0);
   std::stable_sort(idx.begin(), idx.end(), [&](int a, int b) { return ucost[a] > ucost[b]; });
-  std::vector<int> on[8];
+  std::vector<int> on[8];   // units of an XCD
   double load[8] = {};
   for (int u : idx) {
     int best = 0;
     for (int x = 1; x < 8; ++x)
       if (load[x] < load[best]) best = x;
-    on[best].insert(on[best].end(), units[u].begin(), units[u].end());
+    on[best].push_back(u);
     load[best] += ucost[u];
   }
   P.prob.reserve(n);
   for (int x = 0; x < 8; ++x) {
     for (int l = 0; l < kLists; ++l) P.xcd1[l][x] = (int)P.map1[l].size();
     P.xcd2[x] = (int)P.map2.size();
-    for (int i : on[x]) {
-      const dlx_mft_instance& d = inst[i];
-      const FoldTableJob& t = P.tab[P.tab_of[i]];
-      const double sg = d.inverse ? -1.0 : 1.0;
-      const double c = mft_norm(geom_of(d), d.wavelength, d.pixel_scale_in, d.pixel_scale_out);
-      FoldProblem p{};
-      p.src = (const uint8_t*)d.field;
-      p.table = t.out;
-      p.mid = ws + P.U_off[i];
-      p.out = (float*)(ws + P.I_off[i]);
-      // the input half of the shift (the output half is a phase: no intensity)
-      p.cx = sg * t.step * d.shift_x;
-      p.cy = sg * t.step * d.shift_y;
-      p.alpha = (float)(c * std::sqrt(d.weight));
-      p.n = d.n_in;
-      p.m = d.n_out;
-      p.inverse = d.inverse ? 1 : 0;
-      const int w = fold_group_width(d.n_out);
-      const bool vec = d.n_in % 8 == 0 && ((uintptr_t)d.field & 15) == 0;
-      std::vector<uint32_t>& m1 = P.map1[(w == 128 ? 2 : w == 64 ? 1 : 0) * 2 + (vec ? 1 : 0)];
-      p.tile1 = (int)m1.size();
-      p.tile2 = (int)P.map2.size();
-      m1.insert(m1.end(), tiles1(p.n, p.m), (uint32_t)P.prob.size());
-      P.map2.insert(P.map2.end(), tiles2(p.m), (uint32_t)P.prob.size());
-      P.prob.push_back(p);
+    for (int u : on[x]) {
+      // stage 1: this field's column groups of each width
+      for (int l = 0; l < kLists; ++l) {
+        const int L = 128 / kWidth[l], c0 = (int)P.cols.size();
+        for (int i : units[u]) {
+          const dlx_mft_instance& d = inst[i];
+          if (list_of(d.n_out) != l) continue;
+          const FoldTableJob& t = P.tab[P.tab_of[i]];
+          const double sg = d.inverse ? -1.0 : 1.0;
+          for (int c = 0; c < cols1(d.n_out); ++c) {
+            if ((int)P.cols.size() == c0 || P.cols.back().count == L) {
+              FoldColumns g{};
+              g.src = P.fld[P.fld_of[i]].out;
+              g.n = d.n_in;
+              P.cols.push_back(g);
+            }
+            FoldColumns& g = P.cols.back();
+            // the input half of the shift (the output half is a phase: no intensity)
+            g.tile_of[g.count++] = {t.out, ws + P.U_off[i], sg * t.step * d.shift_x,
+                                    sg * t.step * d.shift_y, c * kWidth[l], d.n_out};
+          }
+        }
+        const int nc = (int)P.cols.size() - c0;
+        if (nc == 0) continue;
+        const int base = (int)P.map1[l].size();
+        for (int c = 0; c < nc; ++c) {
+          P.cols[c0 + c].tile = base + c;
+          P.cols[c0 + c].step = nc;
+        }
+        for (int r = 0; r < rows1(P.cols[c0].n); ++r)
+          for (int c = 0; c < nc; ++c) P.map1[l].push_back((uint32_t)(c0 + c));
+      }
+      for (int i : units[u]) {
+        const dlx_mft_instance& d = inst[i];
+        const double c = mft_norm(geom_of(d), d.wavelength, d.pixel_scale_in, d.pixel_scale_out);
+        FoldProblem p{};
+        p.table = P.tab[P.tab_of[i]].out;
+        p.mid = ws + P.U_off[i];
+        p.out = (float*)(ws + P.I_off[i]);
+        p.alpha = (float)(c * std::sqrt(d.weight));
+        p.n = d.n_in;
+        p.m = d.n_out;
+        p.inverse = d.inverse ? 1 : 0;
+        p.tile = (int)P.map2.size();
+        P.map2.insert(P.map2.end(), tiles2(p.m), (uint32_t)P.prob.size());
+        P.prob.push_back(p);
+      }
     }
   }
   for (int l = 0; l < kLists; ++l) P.xcd1[l][8] = (int)P.map1[l].size();
@@ -377,14 +422,16 @@ int launch_plan(const Plan& Q, uint8_t* ws, bool with_matrices, hipStream_t s) {
   if (with_matrices)
     DLX_HIP(launch_fold_group_tables((const FoldTableJob*)(ws + Q.off_tab), (int)Q.tab.size(),
                                      Q.tab_most, s));
+  DLX_HIP(launch_fold_group_fields((const FoldFieldJob*)(ws + Q.off_fld), (int)Q.fld.size(),
+                                   Q.fld_most, s));
   FoldGroup g{};
   g.probs = (const FoldProblem*)(ws + Q.off_prob);
-  const int width[3] = {32, 64, 128};
+  g.cols = (const FoldColumns*)(ws + Q.off_cols);
   for (int l = kLists - 1; l >= 0; --l) {   // the largest outputs first
     if (Q.map1[l].empty()) continue;
     g.map = (const uint32_t*)(ws + Q.off_map1[l]);
     std::memcpy(g.xcd, Q.xcd1[l], sizeof(g.xcd));
-    DLX_HIP(launch_fold_group_stage1(g, width[l / 2], l % 2 != 0, s));
+    DLX_HIP(launch_fold_group_stage1(g, kWidth[l], s));
   }
   g.map = (const uint32_t*)(ws + Q.off_map2);
   std::memcpy(g.xcd, Q.xcd2, sizeof(g.xcd));
@@ -401,7 +448,8 @@ int launch_plan(const Plan& Q, uint8_t* ws, bool with_matrices, hipStream_t s) {
 // Everything launch_plan's grids and by-value arguments depend on.
 std::vector<long> plan_shape(const Plan& Q, const uint8_t* ws, bool fresh, int dev) {
   std::vector<long> k = {(long)dev, (long)(uintptr_t)ws, (long)fresh, (long)Q.off_tab,
-                         (long)Q.tab.size(), Q.tab_most, (long)Q.off_prob, (long)Q.off_map2,
+                         (long)Q.tab.size(), Q.tab_most, (long)Q.off_fld, (long)Q.fld.size(),
+                         (long)Q.fld_most, (long)Q.off_prob, (long)Q.off_cols, (long)Q.off_map2,
                          (long)Q.off_sum, (long)Q.sum.size()};
   for (int l = 0; l < kLists; ++l) {
     k.push_back((long)Q.off_map1[l]);
@@ -571,11 +619,16 @@ int dlx_mft_batched_psf(int32_t n, const dlx_mft_instance* instances, int32_t n_
     const uint8_t* t0 = ws + Q.off_T;
     for (FoldTableJob& j : Q.tab) j.out = (uint8_t*)tcache + (j.out - t0);
     for (FoldProblem& p : Q.prob) p.table = (const uint8_t*)tcache + (p.table - t0);
+    for (FoldColumns& g : Q.cols)
+      for (int i = 0; i < g.count; ++i)
+        g.tile_of[i].table = (const uint8_t*)tcache + (g.tile_of[i].table - t0);
   }
   // all descriptors sit at the front of the workspace: one upload
   std::vector<uint8_t> host(Q.desc, 0);
   put(host, Q.off_tab, Q.tab);
+  put(host, Q.off_fld, Q.fld);
   put(host, Q.off_prob, Q.prob);
+  put(host, Q.off_cols, Q.cols);
   for (int l = 0; l < kLists; ++l) put(host, Q.off_map1[l], Q.map1[l]);
   put(host, Q.off_map2, Q.map2);
   put(host, Q.off_sum, Q.sum);

@@ -17,7 +17,7 @@
 // with zeros to a multiple of 32 (rows start on 128-byte lines); 4 bytes per
 // element in both forms: float32, or split-bf16 chunks of 8 k as 16 bytes of
 // hi = bf16(x) then 16 bytes of lo = bf16(x - hi).
-//   table      [C, S][rows padded to 32][k]
+//   table      [C, S][rows padded to 32][k], in MFMA fragment order
 //   field      rows ((alpha * 2 + beta) * 2 + c) * ceil(n/2) + py,   k = px
 //   stage-1 out rows ((beta * 2 + alpha) * 2 + c) * ceil(m/2) + qx,  k = py
 // with c = 0 real, 1 imaginary.
@@ -122,23 +122,36 @@ struct FoldStage2 {
 hipError_t launch_fold_stage1(const FoldStage1& a, FoldLoad load, bool split, hipStream_t s);
 hipError_t launch_fold_stage2(const FoldStage2& a, FoldEpilogue epi, bool split, hipStream_t s);
 
-// One transform of an uneven batch, in device memory: |alpha W_y P W_x^T|^2 of
-// a complex64 field (times the linear phase cx ux + cy uy) into a float plane.
-// Its stage-1 tiles are [tile1, ...) of its width's list, its stage-2 tiles
-// [tile2, ...), each numbered column-fastest as in the uniform launches.
+// Uneven batches (split form): |alpha W_y P W_x^T|^2 of many (field, sides,
+// step, shift) instances into float planes; descriptors in device memory.
+// Stage 2: one problem per instance, whose tiles are [tile, ...) of the list,
+// numbered column-fastest.
 struct FoldProblem {
-  const uint8_t* src;
   const uint8_t* table;
-  uint8_t* mid;
+  const uint8_t* mid;
   float* out;
-  double cx, cy;
   float alpha;
-  int n, m, inverse, tile1, tile2;
+  int n, m, inverse, tile, pad_;
 };
-// A launch over the tiles of many problems: map[t] is the problem of tile t;
+// Stage 1: up to 128 / width column tiles, of any instances of one pre-folded
+// field, worked through by one workgroup per 32 rows.  cx, cy: the turns per
+// index of an instance's shift.
+struct FoldColumns {
+  const uint8_t* src;
+  int n, count;
+  int tile, step;      // the workgroup of row block r is tile + r step (+ less than step)
+  struct Tile {
+    const uint8_t* table;
+    uint8_t* mid;
+    double cx, cy;
+    int q0, m;
+  } tile_of[4];
+};
+// A launch over tile lists: map[t] is the problem or column group of tile t;
 // XCD x runs [xcd[x], xcd[x + 1]).
 struct FoldGroup {
   const FoldProblem* probs;
+  const FoldColumns* cols;
   const uint32_t* map;
   int xcd[9];
 };
@@ -147,12 +160,19 @@ struct FoldTableJob {
   double step;
   int n, m;
 };
+struct FoldFieldJob {
+  const float2* in;
+  uint8_t* out;        // fold_field_bytes(n)
+  int n, pad_;
+};
 // Output columns per stage-1 tile for an output side m (32, 64 or 128), and
-// the rows and columns of a stage-2 tile.
+// the rows and columns of the tiles.
 int fold_group_width(int m);
 constexpr int kFoldTileQy = 64, kFoldTileQx = 32, kFoldTilePy = 32;
 hipError_t launch_fold_group_tables(const FoldTableJob* jobs, int njobs, long most, hipStream_t s);
-hipError_t launch_fold_group_stage1(const FoldGroup& g, int width, bool vec, hipStream_t s);
+// `most`: the largest field's side.
+hipError_t launch_fold_group_fields(const FoldFieldJob* jobs, int njobs, int most, hipStream_t s);
+hipError_t launch_fold_group_stage1(const FoldGroup& g, int width, hipStream_t s);
 hipError_t launch_fold_group_stage2(const FoldGroup& g, hipStream_t s);
 
 // The folded pupil written to memory (FOLD_MEM rows), bit for bit what
@@ -160,7 +180,9 @@ hipError_t launch_fold_group_stage2(const FoldGroup& g, hipStream_t s);
 hipError_t launch_fold_pupil(const FoldPupil& p, const double* inv_wl, int nb, int n, bool split,
                              uint8_t* out, long stride, hipStream_t s);
 
-// True where forming the pupil in the loader beats writing it first.
-bool fold_pupil_in_loader(int m);
+// True where forming the pupil in the loader beats writing it first: the fast
+// loader takes an amplitude or OPD plane and no phase; each 128-column tile
+// forms the pupil again.
+bool fold_pupil_in_loader(const FoldPupil& p, int m);
 
 }  // namespace dlx

@@ -76,6 +76,19 @@ __device__ __forceinline__ void read_frag(u32x4_t (&f)[2], const uint8_t* tile, 
   for (int j = 0; j < 2; ++j) f[j] = *(const u32x4_t*)(r + (((2 * lk + j) ^ ((lr >> 2) & 3)) << 4));
 }
 
+// A table's pieces in the order MFMAs take them: per 32 rows and stage, 2 KiB
+// = two runs of 64 lanes x 16 bytes.  No two waves of a workgroup need the same
+// rows, so the fragments go straight from memory to registers, a kilobyte per
+// load.
+__device__ __forceinline__ long table_block(int part, int rows_pad, int kp, int row_blk) {
+  return ((long)part * (rows_pad >> 5) + row_blk) * (kp >> 4) * 2048;
+}
+__device__ __forceinline__ void load_frag(u32x4_t (&f)[2], const uint8_t* blk, int s) {
+  const uint8_t* p = blk + (long)s * 2048 + (threadIdx.x & 63) * 16;
+  f[0] = *(const u32x4_t*)p;
+  f[1] = *(const u32x4_t*)(p + 1024);
+}
+
 // acc[i][j] += sum over the stage's 16 k of a_i(m) b_j(n): lane holds column
 // n = lane % 32, register r row m = 8 (r / 4) + 4 (lane / 32) + r % 4.
 template <bool BF, int NI, int NJ>
@@ -131,6 +144,16 @@ __device__ __forceinline__ void put4(uint8_t* row, int quad, int f, const float 
   }
 }
 
+
+__device__ __forceinline__ float2 cmul(float2 a, float2 w) {
+  return make_float2(a.x * w.x - a.y * w.y, a.x * w.y + a.y * w.x);
+}
+// exp(2 pi i t), t in turns (any size): max abs error 1.3e-7.
+__device__ __forceinline__ float2 turn(double t) {
+  t -= rint(t);
+  return make_float2(__builtin_amdgcn_cosf((float)t), __builtin_amdgcn_sinf((float)t));
+}
+
 // ---------------------------------------------------------------------------
 // Field loaders.  Thread t of a workgroup takes row py = t / 8 of a 32-row
 // tile, its mirror side t % 2 and four k of the stage ((t / 2) % 4): it loads
@@ -164,15 +187,19 @@ __device__ __forceinline__ void fold_y(FoldPart& o, int beta) {
 }
 
 // The pupil loader of one thread.  VEC: n a multiple of 8 and 16-byte aligned
-// planes (float4 loads; a run of four is whole or absent).
-template <bool VEC>
+// planes (float4 loads; a run of four is whole or absent).  ANY: any of the
+// planes may be missing and there may be a phase plane, tested as they are
+// read; otherwise the amplitude or the OPD is there, no phase is, and every
+// load is unconditional (a missing plane reads the other one and is replaced
+// by its constant), so that the loads stay in flight over a stage.
+template <bool VEC, bool ANY>
 struct PupilLoad {
-  const float *opd, *amp, *phase;   // rows, or null
-  int n, kh, quad, x0i;     // x0i = n / 2: the first positive column
-  bool row_ok, tilted;
+  const float *opd, *amp, *phase;   // rows
+  int n, kh, quad, x0i;             // x0i = n / 2: the first positive column
+  bool row_ok, tilted, has_opd, has_amp, has_phase;
   double inv_wl, tx, tyY, dx, x0;
   float scale;
-  float4 op, om, ap, am;    // plus and minus runs; minus in memory order (VEC) / reversed index
+  struct Raw { float4 op, om, ap, am; };   // plus runs (k ascending), minus runs (descending)
 
   __device__ __forceinline__ void init(const FoldPupil& p, int n_, int py, int beta, int quad_,
                                        double inv) {
@@ -180,110 +207,91 @@ struct PupilLoad {
     row_ok = py < kh;
     const int yp = x0i + (row_ok ? py : 0);
     const int y = beta ? n - 1 - yp : yp;
-    opd = p.opd ? p.opd + (long)y * n : nullptr;
-    amp = p.amp ? p.amp + (long)y * n : nullptr;
-    phase = p.phase ? p.phase + (long)y * n : nullptr;
+    has_opd = p.opd != nullptr; has_amp = p.amp != nullptr; has_phase = p.phase != nullptr;
+    opd = (has_opd ? p.opd : p.amp) + (long)y * n;
+    amp = (has_amp ? p.amp : p.opd) + (long)y * n;
+    if constexpr (ANY) phase = p.phase + (long)y * n;
     inv_wl = inv; tx = p.tx; dx = p.dx; x0 = p.x0; scale = p.scale;
     tilted = p.tx != 0.0 || p.ty != 0.0;
     tyY = p.ty * pupil_coord(y, p.dx, p.x0);
   }
-  __device__ __forceinline__ void raw(int s) {
-    int p = s * kStageK + quad * 4;
-    if constexpr (VEC) {
-      p = p < kh ? p : 0;
-      const int xp = x0i + p, xm = x0i - 4 - p;
-      op = opd ? *(const float4*)(opd + xp) : make_float4(0.f, 0.f, 0.f, 0.f);
-      om = opd ? *(const float4*)(opd + xm) : make_float4(0.f, 0.f, 0.f, 0.f);
-      ap = amp ? *(const float4*)(amp + xp) : make_float4(1.f, 1.f, 1.f, 1.f);
-      am = amp ? *(const float4*)(amp + xm) : make_float4(1.f, 1.f, 1.f, 1.f);
-    } else {
-      int xp[4], xm[4];
+  __device__ __forceinline__ float4 run_up(const float* row, int p) const {
+    if constexpr (VEC) return *(const float4*)(row + x0i + (p < kh ? p : 0));
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = row[x0i + (p + e < kh ? p + e : kh - 1)];
+    return make_float4(v[0], v[1], v[2], v[3]);
+  }
+  __device__ __forceinline__ float4 run_down(const float* row, int p) const {
+    if constexpr (VEC) return *(const float4*)(row + x0i - 4 - (p < kh ? p : 0));
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = row[n - 1 - x0i - (p + e < kh ? p + e : kh - 1)];
+    return make_float4(v[3], v[2], v[1], v[0]);
+  }
+  __device__ __forceinline__ void raw(int s, Raw& r) const {
+    const int p = s * kStageK + quad * 4;
+    if (!ANY || has_opd) { r.op = run_up(opd, p); r.om = run_down(opd, p); }
+    if (!ANY || has_amp) { r.ap = run_up(amp, p); r.am = run_down(amp, p); }
+  }
+  __device__ __forceinline__ void part(int s, int beta, const Raw& r, FoldPart& o) const {
+    const int p = s * kStageK + quad * 4;
+    float vo[2][4] = {{r.op.x, r.op.y, r.op.z, r.op.w}, {r.om.w, r.om.z, r.om.y, r.om.x}};
+    float va[2][4] = {{r.ap.x, r.ap.y, r.ap.z, r.ap.w}, {r.am.w, r.am.z, r.am.y, r.am.x}};
+    float2 v[2][4];
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int pc = p + e < kh ? p + e : kh - 1;
-        xp[e] = x0i + pc;
-        xm[e] = n - 1 - xp[e];
+        vo[d][e] = has_opd ? vo[d][e] : 0.f;
+        va[d][e] = row_ok && p + e < kh ? scale * (has_amp ? va[d][e] : 1.f) : 0.f;
       }
-      op = opd ? make_float4(opd[xp[0]], opd[xp[1]], opd[xp[2]], opd[xp[3]])
-               : make_float4(0.f, 0.f, 0.f, 0.f);
-      om = opd ? make_float4(opd[xm[3]], opd[xm[2]], opd[xm[1]], opd[xm[0]])
-               : make_float4(0.f, 0.f, 0.f, 0.f);
-      ap = amp ? make_float4(amp[xp[0]], amp[xp[1]], amp[xp[2]], amp[xp[3]])
-               : make_float4(1.f, 1.f, 1.f, 1.f);
-      am = amp ? make_float4(amp[xm[3]], amp[xm[2]], amp[xm[1]], amp[xm[0]])
-               : make_float4(1.f, 1.f, 1.f, 1.f);
-    }
-  }
-  __device__ __forceinline__ void part(int s, int beta, FoldPart& o) const {
-    const int p = s * kStageK + quad * 4;
-    const float vop[4] = {op.x, op.y, op.z, op.w}, vom[4] = {om.w, om.z, om.y, om.x};
-    const float vap[4] = {ap.x, ap.y, ap.z, ap.w}, vam[4] = {am.w, am.z, am.y, am.x};
-    float2 vp[4], vm[4];
+    if (tilted || ANY) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const bool ok = row_ok && p + e < kh;
-      const int xp = x0i + p + e, xm = n - 1 - xp;
-      double tp = 0.0, tm = 0.0;
-      if (phase) {   // rare: not prefetched with the others
-        tp = ok ? (double)phase[xp] * 0.15915494309189535 : 0.0;   // 1 / (2 pi)
-        tm = ok ? (double)phase[xm] * 0.15915494309189535 : 0.0;
-      }
-      double pp = (double)vop[e], pm = (double)vom[e];
-      if (tilted) {
-        pp = pupil_path(tx, pupil_coord(xp, dx, x0), tyY, pp);
-        pm = pupil_path(tx, pupil_coord(xm, dx, x0), tyY, pm);
-      }
-      vp[e] = pupil_phasor(pp, inv_wl, tp, scale * vap[e]);
-      vm[e] = pupil_phasor(pm, inv_wl, tm, scale * vam[e]);
-      if (!ok) vp[e] = vm[e] = make_float2(0.f, 0.f);
+      for (int d = 0; d < 2; ++d)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int pc = p + e < kh ? p + e : kh - 1;
+          const int x = d ? n - 1 - x0i - pc : x0i + pc;
+          double t = 0.0, path = (double)vo[d][e];
+          if (ANY && has_phase) t = (double)phase[x] * 0.15915494309189535;   // 1 / (2 pi)
+          if (tilted) path = pupil_path(tx, pupil_coord(x, dx, x0), tyY, path);
+          v[d][e] = pupil_phasor(path, inv_wl, t, va[d][e]);
+        }
+    } else {
+#pragma unroll
+      for (int d = 0; d < 2; ++d)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[d][e] = pupil_phasor((double)vo[d][e], inv_wl, 0.0, va[d][e]);
     }
-    fold_x(vp, vm, o);
+    fold_x(v[0], v[1], o);
     fold_y(o, beta);
   }
 };
 
-// exp(2 pi i t), t in turns (any size): max abs error 1.3e-7.
-__device__ __forceinline__ float2 turn(double t) {
-  t -= rint(t);
-  return make_float2(__builtin_amdgcn_cosf((float)t), __builtin_amdgcn_sinf((float)t));
-}
-__device__ __forceinline__ float2 cmul(float2 a, float2 w) {
-  return make_float2(a.x * w.x - a.y * w.y, a.x * w.y + a.y * w.x);
-}
-
-// The complex64 field loader of one thread.  VEC as above.  The phase is
-// formed from its FP64 coefficients as the field is folded: the x factor on
-// the loaded values (its linear part is conjugate at k-), the y factor, one
-// per thread, between the x and the y fold.
+// The complex64 field loader of one thread.  VEC as above.  A phase's x factor
+// multiplies the loaded values (w: its values at k+ and k- of the four k, from
+// the stage's window in LDS); the y factor is applied to the stage's results.
 template <bool VEC>
 struct FieldLoad {
   const float2* row;
-  double c2, cx, o;     // o: the centred index of the first positive column
-  float2 ry;
   int n, kh, quad, x0i;
-  bool row_ok, phased;
-  float4 fp[2], fm[2];  // plus run (k ascending), minus run in memory order
+  bool row_ok;
+  struct Raw { float4 fp[2], fm[2]; };   // plus run (k ascending), minus run in memory order
 
-  __device__ __forceinline__ void init(const uint8_t* src, const FoldPhase& ph, int n_, int py,
-                                       int beta, int quad_) {
+  __device__ __forceinline__ void init(const uint8_t* src, int n_, int py, int beta, int quad_) {
     n = n_; kh = (n + 1) >> 1; quad = quad_; x0i = n >> 1;
     row_ok = py < kh;
-    const int pc = row_ok ? py : 0;
-    const int yp = x0i + pc;
+    const int yp = x0i + (row_ok ? py : 0);
     row = (const float2*)src + (long)(beta ? n - 1 - yp : yp) * n;
-    c2 = ph.c2; cx = ph.cx;
-    phased = ph.c2 != 0.0 || ph.cx != 0.0 || ph.cy != 0.0;
-    o = (n & 1) ? 0.0 : 0.5;
-    const double u = beta ? -((double)pc + o) : (double)pc + o;
-    ry = turn(fma(c2 * u, u, ph.cy * u));
   }
-  __device__ __forceinline__ void raw(int s) {
+  __device__ __forceinline__ void raw(int s, Raw& r) const {
     int p = s * kStageK + quad * 4;
     if constexpr (VEC) {
       p = p < kh ? p : 0;
       const float2 *a = row + x0i + p, *b = row + x0i - 4 - p;
-      fp[0] = *(const float4*)a; fp[1] = *(const float4*)(a + 2);
-      fm[0] = *(const float4*)b; fm[1] = *(const float4*)(b + 2);
+      r.fp[0] = *(const float4*)a; r.fp[1] = *(const float4*)(a + 2);
+      r.fm[0] = *(const float4*)b; r.fm[1] = *(const float4*)(b + 2);
     } else {
       float2 a[4], b[4];
 #pragma unroll
@@ -292,39 +300,31 @@ struct FieldLoad {
         a[e] = row[x0i + pc];
         b[3 - e] = row[n - 1 - x0i - pc];
       }
-      fp[0] = make_float4(a[0].x, a[0].y, a[1].x, a[1].y);
-      fp[1] = make_float4(a[2].x, a[2].y, a[3].x, a[3].y);
-      fm[0] = make_float4(b[0].x, b[0].y, b[1].x, b[1].y);
-      fm[1] = make_float4(b[2].x, b[2].y, b[3].x, b[3].y);
+      r.fp[0] = make_float4(a[0].x, a[0].y, a[1].x, a[1].y);
+      r.fp[1] = make_float4(a[2].x, a[2].y, a[3].x, a[3].y);
+      r.fm[0] = make_float4(b[0].x, b[0].y, b[1].x, b[1].y);
+      r.fm[1] = make_float4(b[2].x, b[2].y, b[3].x, b[3].y);
     }
   }
-  __device__ __forceinline__ void part(int s, int beta, FoldPart& out) const {
+  // w: [k][k+, k-] of the stage's phase
+  __device__ __forceinline__ void part(int s, int beta, const Raw& r, bool phased, const float4* w,
+                                       FoldPart& out) const {
+    const float4 *fp = r.fp, *fm = r.fm;
     const int p = s * kStageK + quad * 4;
     float2 vp[4] = {{fp[0].x, fp[0].y}, {fp[0].z, fp[0].w}, {fp[1].x, fp[1].y}, {fp[1].z, fp[1].w}};
     float2 vm[4] = {{fm[1].z, fm[1].w}, {fm[1].x, fm[1].y}, {fm[0].z, fm[0].w}, {fm[0].x, fm[0].y}};
     if (phased) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const double u = (double)(p + e) + o;
-        const float2 w = turn(fma(c2 * u, u, cx * u));
-        vp[e] = cmul(vp[e], w);
-        vm[e] = cmul(vm[e], c2 != 0.0 ? turn(fma(c2 * u, u, -cx * u)) : make_float2(w.x, -w.y));
+        const float4 t = w[quad * 4 + e];
+        vp[e] = cmul(vp[e], make_float2(t.x, t.y));
+        vm[e] = cmul(vm[e], make_float2(t.z, t.w));
       }
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       if (!(row_ok && p + e < kh)) vp[e] = vm[e] = make_float2(0.f, 0.f);
     fold_x(vp, vm, out);
-    if (phased) {
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float2 w = cmul(make_float2(out.v[a][0][e], out.v[a][1][e]), ry);
-          out.v[a][0][e] = w.x;
-          out.v[a][1][e] = w.y;
-        }
-    }
     fold_y(out, beta);
   }
 };
@@ -373,14 +373,38 @@ __device__ __forceinline__ void store_block(uint8_t* patch, const f32x16_t& acc,
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// LDS hand-over between the waves of a workgroup: waits for this wave's LDS
+// accesses only; global loads stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// Trading 32 x 32 blocks between waves through LDS: each wave writes its
+// 1024 floats, and after a barrier reads those of wave ^ XOR.
+__device__ __forceinline__ void put_block(uint8_t* x, const f32x16_t& v) {
+  float4* d = (float4*)(x + (threadIdx.x >> 6) * 4096) + (threadIdx.x & 63);
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    d[64 * q] = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+}
+template <int XOR>
+__device__ __forceinline__ void get_block(const uint8_t* x, f32x16_t& v) {
+  const float4* d = (const float4*)(x + ((threadIdx.x >> 6) ^ XOR) * 4096) + (threadIdx.x & 63);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const float4 t = d[64 * q];
+    v[4 * q] = t.x; v[4 * q + 1] = t.y; v[4 * q + 2] = t.z; v[4 * q + 3] = t.w;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Stage 1: U[(beta, alpha, c), qx][py] = sum_px T_alpha[qx][px] P[(alpha, beta, c), py][px].
 // A workgroup takes 32 rows py of all eight (alpha, beta, c) parts -- the four
 // mirrored pixels of a loaded quad feed both alphas -- and BNQ outputs qx: at
 // 128 the field is formed once per 128-column tile (256 outputs), each wave
-// holds eight 32 x 32 blocks (12 fragment reads per 24 MFMAs of a split
-// stage), and two workgroups share a CU.  Launches with fewer tiles take 64 or
-// 32 columns.
+// holds eight 32 x 32 blocks (eight fragment reads from LDS per 24 MFMAs of a
+// split stage), and two workgroups share a CU.  Launches with fewer tiles take
+// 64 or 32 columns.
 // ---------------------------------------------------------------------------
 struct Stage1Prob {
   const uint8_t* src;
@@ -389,243 +413,212 @@ struct Stage1Prob {
   int n, m;
 };
 
-template <bool BF, int LOAD, bool VEC, int BNQ>
-__device__ __forceinline__ void stage1_tile(uint8_t* lds, const Stage1Prob& g, const FoldPupil& pup,
-                                            double inv_wl, const FoldPhase& ph, int py0, int q0) {
-  constexpr int kA = 256 * kRow, kBuf = kA + 2 * BNQ * kRow;
-  constexpr int NI = BNQ >= 64 ? 4 : 2, NJ = BNQ >= 64 ? BNQ / 64 : 1;
-  const int kh = (g.n + 1) >> 1, mh = (g.m + 1) >> 1;
-  const int mhp = fold_pad(mh);
+template <int BNQ>
+struct S1 {
+  static constexpr int NI = BNQ >= 64 ? 4 : 2, NJ = BNQ >= 64 ? BNQ / 64 : 1;
+  // first A row (in (alpha, beta, c, py) order) and first column of a wave
+  __device__ static __forceinline__ int arow(int wave) {
+    return (wave >> 1) * 128 + (BNQ >= 64 ? 0 : (wave & 1) * 64);
+  }
+  __device__ static __forceinline__ int col(int wave) {
+    return BNQ >= 64 ? (wave & 1) * (BNQ / 2) : 0;
+  }
+};
+
+// The wave's blocks to the stage-1 result.
+template <bool BF, int BNQ>
+__device__ __forceinline__ void stage1_store(uint8_t* patch, f32x16_t (&acc)[S1<BNQ>::NI][S1<BNQ>::NJ],
+                                             int n, int m, uint8_t* out, int py0, int q0) {
+  const int kh = (n + 1) >> 1, mh = (m + 1) >> 1, wave = threadIdx.x >> 6;
   const long rb = 4L * fold_pad(kh);
-  const int nst = (kh + kStageK - 1) / kStageK;
-  const int wave = threadIdx.x >> 6, alpha = wave >> 1;
-  const int arow = alpha * 128 + (BNQ >= 64 ? 0 : (wave & 1) * 64);
-  const int brow = alpha * BNQ + (BNQ >= 64 ? (wave & 1) * (BNQ / 2) : 0);
-
-  f32x16_t acc[NI][NJ];
-  zero_acc(acc);
-  TileRows<2 * BNQ> bt;
-  bt.init([&](int r) {
-    const int a = r / BNQ, q = q0 + r % BNQ;
-    return g.table + (long)(a * mhp + (q < mhp ? q : mhp - 1)) * rb;
-  });
-  TileRows<256> at;
-  PupilLoad<VEC> pl;
-  FieldLoad<VEC> fl;
-  const int py = threadIdx.x >> 3, beta = threadIdx.x & 1, quad = (threadIdx.x >> 1) & 3;
-  if constexpr (LOAD == FOLD_MEM) {
-    at.init([&](int r) {
-      const int y = py0 + (r & 31);
-      return g.src + (long)((r >> 5) * kh + (y < kh ? y : kh - 1)) * rb;
-    });
-  } else if constexpr (LOAD == FOLD_PUPIL) {
-    pl.init(pup, g.n, py0 + py, beta, quad, inv_wl);
-  } else {
-    fl.init(g.src, ph, g.n, py0 + py, beta, quad);
-  }
-  auto raw = [&](int s) {
-    if constexpr (LOAD == FOLD_PUPIL) pl.raw(s);
-    if constexpr (LOAD == FOLD_FIELD) fl.raw(s);
-  };
-  auto convert = [&](int s) {
-    if constexpr (LOAD != FOLD_MEM) {
-      FoldPart o;
-      if constexpr (LOAD == FOLD_PUPIL) pl.part(s, beta, o);
-      else fl.part(s, beta, o);
-      uint8_t* buf = lds + (s & 1) * kBuf;
 #pragma unroll
-      for (int a = 0; a < 2; ++a)
+  for (int i = 0; i < S1<BNQ>::NI; ++i)
 #pragma unroll
-        for (int c = 0; c < 2; ++c)
-          put4<BF>(buf + (((a * 2 + beta) * 2 + c) * 32 + py) * kRow, quad, (py >> 2) & 3, o.v[a][c]);
-    }
-  };
-  auto issue = [&](int s) {
-    uint8_t* buf = lds + (s & 1) * kBuf;
-    if constexpr (LOAD == FOLD_MEM) at.issue(buf, s);
-    bt.issue(buf + kA, s);
-  };
-
-  raw(0);
-  issue(0);
-  convert(0);
-  for (int s = 0; s < nst; ++s) {
-    __builtin_amdgcn_s_waitcnt(0);   // this wave's part of stage s is in LDS
-    __syncthreads();                 // every wave's is; stage s - 1 has been read
-    const uint8_t* la = lds + (s & 1) * kBuf;
-    u32x4_t fa[NI][2], fb[NJ][2];
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) read_frag(fb[j], la + kA, brow + 32 * j);
-#pragma unroll
-    for (int i = 0; i < NI; ++i) read_frag(fa[i], la, arow + 32 * i);
-    const bool more = s + 1 < nst;
-    if (more) {
-      raw(s + 1);
-      issue(s + 1);
-    }
-    __builtin_amdgcn_s_setprio(1);
-    mma_stage<BF, NI, NJ>(acc, fa, fb);
-    __builtin_amdgcn_s_setprio(0);
-    if (more) convert(s + 1);
-  }
-  __syncthreads();
-  uint8_t* patch = lds + wave * kPatch;
-#pragma unroll
-  for (int i = 0; i < NI; ++i)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      // A rows run (beta, c) within alpha
-      const int bc = BNQ >= 64 ? i : (wave & 1) * 2 + i;
-      const int comp = ((bc >> 1) * 2 + alpha) * 2 + (bc & 1);
-      const int q = q0 + (brow - alpha * BNQ) + 32 * j;
+    for (int j = 0; j < S1<BNQ>::NJ; ++j) {
+      const int bc = BNQ >= 64 ? i : (wave & 1) * 2 + i;   // (beta, c)
+      const int comp = ((bc >> 1) * 2 + (wave >> 1)) * 2 + (bc & 1);
+      const int q = q0 + S1<BNQ>::col(wave) + 32 * j;
       if (q < mh)
-        store_block<BF>(patch, acc[i][j], kh - py0, g.out + (long)(comp * mh + q) * rb + 4L * py0,
-                        rb, mh - q);
+        store_block<BF>(patch, acc[i][j], kh - py0, out + (long)(comp * mh + q) * rb + 4L * py0, rb,
+                        mh - q);
     }
 }
 
+// The y factor of a field's phase, applied to the wave's blocks: with
+// exp(i f) at row y+ (its linear part conjugate at y-), the even and odd parts
+// mix as e' = e cos f + i o sin f, o' = o cos f + i e sin f.  `lds`: 32 KiB
+// free of readers (32-column tiles, whose waves hold one beta each, trade).
+template <int BNQ>
+__device__ __forceinline__ void y_phase(uint8_t* lds, f32x16_t (&acc)[S1<BNQ>::NI][S1<BNQ>::NJ],
+                                        double c2, double cy, int n, int py0) {
+  const int lk = (threadIdx.x >> 5) & 1;
+  const double on = (n & 1) ? 0.0 : 0.5;
+  f32x16_t other[2];
+  if constexpr (BNQ == 32) {
+    put_block(lds, acc[0][0]);
+    put_block(lds + 16384, acc[1][0]);
+    lds_barrier();
+    get_block<1>(lds, other[0]);
+    get_block<1>(lds + 16384, other[1]);
+    lds_barrier();
+  }
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const double u = (double)(py0 + 8 * (r >> 2) + 4 * lk + (r & 3)) + on;
+    float2 w = turn(cy * u), q = make_float2(1.f, 0.f);
+    if (c2 != 0.0) q = turn(c2 * u * u);
+    if constexpr (BNQ == 32) {
+      const float2 v = cmul(make_float2(acc[0][0][r] * w.x - other[1][r] * w.y,
+                                        acc[1][0][r] * w.x + other[0][r] * w.y), q);
+      acc[0][0][r] = v.x;
+      acc[1][0][r] = v.y;
+    } else {
+#pragma unroll
+      for (int j = 0; j < S1<BNQ>::NJ; ++j) {
+        const float er = acc[0][j][r], ei = acc[1][j][r], od = acc[2][j][r], oi = acc[3][j][r];
+        const float2 e = cmul(make_float2(er * w.x - oi * w.y, ei * w.x + od * w.y), q);
+        const float2 o = cmul(make_float2(od * w.x - ei * w.y, oi * w.x + er * w.y), q);
+        acc[0][j][r] = e.x; acc[1][j][r] = e.y; acc[2][j][r] = o.x; acc[3][j][r] = o.y;
+      }
+    }
+  }
+}
+
+constexpr int kPupilAny = 3;   // FOLD_PUPIL through the loader that tests for every plane
+
+// Fields formed by the loader: the next stage's parts are formed after this
+// stage's products are issued, from values loaded two stages ahead.
 template <bool BF, int LOAD, bool VEC, int BNQ>
 __global__ void __launch_bounds__(kThreads, 2)
 fold_stage1_kernel(FoldStage1 a) {
-  constexpr int kBuf = (256 + 2 * BNQ) * kRow;
+  using S = S1<BNQ>;
+  constexpr int NI = S::NI, NJ = S::NJ, kBuf = 256 * kRow;
   __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * kBuf];
-  const int tq = (fold_half(a.m) + BNQ - 1) / BNQ, tp = (fold_half(a.n) + 31) / 32;
+  __shared__ float4 win[2][kStageK];   // the x phase of a stage's k, at k+ and k-
+  const int kh = fold_half(a.n), mh = fold_half(a.m), mhp = fold_pad(mh), kp = fold_pad(kh);
+  const int tq = (mh + BNQ - 1) / BNQ, tp = (kh + 31) / 32;
   const int id = xcd_order(blockIdx.x, tq * tp * a.batch);
   const int b = id / (tq * tp), t = id - b * (tq * tp);
-  Stage1Prob g;
-  g.src = a.src ? a.src + (long)b * a.src_stride : nullptr;
-  g.table = a.table + (long)b * a.table_stride;
-  g.out = a.out + (long)b * a.out_stride;
-  g.n = a.n;
-  g.m = a.m;
-  stage1_tile<BF, LOAD, VEC, BNQ>(lds, g, a.pupil, a.inv_wl[b], a.phase[b], (t / tq) * 32,
-                                  (t % tq) * BNQ);
+  const int py0 = (t / tq) * 32, q0 = (t % tq) * BNQ;
+  const int nst = (kh + kStageK - 1) / kStageK;
+  const int wave = threadIdx.x >> 6;
+
+  f32x16_t acc[NI][NJ];
+  zero_acc(acc);
+  const uint8_t* tab[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const int blk = (q0 + S::col(wave)) / 32 + j, last = (mhp >> 5) - 1;
+    tab[j] = a.table + (long)b * a.table_stride +
+             table_block(wave >> 1, mhp, kp, blk < last ? blk : last);
+  }
+  const int py = threadIdx.x >> 3, beta = threadIdx.x & 1, quad = (threadIdx.x >> 1) & 3;
+  std::conditional_t<LOAD == FOLD_FIELD, FieldLoad<VEC>, PupilLoad<VEC, LOAD == kPupilAny>> ld;
+  FoldPhase ph{};
+  bool phased = false;
+  if constexpr (LOAD != FOLD_FIELD) {
+    ld.init(a.pupil, a.n, py0 + py, beta, quad, a.inv_wl[b]);
+  } else {
+    ld.init(a.src + (long)b * a.src_stride, a.n, py0 + py, beta, quad);
+    ph = a.phase[b];
+    phased = ph.c2 != 0.0 || ph.cx != 0.0 || ph.cy != 0.0;
+  }
+  typename decltype(ld)::Raw raw[2];
+  const double on = (a.n & 1) ? 0.0 : 0.5;
+  auto window = [&](int s) {   // formed two stages ahead of its use's products
+    if constexpr (LOAD == FOLD_FIELD) {
+      if (phased && threadIdx.x < kStageK) {
+        const double u = (double)(s * kStageK + (int)threadIdx.x) + on, q = ph.c2 * u * u;
+        const float2 wp = turn(fma(ph.cx, u, q)), wm = turn(fma(-ph.cx, u, q));
+        win[s & 1][threadIdx.x] = make_float4(wp.x, wp.y, wm.x, wm.y);
+      }
+    }
+  };
+  auto convert = [&](int s, const typename decltype(ld)::Raw& r) __attribute__((always_inline)) {
+    FoldPart o;
+    if constexpr (LOAD != FOLD_FIELD) ld.part(s, beta, r, o);
+    else ld.part(s, beta, r, phased, win[s & 1], o);
+    uint8_t* buf = lds + (s & 1) * kBuf;
+#pragma unroll
+    for (int al = 0; al < 2; ++al)
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+        put4<BF>(buf + (((al * 2 + beta) * 2 + c) * 32 + py) * kRow, quad, (py >> 2) & 3, o.v[al][c]);
+  };
+  u32x4_t fb[2][NJ][2];
+  auto load_tab = [&](auto J, int s) __attribute__((always_inline)) {
+    const int sc = s < nst ? s : nst - 1;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) load_frag(fb[decltype(J)::value][j], tab[j], sc);
+  };
+  // one stage: J = s & 1
+  auto step = [&](auto J, int s) __attribute__((always_inline)) {
+    constexpr int j0 = decltype(J)::value;
+    lds_barrier();   // stage s is in LDS, stage s - 1 has been read
+    const uint8_t* la = lds + j0 * kBuf;
+    u32x4_t fa[NI][2];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) read_frag(fa[i], la, S::arow(wave) + 32 * i);
+    load_tab(std::integral_constant<int, 1 - j0>{}, s + 1);
+    ld.raw(s + 2, raw[j0]);
+    window(s + 2);
+    __builtin_amdgcn_s_setprio(1);
+    mma_stage<BF, NI, NJ>(acc, fa, fb[j0]);
+    __builtin_amdgcn_s_setprio(0);
+    if (s + 1 < nst) convert(s + 1, raw[1 - j0]);
+  };
+  load_tab(std::integral_constant<int, 0>{}, 0);
+  ld.raw(0, raw[0]);
+  ld.raw(1, raw[1]);
+  window(0);
+  window(1);
+  if constexpr (LOAD == FOLD_FIELD) lds_barrier();
+  convert(0, raw[0]);
+  int s = 0;
+  for (; s + 1 < nst; s += 2) {   // whole pairs: no path of the loop skips a load
+    step(std::integral_constant<int, 0>{}, s);
+    step(std::integral_constant<int, 1>{}, s + 1);
+  }
+  if (s < nst) step(std::integral_constant<int, 0>{}, s);
+  lds_barrier();
+  if constexpr (LOAD == FOLD_FIELD)
+    if (phased) y_phase<BNQ>(lds, acc, ph.c2, ph.cy, a.n, py0);
+  stage1_store<BF, BNQ>(lds + wave * kPatch, acc, a.n, a.m, a.out + (long)b * a.out_stride, py0, q0);
 }
 
 // ---------------------------------------------------------------------------
-// Stage 2: F[(beta, alpha, c)][qy][qx] = sum_py T_beta[qy][py] U[(beta, alpha, c), qx][py],
-// then the four mirrored outputs.  A workgroup takes BQ rows qy and 32 columns
-// qx of all eight parts; wave (beta, h) holds the four (alpha, c) blocks of BQ / 2
-// rows, combines along x in registers, and trades one sign of x with the wave
-// of the other beta through LDS, after which wave beta holds both signs of y at
-// its sign of x.  With NB stage buffers the loads run NB - 1 stages ahead
-// (counted vmcnt waits; one LDS object per buffer, so that the compiler's own
-// wait before a fragment read covers that buffer's loads alone).
+// A ring of NB stage buffers (16 KiB: 256 folded rows) filled straight from
+// memory NB - 1 stages ahead, with the table fragments of the same stage in
+// registers: the loop of the kernels whose folded operand is in memory.
+// Counted vmcnt waits; one LDS object per buffer, so that the compiler's own
+// wait before a fragment read covers that buffer's loads alone.
+// mma(buffer, fragments) issues one stage's products.
 // ---------------------------------------------------------------------------
 template <int N>
 using IC = std::integral_constant<int, N>;
 
-// The value the partner wave (wave ^ 2) sent: blocks of 1024 floats.
-__device__ __forceinline__ void put_block(uint8_t* x, const f32x16_t& v) {
-  float4* d = (float4*)(x + (threadIdx.x >> 6) * 4096) + (threadIdx.x & 63);
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-    d[64 * q] = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
-}
-__device__ __forceinline__ void get_block(const uint8_t* x, f32x16_t& v) {
-  const float4* d = (const float4*)(x + ((threadIdx.x >> 6) ^ 2) * 4096) + (threadIdx.x & 63);
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const float4 t = d[64 * q];
-    v[4 * q] = t.x; v[4 * q + 1] = t.y; v[4 * q + 2] = t.z; v[4 * q + 3] = t.w;
-  }
-}
-
-struct Stage2Prob {
-  const uint8_t *table, *mid;
-  void* out;
-  float* out2;
-  const float* G;
-  FoldPupil pupil;
-  FoldPhase phase;
-  double inv_wl;
-  float alpha;
-  int n, m, inverse;
-};
-
-template <bool BF, int EPI, int BQ, int NB>
-__device__ __forceinline__ void stage2_tile(const Stage2Prob& a, int qy0, int qx0) {
-  constexpr int kA = 2 * BQ * kRow, kBuf = kA + 256 * kRow;
-  constexpr int NI = BQ / 64;
-  constexpr int kLoads = (2 * BQ + 256) / 64;   // global_load_lds per wave and stage
-  constexpr bool SWAP = EPI == FOLD_VJP;        // lanes run along qy, registers along qx
-  __shared__ __attribute__((aligned(1024))) uint8_t buf0[kBuf], buf1[kBuf];
-  __shared__ __attribute__((aligned(1024))) uint8_t buf2[NB > 2 ? kBuf : 16];
-  __shared__ __attribute__((aligned(1024))) uint8_t buf3[NB > 3 ? kBuf : 16];
-  auto buf = [&](auto J) __attribute__((always_inline)) -> uint8_t* {
-    if constexpr (decltype(J)::value == 0) return buf0;
-    else if constexpr (decltype(J)::value == 1) return buf1;
-    else if constexpr (decltype(J)::value == 2) return buf2;
-    else return buf3;
-  };
-
-  const int kh = fold_half(a.n), mh = fold_half(a.m), mhp = fold_pad(mh);
-  const long rb = 4L * fold_pad(kh);
-  const uint8_t *table = a.table, *mid = a.mid;
-  const int nst = (kh + kStageK - 1) / kStageK;
-  const int lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
-  const int wave = threadIdx.x >> 6, beta = wave >> 1, h = wave & 1;
-
-  TileRows<2 * BQ> at;
-  at.init([&](int r) {
-    const int bt = r / BQ, q = qy0 + r % BQ;
-    return table + (long)(bt * mhp + (q < mhp ? q : mhp - 1)) * rb;
-  });
-  TileRows<256> bt;
-  bt.init([&](int r) {
-    const int q = qx0 + (r & 31);
-    return mid + (long)((r >> 5) * mh + (q < mh ? q : mh - 1)) * rb;
-  });
-  f32x16_t acc[NI][4];
-  zero_acc(acc);
-
+template <int NB, int NT, typename BufF, typename IssueF, typename MmaF>
+__device__ __forceinline__ void ring_loop(int nst, const uint8_t* const (&tab)[NT], BufF buf,
+                                          IssueF issue_rows, MmaF mma) {
+  constexpr int kPer = 2 * NT + 4;   // loads per wave and stage
+  u32x4_t tf[NB][NT][2];
   auto issue = [&](auto J, int s) __attribute__((always_inline)) {
-    at.issue(buf(J), s);
-    bt.issue(buf(J) + kA, s);
+#pragma unroll
+    for (int i = 0; i < NT; ++i) load_frag(tf[decltype(J)::value][i], tab[i], s);
+    issue_rows(J, s);
   };
   // FULL: every stage the step waits past and issues exists (no branches, so
   // the compiler's counts stay exact across the loop's back edge)
   auto step = [&](auto J, auto FULL, int s) __attribute__((always_inline)) {
     constexpr bool full = decltype(FULL)::value;
     if (full || s + NB - 2 < nst)
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kLoads * (NB - 2)) : "memory");
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kPer * (NB - 2)) : "memory");
     else
       asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    const uint8_t* la = buf(J);
-    u32x4_t fa[NI][2], fb[4][2];
-#pragma unroll
-    for (int i = 0; i < NI; ++i) read_frag(fa[i], la, beta * BQ + h * (BQ / 2) + 32 * i);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) read_frag(fb[j], la + kA, (beta * 4 + j) * 32);
-    if (full || s + NB - 1 < nst) issue(IC<(decltype(J)::value + NB - 1) % NB>{}, s + NB - 1);
-    __builtin_amdgcn_s_setprio(1);
-    if constexpr (!SWAP) {
-      mma_stage<BF, NI, 4>(acc, fa, fb);
-    } else {
-      // the same sums with the operands' roles exchanged
-      if constexpr (BF) {
-#pragma unroll
-        for (int t3 = 0; t3 < 3; ++t3)
-#pragma unroll
-          for (int i = 0; i < NI; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                  __builtin_bit_cast(bf16x8_t, fb[j][t3 == 1 ? 1 : 0]),
-                  __builtin_bit_cast(bf16x8_t, fa[i][t3 == 0 ? 1 : 0]), acc[i][j], 0, 0, 0);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-#pragma unroll
-          for (int i = 0; i < NI; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-                  __uint_as_float(fb[j][e >> 2][e & 3]), __uint_as_float(fa[i][e >> 2][e & 3]),
-                  acc[i][j], 0, 0, 0);
-      }
-    }
-    __builtin_amdgcn_s_setprio(0);
+    auto next = [&]() __attribute__((always_inline)) {
+      if (full || s + NB - 1 < nst) issue(IC<(decltype(J)::value + NB - 1) % NB>{}, s + NB - 1);
+    };
+    mma(buf(J), tf[decltype(J)::value], next);
   };
   issue(IC<0>{}, 0);
   if constexpr (NB > 2) { if (nst > 1) issue(IC<1>{}, 1); }
@@ -643,6 +636,122 @@ __device__ __forceinline__ void stage2_tile(const Stage2Prob& a, int qy0, int qx
     if constexpr (NB > 2) { if (s + 2 < nst) step(IC<2>{}, std::false_type{}, s + 2); }
     if constexpr (NB > 3) { if (s + 3 < nst) step(IC<3>{}, std::false_type{}, s + 3); }
   }
+}
+
+#define DLX_RING_BUFFERS(NB)                                                              \
+  __shared__ __attribute__((aligned(1024))) uint8_t buf0[256 * kRow], buf1[256 * kRow];   \
+  __shared__ __attribute__((aligned(1024))) uint8_t buf2[NB > 2 ? 256 * kRow : 16];       \
+  __shared__ __attribute__((aligned(1024))) uint8_t buf3[NB > 3 ? 256 * kRow : 16];       \
+  auto buf = [&](auto J) __attribute__((always_inline)) -> uint8_t* {                     \
+    if constexpr (decltype(J)::value == 0) return buf0;                                   \
+    else if constexpr (decltype(J)::value == 1) return buf1;                              \
+    else if constexpr (decltype(J)::value == 2) return buf2;                              \
+    else return buf3;                                                                     \
+  }
+
+// Stage 1 of a folded field in memory.
+template <bool BF, int BNQ, int NB>
+__global__ void __launch_bounds__(kThreads, 2)
+fold_stage1_mem_kernel(FoldStage1 a) {
+  using S = S1<BNQ>;
+  constexpr int NI = S::NI, NJ = S::NJ;
+  DLX_RING_BUFFERS(NB);
+  const int kh = fold_half(a.n), mh = fold_half(a.m), mhp = fold_pad(mh), kp = fold_pad(kh);
+  const int tq = (mh + BNQ - 1) / BNQ, tp = (kh + 31) / 32;
+  const int id = xcd_order(blockIdx.x, tq * tp * a.batch);
+  const int b = id / (tq * tp), t = id - b * (tq * tp);
+  const int py0 = (t / tq) * 32, q0 = (t % tq) * BNQ;
+  const int wave = threadIdx.x >> 6;
+  const uint8_t* tab[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const int blk = (q0 + S::col(wave)) / 32 + j, last = (mhp >> 5) - 1;
+    tab[j] = a.table + (long)b * a.table_stride +
+             table_block(wave >> 1, mhp, kp, blk < last ? blk : last);
+  }
+  const uint8_t* src = a.src + (long)b * a.src_stride;
+  TileRows<256> at;
+  at.init([&](int r) {
+    const int y = py0 + (r & 31);
+    return src + (long)((r >> 5) * kh + (y < kh ? y : kh - 1)) * 4 * kp;
+  });
+  f32x16_t acc[NI][NJ];
+  zero_acc(acc);
+  ring_loop<NB, NJ>(
+      (kh + kStageK - 1) / kStageK, tab, buf,
+      [&](auto J, int s) __attribute__((always_inline)) { at.issue(buf(J), s); },
+      [&](const uint8_t* la, const u32x4_t (&fb)[NJ][2], auto next) __attribute__((always_inline)) {
+        u32x4_t fa[NI][2];
+#pragma unroll
+        for (int i = 0; i < NI; ++i) read_frag(fa[i], la, S::arow(wave) + 32 * i);
+        next();
+        __builtin_amdgcn_s_setprio(1);
+        mma_stage<BF, NI, NJ>(acc, fa, fb);
+        __builtin_amdgcn_s_setprio(0);
+      });
+  __syncthreads();
+  stage1_store<BF, BNQ>((wave & 1 ? buf1 : buf0) + (wave >> 1) * kPatch, acc, a.n, a.m,
+                        a.out + (long)b * a.out_stride, py0, q0);
+}
+// ---------------------------------------------------------------------------
+// Stage 2: F[(beta, alpha, c)][qy][qx] = sum_py T_beta[qy][py] U[(beta, alpha, c), qx][py],
+// then the four mirrored outputs.  A workgroup takes BQ rows qy and 32 columns
+// qx of all eight parts; wave (beta, h) holds the four (alpha, c) blocks of BQ / 2
+// rows, combines along x in registers, and trades one sign of x with the wave
+// of the other beta through LDS, after which wave beta holds both signs of y at
+// its sign of x.
+// ---------------------------------------------------------------------------
+struct Stage2Prob {
+  const uint8_t *table, *mid;
+  void* out;
+  float* out2;
+  const float* G;
+  FoldPupil pupil;
+  FoldPhase phase;
+  double inv_wl;
+  float alpha;
+  int n, m, inverse;
+};
+
+template <bool BF, int EPI, int BQ, int NB>
+__device__ __forceinline__ void stage2_tile(const Stage2Prob& a, int qy0, int qx0) {
+  constexpr int NI = BQ / 64;
+  constexpr bool SWAP = EPI == FOLD_VJP;        // lanes run along qy, registers along qx
+  DLX_RING_BUFFERS(NB);
+  const int kh = fold_half(a.n), mh = fold_half(a.m), mhp = fold_pad(mh), kp = fold_pad(kh);
+  const int lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
+  const int wave = threadIdx.x >> 6, beta = wave >> 1, h = wave & 1;
+  const uint8_t* tab[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int blk = (qy0 + h * (BQ / 2)) / 32 + i, last = (mhp >> 5) - 1;
+    tab[i] = a.table + table_block(beta, mhp, kp, blk < last ? blk : last);
+  }
+  TileRows<256> bt;
+  bt.init([&](int r) {
+    const int q = qx0 + (r & 31);
+    return a.mid + (long)((r >> 5) * mh + (q < mh ? q : mh - 1)) * 4 * kp;
+  });
+  f32x16_t acc[NI][4];
+  zero_acc(acc);
+  ring_loop<NB, NI>(
+      (kh + kStageK - 1) / kStageK, tab, buf,
+      [&](auto J, int s) __attribute__((always_inline)) { bt.issue(buf(J), s); },
+      [&](const uint8_t* lb, const u32x4_t (&fa)[NI][2], auto next) __attribute__((always_inline)) {
+        u32x4_t fb[4][2];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) read_frag(fb[j], lb, (beta * 4 + j) * 32);
+        next();
+        __builtin_amdgcn_s_setprio(1);
+        if constexpr (!SWAP) {
+          mma_stage<BF, NI, 4>(acc, fa, fb);
+        } else {
+          static_assert(NI == 1, "the exchanged roles accumulate one row block");
+          f32x16_t(&sw)[4][1] = reinterpret_cast<f32x16_t(&)[4][1]>(acc);
+          mma_stage<BF, 4, 1>(sw, fb, fa);
+        }
+        __builtin_amdgcn_s_setprio(0);
+      });
 
   // ---- the mirrored outputs ----
   const float sg = a.inverse ? -1.f : 1.f;
@@ -673,8 +782,8 @@ __device__ __forceinline__ void stage2_tile(const Stage2Prob& a, int qy0, int qx
     put_block(buf0, sr);
     put_block(buf1, si);
     __syncthreads();
-    get_block(buf0, sr);
-    get_block(buf1, si);
+    get_block<2>(buf0, sr);
+    get_block<2>(buf1, si);
     // y+: sum; y-: difference (the beta = 0 value first)
     const float d = beta ? -1.f : 1.f;
     const int q0 = qy0 + h * (BQ / 2) + 32 * i;
@@ -755,8 +864,8 @@ __device__ __forceinline__ void stage2_tile(const Stage2Prob& a, int qy0, int qx
       put_block(buf0, sr);
       put_block(buf1, si);
       __syncthreads();
-      get_block(buf0, sr);
-      get_block(buf1, si);
+      get_block<2>(buf0, sr);
+      get_block<2>(buf1, si);
       __syncthreads();
       uint8_t* patch = buf0 + wave * kPatch;
       uint8_t* out = (uint8_t*)a.out;
@@ -779,7 +888,7 @@ __device__ __forceinline__ void stage2_tile(const Stage2Prob& a, int qy0, int qx
 }
 
 template <bool BF, int EPI, int BQ, int NB>
-__global__ void __launch_bounds__(kThreads, NB * (2 * BQ + 256) * kRow <= 80 * 1024 ? 2 : 1)
+__global__ void __launch_bounds__(kThreads, 2)
 fold_stage2_kernel(FoldStage2 a) {
   const int mh = fold_half(a.m), tx = (mh + 31) / 32, ty = (mh + BQ - 1) / BQ;
   const int id = xcd_order(blockIdx.x, tx * ty * a.batch);
@@ -811,23 +920,161 @@ __device__ __forceinline__ int group_tile(const FoldGroup& l) {
   return t < l.xcd[x + 1] ? t : -1;
 }
 
-template <bool VEC, int BNQ>
+// Stage 1 of an uneven batch, from pre-folded float fields (rows (beta, py) of
+// [px][e re, e im, o re, o im], fold_group_fields): a workgroup takes 32 rows
+// py of one field and L = 128 / BNQ tiles of BNQ columns, each of any instance
+// of that field.  The values loaded for a stage serve all L: per tile the
+// instance's x shift rotates the even and odd parts (e' = e cos f + i o sin f,
+// o' = o cos f + i e sin f; cos and sin of the stage's k from a window in LDS),
+// the parts are split, and the tile's products run; the y shift is applied to
+// the results.
+template <int BNQ>
 __global__ void __launch_bounds__(kThreads, 2)
-fold_group_stage1_kernel(FoldGroup l) {
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * (256 + 2 * BNQ) * kRow];
-  const int t = group_tile(l);
+fold_group_stage1_kernel(FoldGroup g) {
+  using S = S1<BNQ>;
+  constexpr int NI = S::NI, NJ = S::NJ, L = 128 / BNQ, kBuf = 256 * kRow;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * kBuf];
+  __shared__ float2 win[2][L][kStageK];
+  const int t = group_tile(g);
   if (t < 0) return;
-  const FoldProblem& p = l.probs[l.map[t]];
-  Stage1Prob g;
-  g.src = p.src;
-  g.table = p.table;
-  g.out = p.mid;
-  g.n = p.n;
-  g.m = p.m;
-  const FoldPhase ph = {0.0, p.cx, p.cy, 0.0};
-  const int tq = (fold_half(g.m) + BNQ - 1) / BNQ, local = t - p.tile1;
-  stage1_tile<true, FOLD_FIELD, VEC, BNQ>(lds, g, FoldPupil{}, 0.0, ph, (local / tq) * 32,
-                                          (local % tq) * BNQ);
+  const FoldColumns& cg = g.cols[g.map[t]];
+  const int n = cg.n, kh = fold_half(n), kp = fold_pad(kh), count = cg.count;
+  const int py0 = (t - cg.tile) / cg.step * 32;
+  const int nst = (kh + kStageK - 1) / kStageK, wave = threadIdx.x >> 6;
+  const int quad = threadIdx.x & 3, beta = (threadIdx.x >> 2) & 1, py = threadIdx.x >> 3;
+  const float4* row;
+  {
+    const int y = py0 + py < kh ? py0 + py : kh - 1;
+    row = (const float4*)cg.src + ((long)beta * kh + y) * kp + quad * 4;
+  }
+  const uint8_t* tab[L][NJ];
+#pragma unroll
+  for (int l = 0; l < L; ++l) {
+    const FoldColumns::Tile& c = cg.tile_of[l < count ? l : 0];
+    const int mhp = fold_pad(fold_half(c.m)), last = (mhp >> 5) - 1;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int blk = (c.q0 + S::col(wave)) / 32 + j;
+      tab[l][j] = c.table + table_block(wave >> 1, mhp, kp, blk < last ? blk : last);
+    }
+  }
+  f32x16_t acc[L][NI][NJ];
+#pragma unroll
+  for (int l = 0; l < L; ++l) zero_acc(acc[l]);
+  const double on = (n & 1) ? 0.0 : 0.5;
+  const int wl = threadIdx.x / kStageK, we = threadIdx.x % kStageK;   // window entry of a thread
+  const double wcx = wl < L ? cg.tile_of[wl < count ? wl : 0].cx : 0.0;
+  auto window = [&](int s) {
+    if (wl < L) win[s & 1][wl][we] = turn(wcx * ((double)(s * kStageK + we) + on));
+  };
+  float4 raw[2][4];
+  auto load_raw = [&](auto J, int s) __attribute__((always_inline)) {
+    const int sc = s < nst ? s : nst - 1;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) raw[decltype(J)::value][e] = row[sc * kStageK + e];
+  };
+  auto convert = [&](int s, int l, int slot, const float4 (&r)[4]) __attribute__((always_inline)) {
+    float v[2][2][4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float2 w = win[s & 1][l][quad * 4 + e];
+      v[0][0][e] = r[e].x * w.x - r[e].w * w.y;
+      v[0][1][e] = r[e].y * w.x + r[e].z * w.y;
+      v[1][0][e] = r[e].z * w.x - r[e].y * w.y;
+      v[1][1][e] = r[e].w * w.x + r[e].x * w.y;
+    }
+    uint8_t* buf = lds + slot * kBuf;
+#pragma unroll
+    for (int al = 0; al < 2; ++al)
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+        put4<true>(buf + (((al * 2 + beta) * 2 + c) * 32 + py) * kRow, quad, (py >> 2) & 3, v[al][c]);
+  };
+  u32x4_t fb[2][NJ][2];
+  auto load_tab = [&](auto J, const uint8_t* const (&tb)[NJ], int s) __attribute__((always_inline)) {
+    const int sc = s < nst ? s : nst - 1;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) load_frag(fb[decltype(J)::value][j], tb[j], sc);
+  };
+  // step (s, l): P = s & 1; slot and fragment set (s L + l) & 1
+  auto step = [&](auto P, auto LL, int s) __attribute__((always_inline)) {
+    constexpr int p = decltype(P)::value, l = decltype(LL)::value;
+    constexpr int k = (p * L + l) & 1, ln = (l + 1) % L;
+    lds_barrier();
+    const int sn = l + 1 < L ? s : s + 1;   // the next step's stage
+    u32x4_t fa[NI][2];
+    if (l < count) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) read_frag(fa[i], lds + k * kBuf, S::arow(wave) + 32 * i);
+    }
+    load_tab(IC<1 - k>{}, tab[ln], sn);
+    if constexpr (l == 0) {
+      // L = 1 converts the next stage from raw[1 - p] in this step: two ahead
+      if constexpr (L == 1) load_raw(P, s + 2);
+      else load_raw(IC<1 - p>{}, s + 1);
+      // the window of stage s is still read by this stage's converts if L > 1
+      window(L == 1 ? s + 2 : s + 1);
+    }
+    if (l < count) {
+      __builtin_amdgcn_s_setprio(1);
+      mma_stage<true, NI, NJ>(acc[l], fa, fb[k]);
+      __builtin_amdgcn_s_setprio(0);
+    }
+    if (sn < nst && ln < count) {
+      if constexpr (l + 1 < L) convert(sn, ln, 1 - k, raw[p]);
+      else convert(sn, ln, 1 - k, raw[1 - p]);
+    }
+  };
+  auto stage = [&](auto P, int s) __attribute__((always_inline)) {
+    step(P, IC<0>{}, s);
+    if constexpr (L > 1) step(P, IC<1>{}, s);
+    if constexpr (L > 2) { step(P, IC<2>{}, s); step(P, IC<3>{}, s); }
+  };
+  load_tab(IC<0>{}, tab[0], 0);
+  load_raw(IC<0>{}, 0);
+  if constexpr (L == 1) load_raw(IC<1>{}, 1);
+  window(0);
+  if constexpr (L == 1) window(1);
+  lds_barrier();
+  convert(0, 0, 0, raw[0]);
+  int s = 0;
+  for (; s + 1 < nst; s += 2) {
+    stage(IC<0>{}, s);
+    stage(IC<1>{}, s + 1);
+  }
+  if (s < nst) stage(IC<0>{}, s);
+#pragma unroll
+  for (int l = 0; l < L; ++l) {
+    if (l >= count) break;
+    const FoldColumns::Tile& c = cg.tile_of[l];
+    lds_barrier();
+    if (c.cy != 0.0) y_phase<BNQ>(lds, acc[l], 0.0, c.cy, n, py0);
+    lds_barrier();
+    stage1_store<true, BNQ>(lds + wave * kPatch, acc[l], n, c.m, c.mid, py0, c.q0);
+  }
+}
+
+// A distinct field of the batch folded along both axes, once for all its
+// instances: float rows (beta, py) of [px][e re, e im, o re, o im].
+__global__ void __launch_bounds__(256)
+fold_group_field_kernel(const FoldFieldJob* __restrict__ jobs) {
+  const FoldFieldJob j = jobs[blockIdx.z];
+  const int n = j.n, kh = fold_half(n), kp = fold_pad(kh);
+  const int py = blockIdx.y, px = blockIdx.x * blockDim.x + threadIdx.x;
+  if (py >= kh || px >= kp) return;
+  float4 e = make_float4(0.f, 0.f, 0.f, 0.f), o = e;
+  if (px < kh) {
+    const int xp = (n >> 1) + px, xm = n - 1 - xp, yp = (n >> 1) + py, ym = n - 1 - yp;
+    const float2 *rp = j.in + (long)yp * n, *rm = j.in + (long)ym * n;
+    const float2 a = rp[xp], b = rp[xm], c = rm[xp], d = rm[xm];
+    const float2 pe = {a.x + b.x, a.y + b.y}, po = {a.x - b.x, a.y - b.y};
+    const float2 me = {c.x + d.x, c.y + d.y}, mo = {c.x - d.x, c.y - d.y};
+    e = make_float4(pe.x + me.x, pe.y + me.y, po.x + mo.x, po.y + mo.y);
+    o = make_float4(pe.x - me.x, pe.y - me.y, po.x - mo.x, po.y - mo.y);
+  }
+  float4* out = (float4*)j.out + (long)py * kp + px;
+  out[0] = e;
+  out[(long)kh * kp] = o;
 }
 
 __global__ void __launch_bounds__(kThreads, 2)
@@ -843,8 +1090,8 @@ fold_group_stage2_kernel(FoldGroup l) {
   g.n = p.n;
   g.m = p.m;
   g.inverse = p.inverse;
-  const int tx = (fold_half(g.m) + 31) / 32, local = t - p.tile2;
-  stage2_tile<true, FOLD_INTENSITY, kFoldTileQy, 3>(g, (local / tx) * kFoldTileQy, (local % tx) * 32);
+  const int tx = (fold_half(g.m) + 31) / 32, local = t - p.tile;
+  stage2_tile<true, FOLD_INTENSITY, kFoldTileQy, 4>(g, (local / tx) * kFoldTileQy, (local % tx) * 32);
 }
 
 // ---------------------------------------------------------------------------
@@ -880,10 +1127,24 @@ __device__ __forceinline__ void table_entry(int t, double step, int n, int m,
       if (p == 0 && (n & 1)) c[e] *= 0.5f;   // the centre, folded onto itself
     }
   }
-  const long rb = 4L * kp;
-  uint8_t* cr = out + (long)q * rb + (k0 >> 4) * kRow;
-  put4<BF>(cr, (k0 >> 2) & 3, 0, c);
-  put4<BF>(cr + (long)mhp * rb, (k0 >> 2) & 3, 0, s);
+  // the quad's place in its stage: lane half (quad / 2), and, split, the run of
+  // hi and of lo pieces with 8 bytes each; float32, one run of 16 bytes
+  const int quad = (k0 >> 2) & 3;
+#pragma unroll
+  for (int part = 0; part < 2; ++part) {
+    const float(&v)[4] = part ? s : c;
+    uint8_t* d = out + table_block(part, mhp, kp, q >> 5) + (long)(k0 >> 4) * 2048 +
+                 ((quad >> 1) * 32 + (q & 31)) * 16;
+    if constexpr (BF) {
+      uint32_t h[2], lo[2];
+      split2_bf16(v[0], v[1], h[0], lo[0]);
+      split2_bf16(v[2], v[3], h[1], lo[1]);
+      *(uint2*)(d + (quad & 1) * 8) = make_uint2(h[0], h[1]);
+      *(uint2*)(d + 1024 + (quad & 1) * 8) = make_uint2(lo[0], lo[1]);
+    } else {
+      *(float4*)(d + (quad & 1) * 1024) = make_float4(v[0], v[1], v[2], v[3]);
+    }
+  }
 }
 
 template <bool BF>
@@ -909,14 +1170,15 @@ fold_pupil_kernel(FoldPupil pup, FoldSteps wl, int nb, int n,
   const long rb = fold_row_bytes(n);
   const int py = blockIdx.x * 32 + (threadIdx.x >> 3);
   const int beta = threadIdx.x & 1, quad = (threadIdx.x >> 1) & 3, s = blockIdx.y;
-  PupilLoad<VEC> pl;
+  PupilLoad<VEC, true> pl;
   pl.init(pup, n, py, beta, quad, 0.0);
-  pl.raw(s);
+  typename PupilLoad<VEC, true>::Raw raw{};
+  pl.raw(s, raw);
   const int b0 = blockIdx.z * kPupilWl, b1 = b0 + kPupilWl < nb ? b0 + kPupilWl : nb;
   for (int b = b0; b < b1; ++b) {
     pl.inv_wl = wl.step[b];
     FoldPart o;
-    pl.part(s, beta, o);
+    pl.part(s, beta, raw, o);
     if (py >= kh) continue;
     uint8_t* d = out + (long)b * stride + (long)s * kRow;
 #pragma unroll
@@ -929,26 +1191,35 @@ fold_pupil_kernel(FoldPupil pup, FoldSteps wl, int nb, int n,
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+template <bool BF, int LOAD, bool VEC, int BNQ>
+void stage1_go(const FoldStage1& a, long tiles, hipStream_t s) {
+  if constexpr (LOAD == FOLD_MEM)
+    hipLaunchKernelGGL((fold_stage1_mem_kernel<BF, BNQ, BNQ == 128 ? 3 : 4>), dim3((unsigned)tiles), dim3(kThreads), 0,
+                       s, a);
+  else
+    hipLaunchKernelGGL((fold_stage1_kernel<BF, LOAD, VEC, BNQ>), dim3((unsigned)tiles),
+                       dim3(kThreads), 0, s, a);
+}
+
 template <bool BF, int LOAD, bool VEC>
 hipError_t stage1_width(const FoldStage1& a, hipStream_t s) {
   const int mh = fold_half(a.m), tp = (fold_half(a.n) + 31) / 32;
   auto tiles = [&](int w) { return (long)((mh + w - 1) / w) * tp * a.batch; };
-  if (mh > 64 && tiles(128) >= 256) {
-    hipLaunchKernelGGL((fold_stage1_kernel<BF, LOAD, VEC, 128>), dim3((unsigned)tiles(128)),
-                       dim3(kThreads), 0, s, a);
-  } else if (mh > 32 && tiles(64) >= 256) {
-    hipLaunchKernelGGL((fold_stage1_kernel<BF, LOAD, VEC, 64>), dim3((unsigned)tiles(64)),
-                       dim3(kThreads), 0, s, a);
-  } else {
-    hipLaunchKernelGGL((fold_stage1_kernel<BF, LOAD, VEC, 32>), dim3((unsigned)tiles(32)),
-                       dim3(kThreads), 0, s, a);
-  }
+  if (mh > 64 && tiles(128) >= 256) stage1_go<BF, LOAD, VEC, 128>(a, tiles(128), s);
+  else if (mh > 32 && tiles(64) >= 256) stage1_go<BF, LOAD, VEC, 64>(a, tiles(64), s);
+  else stage1_go<BF, LOAD, VEC, 32>(a, tiles(32), s);
   return hipGetLastError();
 }
 
 template <bool BF>
 hipError_t stage1_load(const FoldStage1& a, FoldLoad load, hipStream_t s) {
   if (load == FOLD_MEM) return stage1_width<BF, FOLD_MEM, true>(a, s);
+  if (load == FOLD_PUPIL && (a.pupil.phase || (!a.pupil.opd && !a.pupil.amp))) {
+    // callers write such pupils to memory first where they have the room
+    const long tiles = (long)((fold_half(a.m) + 31) / 32) * ((fold_half(a.n) + 31) / 32) * a.batch;
+    stage1_go<BF, kPupilAny, false, 32>(a, tiles, s);
+    return hipGetLastError();
+  }
   if (load == FOLD_PUPIL) {
     const bool vec = a.n % 8 == 0 && aligned16(a.pupil.opd) && aligned16(a.pupil.amp);
     return vec ? stage1_width<BF, FOLD_PUPIL, true>(a, s) : stage1_width<BF, FOLD_PUPIL, false>(a, s);
@@ -961,7 +1232,7 @@ template <bool BF, int EPI>
 hipError_t stage2_size(const FoldStage2& a, hipStream_t s) {
   const int mh = fold_half(a.m), tx = (mh + 31) / 32;
   auto tiles = [&](int q) { return (long)tx * ((mh + q - 1) / q) * a.batch; };
-  hipLaunchKernelGGL((fold_stage2_kernel<BF, EPI, 64, 3>), dim3((unsigned)tiles(64)), dim3(kThreads),
+  hipLaunchKernelGGL((fold_stage2_kernel<BF, EPI, 64, 4>), dim3((unsigned)tiles(64)), dim3(kThreads),
                      0, s, a);
   return hipGetLastError();
 }
@@ -1049,18 +1320,25 @@ static unsigned group_grid(const FoldGroup& g) {
   return (unsigned)(kXcds * most);
 }
 
-hipError_t launch_fold_group_stage1(const FoldGroup& g, int width, bool vec, hipStream_t s) {
+hipError_t launch_fold_group_stage1(const FoldGroup& g, int width, hipStream_t s) {
   const dim3 grid(group_grid(g)), block(kThreads);
   if (grid.x == 0) return hipSuccess;
-  auto go = [&](auto V) {
-    constexpr bool v = decltype(V)::value;
-    if (width == 128) hipLaunchKernelGGL((fold_group_stage1_kernel<v, 128>), grid, block, 0, s, g);
-    else if (width == 64) hipLaunchKernelGGL((fold_group_stage1_kernel<v, 64>), grid, block, 0, s, g);
-    else hipLaunchKernelGGL((fold_group_stage1_kernel<v, 32>), grid, block, 0, s, g);
-  };
-  if (vec) go(std::true_type{});
-  else go(std::false_type{});
+  if (width == 128) hipLaunchKernelGGL(fold_group_stage1_kernel<128>, grid, block, 0, s, g);
+  else if (width == 64) hipLaunchKernelGGL(fold_group_stage1_kernel<64>, grid, block, 0, s, g);
+  else hipLaunchKernelGGL(fold_group_stage1_kernel<32>, grid, block, 0, s, g);
   return hipGetLastError();
+}
+
+hipError_t launch_fold_group_fields(const FoldFieldJob* jobs, int njobs, int most, hipStream_t s) {
+  const int kh = fold_half(most);
+  for (int j0 = 0; j0 < njobs; j0 += 65535) {
+    const int k = njobs - j0 < 65535 ? njobs - j0 : 65535;
+    hipLaunchKernelGGL(fold_group_field_kernel, dim3((fold_pad(kh) + 255) / 256, kh, k), dim3(256), 0,
+                       s, jobs + j0);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 hipError_t launch_fold_group_stage2(const FoldGroup& g, hipStream_t s) {
@@ -1070,6 +1348,8 @@ hipError_t launch_fold_group_stage2(const FoldGroup& g, hipStream_t s) {
   return hipGetLastError();
 }
 
-bool fold_pupil_in_loader(int m) { return fold_half(m) <= 256; }
+bool fold_pupil_in_loader(const FoldPupil& p, int m) {
+  return !p.phase && (p.opd || p.amp) && fold_half(m) <= 256;
+}
 
 }  // namespace dlx
