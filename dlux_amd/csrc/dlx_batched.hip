@@ -127,7 +127,8 @@ struct Plan {
   int fld_most = 0;                  // side of the largest field
   std::vector<FoldProblem> prob;     // in launch order
   std::vector<FoldColumns> cols;
-  std::vector<uint32_t> map1[kLists], map2;
+  std::vector<FoldRowTile> map1[kLists];
+  std::vector<uint32_t> map2;
   int xcd1[kLists][9], xcd2[9];
   std::vector<SumJob> sum;
   std::vector<size_t> U_off, I_off;  // per instance
@@ -262,7 +263,7 @@ int plan_sizes(int n, const dlx_mft_instance* inst, int n_outputs, Plan& P) {
     nc += c;
   }
   P.off_cols = take(nc * sizeof(FoldColumns));
-  for (int l = 0; l < kLists; ++l) P.off_map1[l] = take(n1[l] * sizeof(uint32_t));
+  for (int l = 0; l < kLists; ++l) P.off_map1[l] = take(n1[l] * sizeof(FoldRowTile));
   P.off_map2 = take(n2 * sizeof(uint32_t));
   P.off_sum = take((size_t)n_outputs * sizeof(SumJob));
   P.desc = off;
@@ -294,110 +295,115 @@ int plan_sizes(int n, const dlx_mft_instance* inst, int n_outputs, Plan& P) {
   return DLX_OK;
 }
 
-// The descriptors.  The instances of one field go to one XCD, their stage-1
-// workgroups for the same rows next to each other (its L2 then serves the
-// field to all of them), fields dealt largest first to the XCD with the least
-// work; with few fields (a scene's shared pupil) the instances are dealt in
-// sets of a column group each.  Stage 2 keeps stage 1's XCDs: it reads what
-// they wrote.
+// Cut a tile list into 8 runs of equal cost, one per XCD.
+void cut_list(const std::vector<float>& cost, int (&xcd)[9]) {
+  double total = 0.0, run = 0.0;
+  for (float c : cost) total += c;
+  int x = 0;
+  xcd[0] = 0;
+  for (size_t t = 0; t < cost.size(); ++t) {
+    while (x < 7 && run >= total * (x + 1) / 8) xcd[++x] = (int)t;
+    run += cost[t];
+  }
+  while (x < 8) xcd[++x] = (int)cost.size();
+}
+
+// The descriptors.  A stage-1 list is dealt to the XCDs in units of an eighth
+// of a field's row blocks with all its column groups, the costliest unit first
+// to the XCD with the least work, and every XCD runs its long tiles first: the
+// launch ends evenly (whole fields dealt to XCDs kept 160 of 512 workgroup
+// slots busy for 48 sources of 256^2 to 1024^2; a list cut into runs of equal
+// cost, an XCD of large fields alone, left a half-empty second round), and the
+// workgroups that share field rows share an L2.
 void plan_fill(int n, const dlx_mft_instance* inst, int n_outputs, float* const* outs, uint8_t* ws,
                Plan& P) {
   for (size_t q = 0; q < P.tab.size(); ++q) P.tab[q].out = ws + P.off_T + P.tab_off[q];
   for (size_t f = 0; f < P.fld.size(); ++f) P.fld[f].out = ws + P.off_P + P.fld_off[f];
-  // stage 1's column blocks over the field's rows and stages, a tile's fixed
-  // part, and stage 2's tiles
-  auto cost = [&](int i) {
-    const int st = (fold_half(inst[i].n_in) + 15) / 16;
-    const int w = fold_group_width(inst[i].n_out);
-    return (double)rows1(inst[i].n_in) * cols1(inst[i].n_out) * (st + 4) * (w + 32) / 160.0 +
-           (double)tiles2(inst[i].n_out) * (st + 8) * 0.5;
+  std::vector<std::vector<int>> members(P.fld.size());
+  for (int i = 0; i < n; ++i) members[P.fld_of[i]].push_back(i);
+  struct Unit {
+    int cols, ncols, row, nrows;
+    float cost;   // of one row block
   };
-  std::vector<std::vector<int>> units(P.fld.size());
-  for (int i = 0; i < n; ++i) units[P.fld_of[i]].push_back(i);
-  if (units.size() < 32) {
-    std::vector<std::vector<int>> cut;
-    for (auto& u : units) {
-      std::stable_sort(u.begin(), u.end(),
-                       [&](int a, int b) { return inst[a].n_out > inst[b].n_out; });
-      for (size_t i = 0; i < u.size();) {
-        const size_t k = 128 / fold_group_width(inst[u[i]].n_out);
-        const size_t e = std::min(u.size(), i + k);
-        cut.emplace_back(u.begin() + i, u.begin() + e);
-        i = e;
+  std::vector<Unit> units;
+  for (int l = kLists - 1; l >= 0; --l) {
+    const int L = 128 / kWidth[l];
+    units.clear();
+    for (size_t f = 0; f < members.size(); ++f) {
+      const int c0 = (int)P.cols.size(), st = (fold_half(P.fld[f].n) + 15) / 16;
+      for (int i : members[f]) {
+        const dlx_mft_instance& d = inst[i];
+        if (list_of(d.n_out) != l) continue;
+        const FoldTableJob& t = P.tab[P.tab_of[i]];
+        const double sg = d.inverse ? -1.0 : 1.0;
+        for (int c = 0; c < cols1(d.n_out); ++c) {
+          if ((int)P.cols.size() == c0 || P.cols.back().count == L) {
+            FoldColumns g{};
+            g.src = P.fld[f].out;
+            g.n = d.n_in;
+            P.cols.push_back(g);
+          }
+          FoldColumns& g = P.cols.back();
+          // the input half of the shift (the output half is a phase: no intensity)
+          g.tile_of[g.count++] = {t.out, ws + P.U_off[i], sg * t.step * d.shift_x,
+                                  sg * t.step * d.shift_y, c * kWidth[l], d.n_out};
+        }
       }
+      const int nc = (int)P.cols.size() - c0;
+      if (nc == 0) continue;
+      float cost = 0.f;   // a step's fixed part and its products, and a tile's store
+      for (int c = c0; c < c0 + nc; ++c)
+        cost += (float)(P.cols[c].count * ((st + 2) * (kWidth[l] + 64) + 256));
+      const int rows = rows1(P.fld[f].n), piece = (rows + 7) / 8;
+      for (int r = 0; r < rows; r += piece)
+        units.push_back({c0, nc, r, std::min(piece, rows - r), cost});
     }
-    units.swap(cut);
-  }
-  std::vector<double> ucost(units.size(), 0.0);
-  for (size_t u = 0; u < units.size(); ++u)
-    for (int i : units[u]) ucost[u] += cost(i);
-  std::vector<int> idx(units.size());
-  std::iota(idx.begin(), idx.end(), 0);
-  std::stable_sort(idx.begin(), idx.end(), [&](int a, int b) { return ucost[a] > ucost[b]; });
-  std::vector<int> on[8];   // units of an XCD
-  double load[8] = {};
-  for (int u : idx) {
-    int best = 0;
-    for (int x = 1; x < 8; ++x)
-      if (load[x] < load[best]) best = x;
-    on[best].push_back(u);
-    load[best] += ucost[u];
+    std::stable_sort(units.begin(), units.end(), [](const Unit& a, const Unit& b) {
+      return a.cost * a.nrows > b.cost * b.nrows;
+    });
+    std::vector<const Unit*> on[8];
+    double load[8] = {};
+    for (const Unit& u : units) {
+      int best = 0;
+      for (int x = 1; x < 8; ++x)
+        if (load[x] < load[best]) best = x;
+      on[best].push_back(&u);
+      load[best] += u.cost * u.nrows;
+    }
+    for (int x = 0; x < 8; ++x) {
+      P.xcd1[l][x] = (int)P.map1[l].size();
+      std::stable_sort(on[x].begin(), on[x].end(), [](const Unit* a, const Unit* b) {
+        return a->cost / a->ncols > b->cost / b->ncols;
+      });
+      for (const Unit* u : on[x])
+        for (int r = u->row; r < u->row + u->nrows; ++r)
+          for (int c = u->cols; c < u->cols + u->ncols; ++c)
+            P.map1[l].push_back({(uint32_t)c, (uint32_t)(r * kFoldTilePy)});
+    }
+    P.xcd1[l][8] = (int)P.map1[l].size();
   }
   P.prob.reserve(n);
-  for (int x = 0; x < 8; ++x) {
-    for (int l = 0; l < kLists; ++l) P.xcd1[l][x] = (int)P.map1[l].size();
-    P.xcd2[x] = (int)P.map2.size();
-    for (int u : on[x]) {
-      // stage 1: this field's column groups of each width
-      for (int l = 0; l < kLists; ++l) {
-        const int L = 128 / kWidth[l], c0 = (int)P.cols.size();
-        for (int i : units[u]) {
-          const dlx_mft_instance& d = inst[i];
-          if (list_of(d.n_out) != l) continue;
-          const FoldTableJob& t = P.tab[P.tab_of[i]];
-          const double sg = d.inverse ? -1.0 : 1.0;
-          for (int c = 0; c < cols1(d.n_out); ++c) {
-            if ((int)P.cols.size() == c0 || P.cols.back().count == L) {
-              FoldColumns g{};
-              g.src = P.fld[P.fld_of[i]].out;
-              g.n = d.n_in;
-              P.cols.push_back(g);
-            }
-            FoldColumns& g = P.cols.back();
-            // the input half of the shift (the output half is a phase: no intensity)
-            g.tile_of[g.count++] = {t.out, ws + P.U_off[i], sg * t.step * d.shift_x,
-                                    sg * t.step * d.shift_y, c * kWidth[l], d.n_out};
-          }
-        }
-        const int nc = (int)P.cols.size() - c0;
-        if (nc == 0) continue;
-        const int base = (int)P.map1[l].size();
-        for (int c = 0; c < nc; ++c) {
-          P.cols[c0 + c].tile = base + c;
-          P.cols[c0 + c].step = nc;
-        }
-        for (int r = 0; r < rows1(P.cols[c0].n); ++r)
-          for (int c = 0; c < nc; ++c) P.map1[l].push_back((uint32_t)(c0 + c));
-      }
-      for (int i : units[u]) {
-        const dlx_mft_instance& d = inst[i];
-        const double c = mft_norm(geom_of(d), d.wavelength, d.pixel_scale_in, d.pixel_scale_out);
-        FoldProblem p{};
-        p.table = P.tab[P.tab_of[i]].out;
-        p.mid = ws + P.U_off[i];
-        p.out = (float*)(ws + P.I_off[i]);
-        p.alpha = (float)(c * std::sqrt(d.weight));
-        p.n = d.n_in;
-        p.m = d.n_out;
-        p.inverse = d.inverse ? 1 : 0;
-        p.tile = (int)P.map2.size();
-        P.map2.insert(P.map2.end(), tiles2(p.m), (uint32_t)P.prob.size());
-        P.prob.push_back(p);
-      }
+  std::vector<float> cost2;
+  // stage 2: instances of one field (a source's wavelengths) together, in runs
+  // of equal cost
+  for (const std::vector<int>& run : members)
+    for (int i : run) {
+      const dlx_mft_instance& d = inst[i];
+      const double c = mft_norm(geom_of(d), d.wavelength, d.pixel_scale_in, d.pixel_scale_out);
+      FoldProblem p{};
+      p.table = P.tab[P.tab_of[i]].out;
+      p.mid = ws + P.U_off[i];
+      p.out = (float*)(ws + P.I_off[i]);
+      p.alpha = (float)(c * std::sqrt(d.weight));
+      p.n = d.n_in;
+      p.m = d.n_out;
+      p.inverse = d.inverse ? 1 : 0;
+      p.tile = (int)P.map2.size();
+      P.map2.insert(P.map2.end(), tiles2(p.m), (uint32_t)P.prob.size());
+      cost2.insert(cost2.end(), tiles2(p.m), (float)((fold_half(p.n) + 15) / 16 + 6));
+      P.prob.push_back(p);
     }
-  }
-  for (int l = 0; l < kLists; ++l) P.xcd1[l][8] = (int)P.map1[l].size();
-  P.xcd2[8] = (int)P.map2.size();
+  cut_list(cost2, P.xcd2);
   std::vector<int> job(n_outputs, -1);
   for (int i = 0; i < n; ++i) {
     int& j = job[inst[i].out_index];
@@ -429,7 +435,7 @@ int launch_plan(const Plan& Q, uint8_t* ws, bool with_matrices, hipStream_t s) {
   g.cols = (const FoldColumns*)(ws + Q.off_cols);
   for (int l = kLists - 1; l >= 0; --l) {   // the largest outputs first
     if (Q.map1[l].empty()) continue;
-    g.map = (const uint32_t*)(ws + Q.off_map1[l]);
+    g.rows = (const FoldRowTile*)(ws + Q.off_map1[l]);
     std::memcpy(g.xcd, Q.xcd1[l], sizeof(g.xcd));
     DLX_HIP(launch_fold_group_stage1(g, kWidth[l], s));
   }

@@ -139,7 +139,6 @@ struct FoldProblem {
 struct FoldColumns {
   const uint8_t* src;
   int n, count;
-  int tile, step;      // the workgroup of row block r is tile + r step (+ less than step)
   struct Tile {
     const uint8_t* table;
     uint8_t* mid;
@@ -147,11 +146,15 @@ struct FoldColumns {
     int q0, m;
   } tile_of[4];
 };
-// A launch over tile lists: map[t] is the problem or column group of tile t;
-// XCD x runs [xcd[x], xcd[x + 1]).
+struct FoldRowTile {
+  uint32_t cols, row;   // column group, first row
+};
+// A launch over a tile list: stage-1 tiles of column groups (rows), or
+// stage-2 tiles' problems (map); XCD x runs [xcd[x], xcd[x + 1]).
 struct FoldGroup {
   const FoldProblem* probs;
   const FoldColumns* cols;
+  const FoldRowTile* rows;
   const uint32_t* map;
   int xcd[9];
 };

@@ -188,32 +188,37 @@ __device__ __forceinline__ void fold_y(FoldPart& o, int beta) {
 
 // The pupil loader of one thread.  VEC: n a multiple of 8 and 16-byte aligned
 // planes (float4 loads; a run of four is whole or absent).  ANY: any of the
-// planes may be missing and there may be a phase plane, tested as they are
-// read; otherwise the amplitude or the OPD is there, no phase is, and every
-// load is unconditional (a missing plane reads the other one and is replaced
-// by its constant), so that the loads stay in flight over a stage.
-template <bool VEC, bool ANY>
+// planes may be missing, there may be a phase plane and a tilt, tested as they
+// are read; otherwise the amplitude or the OPD is there, no phase is, a tilt
+// is if TILT, and every load is unconditional (a missing plane reads the other
+// one, and its constant comes in through the coefficients), so that the loads
+// stay in flight over a stage and the phasors can be scheduled among products.
+template <bool VEC, bool TILT, bool ANY>
 struct PupilLoad {
   const float *opd, *amp, *phase;   // rows
   int n, kh, quad, x0i;             // x0i = n / 2: the first positive column
-  bool row_ok, tilted, has_opd, has_amp, has_phase;
-  double inv_wl, tx, tyY, dx, x0;
-  float scale;
+  bool has_opd, has_amp, has_phase;
+  double inv_wl, tx, tyY, dx, x0, co;   // co: 1 if there is an OPD, else 0
+  float ca, cb;                     // amplitude = ca * value + cb; zero outside the rows
   struct Raw { float4 op, om, ap, am; };   // plus runs (k ascending), minus runs (descending)
 
   __device__ __forceinline__ void init(const FoldPupil& p, int n_, int py, int beta, int quad_,
                                        double inv) {
     n = n_; kh = (n + 1) >> 1; quad = quad_; x0i = n >> 1;
-    row_ok = py < kh;
+    const bool row_ok = py < kh;
     const int yp = x0i + (row_ok ? py : 0);
     const int y = beta ? n - 1 - yp : yp;
     has_opd = p.opd != nullptr; has_amp = p.amp != nullptr; has_phase = p.phase != nullptr;
     opd = (has_opd ? p.opd : p.amp) + (long)y * n;
     amp = (has_amp ? p.amp : p.opd) + (long)y * n;
     if constexpr (ANY) phase = p.phase + (long)y * n;
-    inv_wl = inv; tx = p.tx; dx = p.dx; x0 = p.x0; scale = p.scale;
-    tilted = p.tx != 0.0 || p.ty != 0.0;
+    co = has_opd ? 1.0 : 0.0;
+    inv_wl = TILT || ANY ? inv : has_opd ? inv : 0.0;
+    tx = p.tx; dx = p.dx; x0 = p.x0;
     tyY = p.ty * pupil_coord(y, p.dx, p.x0);
+    const float sc = row_ok ? p.scale : 0.f;
+    ca = has_amp ? sc : 0.f;
+    cb = has_amp ? 0.f : sc;
   }
   __device__ __forceinline__ float4 run_up(const float* row, int p) const {
     if constexpr (VEC) return *(const float4*)(row + x0i + (p < kh ? p : 0));
@@ -236,34 +241,28 @@ struct PupilLoad {
   }
   __device__ __forceinline__ void part(int s, int beta, const Raw& r, FoldPart& o) const {
     const int p = s * kStageK + quad * 4;
-    float vo[2][4] = {{r.op.x, r.op.y, r.op.z, r.op.w}, {r.om.w, r.om.z, r.om.y, r.om.x}};
-    float va[2][4] = {{r.ap.x, r.ap.y, r.ap.z, r.ap.w}, {r.am.w, r.am.z, r.am.y, r.am.x}};
+    const float vo[2][4] = {{r.op.x, r.op.y, r.op.z, r.op.w}, {r.om.w, r.om.z, r.om.y, r.om.x}};
+    const float va[2][4] = {{r.ap.x, r.ap.y, r.ap.z, r.ap.w}, {r.am.w, r.am.z, r.am.y, r.am.x}};
     float2 v[2][4];
+    // VEC: the run is whole or absent
+    const float ra = !VEC || p < kh ? ca : 0.f, rb = !VEC || p < kh ? cb : 0.f;
 #pragma unroll
     for (int d = 0; d < 2; ++d)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        vo[d][e] = has_opd ? vo[d][e] : 0.f;
-        va[d][e] = row_ok && p + e < kh ? scale * (has_amp ? va[d][e] : 1.f) : 0.f;
-      }
-    if (tilted || ANY) {
-#pragma unroll
-      for (int d = 0; d < 2; ++d)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
+        float a = __builtin_fmaf(va[d][e], ra, rb);
+        if constexpr (!VEC) a = p + e < kh ? a : 0.f;
+        double t = 0.0, path = (double)vo[d][e];
+        if constexpr (TILT || ANY) {
           const int pc = p + e < kh ? p + e : kh - 1;
           const int x = d ? n - 1 - x0i - pc : x0i + pc;
-          double t = 0.0, path = (double)vo[d][e];
+          if (ANY && !has_opd) path = 0.0;
           if (ANY && has_phase) t = (double)phase[x] * 0.15915494309189535;   // 1 / (2 pi)
-          if (tilted) path = pupil_path(tx, pupil_coord(x, dx, x0), tyY, path);
-          v[d][e] = pupil_phasor(path, inv_wl, t, va[d][e]);
+          if (ANY && !has_amp) a = p + e < kh ? rb : 0.f;
+          path = fma(path, co, fma(tx, pupil_coord(x, dx, x0), tyY));   // pupil_path's bits
         }
-    } else {
-#pragma unroll
-      for (int d = 0; d < 2; ++d)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[d][e] = pupil_phasor((double)vo[d][e], inv_wl, 0.0, va[d][e]);
-    }
+        v[d][e] = pupil_phasor(path, inv_wl, t, a);
+      }
     fold_x(v[0], v[1], o);
     fold_y(o, beta);
   }
@@ -484,7 +483,8 @@ __device__ __forceinline__ void y_phase(uint8_t* lds, f32x16_t (&acc)[S1<BNQ>::N
   }
 }
 
-constexpr int kPupilAny = 3;   // FOLD_PUPIL through the loader that tests for every plane
+constexpr int kPupilAny = 3;    // FOLD_PUPIL through the loader that tests for every plane
+constexpr int kPupilTilt = 4;   // FOLD_PUPIL with a tilt
 
 // Fields formed by the loader: the next stage's parts are formed after this
 // stage's products are issued, from values loaded two stages ahead.
@@ -513,7 +513,7 @@ fold_stage1_kernel(FoldStage1 a) {
              table_block(wave >> 1, mhp, kp, blk < last ? blk : last);
   }
   const int py = threadIdx.x >> 3, beta = threadIdx.x & 1, quad = (threadIdx.x >> 1) & 3;
-  std::conditional_t<LOAD == FOLD_FIELD, FieldLoad<VEC>, PupilLoad<VEC, LOAD == kPupilAny>> ld;
+  std::conditional_t<LOAD == FOLD_FIELD, FieldLoad<VEC>, PupilLoad<VEC, LOAD == kPupilTilt, LOAD == kPupilAny>> ld;
   FoldPhase ph{};
   bool phased = false;
   if constexpr (LOAD != FOLD_FIELD) {
@@ -551,8 +551,8 @@ fold_stage1_kernel(FoldStage1 a) {
 #pragma unroll
     for (int j = 0; j < NJ; ++j) load_frag(fb[decltype(J)::value][j], tab[j], sc);
   };
-  // one stage: J = s & 1
-  auto step = [&](auto J, int s) __attribute__((always_inline)) {
+  // one stage: J = s & 1; FULL: there is a next one
+  auto step = [&](auto J, auto FULL, int s) __attribute__((always_inline)) {
     constexpr int j0 = decltype(J)::value;
     lds_barrier();   // stage s is in LDS, stage s - 1 has been read
     const uint8_t* la = lds + j0 * kBuf;
@@ -562,10 +562,23 @@ fold_stage1_kernel(FoldStage1 a) {
     load_tab(std::integral_constant<int, 1 - j0>{}, s + 1);
     ld.raw(s + 2, raw[j0]);
     window(s + 2);
+#ifndef V_NOPRIO
     __builtin_amdgcn_s_setprio(1);
+#endif
     mma_stage<BF, NI, NJ>(acc, fa, fb[j0]);
+#ifndef V_NOPRIO
     __builtin_amdgcn_s_setprio(0);
-    if (s + 1 < nst) convert(s + 1, raw[1 - j0]);
+#endif
+    if (decltype(FULL)::value || s + 1 < nst) convert(s + 1, raw[1 - j0]);
+#ifdef V_ILV
+    if constexpr (BF) {
+#pragma unroll
+      for (int q = 0; q < 3 * NI * NJ; ++q) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, V_ILV, 0);
+      }
+    }
+#endif
   };
   load_tab(std::integral_constant<int, 0>{}, 0);
   ld.raw(0, raw[0]);
@@ -575,11 +588,12 @@ fold_stage1_kernel(FoldStage1 a) {
   if constexpr (LOAD == FOLD_FIELD) lds_barrier();
   convert(0, raw[0]);
   int s = 0;
-  for (; s + 1 < nst; s += 2) {   // whole pairs: no path of the loop skips a load
-    step(std::integral_constant<int, 0>{}, s);
-    step(std::integral_constant<int, 1>{}, s + 1);
+  for (; s + 2 < nst; s += 2) {   // whole pairs: no path of the loop skips a load or a part
+    step(std::integral_constant<int, 0>{}, std::true_type{}, s);
+    step(std::integral_constant<int, 1>{}, std::true_type{}, s + 1);
   }
-  if (s < nst) step(std::integral_constant<int, 0>{}, s);
+  step(std::integral_constant<int, 0>{}, std::false_type{}, s);
+  if (s + 1 < nst) step(std::integral_constant<int, 1>{}, std::false_type{}, s + 1);
   lds_barrier();
   if constexpr (LOAD == FOLD_FIELD)
     if (phased) y_phase<BNQ>(lds, acc, ph.c2, ph.cy, a.n, py0);
@@ -937,9 +951,10 @@ fold_group_stage1_kernel(FoldGroup g) {
   __shared__ float2 win[2][L][kStageK];
   const int t = group_tile(g);
   if (t < 0) return;
-  const FoldColumns& cg = g.cols[g.map[t]];
+  const FoldRowTile rt = g.rows[t];
+  const FoldColumns& cg = g.cols[rt.cols];
   const int n = cg.n, kh = fold_half(n), kp = fold_pad(kh), count = cg.count;
-  const int py0 = (t - cg.tile) / cg.step * 32;
+  const int py0 = (int)rt.row;
   const int nst = (kh + kStageK - 1) / kStageK, wave = threadIdx.x >> 6;
   const int quad = threadIdx.x & 3, beta = (threadIdx.x >> 2) & 1, py = threadIdx.x >> 3;
   const float4* row;
@@ -1170,9 +1185,9 @@ fold_pupil_kernel(FoldPupil pup, FoldSteps wl, int nb, int n,
   const long rb = fold_row_bytes(n);
   const int py = blockIdx.x * 32 + (threadIdx.x >> 3);
   const int beta = threadIdx.x & 1, quad = (threadIdx.x >> 1) & 3, s = blockIdx.y;
-  PupilLoad<VEC, true> pl;
+  PupilLoad<VEC, true, true> pl;
   pl.init(pup, n, py, beta, quad, 0.0);
-  typename PupilLoad<VEC, true>::Raw raw{};
+  typename PupilLoad<VEC, true, true>::Raw raw{};
   pl.raw(s, raw);
   const int b0 = blockIdx.z * kPupilWl, b1 = b0 + kPupilWl < nb ? b0 + kPupilWl : nb;
   for (int b = b0; b < b1; ++b) {
@@ -1222,6 +1237,8 @@ hipError_t stage1_load(const FoldStage1& a, FoldLoad load, hipStream_t s) {
   }
   if (load == FOLD_PUPIL) {
     const bool vec = a.n % 8 == 0 && aligned16(a.pupil.opd) && aligned16(a.pupil.amp);
+    if (a.pupil.tx != 0.0 || a.pupil.ty != 0.0)
+      return vec ? stage1_width<BF, kPupilTilt, true>(a, s) : stage1_width<BF, kPupilTilt, false>(a, s);
     return vec ? stage1_width<BF, FOLD_PUPIL, true>(a, s) : stage1_width<BF, FOLD_PUPIL, false>(a, s);
   }
   const bool vec = a.n % 8 == 0 && aligned16(a.src) && a.src_stride % 16 == 0;
