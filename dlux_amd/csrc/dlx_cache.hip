@@ -38,6 +38,11 @@ namespace {
 // takes over its slot.
 constexpr int kMaxUsers = 16;
 
+// The entries' events order work of one device after work of the same device, and
+// the host reads nothing behind them: no system-scope release.  With it a record
+// after a 12 us pair of kernels cost the stream 2.9 us, without it 1.1 us.
+constexpr unsigned kEventFlags = hipEventDisableTiming | hipEventDisableSystemFence;
+
 struct MatEntry {
   std::vector<double> key;
   int dev = 0;
@@ -145,7 +150,7 @@ MatEntry* new_entry(std::vector<double>&& key, int dev, void* mem, size_t bytes,
   e->bytes = bytes;
   e->tick = tick;
   e->pins = 1;
-  if (hipEventCreateWithFlags(&e->ready, hipEventDisableTiming) != hipSuccess) {
+  if (hipEventCreateWithFlags(&e->ready, kEventFlags) != hipSuccess) {
     delete e;
     return nullptr;
   }
@@ -364,7 +369,7 @@ int cache_release(void* handle, hipStream_t s) {
   for (auto& u : e->users)
     if (u.first == s) ev = u.second;
   if (!ev && (int)e->users.size() < kMaxUsers) {
-    if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
+    if (hipEventCreateWithFlags(&ev, kEventFlags) != hipSuccess) {
       (void)hipGetLastError();
       // no event: keep the ordering by syncing the stream before the entry can go
       (void)hipStreamSynchronize(s);

@@ -562,23 +562,13 @@ fold_stage1_kernel(FoldStage1 a) {
     load_tab(std::integral_constant<int, 1 - j0>{}, s + 1);
     ld.raw(s + 2, raw[j0]);
     window(s + 2);
-#ifndef V_NOPRIO
-    __builtin_amdgcn_s_setprio(1);
-#endif
+    // one wave per SIMD (small launches) keeps its products ahead of its
+    // conversion: 17.0 against 19.5 us at 16 wavelengths of 512^2 -> 128^2; with
+    // two, the raised priority cost 90 -> 100 us (float32, 64 of 512^2 -> 256^2)
+    if constexpr (BNQ < 128) __builtin_amdgcn_s_setprio(1);
     mma_stage<BF, NI, NJ>(acc, fa, fb[j0]);
-#ifndef V_NOPRIO
-    __builtin_amdgcn_s_setprio(0);
-#endif
+    if constexpr (BNQ < 128) __builtin_amdgcn_s_setprio(0);
     if (decltype(FULL)::value || s + 1 < nst) convert(s + 1, raw[1 - j0]);
-#ifdef V_ILV
-    if constexpr (BF) {
-#pragma unroll
-      for (int q = 0; q < 3 * NI * NJ; ++q) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, V_ILV, 0);
-      }
-    }
-#endif
   };
   load_tab(std::integral_constant<int, 0>{}, 0);
   ld.raw(0, raw[0]);
@@ -587,10 +577,14 @@ fold_stage1_kernel(FoldStage1 a) {
   window(1);
   if constexpr (LOAD == FOLD_FIELD) lds_barrier();
   convert(0, raw[0]);
+  // whole pairs: no path of the loop skips a load or a part.  A field's parts, with
+  // their choice of a phase, stay in a block of their own: merged with the
+  // products they spilled 567 registers at 128 columns
+  using Whole = std::bool_constant<LOAD != FOLD_FIELD>;
   int s = 0;
-  for (; s + 2 < nst; s += 2) {   // whole pairs: no path of the loop skips a load or a part
-    step(std::integral_constant<int, 0>{}, std::true_type{}, s);
-    step(std::integral_constant<int, 1>{}, std::true_type{}, s + 1);
+  for (; s + 2 < nst; s += 2) {
+    step(std::integral_constant<int, 0>{}, Whole{}, s);
+    step(std::integral_constant<int, 1>{}, Whole{}, s + 1);
   }
   step(std::integral_constant<int, 0>{}, std::false_type{}, s);
   if (s + 1 < nst) step(std::integral_constant<int, 1>{}, std::false_type{}, s + 1);
@@ -1030,11 +1024,7 @@ fold_group_stage1_kernel(FoldGroup g) {
       // the window of stage s is still read by this stage's converts if L > 1
       window(L == 1 ? s + 2 : s + 1);
     }
-    if (l < count) {
-      __builtin_amdgcn_s_setprio(1);
-      mma_stage<true, NI, NJ>(acc[l], fa, fb[k]);
-      __builtin_amdgcn_s_setprio(0);
-    }
+    if (l < count) mma_stage<true, NI, NJ>(acc[l], fa, fb[k]);
     if (sn < nst && ln < count) {
       if constexpr (l + 1 < L) convert(sn, ln, 1 - k, raw[p]);
       else convert(sn, ln, 1 - k, raw[1 - p]);
