@@ -265,5 +265,8 @@ def check(status: int, name: str) -> None:
 
 def dptr(values) -> ctypes.Array:
     """A host double array for the C ABI."""
+    if isinstance(values, np.ndarray) and values.dtype == np.float64 and values.ndim == 1 \
+            and values.size and values.flags.c_contiguous:
+        return (c_double * values.size).from_buffer_copy(values)
     vals = [float(v) for v in values]
     return (c_double * len(vals))(*vals)

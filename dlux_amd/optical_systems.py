@@ -93,6 +93,9 @@ class PupilPlan:
         self.scale = 1.0 / n ** 2          # reference initial phasor ones/N^2
 
     def _t(self, x):
+        if isinstance(x, torch.Tensor) and x.dtype is torch.float32 and x.device == self.dev \
+                and x.shape == (self.n, self.n):
+            return x
         t = x if isinstance(x, torch.Tensor) else torch.as_tensor(np.asarray(x, np.float32))
         t = t.to(device=self.dev, dtype=torch.float32)
         if t.ndim == 0:

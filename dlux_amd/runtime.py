@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import math
 import os
 
 import numpy as np
@@ -49,21 +50,30 @@ def _prec_code(prec: str | None) -> int:
     return _PRECISIONS[name]
 
 
+_gpu_seen = False
+
+
 def device() -> torch.device:
     """The GPU the library runs on; raises if there is none (no CPU fallback)."""
-    if not torch.cuda.is_available():
-        raise RuntimeError("dlux_amd requires a ROCm GPU (gfx950); none is visible")
+    global _gpu_seen
+    if not _gpu_seen:   # a process does not lose its GPU: the query (3 us) is made until one is seen
+        if not torch.cuda.is_available():
+            raise RuntimeError("dlux_amd requires a ROCm GPU (gfx950); none is visible")
+        _gpu_seen = True
     return torch.device("cuda", torch.cuda.current_device())
 
 
 def stream_handle() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # the handle itself, without a Stream object around it: 1 us instead of 6-9
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def as_complex(x, dev=None) -> torch.Tensor:
     """Contiguous complex64 device tensor."""
     dev = dev or device()
     if isinstance(x, torch.Tensor):
+        if x.dtype is torch.complex64 and x.device == dev and x.is_contiguous():
+            return x
         t = x.to(device=dev)
         if not t.is_complex():
             t = t.to(torch.float32).to(torch.complex64)
@@ -75,6 +85,8 @@ def as_float(x, dev=None) -> torch.Tensor:
     """Contiguous float32 device tensor."""
     dev = dev or device()
     if isinstance(x, torch.Tensor):
+        if x.dtype is torch.float32 and x.device == dev and x.is_contiguous():
+            return x
         if x.is_complex():
             raise TypeError("expected a real array, got a complex one")
         return x.to(device=dev, dtype=torch.float32).contiguous()
@@ -218,7 +230,7 @@ def project_basis(basis, grad) -> torch.Tensor:
     dev = device()
     bt = as_float(basis, dev)
     nbasis = int(bt.shape[0])
-    npix = int(np.prod(bt.shape[1:]))
+    npix = math.prod(bt.shape[1:])
     gt = as_float(grad, dev)
     if gt.numel() % max(npix, 1) != 0:
         raise ValueError(f"grad of shape {tuple(gt.shape)} does not match basis pixels {npix}")
@@ -267,14 +279,14 @@ def eval_basis(basis, coeffs, base=None) -> torch.Tensor:
     bt = as_float(basis, dev)
     ct = as_float(coeffs, dev)
     lead = ct.shape
-    nb = int(np.prod(lead)) if ct.ndim else 1
+    nb = math.prod(lead) if ct.ndim else 1
     if tuple(bt.shape[: ct.ndim]) != tuple(lead):
         raise ValueError(
             "The leading basis dimensions must match the coefficient shape, "
             f"received {tuple(bt.shape)} and {tuple(lead)}."
         )
     pix_shape = tuple(bt.shape[ct.ndim:])
-    npix = int(np.prod(pix_shape))
+    npix = math.prod(pix_shape)
     base_t = None if base is None else as_float(base, dev)
     if torch.is_grad_enabled() and any(
             t is not None and t.requires_grad for t in (ct, bt, base_t)):
@@ -724,7 +736,7 @@ def _interp_prepare(images, dev):
     if x.ndim < 2 or x.shape[-1] != x.shape[-2]:
         raise ValueError(f"images must be (..., n, n), got {tuple(x.shape)}")
     lead = tuple(x.shape[:-2])
-    return x, lead, (int(np.prod(lead)) if lead else 1)
+    return x, lead, (math.prod(lead) if lead else 1)
 
 
 def _interp_transform_fwd(x, lead, batch, pixel_scale_in, center_in, n_out, pixel_scale_out,
@@ -899,7 +911,7 @@ def _detector_impl(images, ops) -> torch.Tensor:
         raise ValueError(f"detector input must be (..., n, n), got {tuple(x.shape)}")
     n = int(x.shape[-1])
     lead = tuple(x.shape[:-2])
-    batch = int(np.prod(lead)) if lead else 1
+    batch = math.prod(lead) if lead else 1
     lib = _lib.load()
     arr, keep = _detector_ops(ops, dev)
     side = ctypes.c_int32(0)
@@ -922,7 +934,7 @@ def _detector_vjp_impl(images, ops, dout, param_ops=()):
     g = as_float(dout, dev).contiguous()
     n = int(x.shape[-1])
     lead = tuple(x.shape[:-2])
-    batch = int(np.prod(lead)) if lead else 1
+    batch = math.prod(lead) if lead else 1
     lib = _lib.load()
     arr, keep = _detector_ops(ops, dev)
     side = ctypes.c_int32(0)
