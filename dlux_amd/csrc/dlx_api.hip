@@ -8,7 +8,6 @@
 
 #include "dlx_fold.h"
 #include "dlx_internal.h"
-#include "dlx_split.h"
 
 namespace dlx {
 
@@ -87,159 +86,11 @@ int check_geom(const dlx_mft_geom* g) {
 
 }  // namespace
 
-// Bytes of one batch instance of an R x K complex operand.
 size_t mat_bytes(long rows, long k, bool split) {
-  return split ? (size_t)rows * split4_row_bytes(k) : (size_t)rows * k * sizeof(float2);
-}
-
-// Generate `nb` transfer matrices with per-instance (lambda, dx, p_out, shift,
-// amplitude) into out[b] -- complex64 or split4 -- in launches of DftChunk::kMax.
-// The generator writes exp(sign 2 pi i u_r v_c) over rows r and columns c; the
-// adjoint W^H (rows k of the input plane, columns l of the output plane) is the
-// same phase with the two coordinate vectors swapped and the sign flipped.
-int gen_dft(const dlx_mft_geom& g, int nb, const double* wl, const double* dx,
-            const double* pout, const double* shift, const double* amp, void* out, bool split,
-            hipStream_t s, bool adjoint) {
-  const int rows = adjoint ? g.n_in : g.n_out, cols = adjoint ? g.n_out : g.n_in;
-  const int sign_inv = adjoint ? !g.inverse : g.inverse;
-  const long stride = (long)rows * cols;
-  const long bbytes = (long)mat_bytes(rows, cols, true);
-  for (int b0 = 0; b0 < nb; b0 += DftChunk::kMax) {
-    const int n = nb - b0 < DftChunk::kMax ? nb - b0 : DftChunk::kMax;
-    DftChunk c;
-    for (int i = 0; i < n; ++i) {
-      const int b = b0 + i;
-      DLX_CHECK_ARG(std::isfinite(wl[b]) && wl[b] > 0, "wavelength[%d] must be > 0", b);
-      DLX_CHECK_ARG(std::isfinite(dx[b]) && dx[b] != 0, "pixel_scale_in[%d] must be non-zero", b);
-      DLX_CHECK_ARG(std::isfinite(pout[b]), "pixel_scale_out[%d] must be finite", b);
-      const MftInst p = make_inst(g, wl[b], dx[b], pout[b], shift ? shift[b] : 0.0);
-      // columns carry the a (input-plane) vector, rows the b (output-plane) one
-      c.a_scale[i] = adjoint ? p.b_scale : p.a_scale;
-      c.a_off[i] = adjoint ? p.b_off : p.a_off;
-      c.b_scale[i] = adjoint ? p.a_scale : p.b_scale;
-      c.b_off[i] = adjoint ? p.a_off : p.b_off;
-      c.amp[i] = amp ? amp[b] : 1.0;
-    }
-    if (split) {
-      DLX_HIP(launch_dft_split4(c, n, cols, rows, sign_inv,
-                                (uint8_t*)out + (long)b0 * bbytes, bbytes, s));
-    } else {
-      DLX_HIP(launch_dft_chunk(c, n, cols, rows, sign_inv,
-                               (float2*)out + (long)b0 * stride, stride, s));
-    }
-  }
-  return DLX_OK;
+  return split ? (size_t)rows * ((k + 7) / 8) * 64 : (size_t)rows * k * sizeof(float2);
 }
 
 namespace {
-
-// Transfer matrices for `nb` instances: from the device cache, or generated
-// into `fallback` when the cache is bypassed (graph capture, no memory).
-int get_matrices(const dlx_mft_geom& g, int nb, const double* wl, const double* dx,
-                 const double* pout, const double* shift, bool split, void* fallback,
-                 hipStream_t s, void** out, void** handle, bool adjoint = false) {
-  if (int st = cache_acquire(g, nb, wl, dx, pout, shift, split, s, out, handle, adjoint))
-    return st;
-  if (*out) return DLX_OK;
-  *out = fallback;
-  return gen_dft(g, nb, wl, dx, pout, shift, nullptr, fallback, split, s, adjoint);
-}
-
-// FP32 two-stage MFT of `batch` complex64 fields P (N_in x N_in) against
-// complex64 transfer matrices Wx / Wy (N_out x N_in):
-//   stage 1: U^T = (P Wx^T)^T (complex64, N_out x N_in)
-//   stage 2: E = alpha_b Wy U, stored complex64 (EPI_STORE) or |E|^2 (EPI_INTENSITY).
-int mft_fp32(const dlx_mft_geom& g, int batch, const float2* P, const float2* Wx,
-             const float2* Wy, float2* U, const double* alpha, void* out, int epi,
-             hipStream_t s, bool prof) {
-  const long pstride = (long)g.n_in * g.n_in;
-  const long mstride = (long)g.n_out * g.n_in;
-  const long nout2 = (long)g.n_out * g.n_out;
-  for (int b0 = 0; b0 < batch; b0 += GemmBatch::kMaxBatch) {
-    const int nb = batch - b0 < GemmBatch::kMaxBatch ? batch - b0 : GemmBatch::kMaxBatch;
-    GemmBatch g1{};
-    g1.A = P + (long)b0 * pstride; g1.lda = g.n_in; g1.sA = pstride;
-    g1.B = Wx + (long)b0 * mstride; g1.ldb = g.n_in; g1.sB = mstride;
-    g1.C = U + (long)b0 * mstride; g1.ldc = g.n_in; g1.sC = mstride;
-    g1.M = g.n_in; g1.N = g.n_out; g1.K = g.n_in; g1.batch = nb;
-    g1.epilogue = EPI_STORE_T; g1.precision = DLX_PREC_FP32;
-    for (int i = 0; i < nb; ++i) g1.alpha[i] = 1.0f;
-    int slot = -1;
-    if (prof) { if (int st = prof_begin(1, s, &slot)) return st; }
-    DLX_HIP(launch_cgemm_nt(g1, s));
-    if (prof) { if (int st = prof_end(slot, s)) return st; }
-    GemmBatch g2{};
-    g2.A = Wy + (long)b0 * mstride; g2.lda = g.n_in; g2.sA = mstride;
-    g2.B = U + (long)b0 * mstride; g2.ldb = g.n_in; g2.sB = mstride;
-    g2.C = epi == EPI_STORE ? (void*)((float2*)out + (long)b0 * nout2)
-                            : (void*)((float*)out + (long)b0 * nout2);
-    g2.ldc = g.n_out; g2.sC = nout2;
-    g2.M = g.n_out; g2.N = g.n_out; g2.K = g.n_in; g2.batch = nb;
-    g2.epilogue = epi; g2.precision = DLX_PREC_FP32;
-    for (int i = 0; i < nb; ++i) g2.alpha[i] = (float)alpha[b0 + i];
-    if (prof) { if (int st = prof_begin(2, s, &slot)) return st; }
-    DLX_HIP(launch_cgemm_nt(g2, s));
-    if (prof) { if (int st = prof_end(slot, s)) return st; }
-  }
-  return DLX_OK;
-}
-
-// Split-BF16x3 two-stage MFT of `batch` split4 pupils P (N_in rows, k = N_in)
-// against split4 transfer matrices Wx / Wy (N_out rows, k = N_in):
-//   stage 1: U^T = (P Wx^T)^T written split4 (N_out rows, k = N_in)
-//   stage 2: E = alpha_b Wy U, stored complex64 (EPI_STORE) or |E|^2 (EPI_INTENSITY).
-// Stage 1's launch description for instances [b0, b0 + nb) of a batch.
-GemmSplit stage1_split(const dlx_mft_geom& g, int b0, int nb, const uint8_t* P,
-                       const uint8_t* Wx, uint8_t* U) {
-  const long pbytes = (long)mat_bytes(g.n_in, g.n_in, true);
-  const long wbytes = (long)mat_bytes(g.n_out, g.n_in, true);
-  const long rb = split4_row_bytes(g.n_in);
-  GemmSplit g1{};
-  g1.A = P ? P + (long)b0 * pbytes : nullptr; g1.a_row_bytes = rb; g1.a_batch_bytes = pbytes;
-  g1.B = Wx + (long)b0 * wbytes; g1.b_row_bytes = rb; g1.b_batch_bytes = wbytes;
-  g1.C = U + (long)b0 * wbytes; g1.ldc = rb; g1.c_batch = wbytes;
-  g1.M = g.n_in; g1.N = g.n_out; g1.K = g.n_in; g1.batch = nb; g1.epilogue = EPI_SPLIT_T;
-  for (int i = 0; i < nb; ++i) g1.alpha[i] = 1.0f;
-  return g1;
-}
-
-// With `pg` set, stage 1 generates the pupil in its loader (P unused; the
-// caller has checked cgemm_pupil_supported for every slice).
-int mft_split4(const dlx_mft_geom& g, int batch, const uint8_t* P, const uint8_t* Wx,
-               const uint8_t* Wy, uint8_t* U, const double* alpha, void* out, int epi,
-               hipStream_t s, int (*pb)(int, hipStream_t, int*), int (*pe)(int, hipStream_t),
-               const PupilGen* pg = nullptr) {
-  const long wbytes = (long)mat_bytes(g.n_out, g.n_in, true);
-  const long rb = split4_row_bytes(g.n_in);
-  const long nout2 = (long)g.n_out * g.n_out;
-  for (int b0 = 0; b0 < batch; b0 += GemmSplit::kMaxBatch) {
-    const int nb = batch - b0 < GemmSplit::kMaxBatch ? batch - b0 : GemmSplit::kMaxBatch;
-    const GemmSplit g1 = stage1_split(g, b0, nb, P, Wx, U);
-    int slot = -1;
-    if (pb) { if (int st = pb(1, s, &slot)) return st; }
-    if (pg) {
-      PupilGen p = *pg;
-      for (int i = 0; i < nb; ++i) p.inv_wl[i] = pg->inv_wl[b0 + i];
-      DLX_HIP(launch_cgemm_pupil(g1, p, s));
-    } else {
-      DLX_HIP(launch_cgemm_split4(g1, s));
-    }
-    if (pe) { if (int st = pe(slot, s)) return st; }
-    GemmSplit g2{};
-    g2.A = Wy + (long)b0 * wbytes; g2.a_row_bytes = rb; g2.a_batch_bytes = wbytes;
-    g2.B = U + (long)b0 * wbytes; g2.b_row_bytes = rb; g2.b_batch_bytes = wbytes;
-    g2.ldc = g.n_out;
-    g2.c_batch = nout2;
-    g2.C = epi == EPI_STORE ? (void*)((float2*)out + (long)b0 * nout2)
-                            : (void*)((float*)out + (long)b0 * nout2);
-    g2.M = g.n_out; g2.N = g.n_out; g2.K = g.n_in; g2.batch = nb; g2.epilogue = epi;
-    for (int i = 0; i < nb; ++i) g2.alpha[i] = (float)alpha[b0 + i];
-    if (pb) { if (int st = pb(2, s, &slot)) return st; }
-    DLX_HIP(launch_cgemm_split4(g2, s));
-    if (pe) { if (int st = pe(slot, s)) return st; }
-  }
-  return DLX_OK;
-}
 
 // The psf chain's buffers for a chunk of c wavelengths: the tables (used when
 // they are not taken from the cache), the stage-1 result, the per-wavelength
@@ -390,8 +241,29 @@ int dlx_transfer_matrix(const dlx_mft_geom* geom, int32_t batch, const double* w
   if (batch == 0) return DLX_OK;
   DLX_CHECK_ARG(wavelength && pixel_scale_in && pixel_scale_out && out,
                 "null argument to dlx_transfer_matrix");
-  return gen_dft(*geom, batch, wavelength, pixel_scale_in, pixel_scale_out, shift, nullptr,
-                 out, false, (hipStream_t)stream);
+  const dlx_mft_geom& g = *geom;
+  const long stride = (long)g.n_out * g.n_in;
+  for (int b0 = 0; b0 < batch; b0 += DftChunk::kMax) {
+    const int n = batch - b0 < DftChunk::kMax ? batch - b0 : DftChunk::kMax;
+    DftChunk c;
+    for (int i = 0; i < n; ++i) {
+      const int b = b0 + i;
+      DLX_CHECK_ARG(std::isfinite(wavelength[b]) && wavelength[b] > 0,
+                    "wavelength[%d] must be > 0", b);
+      DLX_CHECK_ARG(std::isfinite(pixel_scale_in[b]) && pixel_scale_in[b] != 0,
+                    "pixel_scale_in[%d] must be non-zero", b);
+      DLX_CHECK_ARG(std::isfinite(pixel_scale_out[b]), "pixel_scale_out[%d] must be finite", b);
+      const MftInst p = make_inst(g, wavelength[b], pixel_scale_in[b], pixel_scale_out[b],
+                                  shift ? shift[b] : 0.0);
+      c.a_scale[i] = p.a_scale;
+      c.a_off[i] = p.a_off;
+      c.b_scale[i] = p.b_scale;
+      c.b_off[i] = p.b_off;
+    }
+    DLX_HIP(launch_dft_chunk(c, n, g.n_in, g.n_out, g.inverse, (float2*)out + (long)b0 * stride,
+                             stride, (hipStream_t)stream));
+  }
+  return DLX_OK;
 }
 
 size_t dlx_mft_workspace_size(const dlx_mft_geom* geom, int32_t batch, int32_t precision) {

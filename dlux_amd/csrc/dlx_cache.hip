@@ -1,14 +1,14 @@
-// Device-resident cache of transfer matrices.
+// Device-resident cache of the contractions' tables.
 //
-// The transfer matrices of an MFT depend only on geometry and per-instance
-// (wavelength, pixel scales, shift) -- not on the field or the weights -- so
-// repeated propagations (phase-retrieval iterations, a serving loop over the
-// same wavelength grid) reuse them instead of regenerating N_out x N_in
-// complex exponentials per call.  An entry holds the matrices of one batch of
-// instances, contiguous, in complex64 or split4 form.
+// The cosine / sine tables of a folded MFT depend only on its sides and phase
+// steps -- not on the field, the shifts or the weights -- so repeated
+// propagations (phase-retrieval iterations, a serving loop over the same
+// wavelength grid) reuse them instead of generating them per call.  An entry
+// holds the tables of one call's wavelengths, in both directions, or the plan
+// and tables of one uneven batch.
 //
 // Stream safety: an entry records an event after its generation; a user on any
-// stream waits on it (hipStreamWaitEvent) before the matrices are read.  Each
+// stream waits on it (hipStreamWaitEvent) before the tables are read.  Each
 // stream that used an entry keeps its own "last use" event on the entry, and
 // eviction synchronises on every one of them before the block is reused, so a
 // block read by work still queued on one stream is never handed to another.
@@ -17,18 +17,15 @@
 // on the device (hipStreamWaitEvent) before writing it; only a release to
 // hipFree synchronises on them.
 // An entry is pinned from its acquire to its release: eviction skips pinned
-// entries (a call that holds two entries, such as the gradient's forward and
-// adjoint matrices, can never have the first evicted to make room for the
-// second), and an acquire that finds no room falls back to the workspace.
+// entries, and an acquire that finds no room falls back to the workspace.
 // The cache is bypassed while the stream is being captured into a graph
-// (allocation and event records are not capturable); callers then generate the
-// matrices into their workspace.
+// (allocation and event records are not capturable); callers then generate
+// the tables into their workspace.
 #include <cstring>
 #include <mutex>
 #include <vector>
 
 #include "dlx_internal.h"
-#include "dlx_split.h"
 
 namespace dlx {
 namespace {
@@ -199,72 +196,6 @@ void* take_block(MatCache& c, size_t need, int dev, hipStream_t s, size_t* bytes
 
 }  // namespace
 
-int cache_acquire(const dlx_mft_geom& g, int nb, const double* wl, const double* dx,
-                  const double* pout, const double* shift, bool split, hipStream_t s,
-                  void** ptr, void** handle, bool adjoint) {
-  *ptr = nullptr;
-  *handle = nullptr;
-  MatCache& c = cache();
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &cs) != hipSuccess) {
-    (void)hipGetLastError();
-    return DLX_OK;
-  }
-  if (cs != hipStreamCaptureStatusNone || c.budget == 0 || t_bypass) return DLX_OK;
-  int dev = 0;
-  DLX_HIP(hipGetDevice(&dev));
-
-  std::vector<double> key;
-  key.reserve(9 + 4 * (size_t)nb);
-  key.insert(key.end(), {(double)dev, (double)g.n_in, (double)g.n_out, (double)g.inverse,
-                         (double)g.has_focal, g.has_focal ? g.focal_length : 0.0,
-                         g.has_focal ? g.focal_shift : 0.0, (split ? 1.0 : 0.0) + (adjoint ? 2.0 : 0.0),
-                         (double)nb});
-  key.insert(key.end(), wl, wl + nb);
-  key.insert(key.end(), dx, dx + nb);
-  key.insert(key.end(), pout, pout + nb);
-  for (int i = 0; i < nb; ++i) key.push_back(shift ? shift[i] : 0.0);
-
-  std::lock_guard<std::mutex> lock(c.mu);
-  for (MatEntry* e : c.entries) {
-    if (e->key.size() == key.size() &&
-        std::memcmp(e->key.data(), key.data(), key.size() * sizeof(double)) == 0) {
-      e->tick = ++c.tick;
-      ++c.hits;
-      DLX_HIP(hipStreamWaitEvent(s, e->ready, 0));
-      ++e->pins;
-      *ptr = e->ptr;
-      *handle = e;
-      return DLX_OK;
-    }
-  }
-  ++c.misses;
-  const size_t per = adjoint ? mat_bytes(g.n_in, g.n_out, split)
-                             : mat_bytes(g.n_out, g.n_in, split);
-  const size_t need = align_up(per * (size_t)nb);
-  if (need > c.budget) return DLX_OK;  // larger than the whole cache: caller generates
-  if (!make_room(c, need)) return DLX_OK;  // pinned entries fill it: caller generates
-  size_t bytes = 0;
-  void* mem = take_block(c, need, dev, s, &bytes);
-  if (!mem) return DLX_OK;  // no memory for the cache: caller generates into its workspace
-  MatEntry* e = new_entry(std::move(key), dev, mem, bytes, ++c.tick);
-  if (!e) {
-    (void)hipFree(mem);
-    set_error("hipEventCreate failed in the matrix cache");
-    return DLX_ERR_HIP;
-  }
-  if (int st = gen_dft(g, nb, wl, dx, pout, shift, nullptr, mem, split, s, adjoint)) {
-    free_entry(c, e, true);
-    return st;
-  }
-  DLX_HIP(hipEventRecord(e->ready, s));
-  c.entries.push_back(e);
-  c.used += bytes;
-  *ptr = mem;
-  *handle = e;
-  return DLX_OK;
-}
-
 uint64_t hash_key(const std::vector<double>& key) {
   uint64_t h = 1469598103934665603ull;   // FNV-1a over the key bytes
   const uint8_t* p = (const uint8_t*)key.data();
@@ -290,9 +221,8 @@ int cache_acquire_raw(const std::vector<double>& key_in, size_t bytes, hipStream
   int dev = 0;
   DLX_HIP(hipGetDevice(&dev));
   std::vector<double> key;
-  key.reserve(key_in.size() + 3);
-  // tag raw entries so they never compare equal to an MFT batch key
-  key.insert(key.end(), {-1.0, (double)dev, (double)bytes});
+  key.reserve(key_in.size() + 2);
+  key.insert(key.end(), {(double)dev, (double)bytes});
   key.insert(key.end(), key_in.begin(), key_in.end());
 
   std::lock_guard<std::mutex> lock(c.mu);

@@ -1,11 +1,11 @@
 // Backward-pass kernels of the polychromatic PSF (gfx950).
 //
-// The adjoint contractions themselves run on the complex GEMMs (dlx_gemm*.hip)
-// with gradient epilogues; this file holds the two reductions around them:
+// The adjoint contractions themselves are the folded ones (dlx_fold.hip) with
+// gradient epilogues; this file holds the two reductions around them:
 //
 //   grad_reduce:    dL/dOPD(p) = sum_l k_l h_l(p),  dL/dphase(p) = sum_l h_l(p)
 //                   over the per-wavelength planes h_l = Im(conj(P_l) Pbar_l)
-//                   written by the last adjoint GEMM (k_l = 2 pi / lambda_l);
+//                   written by the last adjoint contraction (k_l = 2 pi / lambda_l);
 //   project_basis:  dL/dc[s, j] = sum_p basis[j, p] g[s, p]
 //                   (the transpose of eval_basis), deterministic two-pass sum.
 //

@@ -85,98 +85,11 @@ inline double mft_norm(const dlx_mft_geom& g, double wavelength, double dx_in,
 // kernels implemented in the .hip files, launched from the host orchestration
 // ---------------------------------------------------------------------------
 
-// Complex NT GEMM C[b](m,n) = sum_k A[b](m,k) B[b](n,k), then an epilogue.
-enum Epilogue {
-  EPI_STORE = 0,        // C = alpha * acc (complex64), ldc
-  EPI_STORE_T = 1,      // C^T = alpha * acc: written at C[n*ldc + m]
-  EPI_INTENSITY = 2,    // I = |alpha * acc|^2 (float32), ldc
-  EPI_SPLIT_T = 3,      // split4 matrix with rows n and k = m (ldc / c_batch in bytes)
-  // gradient epilogues (G = dL/dPSF, float, ldg / g_batch in elements)
-  EPI_VJP = 4,          // C(m,n) = 2 G(m,n) alpha acc (complex64, ldc)
-  EPI_VJP_SPLIT_T = 5,  // as EPI_SPLIT_T with value 2 G(n,m) alpha acc (split4 rows n, k = m)
-  EPI_GRAD = 6,         // C(m,n) = Im(conj(P(m,n)) alpha acc) (float, ldc); P complex64
-                        // (fp32 kernels, p_ld elements) or split4 (p_ld bytes per row);
-                        // C2 (if set, same layout as C) = Re(conj(U(m,n)) alpha acc),
-                        // U in P's layout
-};
-
-struct GemmBatch {
-  static constexpr int kMaxBatch = 64;   // instances per launch
-  const float2* A; long lda; long sA;
-  const float2* B; long ldb; long sB;
-  void* C; long ldc; long sC;
-  int M, N, K, batch;
-  int epilogue;
-  int precision;        // DLX_PREC_*
-  float alpha[kMaxBatch];   // per-instance scale of the result
-  const float* G; long ldg; long g_batch;          // EPI_VJP
-  const void* P; long p_ld; long p_batch;           // EPI_GRAD
-  float* C2;                                        // EPI_GRAD real part (optional)
-  const void* U;                                    // EPI_GRAD: phasor for C2, P's layout
-};
-
-hipError_t launch_cgemm_nt(const GemmBatch& g, hipStream_t s);
-
-// Split-BF16x3 complex NT GEMM on split4 operands (dlx_split.h).  Row strides
-// and batch strides of A and B are in bytes; C strides are in elements
-// (EPI_STORE / EPI_INTENSITY) or bytes (EPI_SPLIT_T).  alpha is per batch.
-struct GemmSplit {
-  static constexpr int kMaxBatch = 64;
-  const uint8_t* A; long a_row_bytes; long a_batch_bytes;
-  const uint8_t* B; long b_row_bytes; long b_batch_bytes;
-  void* C; long ldc; long c_batch;
-  int M, N, K, batch, epilogue;
-  float alpha[kMaxBatch];
-  const float* G; long ldg; long g_batch;          // EPI_VJP_SPLIT_T
-  const void* P; long p_ld; long p_batch;           // EPI_GRAD (split4, bytes)
-  float* C2;                                        // EPI_GRAD real part (optional)
-  const void* U;                                    // EPI_GRAD: phasor for C2, P's layout
-};
-
-hipError_t launch_cgemm_split4(const GemmSplit& g, hipStream_t s);
-
-// The pupil of instance b, generated in the stage-1 loader instead of read
-// from A:  A[b](y, x) = a(y, x) exp(2 pi i path(y, x) inv_wl[b]) with
-// path = tx X + ty Y + opd (FP64) and a = scale amp, formed from the caller's
-// amplitude and OPD planes (n x n, row-major, float; either may be null) as
-// the pupil kernels form them (dlx_phasor.h).
-struct PupilGen {
-  const float* opd; const float* amp;
-  double dx, x0, tx, ty;
-  float scale;
-  int n;
-  double inv_wl[GemmSplit::kMaxBatch];
-};
-// Stage 1 (EPI_SPLIT_T, K = M = pg.n) with the pupil as A.  Returns
-// hipErrorNotSupported, launching nothing, for shapes it does not cover
-// (cgemm_pupil_supported is false; the caller then writes the pupil and calls
-// launch_cgemm_split4).
-hipError_t launch_cgemm_pupil(const GemmSplit& g, const PupilGen& pg, hipStream_t s);
-bool cgemm_pupil_supported(const GemmSplit& g, const PupilGen& pg);
-
-// One problem of a grouped (uneven) split4 GEMM, in device memory.  Its
-// 128 x tile_n tiles are [tile_start, tile_start + tiles_m * tiles_n) of the
-// launch's tile list, row-major over (tm, tn).
-struct GroupProblem {
-  const uint8_t* A; const uint8_t* B; void* C;
-  long a_row_bytes, b_row_bytes, ldc;
-  int M, N, K, tiles_n, tiles_m, tile_start;
-  float alpha; int pad_;
-};
-struct GroupLaunch {
-  const GroupProblem* probs;   // device array, sorted by tile_start
-  int nprobs;
-  int tile_n;                  // 128, or 64 for launches of problems with N <= 64
-  int xcd_start[9];            // tile range of XCD x: [xcd_start[x], xcd_start[x+1])
-};
-// Epilogues supported: EPI_STORE, EPI_SPLIT_T, EPI_INTENSITY.
-hipError_t launch_cgemm_split4_group(const GroupLaunch& gl, int epilogue, hipStream_t s);
-
 // Per-launch instance parameters passed by value (kernel arguments), so no
 // device-side parameter buffer is needed.
 struct DftChunk {
   static constexpr int kMax = 48;
-  double a_scale[kMax], a_off[kMax], b_scale[kMax], b_off[kMax], amp[kMax];
+  double a_scale[kMax], a_off[kMax], b_scale[kMax], b_off[kMax];
 };
 struct PupilChunk {
   static constexpr int kMax = 128;
@@ -192,35 +105,16 @@ hipError_t launch_dft_chunk(const DftChunk& c, int nb, int n_in, int n_out, int 
                             float2* out, long bstride, hipStream_t s);
 
 // Linear canonical transforms (dlx_lct.hip): per-instance phase polynomials in turns.
-struct LctMatChunk {
-  static constexpr int kMax = 48;
-  double ci2[kMax], co2[kMax], cx[kMax], c0[kMax];
-};
 struct LctChirpChunk {
   static constexpr int kMax = 48;
   double q2[kMax], q1[kMax], q0[kMax], x0[kMax], dx[kMax];   // grid x_k = x0 + k dx
 };
-hipError_t launch_lct_matrix(const LctMatChunk& c, int nb, int n_in, int n_out, double x0_in,
-                             double dx_in, double x0_out, double dx_out, float2* out,
-                             long bstride, hipStream_t s);
-hipError_t launch_lct_matrix_split4(const LctMatChunk& c, int nb, int n_in, int n_out,
-                                    double x0_in, double dx_in, double x0_out, double dx_out,
-                                    uint8_t* out, long batch_bytes, hipStream_t s);
 hipError_t launch_lct_chirp(const LctChirpChunk& c, int nb, int n, const float2* in,
                             float2* out, hipStream_t s);
 hipError_t launch_pupil_chunk(const PupilChunk& c, int nb, int n, double dx, double x0,
                               double tx, double ty, const float* amp, const float* opd,
                               const float* phase, float scale, const float2* in,
                               float2* out, hipStream_t s);
-// split4 producers
-hipError_t launch_dft_split4(const DftChunk& c, int nb, int n_in, int n_out, int inverse,
-                             uint8_t* out, long batch_bytes, hipStream_t s);
-hipError_t launch_pupil_split4(const PupilChunk& c, int nb, int n, double dx, double x0,
-                               double tx, double ty, const float* amp, const float* opd,
-                               const float* phase, float scale, uint8_t* out, long batch_bytes,
-                               hipStream_t s);
-hipError_t launch_to_split4(const float2* in, int batch, long rows, int k, long in_batch,
-                            uint8_t* out, long out_batch_bytes, hipStream_t s);
 hipError_t launch_eval_basis(int nbasis, long npix, int nsets, const float* basis,
                              const float* coeffs, const float* base, float* out,
                              hipStream_t s);
@@ -238,28 +132,17 @@ int project_parts(long npix);
 hipError_t launch_project_basis(int nbasis, long npix, int nsets, const float* basis,
                                 const float* g, float* partial, float* out, hipStream_t s);
 
-// Bytes of one batch instance of an R x K complex operand (complex64 or split4).
+// Bytes of an R x K complex array in the plain layouts that the workspace sizes
+// are stated in: complex64, or (split) four bf16 planes of k in chunks of 8.
 size_t mat_bytes(long rows, long k, bool split);
 
-// Generate `nb` transfer matrices (optionally scaled by amp[b]) into `out`:
-// W (N_out x N_in) or, with `adjoint`, its conjugate transpose W^H (N_in x N_out).
-int gen_dft(const dlx_mft_geom& g, int nb, const double* wl, const double* dx,
-            const double* pout, const double* shift, const double* amp, void* out, bool split,
-            hipStream_t s, bool adjoint = false);
-
-// Device-resident transfer-matrix cache (dlx_cache.hip).  On success *ptr is
-// either the cached matrices (ready for work enqueued on s) or NULL when the
-// cache was bypassed; cache_release records the entry's last use on s.
-int cache_acquire(const dlx_mft_geom& g, int nb, const double* wl, const double* dx,
-                  const double* pout, const double* shift, bool split, hipStream_t s,
-                  void** ptr, void** handle, bool adjoint = false);
+// Device-resident cache of tables (dlx_cache.hip), keyed by the caller: on a
+// hit (*fresh false) the block is ready for work on s; on a miss (*fresh true)
+// the caller fills it on s and then calls cache_ready.  *ptr == NULL (and
+// *fresh true) when bypassed (capture, budget, memory): the caller generates
+// into its own buffer.  The block is allocated on a key's second sighting, or
+// on the first with `eager`.  cache_release records the entry's last use on s.
 int cache_release(void* handle, hipStream_t s);
-// Raw entries keyed by the caller: on a hit (*fresh false) the block is ready
-// for work on s; on a miss (*fresh true) the caller fills it on s and then
-// calls cache_ready.  *ptr == NULL (and *fresh true) when bypassed (capture,
-// budget, memory): the caller generates into its own buffer.
-// The block is allocated on a key's second sighting, or on the first with
-// `eager`.
 int cache_acquire_raw(const std::vector<double>& key, size_t bytes, hipStream_t s,
                       void** ptr, void** handle, bool* fresh, bool eager = false);
 int cache_ready(void* handle, hipStream_t s);

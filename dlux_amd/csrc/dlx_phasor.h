@@ -1,7 +1,7 @@
-// Pupil phasor shared by every pupil producer: the complex64 and split4 pupil
-// kernels and the contraction whose loader generates the pupil on chip.  One
-// definition, with the fused multiply-adds written out, so all of them give
-// the same bits for the same pixel and wavelength.
+// Pupil phasor shared by every pupil producer: the complex64 pupil kernel, the
+// folded pupil kernel, the contraction whose loader forms the pupil on chip and
+// the gradient's epilogue.  One definition, with the fused multiply-adds written
+// out, so all of them give the same bits for the same pixel and wavelength.
 //
 //   P(y, x) = a(y, x) exp(2 pi i t),
 //   t = (opd(y, x) + tx X + ty Y) / lambda + phase(y, x) / (2 pi)   [turns]

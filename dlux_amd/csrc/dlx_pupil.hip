@@ -4,12 +4,11 @@
 // 8/16-byte accesses with one pixel (or four) per lane.
 #include "dlx_internal.h"
 #include "dlx_phasor.h"
-#include "dlx_split.h"
 
 namespace dlx {
 
 // ---------------------------------------------------------------------------
-// Transfer matrix  W[b][l][k] = amp_b * exp(sign * 2 pi i * a_k * b_l)
+// Transfer matrix  W[b][l][k] = exp(sign * 2 pi i * a_k * b_l)
 // (utils/propagation.py:109-127, stored transposed: N_out x N_in).
 // The product a_k*b_l is formed in FP64 and reduced to [-1/2, 1/2] turns, so
 // the FP32 sincospi sees an argument with an absolute error of ~1e-17 turns.
@@ -27,8 +26,7 @@ dft_matrix_kernel(DftChunk c, int n_in, int n_out, int inverse, float2* __restri
   t -= rint(t);
   float s, co;
   sincospif(2.0f * (float)t, &s, &co);
-  const float amp = (float)c.amp[b];
-  out[(long)b * bstride + (long)l * n_in + k] = make_float2(amp * co, inverse ? amp * s : -amp * s);
+  out[(long)b * bstride + (long)l * n_in + k] = make_float2(co, inverse ? s : -s);
 }
 
 hipError_t launch_dft_chunk(const DftChunk& c, int nb, int n_in, int n_out, int inverse,
@@ -74,128 +72,6 @@ hipError_t launch_pupil_chunk(const PupilChunk& c, int nb, int n, double dx, dou
   dim3 grid((unsigned)((npix + 255) / 256), nb);
   hipLaunchKernelGGL(pupil_field_kernel, grid, dim3(256), 0, s, c, n, dx, x0, tx, ty, amp,
                      opd, phase, scale, in, out, npix);
-  return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
-// split4 producers: one lane per 8-element chunk, four 16-byte stores.
-// ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256)
-dft_split4_kernel(DftChunk c, int n_in, int n_out, int inverse, uint8_t* __restrict__ out,
-                  long batch_bytes) {
-  // a quad of lanes per chunk: lane q computes elements 2q, 2q+1 (quad-cooperative store)
-  const long kc = split4_chunks(n_in);
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const int b = blockIdx.y;
-  if (t >= (long)n_out * kc * 4) return;   // whole quads exit together
-  const int q = (int)(t & 3);
-  const long cidx = t >> 2;
-  const int l = (int)(cidx / kc), ch = (int)(cidx - (long)l * kc);
-  const double bb = (double)l * c.b_scale[b] + c.b_off[b];
-  const float amp = (float)c.amp[b];
-  float2 v[2];
-#pragma unroll
-  for (int e = 0; e < 2; ++e) {
-    const int k = ch * 8 + 2 * q + e;
-    if (k < n_in) {
-      const double a = (double)k * c.a_scale[b] + c.a_off[b];
-      double ph = a * bb;
-      ph -= rint(ph);
-      // hardware sin/cos take turns; max abs error 1.3e-7 on [-1/2, 1/2], far below
-      // the 2^-17 relative resolution of the split-BF16 pair
-      const float sn = __builtin_amdgcn_sinf((float)ph), co = __builtin_amdgcn_cosf((float)ph);
-      v[e] = make_float2(amp * co, inverse ? amp * sn : -amp * sn);
-    } else {
-      v[e] = make_float2(0.f, 0.f);
-    }
-  }
-  store_chunk_quad(out + (long)b * batch_bytes, l, split4_row_bytes(n_in), ch, q, v[0], v[1]);
-}
-
-hipError_t launch_dft_split4(const DftChunk& c, int nb, int n_in, int n_out, int inverse,
-                             uint8_t* out, long batch_bytes, hipStream_t s) {
-  const long work = (long)n_out * split4_chunks(n_in) * 4;
-  hipLaunchKernelGGL(dft_split4_kernel, dim3((unsigned)((work + 255) / 256), nb), dim3(256), 0,
-                     s, c, n_in, n_out, inverse, out, batch_bytes);
-  return hipGetLastError();
-}
-
-// Pupil field in split4 (rows y, k = x).  A quad of lanes produces one chunk
-// (8 pixels): lane q loads pixels 2q, 2q+1 of amplitude / OPD / phase once and
-// emits them for up to 16 wavelengths with quad-cooperative 16-byte stores.
-constexpr int kPupilWl = 16;
-
-__global__ void __launch_bounds__(256)
-pupil_split4_kernel(PupilChunk c, int nb, int n, double dx, double x0, double tx, double ty,
-                    const float* __restrict__ amp, const float* __restrict__ opd,
-                    const float* __restrict__ phase, float scale, uint8_t* __restrict__ out,
-                    long batch_bytes) {
-  const long kc = split4_chunks(n);
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  // the work size is a multiple of 4 and of the quad alignment: whole quads exit together
-  if (t >= (long)n * kc * 4) return;
-  const int q = (int)(t & 3);
-  const long cidx = t >> 2;
-  const int y = (int)(cidx / kc), ch = (int)(cidx - (long)y * kc);
-  const double tyY = ty * pupil_coord(y, dx, x0);
-  double path[2], turns0[2];
-  float a[2];
-#pragma unroll
-  for (int e = 0; e < 2; ++e) {
-    const int x = ch * 8 + 2 * q + e;
-    const bool in = x < n;
-    const long p = (long)y * n + x;
-    path[e] = pupil_path(tx, pupil_coord(x, dx, x0), tyY, (in && opd) ? (double)opd[p] : 0.0);
-    turns0[e] = (in && phase) ? (double)phase[p] * 0.15915494309189535 : 0.0;
-    a[e] = in ? scale * (amp ? amp[p] : 1.0f) : 0.f;
-  }
-  const int b0 = blockIdx.y * kPupilWl;
-  const int b1 = b0 + kPupilWl < nb ? b0 + kPupilWl : nb;
-  const long rb = split4_row_bytes(n);
-  for (int b = b0; b < b1; ++b) {
-    float2 v[2];
-#pragma unroll
-    for (int e = 0; e < 2; ++e) v[e] = pupil_phasor(path[e], c.inv_wl[b], turns0[e], a[e]);
-    store_chunk_quad(out + (long)b * batch_bytes, y, rb, ch, q, v[0], v[1]);
-  }
-}
-
-hipError_t launch_pupil_split4(const PupilChunk& c, int nb, int n, double dx, double x0,
-                               double tx, double ty, const float* amp, const float* opd,
-                               const float* phase, float scale, uint8_t* out, long batch_bytes,
-                               hipStream_t s) {
-  const long work = (long)n * split4_chunks(n) * 4;
-  dim3 grid((unsigned)((work + 255) / 256), (nb + kPupilWl - 1) / kPupilWl);
-  hipLaunchKernelGGL(pupil_split4_kernel, grid, dim3(256), 0, s, c, nb, n, dx, x0, tx, ty, amp,
-                     opd, phase, scale, out, batch_bytes);
-  return hipGetLastError();
-}
-
-// complex64 rows x k -> split4 (per batch instance).
-__global__ void __launch_bounds__(256)
-to_split4_kernel(const float2* __restrict__ in, long rows, int k, long in_batch,
-                 uint8_t* __restrict__ out, long out_batch_bytes) {
-  const long kc = split4_chunks(k);
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const int b = blockIdx.y;
-  if (t >= rows * kc) return;
-  const long r = t / kc;
-  const int ch = (int)(t - r * kc);
-  const float2* src = in + (long)b * in_batch + r * k;
-  float2 v[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const int x = ch * 8 + e;
-    v[e] = x < k ? src[x] : make_float2(0.f, 0.f);
-  }
-  store_chunk(out + (long)b * out_batch_bytes, r, split4_row_bytes(k), ch, v);
-}
-
-hipError_t launch_to_split4(const float2* in, int batch, long rows, int k, long in_batch,
-                            uint8_t* out, long out_batch_bytes, hipStream_t s) {
-  const long work = rows * split4_chunks(k);
-  hipLaunchKernelGGL(to_split4_kernel, dim3((unsigned)((work + 255) / 256), batch), dim3(256),
-                     0, s, in, rows, k, in_batch, out, out_batch_bytes);
   return hipGetLastError();
 }
 

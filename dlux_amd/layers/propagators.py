@@ -96,7 +96,7 @@ class ASMPropagator(OpticalLayer):
 # ---------------------------------------------------------------------------
 # ABCD elements and LCT propagators (layers/abcd_propagators.py:23-383).  The
 # matrices are the textbook ray-transfer matrices; the transforms are the
-# Collins integral, run on the device by dlx_lct (two complex GEMMs) and
+# Collins integral, run on the device by dlx_lct (the folded MFT between chirps) and
 # dlx_lct_fft (chirp, centred FFT, chirp).
 # ---------------------------------------------------------------------------
 
@@ -195,8 +195,8 @@ def _wf_grid(wavefront):
 
 
 class MFTPropagator(ABCDPropagator):
-    """LCT to the grid of a CoordSpec (n, d, c) by the Collins integral as two
-    complex GEMMs (dlx_lct).  Replaces abcdLux.lct.lct_prop
+    """LCT to the grid of a CoordSpec (n, d, c) by the Collins integral as the
+    folded MFT between two chirps (dlx_lct).  Replaces abcdLux.lct.lct_prop
     (abcd_propagators.py:245-297)."""
 
     def __call__(self, wavefront: Wavefront) -> Wavefront:
@@ -213,7 +213,7 @@ class FFTPropagator(ABCDPropagator):
     """LCT on the FFT grid of n_padded points, d_out = lambda |B| / (n_padded
     d_in), centred on the spec's c, then the PadSpec crop
     (abcd_propagators.py:300-383).  dlx_lct_fft (chirp, centred FFT, chirp)
-    for power-of-two grids; the same transform by dlx_lct's GEMMs otherwise."""
+    for power-of-two grids; the same transform by dlx_lct otherwise."""
 
     def __init__(self, ABCDs, spec):
         if isinstance(spec, CoordSpec) and spec.d is not None:

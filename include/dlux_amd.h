@@ -501,7 +501,7 @@ int dlx_asm_prop(int32_t n, int32_t m, int32_t batch, const double* wavelength,
  *               exp(i pi / (lambda B) (A x^2 - 2 x x' + D x'^2)),
  * on x = center_in + (k - (N_in-1)/2) pixel_scale_in and
  * x' = center_out + (l - (N_out-1)/2) pixel_scale_out; the 2-D field maps as
- * K u K^T with two complex GEMMs (the MFT's), precision as for dlx_mft.
+ * K u K^T with the MFT's two contractions, precision as for dlx_mft.
  * wavelength[b] per field.  Replaces abcdLux.lct.lct_prop as called by
  * MFTPropagator (layers/abcd_propagators.py:245-297); abcdLux is not
  * available, so this follows the textbook Collins integral (the sign, the
