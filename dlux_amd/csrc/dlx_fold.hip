@@ -594,6 +594,155 @@ fold_stage1_kernel(FoldStage1 a) {
   stage1_store<BF, BNQ>(lds + wave * kPatch, acc, a.n, a.m, a.out + (long)b * a.out_stride, py0, q0);
 }
 
+// Launches with few tiles (fold_stage1_kernel at 32 columns leaves compute units
+// idle): 16 rows py and 32 columns a workgroup, stages of 32 k in two runs of 16.
+// A tile row block is one (alpha, beta) with its real rows 0-15 and imaginary
+// rows 16-31; wave (alpha, beta) accumulates it.  Twice the workgroups, half the
+// products of a wave and half the stages to step through: a chain of load,
+// form, product bounds such launches.  28.6 -> 20.1 us at 2 wavelengths of
+// 1024^2 -> 256^2 (split), 39.1 -> 24.1 at one of 1024^2 -> 512^2 (float32),
+// 20.2 -> 13.9 at 7 of 333^2 -> 111^2 (split, tilted).
+template <bool BF, int LOAD, bool VEC>
+__global__ void __launch_bounds__(kThreads, 2)
+fold_stage1_small_kernel(FoldStage1 a) {
+  constexpr int kRun = 128 * kRow;   // one run of 16 k: 128 tile rows
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[4 * kRun];
+  __shared__ float4 win[2][2 * kStageK];   // the x phase of a stage's k, at k+ and k-
+  const int kh = fold_half(a.n), mh = fold_half(a.m), mhp = fold_pad(mh), kp = fold_pad(kh);
+  const int tq = (mh + 31) / 32, tp = (kh + 15) / 16;
+  const int id = xcd_order(blockIdx.x, tq * tp * a.batch);
+  const int b = id / (tq * tp), t = id - b * (tq * tp);
+  const int py0 = (t / tq) * 16, q0 = (t % tq) * 32;
+  const int nst = kp / (2 * kStageK);
+  const int wave = threadIdx.x >> 6;
+  const uint8_t* tab = a.table + (long)b * a.table_stride + table_block(wave >> 1, mhp, kp, q0 / 32);
+  const int py = threadIdx.x >> 4, beta = threadIdx.x & 1, quad = (threadIdx.x >> 1) & 3;
+  const int run = (threadIdx.x >> 3) & 1;
+  std::conditional_t<LOAD == FOLD_FIELD, FieldLoad<VEC>, PupilLoad<VEC, LOAD == kPupilTilt, false>> ld;
+  FoldPhase ph{};
+  bool phased = false;
+  if constexpr (LOAD != FOLD_FIELD) {
+    ld.init(a.pupil, a.n, py0 + py, beta, quad, a.inv_wl[b]);
+  } else {
+    ld.init(a.src + (long)b * a.src_stride, a.n, py0 + py, beta, quad);
+    ph = a.phase[b];
+    phased = ph.c2 != 0.0 || ph.cx != 0.0 || ph.cy != 0.0;
+  }
+  typename decltype(ld)::Raw raw[2];
+  const double on = (a.n & 1) ? 0.0 : 0.5;
+  auto window = [&](int s) {
+    if constexpr (LOAD == FOLD_FIELD) {
+      if (phased && threadIdx.x < 2 * kStageK) {
+        const double u = (double)(s * 2 * kStageK + (int)threadIdx.x) + on, q = ph.c2 * u * u;
+        const float2 wp = turn(fma(ph.cx, u, q)), wm = turn(fma(-ph.cx, u, q));
+        win[s & 1][threadIdx.x] = make_float4(wp.x, wp.y, wm.x, wm.y);
+      }
+    }
+  };
+  auto convert = [&](int s, const typename decltype(ld)::Raw& r) __attribute__((always_inline)) {
+    FoldPart o;
+    if constexpr (LOAD != FOLD_FIELD) ld.part(2 * s + run, beta, r, o);
+    else ld.part(2 * s + run, beta, r, phased, win[s & 1] + run * kStageK, o);
+    uint8_t* buf = lds + ((s & 1) * 2 + run) * kRun;
+#pragma unroll
+    for (int al = 0; al < 2; ++al)
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+        put4<BF>(buf + ((al * 2 + beta) * 32 + c * 16 + py) * kRow, quad, (py >> 2) & 3, o.v[al][c]);
+  };
+  f32x16_t acc[1][1];
+  zero_acc(acc);
+  u32x4_t fb[2][2][1][2];   // [stage parity][run]
+  auto load_tab = [&](auto J, int s) __attribute__((always_inline)) {
+    const int sc = s < nst ? s : nst - 1;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) load_frag(fb[decltype(J)::value][e][0], tab, 2 * sc + e);
+  };
+  auto step = [&](auto J, int s) __attribute__((always_inline)) {
+    constexpr int j0 = decltype(J)::value;
+    lds_barrier();   // stage s is in LDS, stage s - 1 has been read
+    u32x4_t fa[2][1][2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) read_frag(fa[e][0], lds + (j0 * 2 + e) * kRun, wave * 32);
+    load_tab(std::integral_constant<int, 1 - j0>{}, s + 1);
+    ld.raw(2 * (s + 2) + run, raw[j0]);
+    window(s + 2);
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) mma_stage<BF, 1, 1>(acc, fa[e], fb[j0][e]);
+    __builtin_amdgcn_s_setprio(0);
+    if (s + 1 < nst) convert(s + 1, raw[1 - j0]);
+  };
+  load_tab(std::integral_constant<int, 0>{}, 0);
+  ld.raw(run, raw[0]);
+  ld.raw(2 + run, raw[1]);
+  window(0);
+  window(1);
+  if constexpr (LOAD == FOLD_FIELD) lds_barrier();
+  convert(0, raw[0]);
+  for (int s = 0; s < nst; s += 2) {
+    step(std::integral_constant<int, 0>{}, s);
+    if (s + 1 < nst) step(std::integral_constant<int, 1>{}, s + 1);
+  }
+  lds_barrier();
+  f32x16_t& v = acc[0][0];
+  const int lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
+  if constexpr (LOAD == FOLD_FIELD) {
+    if (phased) {   // the y factor, as y_phase
+      f32x16_t other;
+      put_block(lds, v);
+      lds_barrier();
+      get_block<1>(lds, other);
+      lds_barrier();
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        const double u = (double)(py0 + 8 * (r >> 2) + 4 * lk + (r & 3)) + on;
+        const float2 w = turn(ph.cy * u);
+        float2 q = make_float2(1.f, 0.f);
+        if (ph.c2 != 0.0) q = turn(ph.c2 * u * u);
+        const float2 e = cmul(make_float2(v[r] * w.x - other[r + 8] * w.y,
+                                          v[r + 8] * w.x + other[r] * w.y), q);
+        v[r] = e.x;
+        v[r + 8] = e.y;
+      }
+    }
+  }
+  // rows of 64 bytes (the 16 k of a component), through a wave-private patch
+  constexpr int kSmallRow = 80;
+  uint8_t* patch = lds + wave * kRun;
+  const long rb = 4L * kp;
+  const int kvalid = kh - py0;
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      float x[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = 8 * q + 4 * lk + e < kvalid ? v[8 * c + 4 * q + e] : 0.f;
+      uint8_t* d = patch + (c * 32 + lr) * kSmallRow + q * 32;
+      if constexpr (BF) {
+        uint32_t h[2], l[2];
+        split2_bf16(x[0], x[1], h[0], l[0]);
+        split2_bf16(x[2], x[3], h[1], l[1]);
+        *(uint2*)(d + lk * 8) = make_uint2(h[0], h[1]);
+        *(uint2*)(d + 16 + lk * 8) = make_uint2(l[0], l[1]);
+      } else {
+        *(float4*)(d + lk * 16) = make_float4(x[0], x[1], x[2], x[3]);
+      }
+    }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  uint8_t* out = a.out + (long)b * a.out_stride + 4L * py0;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int c = e >> 1, r = 16 * (e & 1) + (lane >> 2), piece = lane & 3;
+    const uint4 x = *(const uint4*)(patch + (c * 32 + r) * kSmallRow + piece * 16);
+    const int comp = ((wave & 1) * 2 + (wave >> 1)) * 2 + c;
+    if (q0 + r < mh) *(uint4*)(out + (long)(comp * mh + q0 + r) * rb + piece * 16) = x;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // A ring of NB stage buffers (16 KiB: 256 folded rows) filled straight from
 // memory NB - 1 stages ahead, with the table fragments of the same stage in
@@ -1251,9 +1400,27 @@ template <bool BF, int LOAD, bool VEC>
 hipError_t stage1_width(const FoldStage1& a, hipStream_t s) {
   const int mh = fold_half(a.m), tp = (fold_half(a.n) + 31) / 32;
   auto tiles = [&](int w) { return (long)((mh + w - 1) / w) * tp * a.batch; };
-  if (mh > 64 && tiles(128) >= 256) stage1_go<BF, LOAD, VEC, 128>(a, tiles(128), s);
-  else if (mh > 32 && tiles(64) >= 256) stage1_go<BF, LOAD, VEC, 64>(a, tiles(64), s);
-  else stage1_go<BF, LOAD, VEC, 32>(a, tiles(32), s);
+  // A wider tile forms the field fewer times; a launch of fewer tiles leaves
+  // compute units idle.  Measured per launch, us, at 16 / 32 / 64 / 128 columns
+  // (16: the 16-row kernel at 32), 512^2 -> 256^2 pupils:
+  //   tiles of 64   float32                     split
+  //        128      24.7 / 25.0 / 31.1 / 47.2   16.7 / 17.9 / 21.6 / 22.1
+  //        192      33.5 / 39.8 / 33.2 / 49.0   21.2 / 24.8 / 21.4 / 24.0
+  //        256      41.0 / 40.6 / 34.7 / 49.3   26.4 / 25.2 / 22.0 / 24.8
+  //        320      49.4 / 52.3 / 56.3 / 49.1   30.4 / 32.4 / 29.4 / 25.2
+  //       1024       122 /  113 /  102 / 82.9   78.6 / 71.6 / 52.6 / 39.2
+  // and for a folded field in memory, at 32 / 64 / 128:
+  //        128      18.9 / 26.0 / 42.9          12.8 / 14.3 / 20.4
+  //        256      30.0 / 28.2 / 44.9          18.8 / 17.2 / 22.9
+  //       1024      90.7 / 85.6 / 89.0          56.9 / 44.5 / 40.3
+  if (mh > 64 && tiles(64) > 256) stage1_go<BF, LOAD, VEC, 128>(a, tiles(128), s);
+  else if (mh > 32 && tiles(64) >= 192) stage1_go<BF, LOAD, VEC, 64>(a, tiles(64), s);
+  else if (LOAD != FOLD_MEM && tiles(32) < 384) {
+    if constexpr (LOAD != FOLD_MEM)
+      hipLaunchKernelGGL((fold_stage1_small_kernel<BF, LOAD, VEC>),
+                         dim3((unsigned)((mh + 31) / 32 * ((fold_half(a.n) + 15) / 16) * a.batch)),
+                         dim3(kThreads), 0, s, a);
+  } else stage1_go<BF, LOAD, VEC, 32>(a, tiles(32), s);
   return hipGetLastError();
 }
 
@@ -1280,11 +1447,12 @@ template <bool BF, int EPI>
 hipError_t stage2_size(const FoldStage2& a, hipStream_t s) {
   const int mh = fold_half(a.m), tx = (mh + 31) / 32;
   auto tiles = [&](int q) { return (long)tx * ((mh + q - 1) / q) * a.batch; };
-  // 32 rows a workgroup where 64 leave compute units idle (or half of the waves,
-  // at mh <= 32): 24.6 -> 16.7 us at 16 fields 512^2 -> 256^2 (float32, 128 tiles
-  // of 64), 12.4 -> 8.4 at one of 256^2 (float32), 11.1 -> 9.3 at 16 of
-  // 512^2 -> 128^2 (split)
-  if (mh <= 32 || tiles(64) < 256)
+  // 32 rows a workgroup where 64 leave half of the compute units idle (or half of
+  // the waves, at mh <= 32).  us at 32 / 64 rows, 512^2 -> 256^2, by tiles of 64:
+  // 64: 16.8 / 24.8 float32, 10.8 / 13.1 split; 160: 29.4 / 25.4 float32;
+  // 256: 30.2 / 26.8 float32, 18.9 / 15.7 split; one wavelength of 256^2 -> 128^2
+  // (4 tiles) 11.2 / 15.0 float32
+  if (mh <= 32 || tiles(64) <= 128)
     hipLaunchKernelGGL((fold_stage2_kernel<BF, EPI, 32, 4>), dim3((unsigned)tiles(32)),
                        dim3(kThreads), 0, s, a);
   else
