@@ -4,19 +4,19 @@
 // dLux: out = fftshift(fft2(ifftshift(pad(x)))) / M      (utils/propagation.py:52-64)
 //       inverse: fftshift(ifft2(ifftshift(pad(x)))) * M  (= conj-sign DFT / M)
 //
-// A 2-D transform is two launches of one kernel, templated on log2 M so the
-// index arithmetic folds.  Each workgroup loads R rows of length M (power of
-// two) into LDS -- applying the zero pad and ifftshift as an index map on the
-// fly -- runs a Stockham auto-sort FFT on every row (radix-8 stages, then one
-// radix-4 or radix-2 stage; each stage reads its butterfly inputs into
-// registers, synchronises, and writes the outputs in place), and writes the
-// rows out TRANSPOSED.  The second launch therefore reads the first's columns
-// as rows and its transposed write restores the orientation; that write also
-// applies fftshift and the 1/M scale.  HBM traffic is one read and one write of
-// the M x M complex64 array per launch.  The angular-spectrum method takes
-// three launches instead of four (launch_asm): the y transforms of its forward
-// and inverse 2-D transforms, with the transfer function between them, run
-// back to back in LDS.
+// A 2-D transform is two launches of one kernel, templated on log2 M, the rows
+// per workgroup and the pass, so the index arithmetic folds.  A workgroup runs
+// a Stockham auto-sort FFT (stages of radix 16 and 8) on R rows of length M:
+// the first stage reads its butterflies straight from memory -- the zero pad
+// and ifftshift as an index map -- the stages between go through LDS, and the
+// last one writes straight to memory, or through LDS where the rows are stored
+// TRANSPOSED.  The second launch of a transform therefore reads the first's
+// columns as rows and its transposed write restores the orientation; that
+// write also applies fftshift and the 1/M scale.  HBM traffic is one read and
+// one write of the M x M complex64 array per launch.  The angular-spectrum
+// method takes three launches instead of four (launch_asm): the y transforms
+// of its forward and inverse 2-D transforms, with the transfer function
+// between them in the registers of the forward's last stage, run back to back.
 #include <cmath>
 
 #include "dlx_internal.h"
@@ -24,28 +24,12 @@
 namespace dlx {
 namespace {
 
-// At most kLdsElems complex64 of rows per workgroup plus an M-entry twiddle
-// table, within the 160 KiB of LDS; 8 waves per workgroup.
-constexpr int kThreads = 512;
-constexpr int kLdsElems = 16384;
-constexpr int kLdsBudget = 20480;   // complex64 values in 160 KiB
-
 // One 8-byte store of a complex64 (the compiler may otherwise split a float2
 // store into two 4-byte stores, doubling the write requests of the transposed
 // store's short runs).
 typedef float cplx_v __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void store_c64(float2* p, float2 v) {
   *(cplx_v*)p = cplx_v{v.x, v.y};
-}
-
-// LDS position of element x of row rr (row length 2^LOG2M): x with its bits
-// 3..8 XORed into bits 0..5 and a row term XORed in.  A bijection on
-// [0, M) for every row, so each row keeps its own M slots; it spreads the
-// Stockham stages' strided writes (stride RAD p) and the transposed
-// accesses (one column of R rows, M apart) over the LDS banks.
-template <int LOG2M>
-__device__ __forceinline__ int lds_pos(int x, int rr) {
-  return x ^ ((x >> 3) & 63) ^ ((rr * 20) & ((1 << LOG2M) - 1));
 }
 
 __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
@@ -98,90 +82,117 @@ __device__ __forceinline__ void dft_reg<8>(float2 (&x)[8], float sgn) {
   }
 }
 
-// One Stockham stage of radix RAD on rows of length M = 2^LOG2M held in LDS
-// (row stride M): item j (of M/RAD per row) reads x_r = row[j + r M/RAD],
-// twiddles them by exp(sgn 2 pi i r k / (p RAD)) with k = j mod p, transforms,
-// and writes y_q to row[(j - k) RAD + k + q p].  p = 2^LOG2P is the product of
-// earlier radices.  The sizes are template arguments, so the index arithmetic
-// folds into shifts, masks and the LDS instructions' immediate offsets.
-template <int RAD, int LOG2RAD, int LOG2M, int LOG2P, bool INV>
-__device__ __forceinline__ void stockham_stage(float2* buf, const float2* tw, int total) {
-  constexpr float sgn = INV ? 1.f : -1.f;   // the transform's sign, folded into the code
-  constexpr int kItems = kLdsElems / RAD / kThreads;
-  constexpr int log2_per_row = LOG2M - LOG2RAD;
-  constexpr int per_row = 1 << log2_per_row;
-  constexpr int p = 1 << LOG2P;
-  float2 v[kItems][RAD];
+template <>
+__device__ __forceinline__ void dft_reg<16>(float2 (&x)[16], float sgn) {
+  const float c1 = 0.92387953251128674f, s1 = 0.38268343236508977f, h = 0.70710678118654752f;
+  float2 a[4][4];   // [r1][q2]: DFT over r2 of x[r1 + 4 r2], times W16^(r1 q2)
 #pragma unroll
-  for (int it = 0; it < kItems; ++it) {
-    const int t = threadIdx.x + it * kThreads;
-    if (t < total) {
-      const int rr = t >> log2_per_row, j = t & (per_row - 1);
-      const float2* row = buf + (rr << LOG2M);
+  for (int r = 0; r < 4; ++r) {
 #pragma unroll
-      for (int r = 0; r < RAD; ++r) v[it][r] = row[lds_pos<LOG2M>(j + r * per_row, rr)];
-    }
+    for (int q = 0; q < 4; ++q) a[r][q] = x[r + 4 * q];
+    dft_reg<4>(a[r], sgn);
   }
-  __syncthreads();
+  a[1][1] = cmul(a[1][1], make_float2(c1, sgn * s1));
+  a[1][2] = cmul(a[1][2], make_float2(h, sgn * h));
+  a[1][3] = cmul(a[1][3], make_float2(s1, sgn * c1));
+  a[2][1] = cmul(a[2][1], make_float2(h, sgn * h));
+  a[2][2] = mul_si(a[2][2], sgn);
+  a[2][3] = cmul(a[2][3], make_float2(-h, sgn * h));
+  a[3][1] = cmul(a[3][1], make_float2(s1, sgn * c1));
+  a[3][2] = cmul(a[3][2], make_float2(-h, sgn * h));
+  a[3][3] = cmul(a[3][3], make_float2(-c1, -sgn * s1));
 #pragma unroll
-  for (int it = 0; it < kItems; ++it) {
-    const int t = threadIdx.x + it * kThreads;
-    if (t < total) {
-      const int rr = t >> log2_per_row, j = t & (per_row - 1);
-      const int k = j & (p - 1);
-      if (p > 1) {
-        constexpr int sh = LOG2M - LOG2P - LOG2RAD;   // twiddle index r k M / (p RAD)
+  for (int q = 0; q < 4; ++q) {
+    float2 y[4] = {a[0][q], a[1][q], a[2][q], a[3][q]};
+    dft_reg<4>(y, sgn);
 #pragma unroll
-        for (int r = 1; r < RAD; ++r) {
-          const float2 w = tw[(r * k) << sh];
-          v[it][r] = cmul(v[it][r], make_float2(w.x, sgn * w.y));
-        }
-      }
-      dft_reg<RAD>(v[it], sgn);
-      float2* row = buf + (rr << LOG2M);
-      const int i0 = ((j - k) << LOG2RAD) + k;
-#pragma unroll
-      for (int q = 0; q < RAD; ++q) row[lds_pos<LOG2M>(i0 + (q << LOG2P), rr)] = v[it][q];
-    }
+    for (int r = 0; r < 4; ++r) x[q + 4 * r] = y[r];
   }
-  __syncthreads();
 }
 
-// All stages from p = 2^LOG2P: radix 8 while it divides, then one radix-4 or
-// radix-2 stage.
-template <int LOG2M, int LOG2P, bool INV>
-__device__ __forceinline__ void stockham_from(float2* buf, const float2* tw, int total) {
-  if constexpr (LOG2M - LOG2P >= 3) {
-    stockham_stage<8, 3, LOG2M, LOG2P, INV>(buf, tw, total >> 3);
-    stockham_from<LOG2M, LOG2P + 3, INV>(buf, tw, total);
-  } else if constexpr (LOG2M - LOG2P == 2) {
-    stockham_stage<4, 2, LOG2M, LOG2P, INV>(buf, tw, total >> 2);
-  } else if constexpr (LOG2M - LOG2P == 1) {
-    stockham_stage<2, 1, LOG2M, LOG2P, INV>(buf, tw, total >> 1);
-  }
+// log2 of the radices: three stages up to 4096.  A radix-8 first stage is
+// followed by radix 8 and a radix-16 one by radix 16, which the LDS layout
+// needs (lin below).
+constexpr int log2_rad(int log2m, int st) {
+  constexpr int kRad[14][4] = {{},        {1},       {2},       {3},       {4},
+                               {3, 2},    {3, 3},    {4, 3},    {4, 4},    {3, 3, 3},
+                               {3, 3, 4}, {4, 4, 3}, {4, 4, 4}, {4, 4, 3, 2}};
+  return kRad[log2m][st];
 }
+constexpr int stages(int log2m) {
+  int n = 0;
+  while (n < 4 && log2_rad(log2m, n) > 0) ++n;
+  return n;
+}
+constexpr int log2_p(int log2m, int st) {   // product of the earlier radices
+  int l = 0;
+  for (int i = 0; i < st; ++i) l += log2_rad(log2m, i);
+  return l;
+}
+
+// Twiddles exp(2 pi i r k / (p RAD)) of every stage but the first, in the order
+// the stages read them: stage st at p - RAD_0, entry (r - 1) p + k for r = 1 ..
+// RAD - 1 (the sizes telescope to M - RAD_0 in all), rounded from double.
+template <int LOG2M>
+struct Twiddles {
+  float v[2 << LOG2M];
+};
+constexpr double kPi = 3.14159265358979323846;
+constexpr double sin_small(double x) {   // |x| <= pi / 4
+  const double y = x * x;
+  double t = 0.0;
+  for (int i = 10; i >= 1; --i) t = (1.0 + t) * (-y / ((2.0 * i) * (2.0 * i + 1.0)));
+  return x * (1.0 + t);
+}
+constexpr double cos_small(double x) {
+  const double y = x * x;
+  double t = 0.0;
+  for (int i = 10; i >= 1; --i) t = (1.0 + t) * (-y / ((2.0 * i - 1.0) * (2.0 * i)));
+  return 1.0 + t;
+}
+template <int LOG2M>
+constexpr Twiddles<LOG2M> make_twiddles() {
+  constexpr int M = 1 << LOG2M, E = M >= 8 ? M / 8 : 1;   // an octant
+  double c[E + 1] = {}, sn[E + 1] = {};
+  for (int q = 0; q <= E; ++q) {
+    c[q] = cos_small(2.0 * kPi * q / M);
+    sn[q] = sin_small(2.0 * kPi * q / M);
+  }
+  Twiddles<LOG2M> t{};
+  int o = 0;
+  for (int st = 1; st < stages(LOG2M); ++st) {
+    const int p = 1 << log2_p(LOG2M, st), rad = 1 << log2_rad(LOG2M, st);
+    for (int r = 1; r < rad; ++r)
+      for (int k = 0; k < p; ++k, ++o) {
+        const int a = (r * k * (M / (p * rad))) % M;      // M >= 32 where there are two stages
+        const int oct = a / E, f = a % E;
+        const double x = oct & 1 ? sn[E - f] : c[f], y = oct & 1 ? c[E - f] : sn[f];
+        const double u = (oct >> 1) & 1 ? y : x, w = (oct >> 1) & 1 ? x : y;
+        t.v[2 * o] = (float)(oct >= 2 && oct < 6 ? -u : u);
+        t.v[2 * o + 1] = (float)(oct >= 4 ? -w : w);
+      }
+  }
+  return t;
+}
+template <int LOG2M>
+__device__ constexpr Twiddles<LOG2M> kTwiddles = make_twiddles<LOG2M>();
+
+enum FftPass {
+  kFirst = 0,    // padded N x N source, rows stored transposed
+  kSecond = 1,   // plain rows, stored transposed with fftshift and the scale
+  kMid = 2,      // plain rows (y-lines, row index kx): forward, times H, inverse; plain rows
+  kLast = 3,     // rows gathered from columns; plain rows with fftshift and the scale
+};
 
 struct FftParams {
-  int M, log2M, R, log2R, inverse;
-  // 0: centred + zero-padded from an N x N source (ifftshift as an index map);
-  // 1: plain M x M rows; 2: rows gathered from the columns of an M x M array
-  int in_mode;
-  int N, p;         // source side and pad offset (in_mode 0)
+  int N, p;         // source side and pad offset (kFirst)
   long in_bstride, out_bstride;
-  // 0: transposed; 1: transposed + fftshift + scale (+ H); 2: plain rows;
-  // 3: plain rows + fftshift + scale
-  int out_mode;
   float scale;
-  // asm_on with out_mode 1: H(fx, fy) of the centred frequencies, fused into
-  // the store.  asm_mid: the rows are y-lines of a spectrum transformed along
-  // x (row index kx); each is transformed along y, multiplied by H at the
-  // natural-order frequencies (kx, ky), and transformed back along y.
-  int asm_on, asm_mid;
   double asm_z, asm_inv_wl2, asm_df;
-  // rows_lo > 0 (in_mode 0): only the rows that hold the padded field, [0,
+  // rows_lo > 0 (kFirst): only the rows that hold the padded field, [0,
   // rows_lo) and [M - rows_lo, M), are transformed (the others are zero rows
   // whose transforms are zero); the launch has 2 rows_lo / R groups.
-  // zlo < zhi (in_mode 1): positions [zlo, zhi) of every row load as zeros
+  // zlo < zhi (kSecond, kMid): positions [zlo, zhi) of every row load as zeros
   // (the columns the previous launch left unwritten).
   int rows_lo, zlo, zhi;
 };
@@ -202,14 +213,116 @@ __device__ __forceinline__ float2 apply_h(float2 v, int iy, int ix, const FftPar
   return make_float2(v.x * c - v.y * s, v.x * s + v.y * c);
 }
 
-template <int LOG2M>
-__global__ void __launch_bounds__(kThreads)
+// Threads of a workgroup: one radix-16 butterfly each.
+constexpr int fft_threads(int log2m, int log2r) {
+  const int t = (1 << (log2m + log2r)) / 16;
+  return t < 64 ? 64 : t > 1024 ? 1024 : t;
+}
+
+// The workgroup's transforms in LDS.  Element x of row rr sits at x with the 5
+// bits from bit log2 RAD_0 up XORed into its low 5 and a row term XORed in: a
+// bijection on [0, M) for every row that spreads the stages' strided accesses
+// and the transposed ones (one column of R rows, M apart) over the 32 8-byte
+// LDS banks.  It is linear over XOR, so the positions of a butterfly differ by
+// constants.
+template <int LOG2M, int LOG2R>
+struct RowFft {
+  static constexpr int M = 1 << LOG2M, R = 1 << LOG2R, T = fft_threads(LOG2M, LOG2R);
+  static constexpr int kStages = stages(LOG2M);
+  static constexpr uint32_t lin(uint32_t x) { return x ^ ((x >> log2_rad(LOG2M, 0)) & 31); }
+  static __device__ __forceinline__ uint32_t row_off(int rr) {
+    return ((uint32_t)rr << LOG2M) | ((uint32_t)(rr * 20) & (M - 1));
+  }
+  // byte offset of element x of row rr
+  static __device__ __forceinline__ uint32_t off(int rr, int x) {
+    return (row_off(rr) ^ lin((uint32_t)x)) << 3;
+  }
+  static __device__ __forceinline__ float2& at(float2* buf, uint32_t byte) {
+    return *(float2*)((char*)buf + byte);
+  }
+
+  // Stage ST: butterfly j of a row reads x_r = row[j + r M / RAD], twiddles
+  // them by exp(sgn 2 pi i r k / (p RAD)) with k = j mod p, transforms, and
+  // writes y_q to row[(j - k) RAD + k + q p].  load(v, rr, j) fills a butterfly
+  // from elsewhere than LDS (SRC false); post(v, rr, i0) may change it and,
+  // returning true, has stored it (element q at i0 + q p).  RFAST: consecutive
+  // threads take consecutive rows.
+  template <int ST, bool INV, bool SRC, bool DST, bool RFAST, typename Load, typename Post>
+  static __device__ __forceinline__ void stage(float2* buf, const float2* tw, Load load, Post post) {
+    constexpr float sgn = INV ? 1.f : -1.f;
+    constexpr int L = log2_rad(LOG2M, ST), RAD = 1 << L, LP = log2_p(LOG2M, ST), p = 1 << LP;
+    constexpr int LJ = LOG2M - L, total = R << LJ;
+    constexpr int kItems = total > T ? total / T : 1;
+    constexpr bool kAll = total % T == 0;
+    float2 v[kItems][RAD];
+#pragma unroll
+    for (int it = 0; it < kItems; ++it) {
+      const int t = threadIdx.x + it * T;
+      if (kAll || t < total) {
+        const int rr = RFAST ? t & (R - 1) : t >> LJ, j = RFAST ? t >> LOG2R : t & ((1 << LJ) - 1);
+        if constexpr (SRC) {
+          const uint32_t o = off(rr, j);
+#pragma unroll
+          for (int r = 0; r < RAD; ++r) v[it][r] = at(buf, o ^ (lin((uint32_t)r << LJ) << 3));
+        } else {
+          load(v[it], rr, j);
+        }
+      }
+    }
+    if constexpr (SRC && DST) __syncthreads();
+#pragma unroll
+    for (int it = 0; it < kItems; ++it) {
+      const int t = threadIdx.x + it * T;
+      if (kAll || t < total) {
+        const int rr = RFAST ? t & (R - 1) : t >> LJ, j = RFAST ? t >> LOG2R : t & ((1 << LJ) - 1);
+        const int k = j & (p - 1);
+        if constexpr (ST > 0) {
+          const float2* w = tw + (p - (1 << log2_rad(LOG2M, 0))) + k;
+#pragma unroll
+          for (int r = 1; r < RAD; ++r) {
+            const float2 c = w[(r - 1) * p];
+            v[it][r] = cmul(v[it][r], make_float2(c.x, sgn * c.y));
+          }
+        }
+        dft_reg<RAD>(v[it], sgn);
+        const int i0 = ((j - k) << L) + k;
+        post(v[it], rr, i0);
+        if constexpr (DST) {
+          const uint32_t o = off(rr, i0);
+#pragma unroll
+          for (int q = 0; q < RAD; ++q) at(buf, o ^ (lin((uint32_t)q << LP) << 3)) = v[it][q];
+        }
+      }
+    }
+    if constexpr (DST) __syncthreads();
+  }
+
+  // Stages from ST: the first of the transform from `load` unless SRC, the last
+  // through `post`, to LDS if DST.
+  template <int ST, bool INV, bool SRC, bool DST, bool RFAST, typename Load, typename Post>
+  static __device__ __forceinline__ void run(float2* buf, const float2* tw, Load load, Post post) {
+    if constexpr (ST + 1 == kStages) {
+      stage<ST, INV, SRC || (ST > 0), DST, RFAST && ST == 0>(buf, tw, load, post);
+    } else {
+      stage<ST, INV, SRC || (ST > 0), true, RFAST && ST == 0>(buf, tw, load,
+                                                               [](auto&, int, int) {});
+      run<ST + 1, INV, SRC, DST, RFAST>(buf, tw, load, post);
+    }
+  }
+};
+
+// What bounds a launch: LDS and vector work per element beside 16 bytes of HBM
+// traffic.  2048^2 angular spectrum of a 1024^2 field, us per launch (first /
+// mid / last), radix-8 stages with every stage and both ends through LDS: 15.8 /
+// 39.1 / 25.0; this form: FIGURES.
+template <int LOG2M, int LOG2R, int PASS, bool INV>
+__global__ void __launch_bounds__(fft_threads(LOG2M, LOG2R), 4)
 fft_rows_kernel(const float2* __restrict__ in, float2* __restrict__ out, FftParams P) {
+  using F = RowFft<LOG2M, LOG2R>;
   extern __shared__ float2 lds[];
-  constexpr int M = 1 << LOG2M, half_m = M >> 1;
-  constexpr int RS = M;            // LDS row stride
-  const int R = P.R;
-  float2* tw = lds + (long)R * RS;  // M twiddles (cos, sin)(2 pi q / M)
+  constexpr int M = F::M, R = F::R, T = F::T, half_m = M >> 1, kLast_ = F::kStages - 1;
+  constexpr int LP = log2_p(LOG2M, kLast_), RADL = 1 << log2_rad(LOG2M, kLast_);
+  float2* tw = lds + R * M;
   // consecutive row groups on one XCD (workgroups are dealt to the 8 XCDs
   // round-robin), so the short runs of the transposed stores (and loads) that
   // neighbouring groups access in the same cache lines meet in that XCD's L2
@@ -220,110 +333,133 @@ fft_rows_kernel(const float2* __restrict__ in, float2* __restrict__ out, FftPara
   int r0 = (id - b * groups) * R;
   if (P.rows_lo > 0 && r0 >= P.rows_lo) r0 += M - 2 * P.rows_lo;
   const float2* src = in + (long)b * P.in_bstride;
+  float2* dst = out + (long)b * P.out_bstride;
 
-  if constexpr (M >= 4) {
-    // one quadrant by sincospif, the other three by its exact symmetries
-    for (int q = threadIdx.x; q < M / 4; q += kThreads) {
-      float s, c;
-      sincospif(2.0f * (float)q / (float)M, &s, &c);
-      tw[q] = make_float2(c, s);
-      tw[q + M / 4] = make_float2(-s, c);
-      tw[q + M / 2] = make_float2(-c, -s);
-      tw[q + 3 * M / 4] = make_float2(s, -c);
-    }
-  } else {
-    for (int q = threadIdx.x; q < M; q += kThreads) {
-      float s, c;
-      sincospif(2.0f * (float)q / (float)M, &s, &c);
-      tw[q] = make_float2(c, s);
+  if constexpr (F::kStages > 1) {   // read after the first stage's barrier
+    const float2* g = (const float2*)kTwiddles<LOG2M>.v;
+    constexpr int n = M - (1 << log2_rad(LOG2M, 0));
+#pragma unroll
+    for (int q0 = 0; q0 < n; q0 += T) {
+      const int q = q0 + threadIdx.x;
+      if (q < n) tw[q] = g[q];
     }
   }
-  // load (M and R are powers of two: shifts and masks), 16 values per thread
-  // in flight before any is written to LDS
-  const int total = R * M;
-  constexpr int kLoadBatch = 16;
-  for (int t0 = 0; t0 < total; t0 += kLoadBatch * kThreads) {
-    float2 v[kLoadBatch];
+
+  auto load = [&](auto& v, int rr, int j) __attribute__((always_inline)) {
+    constexpr int RAD = sizeof(v) / sizeof(float2), step = M / RAD;
+    if constexpr (PASS == kFirst) {
+      const int sr = ((r0 + rr + half_m) & (M - 1)) - P.p;
+      const bool row_ok = sr >= 0 && sr < P.N;
+      const float2* row = src + (long)(row_ok ? sr : 0) * P.N;
 #pragma unroll
-    for (int i = 0; i < kLoadBatch; ++i) {
-      const int t = t0 + threadIdx.x + i * kThreads;
-      v[i] = make_float2(0.f, 0.f);
-      if (t < total) {
-        if (P.in_mode == 0) {
-          const int rr = t >> LOG2M, nc = t & (M - 1);
-          const int sr = ((r0 + rr + half_m) & (M - 1)) - P.p;
-          const int sc = ((nc + half_m) & (M - 1)) - P.p;
-          if (sr >= 0 && sr < P.N && sc >= 0 && sc < P.N) v[i] = src[(long)sr * P.N + sc];
-        } else if (P.in_mode == 1) {
-          const int y = t & (M - 1);
-          if (y < P.zlo || y >= P.zhi) v[i] = src[(long)r0 * M + t];
+      for (int r = 0; r < RAD; ++r) {
+        const int sc = ((j + r * step + half_m) & (M - 1)) - P.p;
+        const bool ok = row_ok && sc >= 0 && sc < P.N;   // loads stay unconditional, in flight
+        const float2 x = row[ok ? sc : 0];
+        v[r] = ok ? x : make_float2(0.f, 0.f);
+      }
+    } else if constexpr (PASS == kLast) {
+#pragma unroll
+      for (int r = 0; r < RAD; ++r) v[r] = src[(long)(j + r * step) * M + r0 + rr];
+    } else {
+      const float2* row = src + (long)(r0 + rr) * M;
+#pragma unroll
+      for (int r = 0; r < RAD; ++r) {
+        const int y = j + r * step;
+        const bool ok = y < P.zlo || y >= P.zhi;
+        const float2 x = row[ok ? y : 0];
+        v[r] = ok ? x : make_float2(0.f, 0.f);
+      }
+    }
+  };
+  auto none = [](auto&, int, int) {};
+  if constexpr (PASS == kMid) {
+    F::template run<0, false, false, true, false>(
+        lds, tw, load, [&](auto& v, int rr, int i0) __attribute__((always_inline)) {
+          const int ix = ((r0 + rr + half_m) & (M - 1)) - half_m;
+#pragma unroll
+          for (int q = 0; q < RADL; ++q)
+            v[q] = apply_h(v[q], ((i0 + (q << LP) + half_m) & (M - 1)) - half_m, ix, P);
+        });
+    F::template run<0, true, true, false, false>(
+        lds, tw, load, [&](auto& v, int rr, int i0) __attribute__((always_inline)) {
+#pragma unroll
+          for (int q = 0; q < RADL; ++q)
+            store_c64(dst + (long)(r0 + rr) * M + i0 + (q << LP), v[q]);
+        });
+  } else if constexpr (PASS == kLast) {
+    F::template run<0, INV, false, false, true>(
+        lds, tw, load, [&](auto& v, int rr, int i0) __attribute__((always_inline)) {
+          const int oy = (r0 + rr + half_m) & (M - 1);
+#pragma unroll
+          for (int q = 0; q < RADL; ++q) {
+            const int ox = (i0 + (q << LP) + half_m) & (M - 1);
+            store_c64(dst + (long)oy * M + ox, make_float2(v[q].x * P.scale, v[q].y * P.scale));
+          }
+        });
+  } else {
+    F::template run<0, INV, false, true, false>(lds, tw, load, none);
+    // transposed store: out[k][row] (consecutive lanes -> consecutive rows)
+    constexpr int kPer = R * M > T ? R * M / T : 1;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int t = threadIdx.x + i * T;
+      if (R * M % T == 0 || t < R * M) {
+        const int k = t >> LOG2R, rr = t & (R - 1), row = r0 + rr;
+        float2 v = F::at(lds, F::off(rr, k));
+        if constexpr (PASS == kFirst) {
+          store_c64(dst + (long)k * M + row, v);
         } else {
-          // element (rr, x) of the group is column r0 + rr of row x
-          const int x = t >> P.log2R, rr = t & (R - 1);
-          v[i] = src[(long)x * M + r0 + rr];
+          const int oy = (k + half_m) & (M - 1), ox = (row + half_m) & (M - 1);
+          store_c64(dst + (long)oy * M + ox, make_float2(v.x * P.scale, v.y * P.scale));
         }
       }
     }
-#pragma unroll
-    for (int i = 0; i < kLoadBatch; ++i) {
-      const int t = t0 + threadIdx.x + i * kThreads;
-      if (t < total) {
-        const int rr = P.in_mode == 2 ? t & (R - 1) : t >> LOG2M;
-        const int x = P.in_mode == 2 ? t >> P.log2R : t & (M - 1);
-        lds[rr * RS + lds_pos<LOG2M>(x, rr)] = v[i];
-      }
-    }
   }
-  __syncthreads();
+}
 
-  if (P.inverse) stockham_from<LOG2M, 0, true>(lds, tw, total);
-  else stockham_from<LOG2M, 0, false>(lds, tw, total);
+// log2 of the rows per workgroup for length-M rows: within the 160 KiB of LDS
+// beside the twiddles, 4 rows (32-byte runs in the transposed accesses) while
+// that leaves one workgroup per CU.
+constexpr int log2_rows(int log2m) {
+  return log2m <= 8 ? 0 : log2m == 9 ? 1 : log2m <= 12 ? 2 : 0;
+}
 
-  if (P.asm_mid) {
-    // y-line kx = r0 + rr at natural-order frequency ky: multiply by H, then
-    // transform back along y
-    for (int t = threadIdx.x; t < total; t += kThreads) {
-      const int rr = t >> LOG2M, ky = t & (M - 1);
-      const int kx = r0 + rr;
-      float2* e = lds + rr * RS + lds_pos<LOG2M>(ky, rr);
-      *e = apply_h(*e, ((ky + half_m) & (M - 1)) - half_m, ((kx + half_m) & (M - 1)) - half_m, P);
-    }
-    __syncthreads();
-    if (P.inverse) stockham_from<LOG2M, 0, false>(lds, tw, total);
-    else stockham_from<LOG2M, 0, true>(lds, tw, total);
+template <int LOG2M, int LOG2R, int PASS, bool INV>
+hipError_t launch_rows_r(const float2* in, float2* out, int batch, const FftParams& P,
+                         hipStream_t s) {
+  constexpr size_t lds = ((size_t)(1 << (LOG2M + LOG2R)) + (1 << LOG2M)) * sizeof(float2);
+  if constexpr (lds > 64 * 1024) {
+    // Opt in to more than 64 KiB of dynamic LDS (gfx950 has 160 KiB per CU).
+    (void)hipFuncSetAttribute((const void*)fft_rows_kernel<LOG2M, LOG2R, PASS, INV>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    (void)hipGetLastError();
   }
+  const int rows = P.rows_lo > 0 ? 2 * P.rows_lo : 1 << LOG2M;
+  hipLaunchKernelGGL((fft_rows_kernel<LOG2M, LOG2R, PASS, INV>), dim3(rows >> LOG2R, batch),
+                     dim3(fft_threads(LOG2M, LOG2R)), lds, s, in, out, P);
+  return hipGetLastError();
+}
 
-  float2* dst = out + (long)b * P.out_bstride;
-  if (P.out_mode >= 2) {
-    // plain rows (out_mode 3: fftshift on both axes and the scale)
-    for (int t = threadIdx.x; t < total; t += kThreads) {
-      const int rr = t >> LOG2M, k = t & (M - 1);
-      float2 v = lds[rr * RS + lds_pos<LOG2M>(k, rr)];
-      if (P.out_mode == 2) {
-        store_c64(dst + (long)(r0 + rr) * M + k, v);
-      } else {
-        v.x *= P.scale;
-        v.y *= P.scale;
-        const int oy = (r0 + rr + half_m) & (M - 1), ox = (k + half_m) & (M - 1);
-        store_c64(dst + (long)oy * M + ox, v);
-      }
+template <int PASS, bool INV, int LOG2M = 1>
+hipError_t launch_rows(int log2m, const float2* in, float2* out, int batch, const FftParams& P,
+                       hipStream_t s) {
+  if constexpr (LOG2M > 13) {
+    return hipErrorInvalidValue;
+  } else {
+    if (log2m != LOG2M) return launch_rows<PASS, INV, LOG2M + 1>(log2m, in, out, batch, P, s);
+    constexpr int R = log2_rows(LOG2M);
+    if constexpr (PASS == kFirst && R > 0) {
+      // a launch over the field's rows alone has fewer groups: halve the rows per
+      // group while there are fewer than 512
+      int r = R;
+      if (P.rows_lo > 0)
+        while (r > 0 && (2 * P.rows_lo) >> r < 512) --r;
+      if constexpr (R > 1)
+        if (r == 1) return launch_rows_r<LOG2M, 1, PASS, INV>(in, out, batch, P, s);
+      if (r == 0) return launch_rows_r<LOG2M, 0, PASS, INV>(in, out, batch, P, s);
     }
-    return;
-  }
-  // transposed store: out[k][row] (consecutive lanes -> consecutive rows)
-  for (int t = threadIdx.x; t < total; t += kThreads) {
-    const int k = t >> P.log2R, rr = t & (R - 1);
-    const int row = r0 + rr;
-    float2 v = lds[rr * RS + lds_pos<LOG2M>(k, rr)];
-    if (P.out_mode == 0) {
-      store_c64(dst + (long)k * M + row, v);
-    } else {
-      const int oy = (k + half_m) & (M - 1), ox = (row + half_m) & (M - 1);
-      v.x *= P.scale;
-      v.y *= P.scale;
-      if (P.asm_on) v = apply_h(v, oy - half_m, ox - half_m, P);
-      store_c64(dst + (long)oy * M + ox, v);
-    }
+    return launch_rows_r<LOG2M, R, PASS, INV>(in, out, batch, P, s);
   }
 }
 
@@ -333,120 +469,50 @@ int ilog2(int m) {
   return l;
 }
 
-template <int LOG2M>
-hipError_t launch_rows_m(const float2* in, float2* out, int batch, const FftParams& P,
-                         size_t lds, hipStream_t s) {
-  if (lds > 64 * 1024) {
-    // Opt in to more than 64 KiB of dynamic LDS (gfx950 has 160 KiB per CU).
-    (void)hipFuncSetAttribute((const void*)fft_rows_kernel<LOG2M>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    (void)hipGetLastError();
-  }
-  const int rows = P.rows_lo > 0 ? 2 * P.rows_lo : P.M;
-  hipLaunchKernelGGL(fft_rows_kernel<LOG2M>, dim3(rows / P.R, batch), dim3(kThreads), lds, s, in,
-                     out, P);
-  return hipGetLastError();
-}
-
-// Rows per workgroup for length-M rows: about two workgroups per CU (512)
-// when the rows fit, within kLdsElems and the LDS left beside the M-entry
-// twiddle table, at least 4 rows (32-byte runs in the transposed store) while
-// that still leaves one workgroup per CU; a power of two.
-int rows_per_group(int M) {
-  int cap = (kLdsBudget - M) / M;
-  if (cap > kLdsElems / M) cap = kLdsElems / M;
-  if (cap < 1) cap = 1;
-  int r = M / 512;
-  const int r_min = M / 256 < 4 ? M / 256 : 4;
-  if (r < r_min) r = r_min;
-  if (r < 1) r = 1;
-  if (r > cap) r = cap;
-  int R = 1 << (ilog2(r + 1) - 1);   // largest power of two <= r
-  return R > M ? M : R;
-}
-
-hipError_t launch_rows(const float2* in, float2* out, int batch, FftParams P, hipStream_t s) {
-  P.log2M = ilog2(P.M);
-  P.R = rows_per_group(P.M);
-  // a launch over the field's rows alone has fewer groups: halve the rows per
-  // group while there are fewer than 512 groups (2048^2 padded from 1024^2:
-  // 512 groups of 2 rows measured 1 % faster than 256 of 4)
-  if (P.rows_lo > 0)
-    while (P.R > 1 && 2 * P.rows_lo / P.R < 512 && P.rows_lo % (P.R / 2) == 0) P.R /= 2;
-  P.log2R = ilog2(P.R);
-  const size_t lds = ((size_t)P.R * P.M + P.M) * sizeof(float2);
-  if (lds > 160 * 1024) return hipErrorInvalidValue;
-  switch (P.log2M) {
-    case 1: return launch_rows_m<1>(in, out, batch, P, lds, s);
-    case 2: return launch_rows_m<2>(in, out, batch, P, lds, s);
-    case 3: return launch_rows_m<3>(in, out, batch, P, lds, s);
-    case 4: return launch_rows_m<4>(in, out, batch, P, lds, s);
-    case 5: return launch_rows_m<5>(in, out, batch, P, lds, s);
-    case 6: return launch_rows_m<6>(in, out, batch, P, lds, s);
-    case 7: return launch_rows_m<7>(in, out, batch, P, lds, s);
-    case 8: return launch_rows_m<8>(in, out, batch, P, lds, s);
-    case 9: return launch_rows_m<9>(in, out, batch, P, lds, s);
-    case 10: return launch_rows_m<10>(in, out, batch, P, lds, s);
-    case 11: return launch_rows_m<11>(in, out, batch, P, lds, s);
-    case 12: return launch_rows_m<12>(in, out, batch, P, lds, s);
-    case 13: return launch_rows_m<13>(in, out, batch, P, lds, s);
-    default: return hipErrorInvalidValue;
-  }
-}
-
 }  // namespace
 
-// Maximum transform side handled by the LDS kernel (one row + twiddles fit).
+// Maximum transform side (one row + twiddles fit in LDS).
 constexpr int kMaxFftSide = 8192;
 
 bool fft_supported(int m) { return m >= 2 && m <= kMaxFftSide && (m & (m - 1)) == 0; }
 
-// Full centred 2-D transform of `batch` N x N fields, padded to M x M.
-// tmp: batch * M * M complex64 scratch.
 // A launch over the rows of an N x N field padded to M x M (ifftshifted):
 // the rows that hold the field are [0, N/2) and [M - N/2, M); transform only
-// those when N/2 is a multiple of the rows per workgroup.
-static void set_padded_rows(int N, int M, FftParams& A) {
-  const int half = N / 2;
-  A.rows_lo = N < M && half > 0 && half % rows_per_group(M) == 0 ? half : 0;
-}
-
-// The launch after one that skipped zero rows reads, in each of its rows, the
-// positions those rows would have written as zeros.
-static void set_zero_columns(const FftParams& A, FftParams& B) {
-  B.zlo = A.rows_lo > 0 ? A.rows_lo : 0;
-  B.zhi = A.rows_lo > 0 ? A.M - A.rows_lo : 0;
-}
-
-hipError_t launch_fft2_centred(const float2* in, int N, int M, int batch, int inverse,
-                               float scale, float2* tmp, float2* out, int asm_on, double z,
-                               double wavelength, double dx, hipStream_t s) {
+// those when N/2 is a multiple of the rows per workgroup.  The launch after it
+// reads, in each of its rows, the positions the others would have written as
+// zeros.
+static FftParams first_params(int N, int M) {
   FftParams A{};
-  A.M = M;
-  A.inverse = inverse;
-  A.in_mode = 0;
   A.N = N;
   A.p = (M - N) / 2;
   A.in_bstride = (long)N * N;
   A.out_bstride = (long)M * M;
-  A.out_mode = 0;
-  set_padded_rows(N, M, A);
-  hipError_t e = launch_rows(in, tmp, batch, A, s);
-  if (e != hipSuccess) return e;
+  const int half = N / 2;
+  A.rows_lo = N < M && half > 0 && half % (1 << log2_rows(ilog2(M))) == 0 ? half : 0;
+  return A;
+}
+static FftParams next_params(const FftParams& A, int M) {
   FftParams B = A;
   B.rows_lo = 0;
-  B.in_mode = 1;
   B.in_bstride = (long)M * M;
-  B.out_mode = 1;
+  B.zlo = A.rows_lo;
+  B.zhi = A.rows_lo > 0 ? M - A.rows_lo : 0;
+  return B;
+}
+
+// Full centred 2-D transform of `batch` N x N fields, padded to M x M.
+// tmp: batch * M * M complex64 scratch.
+hipError_t launch_fft2_centred(const float2* in, int N, int M, int batch, int inverse,
+                               float scale, float2* tmp, float2* out, hipStream_t s) {
+  const int l = ilog2(M);
+  const FftParams A = first_params(N, M);
+  hipError_t e = inverse ? launch_rows<kFirst, true>(l, in, tmp, batch, A, s)
+                         : launch_rows<kFirst, false>(l, in, tmp, batch, A, s);
+  if (e != hipSuccess) return e;
+  FftParams B = next_params(A, M);
   B.scale = scale;
-  set_zero_columns(A, B);
-  B.asm_on = asm_on;
-  if (asm_on) {
-    B.asm_z = z;
-    B.asm_inv_wl2 = 1.0 / (wavelength * wavelength);
-    B.asm_df = 1.0 / ((double)M * dx);
-  }
-  return launch_rows(tmp, out, batch, B, s);
+  return inverse ? launch_rows<kSecond, true>(l, tmp, out, batch, B, s)
+                 : launch_rows<kSecond, false>(l, tmp, out, batch, B, s);
 }
 
 // Angular-spectrum propagation of one N x N field padded to M x M:
@@ -455,41 +521,22 @@ hipError_t launch_fft2_centred(const float2* in, int N, int M, int batch, int in
 // inverse transforms with their fftshift / ifftshift pairs cancelled between
 // them.  Three launches: x transforms of the padded field (transposed store);
 // per y-line (fixed kx) the forward y transform, H', and the inverse y
-// transform, in LDS; the inverse x transforms of rows gathered from columns,
-// stored with fftshift and the 1/M^2 scale.
+// transform; the inverse x transforms of rows gathered from columns, stored
+// with fftshift and the 1/M^2 scale.
 hipError_t launch_asm(const float2* in, int N, int M, double z, double wavelength, double dx,
                       float2* tmp, float2* tmp2, float2* out, hipStream_t s) {
-  FftParams A{};
-  A.M = M;
-  A.in_mode = 0;
-  A.N = N;
-  A.p = (M - N) / 2;
-  A.in_bstride = (long)N * N;
-  A.out_bstride = (long)M * M;
-  A.out_mode = 0;
-  set_padded_rows(N, M, A);
-  hipError_t e = launch_rows(in, tmp, 1, A, s);
+  const int l = ilog2(M);
+  const FftParams A = first_params(N, M);
+  hipError_t e = launch_rows<kFirst, false>(l, in, tmp, 1, A, s);
   if (e != hipSuccess) return e;
-  FftParams B = A;
-  B.rows_lo = 0;
-  B.in_mode = 1;
-  B.in_bstride = (long)M * M;
-  B.out_mode = 2;
-  set_zero_columns(A, B);
-  B.asm_mid = 1;
+  FftParams B = next_params(A, M);
   B.asm_z = z;
   B.asm_inv_wl2 = 1.0 / (wavelength * wavelength);
   B.asm_df = 1.0 / ((double)M * dx);
-  e = launch_rows(tmp, tmp2, 1, B, s);
+  e = launch_rows<kMid, false>(l, tmp, tmp2, 1, B, s);
   if (e != hipSuccess) return e;
-  FftParams C = A;
-  C.rows_lo = 0;
-  C.inverse = 1;
-  C.in_mode = 2;
-  C.in_bstride = (long)M * M;
-  C.out_mode = 3;
-  C.scale = (float)(1.0 / ((double)M * M));
-  return launch_rows(tmp2, out, 1, C, s);
+  B.scale = (float)(1.0 / ((double)M * M));
+  return launch_rows<kLast, true>(l, tmp2, out, 1, B, s);
 }
 
 }  // namespace dlx
@@ -520,8 +567,7 @@ extern "C" int dlx_fft2(int32_t n, int32_t m, int32_t batch, int32_t inverse, co
     return DLX_ERR_WORKSPACE;
   }
   DLX_HIP(launch_fft2_centred((const float2*)in, n, m, batch, inverse, 1.0f / (float)m,
-                              (float2*)workspace, (float2*)out, 0, 0, 0, 0,
-                              (hipStream_t)stream));
+                              (float2*)workspace, (float2*)out, (hipStream_t)stream));
   return DLX_OK;
 }
 
