@@ -314,7 +314,7 @@ struct RowFft {
 // What bounds a launch: LDS and vector work per element beside 16 bytes of HBM
 // traffic.  2048^2 angular spectrum of a 1024^2 field, us per launch (first /
 // mid / last), radix-8 stages with every stage and both ends through LDS: 15.8 /
-// 39.1 / 25.0; this form: FIGURES.
+// 39.1 / 25.0; this form: 11.8 / 24.2 / 15.6.
 template <int LOG2M, int LOG2R, int PASS, bool INV>
 __global__ void __launch_bounds__(fft_threads(LOG2M, LOG2R), 4)
 fft_rows_kernel(const float2* __restrict__ in, float2* __restrict__ out, FftParams P) {
@@ -419,10 +419,12 @@ fft_rows_kernel(const float2* __restrict__ in, float2* __restrict__ out, FftPara
 }
 
 // log2 of the rows per workgroup for length-M rows: within the 160 KiB of LDS
-// beside the twiddles, 4 rows (32-byte runs in the transposed accesses) while
-// that leaves one workgroup per CU.
-constexpr int log2_rows(int log2m) {
-  return log2m <= 8 ? 0 : log2m == 9 ? 1 : log2m <= 12 ? 2 : 0;
+// beside the twiddles, enough for long runs in the transposed accesses while
+// that leaves one workgroup per CU.  2048^2, us at 2 / 4 / 8 rows: kFirst (1024
+// rows) 14.4 / 11.8 / 12.0, kLast 20.3 / 17.0 / 15.6; kMid has no transposed
+// access, and two workgroups on a CU overlap: 26.4 / 24.2 at 2 / 4 (1: 31.4).
+constexpr int log2_rows(int log2m, int pass) {
+  return log2m <= 8 ? 0 : log2m == 9 ? 1 : log2m == 11 && pass != kMid ? 3 : log2m <= 12 ? 2 : 0;
 }
 
 template <int LOG2M, int LOG2R, int PASS, bool INV>
@@ -448,13 +450,15 @@ hipError_t launch_rows(int log2m, const float2* in, float2* out, int batch, cons
     return hipErrorInvalidValue;
   } else {
     if (log2m != LOG2M) return launch_rows<PASS, INV, LOG2M + 1>(log2m, in, out, batch, P, s);
-    constexpr int R = log2_rows(LOG2M);
+    constexpr int R = log2_rows(LOG2M, PASS);
     if constexpr (PASS == kFirst && R > 0) {
       // a launch over the field's rows alone has fewer groups: halve the rows per
-      // group while there are fewer than 512
+      // group while there are fewer than 256
       int r = R;
       if (P.rows_lo > 0)
-        while (r > 0 && (2 * P.rows_lo) >> r < 512) --r;
+        while (r > 0 && ((2 * P.rows_lo) >> r < 256 || P.rows_lo % (1 << r))) --r;
+      if constexpr (R > 2)
+        if (r == 2) return launch_rows_r<LOG2M, 2, PASS, INV>(in, out, batch, P, s);
       if constexpr (R > 1)
         if (r == 1) return launch_rows_r<LOG2M, 1, PASS, INV>(in, out, batch, P, s);
       if (r == 0) return launch_rows_r<LOG2M, 0, PASS, INV>(in, out, batch, P, s);
@@ -478,7 +482,7 @@ bool fft_supported(int m) { return m >= 2 && m <= kMaxFftSide && (m & (m - 1)) =
 
 // A launch over the rows of an N x N field padded to M x M (ifftshifted):
 // the rows that hold the field are [0, N/2) and [M - N/2, M); transform only
-// those when N/2 is a multiple of the rows per workgroup.  The launch after it
+// those when N/2 is a multiple of the middle pass's rows per workgroup.  The launch after it
 // reads, in each of its rows, the positions the others would have written as
 // zeros.
 static FftParams first_params(int N, int M) {
@@ -488,7 +492,7 @@ static FftParams first_params(int N, int M) {
   A.in_bstride = (long)N * N;
   A.out_bstride = (long)M * M;
   const int half = N / 2;
-  A.rows_lo = N < M && half > 0 && half % (1 << log2_rows(ilog2(M))) == 0 ? half : 0;
+  A.rows_lo = N < M && half > 0 && half % (1 << log2_rows(ilog2(M), kMid)) == 0 ? half : 0;
   return A;
 }
 static FftParams next_params(const FftParams& A, int M) {
