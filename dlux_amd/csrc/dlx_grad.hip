@@ -10,60 +10,54 @@
 //                   (the transpose of eval_basis), deterministic two-pass sum.
 //
 // Both are HBM-bound streaming passes: float4 loads, one pass over the planes.
+#include <type_traits>
+
 #include "dlx_internal.h"
 
 namespace dlx {
 namespace {
 
+// V pixels and 8 planes in flight per lane.
+template <int V>
 __global__ void __launch_bounds__(256)
 grad_reduce_kernel(GradChunk c, int nb, long npix, const float* __restrict__ h,
-                   int accumulate, int vec_ok, float* __restrict__ g_opd,
-                   float* __restrict__ g_phase) {
-  const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;   // float4 index
-  const long p = 4 * q;
+                   int accumulate, float* __restrict__ g_opd, float* __restrict__ g_phase) {
+  constexpr int kDepth = 8;
+  const long p = ((long)blockIdx.x * blockDim.x + threadIdx.x) * V;
   if (p >= npix) return;
-  // float4 accesses need every plane 16-byte aligned (npix % 4 == 0)
-  const bool full = vec_ok && p + 4 <= npix;
-  float4 so = make_float4(0.f, 0.f, 0.f, 0.f), sp = so;
-  for (int b = 0; b < nb; ++b) {
-    const float* hb = h + (long)b * npix + p;
-    float4 v;
-    if (full) {
-      v = *(const float4*)hb;
-    } else {
-      v.x = hb[0];
-      v.y = p + 1 < npix ? hb[1] : 0.f;
-      v.z = p + 2 < npix ? hb[2] : 0.f;
-      v.w = p + 3 < npix ? hb[3] : 0.f;
-    }
-    const float k = c.kw[b];
-    so.x += k * v.x; so.y += k * v.y; so.z += k * v.z; so.w += k * v.w;
-    sp.x += v.x; sp.y += v.y; sp.z += v.z; sp.w += v.w;
-  }
-  const float ov[4] = {so.x, so.y, so.z, so.w}, pv[4] = {sp.x, sp.y, sp.z, sp.w};
-  if (full) {
-    if (g_opd) {
-      float4 o = so;
-      if (accumulate) {
-        const float4 a = *(const float4*)(g_opd + p);
-        o.x += a.x; o.y += a.y; o.z += a.z; o.w += a.w;
+  PixelRun<V> so{}, sp{};
+  auto group = [&](auto FULL, int b0) __attribute__((always_inline)) {
+    PixelRun<V> v[kDepth];
+#pragma unroll
+    for (int e = 0; e < kDepth; ++e)
+      v[e].load(h + (long)(decltype(FULL)::value || b0 + e < nb ? b0 + e : nb - 1) * npix + p);
+#pragma unroll
+    for (int e = 0; e < kDepth; ++e) {
+      if (decltype(FULL)::value || b0 + e < nb) {
+        const float k = c.kw[b0 + e];
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+          so.v[q] += k * v[e].v[q];
+          sp.v[q] += v[e].v[q];
+        }
       }
-      *(float4*)(g_opd + p) = o;
     }
-    if (g_phase) {
-      float4 o = sp;
-      if (accumulate) {
-        const float4 a = *(const float4*)(g_phase + p);
-        o.x += a.x; o.y += a.y; o.z += a.z; o.w += a.w;
-      }
-      *(float4*)(g_phase + p) = o;
+  };
+  int b0 = 0;
+  for (; b0 + kDepth <= nb; b0 += kDepth) group(std::true_type{}, b0);
+  if (b0 < nb) group(std::false_type{}, b0);
+  auto put = [&](float* g, PixelRun<V> r) __attribute__((always_inline)) {
+    if (!g) return;
+    if (accumulate) {
+      PixelRun<V> o;
+      o.load(g + p);
+#pragma unroll
+      for (int q = 0; q < V; ++q) r.v[q] += o.v[q];
     }
-  } else {
-    for (int e = 0; e < 4 && p + e < npix; ++e) {
-      if (g_opd) g_opd[p + e] = ov[e] + (accumulate ? g_opd[p + e] : 0.f);
-      if (g_phase) g_phase[p + e] = pv[e] + (accumulate ? g_phase[p + e] : 0.f);
-    }
-  }
+    r.store(g + p);
+  };
+  put(g_opd, so);
+  put(g_phase, sp);
 }
 
 // Pass 1: partial[(s * nbasis + j) * S + part] = sum over the part's pixel range.
@@ -121,11 +115,13 @@ project_final_kernel(int total, int nparts, const float* __restrict__ partial,
 
 hipError_t launch_grad_reduce(const GradChunk& c, int nb, long npix, const float* h,
                               int accumulate, float* g_opd, float* g_phase, hipStream_t s) {
-  const long quads = (npix + 3) / 4;
-  const int vec_ok = (npix % 4 == 0) && ((uintptr_t)h % 16 == 0) &&
-                     ((uintptr_t)g_opd % 16 == 0) && ((uintptr_t)g_phase % 16 == 0);
-  hipLaunchKernelGGL(grad_reduce_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, s,
-                     c, nb, npix, h, accumulate, vec_ok, g_opd, g_phase);
+  if ((npix % 4 == 0) && ((uintptr_t)h % 16 == 0) && ((uintptr_t)g_opd % 16 == 0) &&
+      ((uintptr_t)g_phase % 16 == 0))
+    hipLaunchKernelGGL(grad_reduce_kernel<4>, dim3((unsigned)((npix / 4 + 255) / 256)), dim3(256), 0,
+                       s, c, nb, npix, h, accumulate, g_opd, g_phase);
+  else
+    hipLaunchKernelGGL(grad_reduce_kernel<1>, dim3((unsigned)((npix + 255) / 256)), dim3(256), 0, s,
+                       c, nb, npix, h, accumulate, g_opd, g_phase);
   return hipGetLastError();
 }
 

@@ -44,6 +44,24 @@ inline int launch_status(const char* what) {
   return DLX_OK;
 }
 
+// V consecutive floats of a plane, one access (V = 4: 16-byte aligned).
+template <int V>
+struct PixelRun {
+  float v[V];
+  __device__ __forceinline__ void load(const float* p) {
+    if constexpr (V == 4) {
+      const float4 t = *(const float4*)p;
+      v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
+    } else {
+      v[0] = *p;
+    }
+  }
+  __device__ __forceinline__ void store(float* p) const {
+    if constexpr (V == 4) *(float4*)p = make_float4(v[0], v[1], v[2], v[3]);
+    else *p = v[0];
+  }
+};
+
 inline size_t align_up(size_t x, size_t a = 256) { return (x + a - 1) / a * a; }
 
 // Device-side per-instance MFT parameters (one per wavelength / source).

@@ -2,6 +2,8 @@
 // of the hot path (gfx950): pupil-field synthesis, basis evaluation, power and
 // intensity reductions.  All are HBM-bound; they are written for coalesced
 // 8/16-byte accesses with one pixel (or four) per lane.
+#include <type_traits>
+
 #include "dlx_internal.h"
 #include "dlx_phasor.h"
 
@@ -77,91 +79,91 @@ hipError_t launch_pupil_chunk(const PupilChunk& c, int nb, int n, double dx, dou
 
 // ---------------------------------------------------------------------------
 // Basis evaluation: out[s][p] = sum_j coeffs[s][j] * basis[j][p] (+ base[p]).
-// One lane per 4 pixels (16-byte loads); the basis is streamed once for up to
-// kSets coefficient sets (utils/math.py:177-196 tensordot).
+// V pixels a lane: four (16-byte accesses) where the planes are aligned, one
+// elsewhere.  The basis is streamed once for up to kSets coefficient sets
+// (utils/math.py:177-196 tensordot), kDepth planes of it in flight per lane, and
+// kRest of the last ones, missing planes loading the last again: a plane loaded
+// by itself costs a full latency.  21 planes of 401^2 (one-pixel lanes, which
+// coalesce) 8.8 -> 5.6 us; 36 of 512^2 7.6 -> 7.0 us, 5.4 TB/s.
 // ---------------------------------------------------------------------------
 constexpr int kSets = 8;
 
-// NS coefficient sets per launch; the basis loop is unrolled so several
-// 16-byte loads per lane are in flight (the kernel streams the basis once).
-template <int NS>
+template <int NS, int V>
 __global__ void __launch_bounds__(256)
 eval_basis_kernel(int nbasis, long npix, int nsets, const float* __restrict__ basis,
                   const float* __restrict__ coeffs, const float* __restrict__ base,
-                  float* __restrict__ out, int vec_ok) {
-  const long p4 = ((long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-  if (p4 >= npix) return;
-  const bool full = vec_ok && (p4 + 4 <= npix);
-  float acc[NS][4];
+                  float* __restrict__ out) {
+  constexpr int kDepth = NS == 1 ? 12 : 6, kRest = NS == 1 ? 6 : 3;
+  const long p = ((long)blockIdx.x * blockDim.x + threadIdx.x) * V;
+  if (p >= npix) return;
+  float acc[NS][V];
 #pragma unroll
   for (int s = 0; s < NS; ++s)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) acc[s][q] = 0.f;
-#pragma unroll 6
-  for (int j = 0; j < nbasis; ++j) {
-    float v[4];
-    const float* row = basis + (long)j * npix + p4;
-    if (full) {
-      const float4 t = *(const float4*)row;
-      v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
-    } else {
+    for (int q = 0; q < V; ++q) acc[s][q] = 0.f;
+  auto group = [&](auto FULL, int j0) __attribute__((always_inline)) {
+    constexpr int D = decltype(FULL)::value ? kDepth : kRest;
+    PixelRun<V> v[D];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) v[q] = (p4 + q < npix) ? row[q] : 0.f;
-    }
+    for (int e = 0; e < D; ++e)
+      v[e].load(basis + (long)(decltype(FULL)::value || j0 + e < nbasis ? j0 + e : nbasis - 1) * npix + p);
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      if (NS == 1 || s < nsets) {
-        const float cj = coeffs[(long)s * nbasis + j];
+    for (int e = 0; e < D; ++e) {
+      if (decltype(FULL)::value || j0 + e < nbasis) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) acc[s][q] = fmaf(cj, v[q], acc[s][q]);
-      }
-    }
-  }
+        for (int s = 0; s < NS; ++s) {
+          if (NS == 1 || s < nsets) {
+            const float cj = coeffs[(long)s * nbasis + j0 + e];
 #pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    if (NS > 1 && s >= nsets) break;
-    if (full) {
-      float4 r = make_float4(acc[s][0], acc[s][1], acc[s][2], acc[s][3]);
-      if (base) {
-        const float4 bb = *(const float4*)(base + p4);
-        r.x += bb.x; r.y += bb.y; r.z += bb.z; r.w += bb.w;
-      }
-      *(float4*)(out + (long)s * npix + p4) = r;
-    } else {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        if (p4 + q < npix) {
-          float r = acc[s][q];
-          if (base) r += base[p4 + q];
-          out[(long)s * npix + p4 + q] = r;
+            for (int q = 0; q < V; ++q) acc[s][q] = fmaf(cj, v[e].v[q], acc[s][q]);
+          }
         }
       }
     }
+  };
+  int j0 = 0;
+  for (; j0 + kDepth <= nbasis; j0 += kDepth) group(std::true_type{}, j0);
+  for (; j0 < nbasis; j0 += kRest) group(std::false_type{}, j0);
+  PixelRun<V> bb{};
+  if (base) bb.load(base + p);
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    if (NS > 1 && s >= nsets) break;
+    PixelRun<V> r;
+#pragma unroll
+    for (int q = 0; q < V; ++q) r.v[q] = base ? acc[s][q] + bb.v[q] : acc[s][q];
+    r.store(out + (long)s * npix + p);
   }
+}
+
+template <int V>
+hipError_t eval_basis_go(int nbasis, long npix, int nsets, const float* basis, const float* coeffs,
+                         const float* base, float* out, hipStream_t s) {
+  const dim3 grid((unsigned)((npix / V + 255) / 256));
+  if (nsets == 1) {
+    hipLaunchKernelGGL((eval_basis_kernel<1, V>), grid, dim3(256), 0, s, nbasis, npix, 1, basis,
+                       coeffs, base, out);
+    return hipGetLastError();
+  }
+  for (int s0 = 0; s0 < nsets; s0 += kSets) {
+    const int ns = nsets - s0 < kSets ? nsets - s0 : kSets;
+    hipLaunchKernelGGL((eval_basis_kernel<kSets, V>), grid, dim3(256), 0, s, nbasis, npix, ns, basis,
+                       coeffs + (long)s0 * nbasis, base, out + (long)s0 * npix);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 hipError_t launch_eval_basis(int nbasis, long npix, int nsets, const float* basis,
                              const float* coeffs, const float* base, float* out,
                              hipStream_t s) {
   // 16-byte loads and stores need 16-byte aligned rows
-  const int vec_ok = ((npix & 3) == 0) && ((reinterpret_cast<uintptr_t>(basis) & 15) == 0) &&
-                     ((reinterpret_cast<uintptr_t>(out) & 15) == 0) &&
-                     (!base || (reinterpret_cast<uintptr_t>(base) & 15) == 0);
-  const long lanes = (npix + 3) / 4;
-  const dim3 grid((unsigned)((lanes + 255) / 256));
-  if (nsets == 1) {
-    hipLaunchKernelGGL(eval_basis_kernel<1>, grid, dim3(256), 0, s, nbasis, npix, 1, basis,
-                       coeffs, base, out, vec_ok);
-    return hipGetLastError();
-  }
-  for (int s0 = 0; s0 < nsets; s0 += kSets) {
-    const int ns = nsets - s0 < kSets ? nsets - s0 : kSets;
-    hipLaunchKernelGGL(eval_basis_kernel<kSets>, grid, dim3(256), 0, s, nbasis, npix, ns, basis,
-                       coeffs + (long)s0 * nbasis, base, out + (long)s0 * npix, vec_ok);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
+  const bool vec = ((npix & 3) == 0) && ((reinterpret_cast<uintptr_t>(basis) & 15) == 0) &&
+                   ((reinterpret_cast<uintptr_t>(out) & 15) == 0) &&
+                   (!base || (reinterpret_cast<uintptr_t>(base) & 15) == 0);
+  return vec ? eval_basis_go<4>(nbasis, npix, nsets, basis, coeffs, base, out, s)
+             : eval_basis_go<1>(nbasis, npix, nsets, basis, coeffs, base, out, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -223,38 +225,54 @@ hipError_t launch_intensity(long npix, int batch, const float2* f, int sum_batch
   return hipGetLastError();
 }
 
-// psf[p] (=|+=) sum_b planes[b][p] in index order (deterministic); four
-// pixels per lane and a plane loop unrolled 16 deep keep 256 bytes per lane in
-// flight (a 256^2 PSF has only 16 Ki lanes).
+// psf[p] (=|+=) sum_b planes[b][p] in index order (deterministic): V pixels and
+// 16 planes in flight per lane, then kRest of the rest (one after another they
+// cost a full latency each): 7.9 -> 3.1 us at 11 planes of 173^2; 64 planes of
+// 256^2 take 4.7 us, 3.6 TB/s (a 256^2 image has only 256 waves of 4 pixels; one
+// pixel a lane took 5.2).
+template <int V>
 __global__ void __launch_bounds__(256)
 sum_planes_kernel(long npix, int nplanes, const float* __restrict__ planes, int accumulate,
-                  float* __restrict__ psf, int vec_ok) {
-  const long p4 = ((long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-  if (p4 >= npix) return;
-  if (vec_ok) {
-    float4 acc = accumulate ? *(const float4*)(psf + p4) : make_float4(0.f, 0.f, 0.f, 0.f);
+                  float* __restrict__ psf) {
+  constexpr int kRest = 8;
+  const long p = ((long)blockIdx.x * blockDim.x + threadIdx.x) * V;
+  if (p >= npix) return;
+  PixelRun<V> acc{};
+  if (accumulate) acc.load(psf + p);
+  int b0 = 0;
 #pragma unroll 16
-    for (int b = 0; b < nplanes; ++b) {
-      const float4 v = *(const float4*)(planes + (long)b * npix + p4);
-      acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w;
-    }
-    *(float4*)(psf + p4) = acc;
-  } else {
-    for (long p = p4; p < p4 + 4 && p < npix; ++p) {
-      float acc = accumulate ? psf[p] : 0.f;
-      for (int b = 0; b < nplanes; ++b) acc += planes[(long)b * npix + p];
-      psf[p] = acc;
+  for (; b0 < (nplanes & ~15); ++b0) {
+    PixelRun<V> v;
+    v.load(planes + (long)b0 * npix + p);
+#pragma unroll
+    for (int q = 0; q < V; ++q) acc.v[q] += v.v[q];
+  }
+  for (; b0 < nplanes; b0 += kRest) {
+    PixelRun<V> v[kRest];
+#pragma unroll
+    for (int e = 0; e < kRest; ++e)
+      v[e].load(planes + (long)(b0 + e < nplanes ? b0 + e : nplanes - 1) * npix + p);
+#pragma unroll
+    for (int e = 0; e < kRest; ++e) {
+      if (b0 + e < nplanes) {
+#pragma unroll
+        for (int q = 0; q < V; ++q) acc.v[q] += v[e].v[q];
+      }
     }
   }
+  acc.store(psf + p);
 }
 
 hipError_t launch_sum_planes(long npix, int nplanes, const float* planes, int accumulate,
                              float* psf, hipStream_t s) {
-  const long lanes = (npix + 3) / 4;
-  const int vec_ok = ((npix & 3) == 0) && ((reinterpret_cast<uintptr_t>(planes) & 15) == 0) &&
-                     ((reinterpret_cast<uintptr_t>(psf) & 15) == 0);
-  hipLaunchKernelGGL(sum_planes_kernel, dim3((unsigned)((lanes + 255) / 256)), dim3(256), 0, s,
-                     npix, nplanes, planes, accumulate, psf, vec_ok);
+  const bool vec = ((npix & 3) == 0) && ((reinterpret_cast<uintptr_t>(planes) & 15) == 0) &&
+                   ((reinterpret_cast<uintptr_t>(psf) & 15) == 0);
+  if (vec)
+    hipLaunchKernelGGL(sum_planes_kernel<4>, dim3((unsigned)((npix / 4 + 255) / 256)), dim3(256), 0,
+                       s, npix, nplanes, planes, accumulate, psf);
+  else
+    hipLaunchKernelGGL(sum_planes_kernel<1>, dim3((unsigned)((npix + 255) / 256)), dim3(256), 0, s,
+                       npix, nplanes, planes, accumulate, psf);
   return hipGetLastError();
 }
 
