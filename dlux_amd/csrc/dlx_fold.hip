@@ -24,6 +24,17 @@ typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t u32x4_t;
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef const __attribute__((address_space(1))) void gbl_void_t;
 
+// Global accesses through pointers that may come from descriptors in memory,
+// whose address space the compiler does not see: as flat accesses they would
+// count with the LDS ones, and every wait for LDS would wait for memory (48
+// sources of 256^2 to 1024^2, with the branch-free steps: 728 -> 675 us).
+__device__ __forceinline__ u32x4_t load_global(const void* p) {
+  return *(const __attribute__((address_space(1))) u32x4_t*)p;
+}
+__device__ __forceinline__ void store_global(void* p, u32x4_t v) {
+  *(__attribute__((address_space(1))) u32x4_t*)p = v;
+}
+
 constexpr int kThreads = 256;   // 4 waves
 constexpr int kStageK = 16;     // k per stage
 constexpr int kRow = 64;        // bytes of a tile row per stage
@@ -35,10 +46,6 @@ __device__ __forceinline__ int xcd_order(int hw, int total) {
   const int per = total / kXcds;
   if (hw >= per * kXcds) return hw;   // tail that does not fill all XCDs evenly
   return (hw % kXcds) * per + hw / kXcds;
-}
-
-__device__ __forceinline__ float quad_swap1(float v) {   // the value of lane ^ 1
-  return __uint_as_float(quad_xor<1>(__float_as_uint(v)));
 }
 
 // ---------------------------------------------------------------------------
@@ -69,11 +76,14 @@ struct TileRows {
 };
 
 // A lane's two pieces of tile row row0 + lane % 32 (row0 a multiple of 32).
-__device__ __forceinline__ void read_frag(u32x4_t (&f)[2], const uint8_t* tile, int row0) {
+// `odd`: the rows are parts of beta = 1 as a loader writes them (part_row).
+__device__ __forceinline__ void read_frag(u32x4_t (&f)[2], const uint8_t* tile, int row0,
+                                          int odd = 0) {
   const int lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
-  const uint8_t* r = tile + (row0 + lr) * kRow;
+  const uint8_t* r = tile + (row0 + (lr ^ (2 * odd))) * kRow;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) f[j] = *(const u32x4_t*)(r + (((2 * lk + j) ^ ((lr >> 2) & 3)) << 4));
+  for (int j = 0; j < 2; ++j)
+    f[j] = *(const u32x4_t*)(r + (((2 * lk + j) ^ ((lr >> 2) & 3) ^ odd) << 4));
 }
 
 // A table's pieces in the order MFMAs take them: per 32 rows and stage, 2 KiB
@@ -85,8 +95,8 @@ __device__ __forceinline__ long table_block(int part, int rows_pad, int kp, int 
 }
 __device__ __forceinline__ void load_frag(u32x4_t (&f)[2], const uint8_t* blk, int s) {
   const uint8_t* p = blk + (long)s * 2048 + (threadIdx.x & 63) * 16;
-  f[0] = *(const u32x4_t*)p;
-  f[1] = *(const u32x4_t*)(p + 1024);
+  f[0] = load_global(p);
+  f[1] = load_global(p + 1024);
 }
 
 // acc[i][j] += sum over the stage's 16 k of a_i(m) b_j(n): lane holds column
@@ -144,6 +154,10 @@ __device__ __forceinline__ void put4(uint8_t* row, int quad, int f, const float 
   }
 }
 
+// Where a loader puts row py of a part: the lanes of beta = 1 write beside those
+// of beta = 0, whose banks they would otherwise share.
+__device__ __forceinline__ int part_row(int py, int beta) { return py ^ (2 * beta); }
+__device__ __forceinline__ int part_slot(int py, int beta) { return ((py >> 2) & 3) ^ beta; }
 
 __device__ __forceinline__ float2 cmul(float2 a, float2 w) {
   return make_float2(a.x * w.x - a.y * w.y, a.x * w.y + a.y * w.x);
@@ -164,7 +178,11 @@ struct FoldPart {
   float v[2][2][4];   // [alpha][c][k]
 };
 
-// x and y folds; vp / vm: the values at k+ and k- of the thread's own row.
+// x and y folds; vp / vm: the values at k+ and k- of the thread's own row, times
+// -1 in the lanes of row y- (beta = 1): then own + other's * (beta ? 1 : -1) is
+// the even part in one lane and the odd part in the other, one instruction a
+// value (a swap, a copy and a multiply-add before: 64 of 423 vector
+// instructions of two split stages).
 __device__ __forceinline__ void fold_x(const float2 (&vp)[4], const float2 (&vm)[4], FoldPart& o) {
 #pragma clang fp contract(off)
 #pragma unroll
@@ -176,14 +194,19 @@ __device__ __forceinline__ void fold_x(const float2 (&vp)[4], const float2 (&vm)
   }
 }
 __device__ __forceinline__ void fold_y(FoldPart& o, int beta) {
-  const float sg = beta ? -1.f : 1.f;   // lane beta = 1 (row y-): v(y+) - v(y-)
+  const float sg = beta ? 1.f : -1.f;
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        o.v[a][c][e] = __builtin_fmaf(o.v[a][c][e], sg, quad_swap1(o.v[a][c][e]));
+  for (int a = 0; a < 2; ++a) {
+    float(&x)[4] = o.v[a][0], (&y)[4] = o.v[a][1];
+    // x = x of lane ^ 1 * sg + x; a DPP operand is read two states after its write
+#define DLX_FOLD(i) "v_fmac_f32_dpp %" #i ", %" #i ", %8 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+    asm("s_nop 1\n\t" DLX_FOLD(0) DLX_FOLD(1) DLX_FOLD(2) DLX_FOLD(3) DLX_FOLD(4) DLX_FOLD(5)
+            DLX_FOLD(6) DLX_FOLD(7)
+        : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(y[0]), "+v"(y[1]), "+v"(y[2]),
+          "+v"(y[3])
+        : "v"(sg));
+#undef DLX_FOLD
+  }
 }
 
 // The pupil loader of one thread.  VEC: n a multiple of 8 and 16-byte aligned
@@ -199,7 +222,7 @@ struct PupilLoad {
   int n, kh, quad, x0i;             // x0i = n / 2: the first positive column
   bool has_opd, has_amp, has_phase;
   double inv_wl, tx, tyY, dx, x0, co;   // co: 1 if there is an OPD, else 0
-  float ca, cb;                     // amplitude = ca * value + cb; zero outside the rows
+  float ca, cb;                     // amplitude = ca * value + cb, signed; zero outside the rows
   struct Raw { float4 op, om, ap, am; };   // plus runs (k ascending), minus runs (descending)
 
   __device__ __forceinline__ void init(const FoldPupil& p, int n_, int py, int beta, int quad_,
@@ -216,7 +239,7 @@ struct PupilLoad {
     inv_wl = TILT || ANY ? inv : has_opd ? inv : 0.0;
     tx = p.tx; dx = p.dx; x0 = p.x0;
     tyY = p.ty * pupil_coord(y, p.dx, p.x0);
-    const float sc = row_ok ? p.scale : 0.f;
+    const float sc = !row_ok ? 0.f : beta ? -p.scale : p.scale;   // the y fold's sign
     ca = has_amp ? sc : 0.f;
     cb = has_amp ? 0.f : sc;
   }
@@ -321,8 +344,13 @@ struct FieldLoad {
       }
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
+    for (int e = 0; e < 4; ++e) {
       if (!(row_ok && p + e < kh)) vp[e] = vm[e] = make_float2(0.f, 0.f);
+      if (beta) {   // the y fold's sign
+        vp[e] = make_float2(-vp[e].x, -vp[e].y);
+        vm[e] = make_float2(-vm[e].x, -vm[e].y);
+      }
+    }
     fold_x(vp, vm, out);
     fold_y(out, beta);
   }
@@ -364,8 +392,8 @@ __device__ __forceinline__ void store_block(uint8_t* patch, const f32x16_t& acc,
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
     const int r = 8 * t + (lane >> 3), piece = lane & 7;
-    const uint4 v = *(const uint4*)(patch + r * kPatchRow + piece * 16);
-    if (r < rows) *(uint4*)(out + (long)r * row_bytes + piece * 16) = v;
+    const u32x4_t v = *(const u32x4_t*)(patch + r * kPatchRow + piece * 16);
+    if (r < rows) store_global(out + (long)r * row_bytes + piece * 16, v);
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -418,6 +446,9 @@ struct S1 {
   // first A row (in (alpha, beta, c, py) order) and first column of a wave
   __device__ static __forceinline__ int arow(int wave) {
     return (wave >> 1) * 128 + (BNQ >= 64 ? 0 : (wave & 1) * 64);
+  }
+  __device__ static __forceinline__ int beta(int wave, int i) {
+    return BNQ >= 64 ? i >> 1 : wave & 1;
   }
   __device__ static __forceinline__ int col(int wave) {
     return BNQ >= 64 ? (wave & 1) * (BNQ / 2) : 0;
@@ -539,11 +570,12 @@ fold_stage1_kernel(FoldStage1 a) {
     if constexpr (LOAD != FOLD_FIELD) ld.part(s, beta, r, o);
     else ld.part(s, beta, r, phased, win[s & 1], o);
     uint8_t* buf = lds + (s & 1) * kBuf;
+    const int pr = part_row(py, beta), fl = part_slot(py, beta);
 #pragma unroll
     for (int al = 0; al < 2; ++al)
 #pragma unroll
       for (int c = 0; c < 2; ++c)
-        put4<BF>(buf + (((al * 2 + beta) * 2 + c) * 32 + py) * kRow, quad, (py >> 2) & 3, o.v[al][c]);
+        put4<BF>(buf + (((al * 2 + beta) * 2 + c) * 32 + pr) * kRow, quad, fl, o.v[al][c]);
   };
   u32x4_t fb[2][NJ][2];
   auto load_tab = [&](auto J, int s) __attribute__((always_inline)) {
@@ -558,7 +590,8 @@ fold_stage1_kernel(FoldStage1 a) {
     const uint8_t* la = lds + j0 * kBuf;
     u32x4_t fa[NI][2];
 #pragma unroll
-    for (int i = 0; i < NI; ++i) read_frag(fa[i], la, S::arow(wave) + 32 * i);
+    for (int i = 0; i < NI; ++i)
+      read_frag(fa[i], la, S::arow(wave) + 32 * i, S::beta(wave, i));
     load_tab(std::integral_constant<int, 1 - j0>{}, s + 1);
     ld.raw(s + 2, raw[j0]);
     window(s + 2);
@@ -644,11 +677,12 @@ fold_stage1_small_kernel(FoldStage1 a) {
     if constexpr (LOAD != FOLD_FIELD) ld.part(2 * s + run, beta, r, o);
     else ld.part(2 * s + run, beta, r, phased, win[s & 1] + run * kStageK, o);
     uint8_t* buf = lds + ((s & 1) * 2 + run) * kRun;
+    const int pr = part_row(py, beta), fl = part_slot(py, beta);
 #pragma unroll
     for (int al = 0; al < 2; ++al)
 #pragma unroll
       for (int c = 0; c < 2; ++c)
-        put4<BF>(buf + ((al * 2 + beta) * 32 + c * 16 + py) * kRow, quad, (py >> 2) & 3, o.v[al][c]);
+        put4<BF>(buf + ((al * 2 + beta) * 32 + c * 16 + pr) * kRow, quad, fl, o.v[al][c]);
   };
   f32x16_t acc[1][1];
   zero_acc(acc);
@@ -663,7 +697,7 @@ fold_stage1_small_kernel(FoldStage1 a) {
     lds_barrier();   // stage s is in LDS, stage s - 1 has been read
     u32x4_t fa[2][1][2];
 #pragma unroll
-    for (int e = 0; e < 2; ++e) read_frag(fa[e][0], lds + (j0 * 2 + e) * kRun, wave * 32);
+    for (int e = 0; e < 2; ++e) read_frag(fa[e][0], lds + (j0 * 2 + e) * kRun, wave * 32, wave & 1);
     load_tab(std::integral_constant<int, 1 - j0>{}, s + 1);
     ld.raw(2 * (s + 2) + run, raw[j0]);
     window(s + 2);
@@ -994,7 +1028,7 @@ __device__ __forceinline__ void stage2_tile(const Stage2Prob& a, int qy0, int qx
         im *= alpha;
         const long o = (long)y * m + x;
         if constexpr (EPI == FOLD_INTENSITY) {
-          ((float*)a.out)[o] = re * re + im * im;
+          ((__attribute__((address_space(1))) float*)a.out)[o] = re * re + im * im;
         } else if constexpr (EPI == FOLD_STORE) {
           float2 v = make_float2(re, im);
           if (phased) {
@@ -1170,7 +1204,8 @@ fold_group_stage1_kernel(FoldGroup g) {
   auto load_raw = [&](auto J, int s) __attribute__((always_inline)) {
     const int sc = s < nst ? s : nst - 1;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) raw[decltype(J)::value][e] = row[sc * kStageK + e];
+    for (int e = 0; e < 4; ++e)
+      raw[decltype(J)::value][e] = __builtin_bit_cast(float4, load_global(row + sc * kStageK + e));
   };
   auto convert = [&](int s, int l, int slot, const float4 (&r)[4]) __attribute__((always_inline)) {
     float v[2][2][4];
@@ -1183,11 +1218,12 @@ fold_group_stage1_kernel(FoldGroup g) {
       v[1][1][e] = r[e].w * w.x + r[e].x * w.y;
     }
     uint8_t* buf = lds + slot * kBuf;
+    const int pr = part_row(py, beta), fl = part_slot(py, beta);
 #pragma unroll
     for (int al = 0; al < 2; ++al)
 #pragma unroll
       for (int c = 0; c < 2; ++c)
-        put4<true>(buf + (((al * 2 + beta) * 2 + c) * 32 + py) * kRow, quad, (py >> 2) & 3, v[al][c]);
+        put4<true>(buf + (((al * 2 + beta) * 2 + c) * 32 + pr) * kRow, quad, fl, v[al][c]);
   };
   u32x4_t fb[2][NJ][2];
   auto load_tab = [&](auto J, const uint8_t* const (&tb)[NJ], int s) __attribute__((always_inline)) {
@@ -1195,16 +1231,19 @@ fold_group_stage1_kernel(FoldGroup g) {
 #pragma unroll
     for (int j = 0; j < NJ; ++j) load_frag(fb[decltype(J)::value][j], tb[j], sc);
   };
-  // step (s, l): P = s & 1; slot and fragment set (s L + l) & 1
-  auto step = [&](auto P, auto LL, int s) __attribute__((always_inline)) {
+  // step (s, l): P = s & 1; slot and fragment set (s L + l) & 1.  ALL: the group
+  // has L tiles; MORE: there is a next stage -- then no branch splits the step.
+  auto step = [&](auto P, auto LL, auto ALL, auto MORE, int s) __attribute__((always_inline)) {
+    constexpr bool all = decltype(ALL)::value, more = decltype(MORE)::value;
     constexpr int p = decltype(P)::value, l = decltype(LL)::value;
     constexpr int k = (p * L + l) & 1, ln = (l + 1) % L;
     lds_barrier();
     const int sn = l + 1 < L ? s : s + 1;   // the next step's stage
     u32x4_t fa[NI][2];
-    if (l < count) {
+    if (all || l < count) {
 #pragma unroll
-      for (int i = 0; i < NI; ++i) read_frag(fa[i], lds + k * kBuf, S::arow(wave) + 32 * i);
+      for (int i = 0; i < NI; ++i)
+        read_frag(fa[i], lds + k * kBuf, S::arow(wave) + 32 * i, S::beta(wave, i));
     }
     load_tab(IC<1 - k>{}, tab[ln], sn);
     if constexpr (l == 0) {
@@ -1214,16 +1253,28 @@ fold_group_stage1_kernel(FoldGroup g) {
       // the window of stage s is still read by this stage's converts if L > 1
       window(L == 1 ? s + 2 : s + 1);
     }
-    if (l < count) mma_stage<true, NI, NJ>(acc[l], fa, fb[k]);
-    if (sn < nst && ln < count) {
+    if (all || l < count) mma_stage<true, NI, NJ>(acc[l], fa, fb[k]);
+    if ((l + 1 < L || more || sn < nst) && (all || ln < count)) {
       if constexpr (l + 1 < L) convert(sn, ln, 1 - k, raw[p]);
       else convert(sn, ln, 1 - k, raw[1 - p]);
     }
   };
-  auto stage = [&](auto P, int s) __attribute__((always_inline)) {
-    step(P, IC<0>{}, s);
-    if constexpr (L > 1) step(P, IC<1>{}, s);
-    if constexpr (L > 2) { step(P, IC<2>{}, s); step(P, IC<3>{}, s); }
+  auto stage = [&](auto P, auto ALL, auto MORE, int s) __attribute__((always_inline)) {
+    step(P, IC<0>{}, ALL, MORE, s);
+    if constexpr (L > 1) step(P, IC<1>{}, ALL, MORE, s);
+    if constexpr (L > 2) {
+      step(P, IC<2>{}, ALL, MORE, s);
+      step(P, IC<3>{}, ALL, MORE, s);
+    }
+  };
+  auto run = [&](auto ALL) __attribute__((always_inline)) {
+    int s = 0;
+    for (; s + 2 < nst; s += 2) {
+      stage(IC<0>{}, ALL, std::true_type{}, s);
+      stage(IC<1>{}, ALL, std::true_type{}, s + 1);
+    }
+    stage(IC<0>{}, ALL, std::false_type{}, s);
+    if (s + 1 < nst) stage(IC<1>{}, ALL, std::false_type{}, s + 1);
   };
   load_tab(IC<0>{}, tab[0], 0);
   load_raw(IC<0>{}, 0);
@@ -1232,12 +1283,8 @@ fold_group_stage1_kernel(FoldGroup g) {
   if constexpr (L == 1) window(1);
   lds_barrier();
   convert(0, 0, 0, raw[0]);
-  int s = 0;
-  for (; s + 1 < nst; s += 2) {
-    stage(IC<0>{}, s);
-    stage(IC<1>{}, s + 1);
-  }
-  if (s < nst) stage(IC<0>{}, s);
+  if (L == 1 || count == L) run(std::true_type{});
+  else run(std::false_type{});
 #pragma unroll
   for (int l = 0; l < L; ++l) {
     if (l >= count) break;

@@ -32,7 +32,7 @@ template <int M>
 __device__ __forceinline__ uint32_t quad_xor(uint32_t v) {
   // quad_perm [q ^ M for q in 0..3]
   constexpr int ctrl = M == 1 ? 0xB1 : (M == 2 ? 0x4E : 0x1B);
-  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xF, 0xF, false);
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xF, 0xF, true);
 }
 
 }  // namespace dlx
