@@ -35,6 +35,9 @@ __device__ __forceinline__ void store_global(void* p, u32x4_t v) {
   *(__attribute__((address_space(1))) u32x4_t*)p = v;
 }
 
+template <int N>
+using IC = std::integral_constant<int, N>;
+
 constexpr int kThreads = 256;   // 4 waves
 constexpr int kStageK = 16;     // k per stage
 constexpr int kRow = 64;        // bytes of a tile row per stage
@@ -558,17 +561,17 @@ fold_stage1_kernel(FoldStage1 a) {
   const double on = (a.n & 1) ? 0.0 : 0.5;
   auto window = [&](int s) {   // formed two stages ahead of its use's products
     if constexpr (LOAD == FOLD_FIELD) {
-      if (phased && threadIdx.x < kStageK) {
+      if (threadIdx.x < kStageK) {
         const double u = (double)(s * kStageK + (int)threadIdx.x) + on, q = ph.c2 * u * u;
         const float2 wp = turn(fma(ph.cx, u, q)), wm = turn(fma(-ph.cx, u, q));
         win[s & 1][threadIdx.x] = make_float4(wp.x, wp.y, wm.x, wm.y);
       }
     }
   };
-  auto convert = [&](int s, const typename decltype(ld)::Raw& r) __attribute__((always_inline)) {
+  auto convert = [&](auto PH, int s, const typename decltype(ld)::Raw& r) __attribute__((always_inline)) {
     FoldPart o;
     if constexpr (LOAD != FOLD_FIELD) ld.part(s, beta, r, o);
-    else ld.part(s, beta, r, phased, win[s & 1], o);
+    else ld.part(s, beta, r, decltype(PH)::value, win[s & 1], o);
     uint8_t* buf = lds + (s & 1) * kBuf;
     const int pr = part_row(py, beta), fl = part_slot(py, beta);
 #pragma unroll
@@ -583,8 +586,8 @@ fold_stage1_kernel(FoldStage1 a) {
 #pragma unroll
     for (int j = 0; j < NJ; ++j) load_frag(fb[decltype(J)::value][j], tab[j], sc);
   };
-  // one stage: J = s & 1; FULL: there is a next one
-  auto step = [&](auto J, auto FULL, int s) __attribute__((always_inline)) {
+  // one stage: J = s & 1; FULL: there is a next one; PH: the field has a phase
+  auto step = [&](auto J, auto FULL, auto PH, int s) __attribute__((always_inline)) {
     constexpr int j0 = decltype(J)::value;
     lds_barrier();   // stage s is in LDS, stage s - 1 has been read
     const uint8_t* la = lds + j0 * kBuf;
@@ -592,35 +595,42 @@ fold_stage1_kernel(FoldStage1 a) {
 #pragma unroll
     for (int i = 0; i < NI; ++i)
       read_frag(fa[i], la, S::arow(wave) + 32 * i, S::beta(wave, i));
-    load_tab(std::integral_constant<int, 1 - j0>{}, s + 1);
+    load_tab(IC<1 - j0>{}, s + 1);
     ld.raw(s + 2, raw[j0]);
-    window(s + 2);
+    if constexpr (decltype(PH)::value) window(s + 2);
     // one wave per SIMD (small launches) keeps its products ahead of its
     // conversion: 17.0 against 19.5 us at 16 wavelengths of 512^2 -> 128^2; with
     // two, the raised priority cost 90 -> 100 us (float32, 64 of 512^2 -> 256^2)
     if constexpr (BNQ < 128) __builtin_amdgcn_s_setprio(1);
     mma_stage<BF, NI, NJ>(acc, fa, fb[j0]);
     if constexpr (BNQ < 128) __builtin_amdgcn_s_setprio(0);
-    if (decltype(FULL)::value || s + 1 < nst) convert(s + 1, raw[1 - j0]);
+    if (decltype(FULL)::value || s + 1 < nst) convert(PH, s + 1, raw[1 - j0]);
   };
-  load_tab(std::integral_constant<int, 0>{}, 0);
-  ld.raw(0, raw[0]);
-  ld.raw(1, raw[1]);
-  window(0);
-  window(1);
-  if constexpr (LOAD == FOLD_FIELD) lds_barrier();
-  convert(0, raw[0]);
-  // whole pairs: no path of the loop skips a load or a part.  A field's parts, with
-  // their choice of a phase, stay in a block of their own: merged with the
-  // products they spilled 567 registers at 128 columns
-  using Whole = std::bool_constant<LOAD != FOLD_FIELD>;
-  int s = 0;
-  for (; s + 2 < nst; s += 2) {
-    step(std::integral_constant<int, 0>{}, Whole{}, s);
-    step(std::integral_constant<int, 1>{}, Whole{}, s + 1);
-  }
-  step(std::integral_constant<int, 0>{}, std::false_type{}, s);
-  if (s + 1 < nst) step(std::integral_constant<int, 1>{}, std::false_type{}, s + 1);
+  auto run = [&](auto PH) __attribute__((always_inline)) {
+    load_tab(IC<0>{}, 0);
+    ld.raw(0, raw[0]);
+    ld.raw(1, raw[1]);
+    if constexpr (decltype(PH)::value) {
+      window(0);
+      window(1);
+      lds_barrier();
+    }
+    convert(PH, 0, raw[0]);
+    // whole pairs: no path of the loop skips a load or a part, and the choice of a
+    // field's phase is made outside it (16 fields 512^2 -> 256^2, float32: 48.0 ->
+    // 46.4 us).  At 128 columns a field's parts stay in a block of their own:
+    // merged with the products they spilled 567 registers
+    using Whole = std::bool_constant<LOAD != FOLD_FIELD || BNQ < 128>;
+    int s = 0;
+    for (; s + 2 < nst; s += 2) {
+      step(IC<0>{}, Whole{}, PH, s);
+      step(IC<1>{}, Whole{}, PH, s + 1);
+    }
+    step(IC<0>{}, std::false_type{}, PH, s);
+    if (s + 1 < nst) step(IC<1>{}, std::false_type{}, PH, s + 1);
+  };
+  if (LOAD == FOLD_FIELD && phased) run(std::bool_constant<LOAD == FOLD_FIELD>{});
+  else run(std::false_type{});
   lds_barrier();
   if constexpr (LOAD == FOLD_FIELD)
     if (phased) y_phase<BNQ>(lds, acc, ph.c2, ph.cy, a.n, py0);
@@ -665,17 +675,17 @@ fold_stage1_small_kernel(FoldStage1 a) {
   const double on = (a.n & 1) ? 0.0 : 0.5;
   auto window = [&](int s) {
     if constexpr (LOAD == FOLD_FIELD) {
-      if (phased && threadIdx.x < 2 * kStageK) {
+      if (threadIdx.x < 2 * kStageK) {
         const double u = (double)(s * 2 * kStageK + (int)threadIdx.x) + on, q = ph.c2 * u * u;
         const float2 wp = turn(fma(ph.cx, u, q)), wm = turn(fma(-ph.cx, u, q));
         win[s & 1][threadIdx.x] = make_float4(wp.x, wp.y, wm.x, wm.y);
       }
     }
   };
-  auto convert = [&](int s, const typename decltype(ld)::Raw& r) __attribute__((always_inline)) {
+  auto convert = [&](auto PH, int s, const typename decltype(ld)::Raw& r) __attribute__((always_inline)) {
     FoldPart o;
     if constexpr (LOAD != FOLD_FIELD) ld.part(2 * s + run, beta, r, o);
-    else ld.part(2 * s + run, beta, r, phased, win[s & 1] + run * kStageK, o);
+    else ld.part(2 * s + run, beta, r, decltype(PH)::value, win[s & 1] + run * kStageK, o);
     uint8_t* buf = lds + ((s & 1) * 2 + run) * kRun;
     const int pr = part_row(py, beta), fl = part_slot(py, beta);
 #pragma unroll
@@ -692,32 +702,42 @@ fold_stage1_small_kernel(FoldStage1 a) {
 #pragma unroll
     for (int e = 0; e < 2; ++e) load_frag(fb[decltype(J)::value][e][0], tab, 2 * sc + e);
   };
-  auto step = [&](auto J, int s) __attribute__((always_inline)) {
+  auto step = [&](auto J, auto FULL, auto PH, int s) __attribute__((always_inline)) {
     constexpr int j0 = decltype(J)::value;
     lds_barrier();   // stage s is in LDS, stage s - 1 has been read
     u32x4_t fa[2][1][2];
 #pragma unroll
-    for (int e = 0; e < 2; ++e) read_frag(fa[e][0], lds + (j0 * 2 + e) * kRun, wave * 32, wave & 1);
-    load_tab(std::integral_constant<int, 1 - j0>{}, s + 1);
+    for (int e = 0; e < 2; ++e)
+      read_frag(fa[e][0], lds + (j0 * 2 + e) * kRun, wave * 32, wave & 1);
+    load_tab(IC<1 - j0>{}, s + 1);
     ld.raw(2 * (s + 2) + run, raw[j0]);
-    window(s + 2);
+    if constexpr (decltype(PH)::value) window(s + 2);
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int e = 0; e < 2; ++e) mma_stage<BF, 1, 1>(acc, fa[e], fb[j0][e]);
     __builtin_amdgcn_s_setprio(0);
-    if (s + 1 < nst) convert(s + 1, raw[1 - j0]);
+    if (decltype(FULL)::value || s + 1 < nst) convert(PH, s + 1, raw[1 - j0]);
   };
-  load_tab(std::integral_constant<int, 0>{}, 0);
-  ld.raw(run, raw[0]);
-  ld.raw(2 + run, raw[1]);
-  window(0);
-  window(1);
-  if constexpr (LOAD == FOLD_FIELD) lds_barrier();
-  convert(0, raw[0]);
-  for (int s = 0; s < nst; s += 2) {
-    step(std::integral_constant<int, 0>{}, s);
-    if (s + 1 < nst) step(std::integral_constant<int, 1>{}, s + 1);
-  }
+  auto loop = [&](auto PH) __attribute__((always_inline)) {
+    load_tab(IC<0>{}, 0);
+    ld.raw(run, raw[0]);
+    ld.raw(2 + run, raw[1]);
+    if constexpr (decltype(PH)::value) {
+      window(0);
+      window(1);
+      lds_barrier();
+    }
+    convert(PH, 0, raw[0]);
+    int s = 0;
+    for (; s + 2 < nst; s += 2) {
+      step(IC<0>{}, std::true_type{}, PH, s);
+      step(IC<1>{}, std::true_type{}, PH, s + 1);
+    }
+    step(IC<0>{}, std::false_type{}, PH, s);
+    if (s + 1 < nst) step(IC<1>{}, std::false_type{}, PH, s + 1);
+  };
+  if (LOAD == FOLD_FIELD && phased) loop(std::bool_constant<LOAD == FOLD_FIELD>{});
+  else loop(std::false_type{});
   lds_barrier();
   f32x16_t& v = acc[0][0];
   const int lane = threadIdx.x & 63, lr = lane & 31, lk = lane >> 5;
@@ -785,9 +805,6 @@ fold_stage1_small_kernel(FoldStage1 a) {
 // wait before a fragment read covers that buffer's loads alone.
 // mma(buffer, fragments) issues one stage's products.
 // ---------------------------------------------------------------------------
-template <int N>
-using IC = std::integral_constant<int, N>;
-
 template <int NB, int NT, typename BufF, typename IssueF, typename MmaF>
 __device__ __forceinline__ void ring_loop(int nst, const uint8_t* const (&tab)[NT], BufF buf,
                                           IssueF issue_rows, MmaF mma) {
