@@ -109,14 +109,16 @@ PsfLayout psf_layout(const dlx_mft_geom& g, int c) {
 }
 
 // Workspace of the psf chain: a complex pupil, two complex matrices and the
-// planes per wavelength -- which the folded buffers fit in on all but the
-// smallest grids -- so that the limits a caller meets do not depend on how the
-// chain lays its buffers out.
+// planes per wavelength (psf_plain_bytes) -- which the folded buffers fit in on
+// all but the smallest grids -- so that the limits a caller meets do not depend
+// on how the chain lays its buffers out.
+size_t psf_plain_bytes(const dlx_mft_geom& g, int c, bool split) {
+  return align_up((size_t)c * mat_bytes(g.n_in, g.n_in, split)) +
+         2 * align_up((size_t)c * mat_bytes(g.n_out, g.n_in, split)) +
+         align_up((size_t)c * g.n_out * g.n_out * sizeof(float));
+}
 size_t psf_poly_bytes(const dlx_mft_geom& g, int c, bool split) {
-  const size_t P = align_up((size_t)c * mat_bytes(g.n_in, g.n_in, split));
-  const size_t W = align_up((size_t)c * mat_bytes(g.n_out, g.n_in, split));
-  const size_t I = align_up((size_t)c * g.n_out * g.n_out * sizeof(float));
-  const size_t plain = P + 2 * W + I, fold = psf_layout(g, c).total;
+  const size_t plain = psf_plain_bytes(g, c, split), fold = psf_layout(g, c).total;
   return plain > fold ? plain : fold;
 }
 
@@ -884,7 +886,11 @@ int dlx_profile_read(int32_t stage, double* total_ms, int32_t* count) {
 namespace dlx {
 
 constexpr size_t kNoallocScratchBytes = (size_t)64 << 20;   // 64 MiB per GPU
-static __device__ __align__(256) uint8_t scratch[kNoallocScratchBytes];
+// Room beyond it for grids of a few pixels, whose folded buffers pad n to 64:
+// with at most 64 MiB of plain buffers the output side is at most 4096, and the
+// folded ones exceed them by less than 640 n_out + 8192 bytes.
+constexpr size_t kNoallocSlack = (size_t)4 << 20;
+static __device__ __align__(256) uint8_t scratch[kNoallocScratchBytes + kNoallocSlack];
 
 namespace {
 
@@ -933,7 +939,7 @@ int dlx_psf_poly_noalloc(const dlx_mft_geom* geom, int32_t nwl, const double* wa
                                    precision))
     return st;
   const bool split = precision == DLX_PREC_BF16X3;
-  const size_t one = psf_poly_bytes(*geom, 1, split);
+  const size_t one = psf_plain_bytes(*geom, 1, split);
   if (one > kNoallocScratchBytes) {
     set_error("dlx_psf_poly_noalloc: one wavelength of a %d^2 -> %d^2 PSF needs %zu bytes, "
               "more than the %zu-byte scratch array; use dlx_psf_poly with a workspace",

@@ -172,3 +172,23 @@ def test_batch_partial_groups(rt):
         for o, x in enumerate(rt.mft_batched_psf(inst, n_outputs=len(exact))):
             n = [d["field"].shape[0] for d in inst if d["out_index"] == o][0]
             assert _err(x, exact[o]) < 12 * _sigma(n, "bf16x3"), o
+
+
+@pytest.mark.parametrize("prec", ["fp32", "bf16x3"])
+def test_noalloc_smallest_pupil_largest_image(rt, prec):
+    """A geometry whose plain buffers fit the 64 MiB array and whose padded ones exceed it."""
+    import ctypes
+    from dlux_amd import _lib
+    n, m = 2, 4050
+    print(f"[fold-noalloc] n={n} m={m} {prec}", flush=True)
+    dev, _ = _planes(n, "amp opd", 5, 0)
+    wls, w = np.array([0.9e-6, 1.1e-6]), np.array([0.4, 0.6])
+    ref = rt.psf_poly(n, m, wls, w, 1.0 / n, P_OUT, scale=0.25, precision=prec, **dev)
+    out = torch.full((m, m), float("nan"), device="cuda")
+    g = rt.geom(n, m)
+    st = _lib.load().dlx_psf_poly_noalloc(
+        ctypes.byref(g), 2, _lib.dptr(wls), _lib.dptr(w), 1.0 / n, P_OUT, 0.0, 0.0, 0.0,
+        dev["amp"].data_ptr(), dev["opd"].data_ptr(), None, 0.25, out.data_ptr(),
+        rt._prec_code(prec), rt.stream_handle())
+    _lib.check(st, "dlx_psf_poly_noalloc")
+    assert _err(out, ref.double().cpu().numpy()) < 12 * _sigma(n, prec)
