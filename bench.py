@@ -36,30 +36,29 @@ ERR_BOUND = 1e-5
 # known size (profiles/mft_poly_512to256_64wl_hbm_traffic.md).  The counters cannot
 # be read from inside this process.
 # Keyed by (form, pupil generated in stage 1's loader).
-TRAFFIC_BYTES = {("bf16x3", True): 151.2e6}
+TRAFFIC_BYTES = {("bf16x3", True): 113.9e6}
 # MFMA busy fraction of the stage-1 kernel from rocprofv3 SQ_VALU_MFMA_BUSY_CYCLES /
 # (GRBM_GUI_ACTIVE / 8 x 1024 SIMDs) (profiles/mft_poly_512to256_64wl_mfma_counters.md).
-MFMA_BUSY_PMC = {("bf16x3", True): 0.515}
+MFMA_BUSY_PMC = {("bf16x3", True): 0.261}
 
 
 def _stage1_kernel(head, prologue):
-    if head == "fp32":
-        return "cgemm_nt_fp32 stage 1 (pupil x transfer matrix)"
+    form = "split-BF16x3" if head == "bf16x3" else "float32"
     if prologue:
-        return ("cgemm_pupil_kernel stage 1 (pupil generated in the loader x transfer "
-                "matrix)")
-    return "cgemm_split4_deep_kernel stage 1 (pupil x transfer matrix)"
+        return (f"fold_stage1_kernel ({form}; pupil formed and folded in the loader x cosine / "
+                "sine tables)")
+    return f"fold_stage1_mem_kernel ({form}; folded pupil x cosine / sine tables)"
 
 
 def _stage1_bytes(cfg, head, prologue):
-    """Algorithmic HBM bytes of one stage-1 launch: the split4 (8 B) or complex64
-    (8 B) transfer matrices read and U^T written, plus the pupil: read as split4
-    or complex64 (8 B per pixel per wavelength), or, with the pupil generated in
-    the loader, its wavelength-independent path (8 B) and amplitude (4 B) planes
-    read once."""
-    mats = cfg.n_wl * 8.0 * 2 * cfg.n_out * cfg.n_in
+    """Algorithmic HBM bytes of one stage-1 launch: the cosine and sine tables
+    (4 B per real, over half of either side) read and the eight real parts of the
+    result written, per wavelength, plus the pupil: its OPD and amplitude planes (8 B
+    per pixel) read once, or the folded pupil (8 B per pixel and wavelength)."""
+    kh, mh = (cfg.n_in + 1) // 2, (cfg.n_out + 1) // 2
+    mats = cfg.n_wl * 4.0 * (2 + 8) * mh * kh
     if prologue:
-        return mats + 12.0 * cfg.n_in * cfg.n_in
+        return mats + 8.0 * cfg.n_in * cfg.n_in
     return mats + cfg.n_wl * 8.0 * cfg.n_in * cfg.n_in
 
 
@@ -520,7 +519,7 @@ def _aperture_leg(torch, steps, warmup=3):
 def _lct_leg(torch, steps, check, warmup=3):
     """Linear canonical transforms of a lens + free-space system (B = 0.5 m):
     the Collins integral of 64 wavelengths of a 512^2 field to 256^2 on the
-    MFT's split-BF16x3 GEMMs (dlx_lct), and the FFT form of one 1024^2 field
+    MFT's split-BF16x3 contractions (dlx_lct), and the FFT form of one 1024^2 field
     on a 2048^2 grid (dlx_lct_fft).  Algorithmic work: 8 (N_out N_in^2 +
     N_out^2 N_in) FLOPs per wavelength for the matrix form; two FFT passes
     reading and writing M^2 complex64 values plus the two chirp passes for
@@ -566,7 +565,7 @@ def _lct_leg(torch, steps, check, warmup=3):
     ms_fft = beg.elapsed_time(end) / steps
     fft_bytes = 2 * 2 * 8 * m * m + 2 * 8 * nf * nf + 2 * 8 * m * m
     return {"workload": "lct: lens f = 0.8 m between 0.3 m and 0.2 m of free space; "
-                        "64 lambda x 512^2 -> 256^2 (split-BF16x3 GEMMs)",
+                        "64 lambda x 512^2 -> 256^2 (split-BF16x3)",
             "ms_per_call": ms, "tflops": flops / (ms * 1e-3) / 1e12,
             "frac_of_bf16_peak": flops / (ms * 1e-3) / 1e12 / 2500.0,
             "max_rel_err_vs_fp64": err,
@@ -687,8 +686,10 @@ def main():
     else:
         head = "fp32"
     ms = res[head]["ms"]
-    prologue = head == "bf16x3" and os.environ.get("DLUX_AMD_PUPIL_PROLOGUE", "1") != "0"
-    n1 = cfg.n_out * cfg.n_in ** 2 * 8.0 * cfg.n_wl        # stage-1 algorithmic flops/launch
+    prologue = os.environ.get("DLUX_AMD_PUPIL_PROLOGUE", "1") != "0"
+    # stage-1 algorithmic flops per launch: on symmetric grids the transfer matrix is a
+    # cosine and a sine over half of either side, a quarter of the complex products
+    n1 = cfg.n_out * cfg.n_in ** 2 * 2.0 * cfg.n_wl
     t1_ms, c1 = res[head]["s1"]
     t2_ms, c2 = res[head]["s2"]
     avg1 = t1_ms / max(c1, 1)
@@ -727,6 +728,7 @@ def main():
                      "frac_of_measured_ceiling": (achieved * terms /
                                                   ceiling["random_operands_tflops"]
                                                   if head == "bf16x3" else None),
+                     # both contractions at the plain complex products' operation count
                      "mft_pair_tflops": pair},
         "cpu_baseline": cpu,
         "forms": {p: {"psf_per_s": 1e3 / res[p]["ms"], "ms_per_step": res[p]["ms"],

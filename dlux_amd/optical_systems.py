@@ -10,7 +10,7 @@ BasisLayer, Optic, BasisOptic, Tilt, Normalise), the chain collapses to
 
 because |exp(i.)| = 1 makes every normalisation factor lambda-independent.
 The system then computes sum_l w_l |MFT_l(E_l)|^2 in one dlx_psf_poly call
-(pupil synthesis, per-wavelength DFT matrices, two MFMA contractions and the
+(pupil synthesis, per-wavelength tables, two MFMA contractions and the
 weighted |E|^2 reduction).  Any other layer makes it fall back to applying the
 layers one by one on a wavelength-vectorised Wavefront (still on the GPU).
 """

@@ -1225,12 +1225,12 @@ def batched_graph_stats() -> dict:
 
 
 def cache_clear() -> None:
-    """Free every cached transfer matrix (after their pending uses)."""
+    """Free every cached table (after their pending uses)."""
     _lib.check(_lib.load().dlx_cache_clear(), "dlx_cache_clear")
 
 
 def cache_set_budget(nbytes: int) -> None:
-    """Device memory the transfer-matrix cache may hold (0 disables it)."""
+    """Device memory the table cache may hold (0 disables it)."""
     _lib.check(_lib.load().dlx_cache_set_budget(int(nbytes)), "dlx_cache_set_budget")
 
 
@@ -1250,7 +1250,7 @@ def mfma_rate(random_operands: bool = True) -> float:
 
 class cache_bypass:
     """Context manager: calls made from this thread inside it skip the
-    transfer-matrix cache (dlx_cache_bypass), generating their matrices into
+    table cache (dlx_cache_bypass), generating their tables into
     their workspace -- no allocation, eviction or wait."""
 
     def __enter__(self):
@@ -1263,7 +1263,7 @@ class cache_bypass:
 
 
 def cache_stats() -> dict:
-    """{'hits', 'misses', 'bytes', 'entries'} of the transfer-matrix cache."""
+    """{'hits', 'misses', 'bytes', 'entries'} of the table cache."""
     import ctypes
     h, m = ctypes.c_uint64(), ctypes.c_uint64()
     b, e = ctypes.c_size_t(), ctypes.c_int32()
@@ -1283,7 +1283,7 @@ class graph_step:
     gradients in place (``p.grad.zero_()`` when ``p.grad`` exists), never
     ``p.grad = None``.  Calling the object replays the graph and returns fn's
     outputs from the capture: static tensors overwritten by every replay.
-    fn is run ``warmup`` times on a side stream first (the transfer matrices
+    fn is run ``warmup`` times on a side stream first (the tables
     are cached then, and parameter gradients allocated)."""
 
     def __init__(self, fn, warmup: int = 3):

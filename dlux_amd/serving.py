@@ -23,7 +23,7 @@ runs on one host thread:
     runs and their kernels overlap on the device;
   * every stream has one workspace arena, grown to the largest group it ran
     and reused (work on a stream is ordered), and the loop's thread skips the
-    library's transfer-matrix cache (the mix's wavelength grids rarely
+    library's table cache (the mix's wavelength grids rarely
     repeat), so serving allocates nothing per request beyond its results
     and never waits on the host for an eviction.
 
@@ -178,7 +178,8 @@ class Server:
                 r.n_in ** 2 + r.n_out ** 2)
         nwl = len(r.wavelengths)
         if r.kind == "psf":
-            # fields + split4 pupils + two matrices + U^T + intensity planes + output
+            # fields, folded fields, tables, stage-1 results, intensity planes, output (the
+            # batch's own bound is the unfolded layout's)
             per = 16 * r.n_in ** 2 + 3 * 8 * r.n_out * r.n_in + 4 * r.n_out ** 2
             return nwl * per + 4 * r.n_out ** 2 + (1 << 16)
         g = runtime.geom(r.n_in, r.n_out)

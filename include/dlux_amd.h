@@ -168,12 +168,12 @@ int dlx_psf_poly(const dlx_mft_geom* geom, int32_t nwl, const double* wavelength
                  void* workspace, size_t workspace_bytes, void* stream);
 
 /*
- * dlx_psf_poly that allocates nothing and takes no workspace: the pupils,
- * transfer matrices and per-wavelength planes live in a fixed 64 MiB device
+ * dlx_psf_poly that allocates nothing and takes no workspace: the tables,
+ * intermediates and per-wavelength planes live in a fixed 64 MiB device
  * array of the library (one copy per GPU, held until the process ends; its
  * size is dlx_psf_poly_noalloc_scratch_bytes()), the wavelengths run in
- * chunks that fit it, and the transfer matrices are generated every call (the
- * device matrix cache, which allocates, is not used).  Same arguments and
+ * chunks that fit it, and the tables are generated every call (the
+ * device table cache, which allocates, is not used).  Same arguments and
  * result as dlx_psf_poly.  Rejects, with DLX_ERR_INVALID, a geometry whose
  * one-wavelength buffers exceed the array.  Calls that overlap on one GPU
  * (two host threads or two streams) race on the array; callers serialise them.
@@ -259,7 +259,7 @@ typedef struct dlx_mft_instance {
  * captured into a caller's graph (it uploads per-call descriptors); instead,
  * when enabled, the launches themselves run as a HIP graph that the library captures (on a
  * private stream) at the second call with the same workspace, batch shape
- * (sizes, output grouping, shared fields) and matrix state (generated or
+ * (sizes, output grouping, shared fields) and table state (generated or
  * resident), and launches on `stream` after uploading that call's
  * descriptors (dlx_batched_graphs).
  * Replaces the vmapped source x wavelength propagation of
@@ -641,10 +641,10 @@ int dlx_detector_vjp_params(int32_t n, int32_t batch, const float* in,
                             size_t workspace_bytes, void* stream);
 
 /*
- * Transfer-matrix cache (no counterpart in the reference: dLux rebuilds the
- * matrices inside every traced call).  dlx_mft, dlx_psf_poly,
- * dlx_psf_poly_vjp and dlx_mft_batched_psf keep the matrices of each
- * (geometry, wavelengths, pixel scales, shifts) batch resident on the device
+ * Table cache (no counterpart in the reference: dLux rebuilds its transfer
+ * matrices inside every traced call).  dlx_mft, dlx_lct, dlx_psf_poly,
+ * dlx_psf_poly_vjp and dlx_mft_batched_psf keep the cosine / sine tables of each
+ * batch of (sides, phase steps) resident on the device
  * and reuse them; least-recently-used batches are
  * evicted beyond the budget (default 16 GiB, environment DLUX_AMD_CACHE_MB).
  * A budget of 0 disables caching.  The cache is bypassed for streams under
@@ -652,7 +652,7 @@ int dlx_detector_vjp_params(int32_t n, int32_t batch, const float* in,
  * every entry.  An evicted entry's block is reused without the host waiting:
  * the stream that takes it next waits on the device for the work that last
  * read it.  dlx_cache_bypass(1) makes the calling thread's calls skip the cache
- * (matrices generated into their workspace, nothing allocated, evicted or
+ * (tables generated into their workspace, nothing allocated, evicted or
  * waited on) until dlx_cache_bypass(0): for request loops whose wavelength
  * grids rarely repeat.
  */
@@ -676,7 +676,7 @@ int dlx_cache_stats(uint64_t* hits, uint64_t* misses, size_t* bytes, int32_t* en
 /*
  * Diagnostics (no counterpart in the reference): live timing of the MFT
  * contraction launches inside dlx_psf_poly.  While enabled, each stage-1
- * (pupil x transfer matrix) and stage-2 (transfer matrix x intermediate, with
+ * (pupil x tables) and stage-2 (tables x intermediate, with
  * the |E|^2 epilogue) launch is bracketed by hipEvents on the caller's stream
  * (at most 8192 launches are recorded).  enable resets the record;
  * dlx_profile_read waits for the recorded events and returns the summed
