@@ -951,7 +951,7 @@ int dlx_psf_poly_noalloc(const dlx_mft_geom* geom, int32_t nwl, const double* wa
   while (c > 1 && psf_poly_bytes(*geom, c, split) > kNoallocScratchBytes) --c;
   void* ws = nullptr;
   if (int st = scratch_address(&ws)) return st;
-  // matrices are generated into the array every call: the device cache allocates
+  // tables are generated into the array every call: the device cache allocates
   return psf_poly_run(*geom, nwl, wavelength, weight, pixel_scale_in, pixel_scale_out, center,
                       tilt_x, tilt_y, amp, opd, phase, scale, psf, split, (uint8_t*)ws, c,
                       false, false, (hipStream_t)stream);

@@ -439,9 +439,9 @@ void plan_fill(int n, const dlx_mft_instance* inst, int n_outputs, float* const*
 // the workspace; its grid and by-value arguments depend on the plan's shape
 // only.  So one captured graph serves every call with the same workspace and
 // the same shape, whatever the fields, wavelengths, weights, shifts, outputs
-// and matrix addresses (all uploaded before the launch).
-int launch_plan(const Plan& Q, uint8_t* ws, bool with_matrices, hipStream_t s) {
-  if (with_matrices)
+// and table addresses (all uploaded before the launch).
+int launch_plan(const Plan& Q, uint8_t* ws, bool with_tables, hipStream_t s) {
+  if (with_tables)
     DLX_HIP(launch_fold_group_tables((const FoldTableJob*)(ws + Q.off_tab), (int)Q.tab.size(),
                                      Q.tab_most, s));
   DLX_HIP(launch_fold_group_fields((const FoldFieldJob*)(ws + Q.off_fld), (int)Q.fld.size(),

@@ -77,7 +77,7 @@ struct MatCache {
 };
 
 // Per-thread bypass (dlx_cache_bypass): calls from this thread generate their
-// matrices into their workspace and never allocate, evict or wait.
+// tables into their workspace and never allocate, evict or wait.
 thread_local bool t_bypass = false;
 
 MatCache& cache() {
@@ -265,7 +265,7 @@ int cache_acquire_raw(const std::vector<double>& key_in, size_t bytes, hipStream
   MatEntry* e = new_entry(std::move(key), dev, mem, got, ++c.tick);
   if (!e) {
     (void)hipFree(mem);
-    set_error("hipEventCreate failed in the matrix cache");
+    set_error("hipEventCreate failed in the table cache");
     return DLX_ERR_HIP;
   }
   e->pending = true;

@@ -434,7 +434,9 @@ __device__ __forceinline__ void get_block(const uint8_t* x, f32x16_t& v) {
 // 128 the field is formed once per 128-column tile (256 outputs), each wave
 // holds eight 32 x 32 blocks (eight fragment reads from LDS per 24 MFMAs of a
 // split stage), and two workgroups share a CU.  Launches with fewer tiles take
-// 64 or 32 columns.
+// 64 or 32 columns.  Issue bounds the loop: 24 MFMAs and 180 vector instructions
+// (phasors, folds, split) per wave and split stage.  64 wavelengths of 512^2 ->
+// 256^2: 38 us split, 88 float32, where the complex contractions took 101 and 332.
 // ---------------------------------------------------------------------------
 struct Stage1Prob {
   const uint8_t* src;
@@ -909,7 +911,9 @@ fold_stage1_mem_kernel(FoldStage1 a) {
 // with the wave of the other beta through LDS, after which wave beta holds both
 // signs of y at its sign of x.  BQ = 32, for launches that leave compute units
 // idle: wave (beta, alpha) holds both components of one part, and two trades
-// leave it the outputs of one sign of x (alpha) and one of y (beta).
+// leave it the outputs of one sign of x (alpha) and one of y (beta).  Reading U
+// and the products take similar times: 23.5 us split, 50 float32 at 64 wavelengths
+// of 512^2 -> 256^2 (64 MB of U; the complex contraction took 50 and 176).
 // ---------------------------------------------------------------------------
 struct Stage2Prob {
   const uint8_t *table, *mid;
@@ -1176,7 +1180,9 @@ __device__ __forceinline__ int group_tile(const FoldGroup& l) {
 // instance's x shift rotates the even and odd parts (e' = e cos f + i o sin f,
 // o' = o cos f + i e sin f; cos and sin of the stage's k from a window in LDS),
 // the parts are split, and the tile's products run; the y shift is applied to
-// the results.
+// the results.  768 instances of 256^2 to 1024^2 take 182 + 141 + 96 us in the
+// three widths and 172 in stage 2 (the complex contractions 1360 in all); issue
+// bounds it as the stage above.
 template <int BNQ>
 __global__ void __launch_bounds__(kThreads, 2)
 fold_group_stage1_kernel(FoldGroup g) {
