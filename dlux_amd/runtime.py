@@ -69,27 +69,31 @@ def stream_handle() -> int:
 
 
 def as_complex(x, dev=None) -> torch.Tensor:
-    """Contiguous complex64 device tensor."""
+    """Contiguous complex64 device tensor whose memory holds its values: a lazily
+    conjugated view is materialised."""
     dev = dev or device()
     if isinstance(x, torch.Tensor):
-        if x.dtype is torch.complex64 and x.device == dev and x.is_contiguous():
+        if x.dtype is torch.complex64 and x.device == dev and x.is_contiguous() \
+                and not (x.is_conj() or x.is_neg()):
             return x
         t = x.to(device=dev)
         if not t.is_complex():
             t = t.to(torch.float32).to(torch.complex64)
-        return t.to(torch.complex64).contiguous()
+        return t.to(torch.complex64).resolve_conj().resolve_neg().contiguous()
     return torch.as_tensor(np.asarray(x, np.complex64), device=dev).contiguous()
 
 
 def as_float(x, dev=None) -> torch.Tensor:
-    """Contiguous float32 device tensor."""
+    """Contiguous float32 device tensor whose memory holds its values: a lazily
+    negated view (the imaginary part of a conjugate) is materialised."""
     dev = dev or device()
     if isinstance(x, torch.Tensor):
-        if x.dtype is torch.float32 and x.device == dev and x.is_contiguous():
+        if x.dtype is torch.float32 and x.device == dev and x.is_contiguous() \
+                and not x.is_neg():
             return x
         if x.is_complex():
             raise TypeError("expected a real array, got a complex one")
-        return x.to(device=dev, dtype=torch.float32).contiguous()
+        return x.to(device=dev, dtype=torch.float32).resolve_neg().contiguous()
     return torch.as_tensor(np.asarray(x, np.float32), device=dev).contiguous()
 
 
@@ -643,9 +647,7 @@ def soft_apertures_vjp(npix: int, pixel_scale: float, apertures, dout: torch.Ten
     n = len(apertures)
     dev = device()
     lib = _lib.load()
-    dout = dout.detach()
-    if dout.dtype != torch.float32 or not dout.is_contiguous() or dout.device != dev:
-        dout = dout.to(device=dev, dtype=torch.float32).contiguous()
+    dout = as_float(dout.detach(), dev)
     if tuple(dout.shape) != (npix, npix):
         raise ValueError(f"dout must be ({npix}, {npix}), got {tuple(dout.shape)}")
     arr = (_lib.SoftAperture * max(n, 1))(*apertures)
@@ -779,7 +781,7 @@ class _InterpFn(torch.autograd.Function):
     def backward(ctx, gout):
         shape, lead, batch, spec = ctx.meta
         n_in = shape[-1]
-        g = gout.to(torch.float32).contiguous()
+        g = as_float(gout, gout.device)
         din = torch.empty(shape, dtype=torch.float32, device=g.device)
         ws = torch.empty(max(batch * n_in * n_in, 1), dtype=torch.float64, device=g.device)
         lib = _lib.load()
@@ -830,8 +832,8 @@ def interp_points(images, pixel_scale_in: float, center_in: float, xs, ys,
     (dlx_interp_points_vjp); the points are constants."""
     dev = device()
     _interp_method(method)
-    qx = torch.as_tensor(xs, device=dev).detach().to(torch.float64).contiguous()
-    qy = torch.as_tensor(ys, device=dev).detach().to(torch.float64).contiguous()
+    qx = torch.as_tensor(xs, device=dev).detach().to(torch.float64).resolve_neg().contiguous()
+    qy = torch.as_tensor(ys, device=dev).detach().to(torch.float64).resolve_neg().contiguous()
     if qx.shape != qy.shape:
         raise ValueError("xs and ys must have the same shape")
     if _tracks(images):

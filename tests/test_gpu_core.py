@@ -347,3 +347,20 @@ def test_mfma_rate_probe(rt):
     print(f"  low-entropy {hi:.0f} TF/s, full-entropy {lo:.0f} TF/s")
     assert 0 < hi < 2750 and 0 < lo < 2750
     assert lo < 1.1 * hi
+
+
+def test_conjugated_field_views(rt):
+    """field.conj() is a view of the field's memory: the transform of the view
+    is the transform of its values, bit for bit."""
+    rng = np.random.default_rng(11)
+    f = torch.as_tensor(_rand_field(rng, 48).astype(np.complex64), device="cuda")
+    c = f.conj()
+    assert c.is_conj()
+    plain = c.resolve_conj()
+    print("[conj] mft", flush=True)
+    assert torch.equal(rt.mft(c, 1e-6, 1 / 48, 24, 0.25e-6), rt.mft(plain, 1e-6, 1 / 48, 24, 0.25e-6))
+    print("[conj] batch", flush=True)
+    inst = dict(wavelength=1e-6, pixel_scale_in=1 / 48, n_out=24, pixel_scale_out=0.25e-6)
+    images = [rt.MftBatch([dict(inst, field=x)], n_outputs=1)()[0] for x in (c, plain, f)]
+    assert torch.equal(images[0], images[1])
+    assert not torch.equal(images[0], images[2])

@@ -711,3 +711,27 @@ def test_interp_vjp_abi_validation_without_gpu(lib):
                                      None) != 0
     assert lib.dlx_interp_points_vjp(4, 1.0, 0.0, 3, None, None, 1, 0, None, None, None,
                                      None) == 0
+
+
+def test_lazily_conjugated_and_negated_tensors_are_materialised():
+    """The library reads a tensor's memory, where a conjugated or negated view
+    still holds the values it was made from."""
+    torch = pytest.importorskip("torch")
+    from dlux_amd import runtime
+    cpu = torch.device("cpu")
+    z = torch.complex(torch.arange(6.0).reshape(2, 3), 1.0 + torch.arange(6.0).reshape(2, 3))
+    memory = lambda t: np.ctypeslib.as_array(  # noqa: E731
+        ctypes.cast(t.data_ptr(), ctypes.POINTER(ctypes.c_float)), (t.numel() * (
+            2 if t.is_complex() else 1),)).copy()
+    for view in (z.conj(), z.T.conj(), z.to(torch.complex128).conj(), torch._neg_view(z)):
+        out = runtime.as_complex(view, cpu)
+        ref = view.resolve_conj().resolve_neg().to(torch.complex64).contiguous()
+        assert np.array_equal(memory(out), memory(ref))
+    for view in (z.conj().imag, torch._neg_view(z.real.contiguous()),
+                 torch._neg_view(z.real.contiguous()).double()):
+        out = runtime.as_float(view, cpu)
+        assert np.array_equal(memory(out), view.resolve_neg().float().contiguous().numpy().ravel())
+    # an ordinary tensor is passed as it is
+    assert runtime.as_complex(z, cpu).data_ptr() == z.data_ptr()
+    r = z.real.contiguous()
+    assert runtime.as_float(r, cpu).data_ptr() == r.data_ptr()
