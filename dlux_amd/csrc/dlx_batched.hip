@@ -136,7 +136,7 @@ struct Plan {
   std::vector<FoldTableJob> tab;
   std::vector<size_t> tab_off;       // of each distinct table, from off_T
   std::vector<int> tab_of;           // instance -> table
-  long tab_most = 0;                 // threads of the largest table
+  int tab_most = 0;                  // threads of the largest table
   std::vector<FoldFieldJob> fld;     // distinct fields
   std::vector<size_t> fld_off;
   std::vector<int> fld_of;           // instance -> field
@@ -260,8 +260,7 @@ int plan_sizes(int n, const dlx_mft_instance* inst, int n_outputs, Plan& P) {
       P.tab.push_back({nullptr, k.step, k.n, k.m});
       P.tab_off.push_back(P.tab_bytes);
       P.tab_bytes += fold_table_bytes(k.n, k.m);
-      const long work = (long)fold_pad(fold_half(k.m)) * fold_pad(fold_half(k.n)) / 4;
-      P.tab_most = std::max(P.tab_most, work);
+      P.tab_most = std::max(P.tab_most, fold_group_table_threads(k.n, k.m));
     }
     P.tab_of[i] = it.first->second;
   }
@@ -470,7 +469,7 @@ int launch_plan(const Plan& Q, uint8_t* ws, bool with_tables, hipStream_t s) {
 // Everything launch_plan's grids and by-value arguments depend on.
 std::vector<long> plan_shape(const Plan& Q, const uint8_t* ws, bool fresh, int dev) {
   std::vector<long> k = {(long)dev, (long)(uintptr_t)ws, (long)fresh, (long)Q.off_tab,
-                         (long)Q.tab.size(), Q.tab_most, (long)Q.off_fld, (long)Q.fld.size(),
+                         (long)Q.tab.size(), (long)Q.tab_most, (long)Q.off_fld, (long)Q.fld.size(),
                          (long)Q.fld_most, (long)Q.off_prob, (long)Q.off_cols, (long)Q.off_map2,
                          (long)Q.off_sum, (long)Q.sum.size()};
   for (int l = 0; l < kLists; ++l) {

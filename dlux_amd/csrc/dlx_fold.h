@@ -172,7 +172,9 @@ struct FoldFieldJob {
 // the rows and columns of the tiles.
 int fold_group_width(int m);
 constexpr int kFoldTileQy = 64, kFoldTileQx = 32, kFoldTilePy = 32;
-hipError_t launch_fold_group_tables(const FoldTableJob* jobs, int njobs, long most, hipStream_t s);
+// `most`: fold_group_table_threads of the largest table.
+int fold_group_table_threads(int n, int m);
+hipError_t launch_fold_group_tables(const FoldTableJob* jobs, int njobs, int most, hipStream_t s);
 // `most`: the largest field's side.
 hipError_t launch_fold_group_fields(const FoldFieldJob* jobs, int njobs, int most, hipStream_t s);
 hipError_t launch_fold_group_stage1(const FoldGroup& g, int width, hipStream_t s);

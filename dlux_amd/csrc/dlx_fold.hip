@@ -1,7 +1,7 @@
 // The folded MFT's kernels (dlx_fold.h): cosine / sine tables, the pupil and
 // field loaders, and the two contractions with their epilogues, in complex64
 // (v_mfma_f32_32x32x2_f32) and split-BF16x3 form (v_mfma_f32_32x32x16_bf16,
-// hi*hi + hi*lo + lo*hi), on one tile geometry: both forms hold 4 bytes per
+// lo*lo + lo*hi + hi*lo + hi*hi), on one tile geometry: both forms hold 4 bytes per
 // real, so a stage of 16 k is 64 bytes of every tile row -- four 16-byte
 // pieces, of which a lane's half (lane / 32) takes two:
 //   split-BF16x3  [hi k 0-7][lo k 0-7][hi k 8-15][lo k 8-15]
@@ -108,16 +108,16 @@ template <bool BF, int NI, int NJ>
 __device__ __forceinline__ void mma_stage(f32x16_t (&acc)[NI][NJ], const u32x4_t (&a)[NI][2],
                                           const u32x4_t (&b)[NJ][2]) {
   if constexpr (BF) {
-    // lo*hi, hi*lo, hi*hi: the small terms first
+    // lo*lo, lo*hi, hi*lo, hi*hi: the small terms first
 #pragma unroll
-    for (int t = 0; t < 3; ++t)
+    for (int t = 0; t < 4; ++t)
 #pragma unroll
       for (int i = 0; i < NI; ++i)
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              __builtin_bit_cast(bf16x8_t, a[i][t == 0 ? 1 : 0]),
-              __builtin_bit_cast(bf16x8_t, b[j][t == 1 ? 1 : 0]), acc[i][j], 0, 0, 0);
+              __builtin_bit_cast(bf16x8_t, a[i][t < 2 ? 1 : 0]),
+              __builtin_bit_cast(bf16x8_t, b[j][t & 1 ? 0 : 1]), acc[i][j], 0, 0, 0);
   } else {
 #pragma unroll
     for (int e = 0; e < 8; ++e)
@@ -1363,51 +1363,85 @@ fold_group_stage2_kernel(FoldGroup l) {
 // Tables and the pupil in memory
 // ---------------------------------------------------------------------------
 
-// One table: four consecutive k of a row of both the cosine and the sine per
-// thread.  Hardware sin / cos take turns (max abs error 1.3e-7, below the split
-// pair's 2^-17); the float32 form takes the library's functions.
+// One table: `table_quads` runs of four consecutive k of a row of both the cosine
+// and the sine per thread, from the library's functions: the hardware's (max abs
+// error 1.3e-7) are off alike in every table, which a sum over sources and
+// wavelengths does not average out (24 stars of 8 wavelengths, relative error in
+// 1e-7: 6.9 with them, 5.7 without).
+//
+// The split form rounds the 16 k of a stage one after another and adds what the
+// pair hi + lo leaves of a value to the next: over neighbouring k, where a field
+// varies slowly, the errors cancel.  Each rounded by itself they add coherently
+// at the peak: the folds pair k with its mirror, so a table holds a quarter of
+// the complex form's independent roundings.  Rms error of six fields 256^2 ->
+// 256^2, shifted, in 1e-7 of the field / the intensity: 22.1 / 8.1 so, 12.9 /
+// 4.1 with the carry, these functions and the lo * lo products of mma_stage, 20.3 /
+// 5.8 in the unfolded complex form of three products; white fields 54.6 / 54.9,
+// 52.1 / 52.0 and 54.2 / 54.4.  The fourth product costs 64 wavelengths of 512^2
+// -> 256^2 76.6 -> 81.1 us, 768 uneven instances 658 -> 691.
+template <bool BF>
+__host__ __device__ constexpr int table_quads() { return BF ? 4 : 1; }
+// Threads of the table contracting side n into side m.
+template <bool BF>
+__host__ __device__ inline int table_threads(int n, int m) {
+  return fold_pad(fold_half(m)) * (fold_pad(fold_half(n)) / (4 * table_quads<BF>()));
+}
+
 template <bool BF>
 __device__ __forceinline__ void table_entry(int t, double step, int n, int m,
                                             uint8_t* __restrict__ out) {
+  constexpr int Q = table_quads<BF>();
   const int kh = fold_half(n), mh = fold_half(m), kp = fold_pad(kh), mhp = fold_pad(mh);
-  const int quads = kp >> 2;
-  if (t >= mhp * quads) return;
-  const int q = t / quads, k0 = (t - q * quads) * 4;
+  if (t >= table_threads<BF>(n, m)) return;
+  // consecutive threads take the 32 rows of a block
+  const int runs = kp / (4 * Q), q = (t / (32 * runs)) * 32 + (t & 31);
+  const int k0 = ((t >> 5) % runs) * 4 * Q;
   const double on = (n & 1) ? 0.0 : 0.5, om = (m & 1) ? 0.0 : 0.5;
   const double u = step * ((double)q + om);
-  float c[4], s[4];
+  uint8_t* d[2];   // the stage's rows in the cosine and the sine
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int p = k0 + e;
-    c[e] = s[e] = 0.f;
-    if (p < kh && q < mh) {
-      double ph = u * ((double)p + on);
-      ph -= rint(ph);
-      if constexpr (BF) {
-        s[e] = __builtin_amdgcn_sinf((float)ph);
-        c[e] = __builtin_amdgcn_cosf((float)ph);
-      } else {
-        sincospif(2.0f * (float)ph, &s[e], &c[e]);
+  for (int part = 0; part < 2; ++part)
+    d[part] = out + table_block(part, mhp, kp, q >> 5) + (long)(k0 >> 4) * 2048 + (q & 31) * 16;
+  float left[2] = {0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < Q; ++i) {
+    const int quad = ((k0 >> 2) & 3) + i;
+    float v[2][4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int p = k0 + 4 * i + e;
+      float c = 0.f, s = 0.f;
+      if (p < kh && q < mh) {
+        double ph = u * ((double)p + on);
+        ph -= rint(ph);
+        sincospif(2.0f * (float)ph, &s, &c);
+        if (p == 0 && (n & 1)) c *= 0.5f;   // the centre, folded onto itself
       }
-      if (p == 0 && (n & 1)) c[e] *= 0.5f;   // the centre, folded onto itself
+      v[0][e] = c;
+      v[1][e] = s;
     }
-  }
-  // the quad's place in its stage: lane half (quad / 2), and, split, the run of
-  // hi and of lo pieces with 8 bytes each; float32, one run of 16 bytes
-  const int quad = (k0 >> 2) & 3;
+    // the quad's place in its stage: lane half (quad / 2), and, split, the run of
+    // hi and of lo pieces with 8 bytes each; float32, one run of 16 bytes
 #pragma unroll
-  for (int part = 0; part < 2; ++part) {
-    const float(&v)[4] = part ? s : c;
-    uint8_t* d = out + table_block(part, mhp, kp, q >> 5) + (long)(k0 >> 4) * 2048 +
-                 ((quad >> 1) * 32 + (q & 31)) * 16;
-    if constexpr (BF) {
-      uint32_t h[2], lo[2];
-      split2_bf16(v[0], v[1], h[0], lo[0]);
-      split2_bf16(v[2], v[3], h[1], lo[1]);
-      *(uint2*)(d + (quad & 1) * 8) = make_uint2(h[0], h[1]);
-      *(uint2*)(d + 1024 + (quad & 1) * 8) = make_uint2(lo[0], lo[1]);
-    } else {
-      *(float4*)(d + (quad & 1) * 1024) = make_float4(v[0], v[1], v[2], v[3]);
+    for (int part = 0; part < 2; ++part) {
+      uint8_t* o = d[part] + (quad >> 1) * 512;
+      if constexpr (BF) {
+        uint32_t h[4], lo[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+#pragma clang fp contract(off)
+          const bool in = k0 + 4 * i + e < kh && q < mh;
+          const float x = in ? v[part][e] + left[part] : 0.f;
+          h[e] = bf16x2_rne(x, 0.f);
+          const float r = x - __uint_as_float(h[e] << 16);
+          lo[e] = bf16x2_rne(r, 0.f);
+          left[part] = r - __uint_as_float(lo[e] << 16);
+        }
+        *(uint2*)(o + (quad & 1) * 8) = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
+        *(uint2*)(o + 1024 + (quad & 1) * 8) = make_uint2(lo[0] | lo[1] << 16, lo[2] | lo[3] << 16);
+      } else {
+        *(float4*)(o + (quad & 1) * 1024) = make_float4(v[part][0], v[part][1], v[part][2], v[part][3]);
+      }
     }
   }
 }
@@ -1558,7 +1592,7 @@ hipError_t launch_fold_tables(const double* step, int nb, int n, int m, bool spl
     for (int adj = 0; adj < (adjoint ? 2 : 1); ++adj) {
       const int kn = adj ? m : n, km = adj ? n : m;
       uint8_t* o = out + (long)b0 * stride + (adj ? fold_table_bytes(n, m) : 0);
-      const int work = fold_pad(fold_half(km)) * (fold_pad(fold_half(kn)) / 4);
+      const int work = split ? table_threads<true>(kn, km) : table_threads<false>(kn, km);
       const dim3 grid((unsigned)((work + 255) / 256), k);
       if (split)
         hipLaunchKernelGGL(fold_table_kernel<true>, grid, dim3(256), 0, s, st, kn, km, o, stride);
@@ -1608,7 +1642,9 @@ int fold_group_width(int m) {
   return mh > 64 ? 128 : mh > 32 ? 64 : 32;
 }
 
-hipError_t launch_fold_group_tables(const FoldTableJob* jobs, int njobs, long most, hipStream_t s) {
+int fold_group_table_threads(int n, int m) { return table_threads<true>(n, m); }
+
+hipError_t launch_fold_group_tables(const FoldTableJob* jobs, int njobs, int most, hipStream_t s) {
   hipLaunchKernelGGL(fold_group_table_kernel, dim3(njobs, (unsigned)((most + 255) / 256)), dim3(256),
                      0, s, jobs);
   return hipGetLastError();

@@ -1,5 +1,5 @@
 // Split of FP32 values into two bf16, the operand form of the split-BF16x3
-// contractions: x = hi + lo + O(2^-17 |x|), products hi hi + hi lo + lo hi.
+// contractions: x = hi + lo + O(2^-17 |x|), all four products of the pairs.
 #pragma once
 
 #include <hip/hip_runtime.h>

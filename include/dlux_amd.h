@@ -40,7 +40,8 @@ enum dlx_status {
 
 enum dlx_precision {
   DLX_PREC_FP32 = 0,   /* complex64 operands, FP32 MFMA, FP32 accumulate         */
-  DLX_PREC_BF16X3 = 1  /* split-BF16 3-term (hi*hi + hi*lo + lo*hi) MFMA, FP32 acc */
+  DLX_PREC_BF16X3 = 1  /* operands split into two BF16 (hi + lo), MFMA, FP32 acc; leading
+                           terms hi*hi + hi*lo + lo*hi, and lo*lo */
 };
 
 /* Library version string ("dlux_amd x.y.z gfx950"). */

@@ -6,8 +6,8 @@ a phase plane, a tilt, a field with and without shifts, a folded pupil in
 memory); the gradient's epilogues; uneven batches whose tile groups are not full.
 
 Bounds.  The split form drops 2^-18 of a product's terms twice over (each
-operand's third part) and the lo * lo product: 3 * 2^-18 per term and
-contraction.  The hardware sine and cosine are good to 1.3e-7.  float32 sums of
+operand's third part); 3 * 2^-18 per term and contraction covers that and the
+carrying of a table value's rest to its neighbour.  The hardware sine and cosine are good to 1.3e-7.  float32 sums of
 K terms round by 2^-24 of the running sum each.  Independent errors of the K =
 N_in terms of a contraction add in quadrature against a sum that adds
 coherently at the peak, so relative to it a field is off by
@@ -193,3 +193,61 @@ def test_noalloc_smallest_pupil_largest_image(rt, prec):
         rt._prec_code(prec), rt.stream_handle())
     _lib.check(st, "dlx_psf_poly_noalloc")
     assert _err(out, ref.double().cpu().numpy()) < 12 * _sigma(n, prec)
+
+
+def _unfolded_split(f, wl, m, shift):
+    """The transform as split operands of the unfolded complex form give it: the
+    field, the kernels and the intermediate each hi + lo in bf16, products hi hi
+    + hi lo + lo hi, sums in 64 bits."""
+    def split(x):
+        x = x.float()
+        hi = x.bfloat16().float()
+        return hi.double(), (x - hi).bfloat16().double()
+
+    def real_nt(a, b):
+        (ah, al), (bh, bl) = split(a), split(b)
+        return al @ bh.T + ah @ bl.T + ah @ bh.T
+
+    def nt(a, b):
+        return torch.complex(real_nt(a.real, b.real) - real_nt(a.imag, b.imag),
+                             real_nt(a.real, b.imag) + real_nt(a.imag, b.real))
+
+    n = f.shape[-1]
+    wx, wy = (torch.as_tensor(orc.transfer_matrix(wl, n, 1.0 / n, m, P_OUT, shift=s).T.copy()).cuda()
+              for s in shift)
+    c = orc.calc_nfringes(wl, n, 1.0 / n, m, P_OUT) / (n * m)
+    return c * nt(wy, nt(f, wx).T)
+
+
+@pytest.mark.parametrize("white", [False, True])
+@pytest.mark.parametrize("n,m,shift", [(64, 64, (10.0, -7.0)), (256, 256, (20.0, -30.0)),
+                                       (131, 101, (0.0, 0.0))])
+def test_split_error_not_above_the_unfolded_form(rt, n, m, shift, white):
+    """The folds add mirrored values before the split, so its rounding errors
+    meet at the peak; the products and the tables must make up for that.  Rms
+    over fields of the 2-norm error of the field and of its intensity against
+    complex128, beside that of the unfolded split form with exact sums."""
+    print(f"[fold-split-error] n={n} m={m} shift={shift} white={white}", flush=True)
+    x = (torch.arange(n, device="cuda") - (n - 1) / 2) / n * 2
+    yy, xx = torch.meshgrid(x, x, indexing="ij")
+    err = torch.zeros(2, 2, dtype=torch.float64)
+    for seed in range(6):
+        g = torch.Generator(device="cuda").manual_seed(seed)
+        if white:
+            f = torch.complex(*torch.randn((2, n, n), generator=g, device="cuda")) / n ** 2
+        else:
+            c = 0.2 * torch.randn(5, generator=g, device="cuda")
+            ph = c[0] * xx + c[1] * yy + c[2] * (2 * xx ** 2 - 1) + c[3] * xx * yy + c[4] * yy ** 3
+            f = torch.polar((xx ** 2 + yy ** 2 < 1).float() / n ** 2, ph)
+        wl = 0.8e-6 + 0.07e-6 * seed
+        ref = torch.as_tensor(orc.mft(f.cpu().numpy().astype(complex), wl, 1.0 / n, m, P_OUT,
+                                      shift=shift)).cuda()
+        got = rt.mft(f, wl, 1.0 / n, m, P_OUT, shift_x=shift[0], shift_y=shift[1],
+                     precision="bf16x3")
+        plain = _unfolded_split(f.to(torch.complex128), wl, m, shift)
+        for i, e in enumerate((got.to(torch.complex128), plain)):
+            for j, (a, b) in enumerate(((e, ref), (e.abs() ** 2, ref.abs() ** 2))):
+                err[i, j] += float(torch.linalg.vector_norm(a - b) / torch.linalg.vector_norm(b)) ** 2
+    err = (err / 6).sqrt()
+    print(err.tolist(), flush=True)
+    assert bool((err[0] <= err[1]).all())
