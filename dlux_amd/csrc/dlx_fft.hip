@@ -131,10 +131,14 @@ __device__ __forceinline__ void dft_reg<16>(float2 (&x)[16], float sgn) {
 
 // log2 of the radices: three stages up to 4096.  A radix-8 first stage is
 // followed by radix 8 and a radix-16 one by radix 16, which the LDS layout
-// needs (lin below).
+// needs (lin below).  256 points take three stages too: two of radix 16 leave a
+// row 16 lanes, each with 16 transfer functions to form one after another, and
+// the angular spectrum of eight 128^2 fields took 142 us (131 in stages of radix
+// 8 on 512 threads) where these on two rows take 99; eight transforms of 256^2 15.1
+// and 12.3 (33.1).
 constexpr int log2_rad(int log2m, int st) {
   constexpr int kRad[14][4] = {{},        {1},       {2},       {3},       {4},
-                               {3, 2},    {3, 3},    {4, 3},    {4, 4},    {3, 3, 3},
+                               {3, 2},    {3, 3},    {4, 3},    {3, 3, 2}, {3, 3, 3},
                                {3, 3, 4}, {4, 4, 3}, {4, 4, 4}, {4, 4, 3, 2}};
   return kRad[log2m][st];
 }
@@ -442,8 +446,9 @@ fft_rows_kernel(const float2* __restrict__ in, float2* __restrict__ out, FftPara
 // that leaves one workgroup per CU.  2048^2, us at 2 / 4 / 8 rows: kFirst (1024
 // rows) 14.4 / 11.8 / 12.0, kLast 20.3 / 17.0 / 15.6; kMid has no transposed
 // access, and two workgroups on a CU overlap: 26.4 / 24.2 at 2 / 4 (1: 31.4).
+// 64 transforms of 256^2, us at 1 / 2 rows: 55.2 / 35.9.
 constexpr int log2_rows(int log2m, int pass) {
-  return log2m <= 8 ? 0 : log2m == 9 ? 1 : log2m == 11 && pass != kMid ? 3 : log2m <= 12 ? 2 : 0;
+  return log2m <= 7 ? 0 : log2m <= 9 ? 1 : log2m == 11 && pass != kMid ? 3 : log2m <= 12 ? 2 : 0;
 }
 
 template <int LOG2M, int LOG2R, int PASS, bool INV>

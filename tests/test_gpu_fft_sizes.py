@@ -46,8 +46,8 @@ def _rel(x, ref):
 
 
 SIZES = [(2, 2), (2, 4), (4, 8), (6, 16), (20, 32), (64, 64), (96, 128), (130, 256),
-         (256, 512), (300, 512), (512, 1024), (1000, 1024), (1024, 2048), (600, 2048),
-         (2048, 4096), (130, 8192)]
+         (254, 256), (256, 256), (256, 512), (300, 512), (512, 1024), (1000, 1024),
+         (1024, 2048), (600, 2048), (2048, 4096), (130, 8192)]
 
 
 @pytest.mark.parametrize("inverse", [False, True])
