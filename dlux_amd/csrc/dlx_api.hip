@@ -124,33 +124,42 @@ size_t psf_poly_bytes(const dlx_mft_geom& g, int c, bool split) {
 
 // The cosine / sine tables of nb phase steps contracting side n into side m
 // (and, with `adjoint`, of the transposed contraction), from the device cache
-// -- an entry holds both -- or generated into `ws` when the cache is bypassed.
-// Equal steps share one table (stride 0).
+// or generated into `ws` when the cache is bypassed.  Equal steps share one table
+// (stride 0).
 struct FoldTables {
   const uint8_t *fwd, *adj;
   long stride;
 };
+// What a call leaves in the cache: the PSF's entry holds both directions, for the
+// gradient that may follow, and is made on the first sighting of its steps, as a
+// field transform's of the forward direction is; a canonical transform's is made on
+// the second, as a caller that scans planes or wavelengths never asks for one again.
+enum TableUse { TABLES_PSF, TABLES_FIELD, TABLES_LCT };
 int fold_tables(int n, int m, const std::vector<double>& steps, bool split, bool adjoint,
-                bool use_cache, uint8_t* ws, hipStream_t s, FoldTables* out, CacheLease* lease) {
+                TableUse use, bool use_cache, uint8_t* ws, hipStream_t s, FoldTables* out,
+                CacheLease* lease) {
   const long tf = fold_table_bytes(n, m), ta = fold_table_bytes(m, n);
   bool one = true;
   for (double v : steps) one = one && v == steps[0];
   const int nb = one ? 1 : (int)steps.size();
+  const bool both = use == TABLES_PSF;
   void* mem = nullptr;
   bool fresh = true;
   if (use_cache) {
-    std::vector<double> key = {2001.0, (double)n, (double)m, split ? 1.0 : 0.0};
+    std::vector<double> key = {2001.0, (double)n, (double)m, split ? 1.0 : 0.0, both ? 1.0 : 0.0};
     key.insert(key.end(), steps.begin(), steps.begin() + nb);
-    if (int st = cache_acquire_raw(key, (size_t)nb * (tf + ta), s, &mem, &lease->h, &fresh, true))
+    if (int st = cache_acquire_raw(key, (size_t)nb * (both ? tf + ta : tf), s, &mem, &lease->h,
+                                   &fresh, use != TABLES_LCT))
       return st;
   }
   uint8_t* base = mem ? (uint8_t*)mem : ws;
-  const long stride = mem || adjoint ? tf + ta : tf;
+  const bool adj = adjoint || (mem && both);
+  const long stride = adj ? tf + ta : tf;
   out->stride = one ? 0 : stride;
   out->fwd = base;
   out->adj = base + tf;
   if (fresh) {
-    DLX_HIP(launch_fold_tables(steps.data(), nb, n, m, split, mem || adjoint, base, stride, s));
+    DLX_HIP(launch_fold_tables(steps.data(), nb, n, m, split, adj, base, stride, s));
     if (int st = cache_ready(lease->h, s)) return st;
   }
   return DLX_OK;
@@ -174,11 +183,11 @@ size_t field_transform_bytes(int n, int m, int batch) {
          align_up((size_t)c * fold_mid_bytes(n, m));
 }
 int field_transform(int n, int m, int batch, bool inverse, const std::vector<double>& steps,
-                    const FoldPhase* pin, const FoldPhase* pout, const double* alpha,
+                    TableUse use, const FoldPhase* pin, const FoldPhase* pout, const double* alpha,
                     const void* in, void* out, bool split, uint8_t* ws, hipStream_t s) {
   CacheLease h(s);
   FoldTables tab;
-  if (int st = fold_tables(n, m, steps, split, false, true, ws, s, &tab, &h)) return st;
+  if (int st = fold_tables(n, m, steps, split, false, use, true, ws, s, &tab, &h)) return st;
   uint8_t* U = ws + align_up((size_t)batch * fold_table_bytes(n, m));
   for (int b0 = 0; b0 < batch; b0 += kFieldChunk) {
     const int nb = batch - b0 < kFieldChunk ? batch - b0 : kFieldChunk;
@@ -323,7 +332,7 @@ int dlx_mft(const dlx_mft_geom* geom, int32_t batch, const void* in, void* out,
     c[b] = mft_norm(g, wavelength[b], pixel_scale_in[b], pixel_scale_out[b]) *
            (field_scale ? field_scale[b] : 1.0);
   }
-  return field_transform(g.n_in, g.n_out, batch, g.inverse != 0, steps,
+  return field_transform(g.n_in, g.n_out, batch, g.inverse != 0, steps, TABLES_FIELD,
                          shifted ? pin.data() : nullptr, shifted ? pout.data() : nullptr, c.data(),
                          in, out, precision == DLX_PREC_BF16X3, (uint8_t*)workspace, s);
 }
@@ -383,8 +392,9 @@ int dlx_lct(int32_t n_in, int32_t n_out, int32_t batch, const double* abcd,
                2.0 * ((A * xc * xc - 2.0 * xc * xo + D * xo * xo) / (2.0 * lb)) +
                    (B > 0 ? -0.25 : 0.25)};
   }
-  return field_transform(n_in, n_out, batch, B < 0, steps, pin.data(), pout.data(), alpha.data(),
-                         in, out, precision == DLX_PREC_BF16X3, (uint8_t*)workspace, s);
+  return field_transform(n_in, n_out, batch, B < 0, steps, TABLES_LCT, pin.data(), pout.data(),
+                         alpha.data(), in, out, precision == DLX_PREC_BF16X3, (uint8_t*)workspace,
+                         s);
 }
 
 size_t dlx_lct_fft_workspace_size(int32_t n, int32_t m, int32_t batch) {
@@ -588,7 +598,7 @@ int psf_poly_run(const dlx_mft_geom& g, int32_t nwl, const double* wavelength,
     FoldTables tab;
     if (int st = fold_tables(g.n_in, g.n_out,
                              psf_steps(g, nb, wavelength + l0, pixel_scale_in, pixel_scale_out),
-                             split, false, use_cache, T_ws, s, &tab, &h))
+                             split, false, TABLES_PSF, use_cache, T_ws, s, &tab, &h))
       return st;
     f1.batch = nb;
     f1.table = tab.fwd;
@@ -769,7 +779,7 @@ int dlx_psf_poly_vjp(const dlx_mft_geom* geom, int32_t nwl, const double* wavele
     FoldTables tab;
     if (int st = fold_tables(g.n_in, g.n_out,
                              psf_steps(g, nb, wavelength + l0, pixel_scale_in, pixel_scale_out),
-                             split, true, true, T_ws, s, &tab, &h))
+                             split, true, TABLES_PSF, true, T_ws, s, &tab, &h))
       return st;
     FoldStage2 e{}, b{};
     for (int i = 0; i < nb; ++i) {

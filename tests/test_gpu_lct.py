@@ -63,6 +63,28 @@ def test_lct_vs_oracle(rt, case, prec):
         assert err < tol
 
 
+def test_lct_tables_enter_the_cache_on_the_second_sighting(rt):
+    """A scan over planes or wavelengths, which never comes back to one, allocates
+    nothing; an entry holds the one direction that a transform without a gradient
+    uses (a 64 -> 48 axis: 2 tables of 32 x 32 reals, 4 bytes each)."""
+    print("[lct] cache", flush=True)
+    u = torch.ones((1, 64, 64), dtype=torch.complex64, device="cuda")
+    call = lambda wl: rt.lct(u, [wl], _MATS["free"], 40e-6, 0.0, 48, 35e-6, 0.0)  # noqa: E731
+    rt.cache_clear()
+    for i in range(4):
+        call(0.91e-6 + 1e-9 * i)
+    assert rt.cache_stats()["entries"] == 0
+    call(0.91e-6)
+    s = rt.cache_stats()
+    assert (s["entries"], s["bytes"]) == (1, 2 * 32 * 32 * 4)
+    hits = s["hits"]
+    call(0.91e-6)
+    assert rt.cache_stats()["hits"] == hits + 1
+    rt.mft(u, [1e-6], 40e-6, 48, 1e-3)
+    s = rt.cache_stats()
+    assert (s["entries"], s["bytes"]) == (2, 2 * 2 * 32 * 32 * 4)
+
+
 @pytest.mark.parametrize("n,m", [(48, 64), (64, 128), (32, 32)])
 def test_lct_fft_vs_oracle(rt, n, m):
     print(f"[lct fft] n={n} m={m}", flush=True)
