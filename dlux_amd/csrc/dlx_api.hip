@@ -589,7 +589,7 @@ int psf_poly_run(const dlx_mft_geom& g, int32_t nwl, const double* wavelength,
   // the pupil formed in stage 1's loader (no pupil array in HBM), or written
   // first where many column tiles would each form it again
   const bool in_loader =
-      !room || (pupil_prologue_enabled() && fold_pupil_in_loader(f1.pupil, g.n_out));
+      !room || (pupil_prologue_enabled() && fold_pupil_in_loader(f1.pupil, g.n_in, g.n_out));
   for (int l0 = 0; l0 < nwl; l0 += c) {
     const int nb = nwl - l0 < c ? nwl - l0 : c;
     // one wavelength is its own sum
@@ -796,7 +796,7 @@ int dlx_psf_poly_vjp(const dlx_mft_geom* geom, int32_t nwl, const double* wavele
     f.out = U; f.out_stride = fold_mid_bytes(g.n_in, g.n_out);
     f.pupil = pup;
     for (int i = 0; i < nb; ++i) f.inv_wl[i] = b.inv_wl[i];
-    const bool in_loader = fold_pupil_in_loader(pup, g.n_out);
+    const bool in_loader = fold_pupil_in_loader(pup, g.n_in, g.n_out);
     if (!in_loader) {
       f.src = P;
       f.src_stride = fold_field_bytes(g.n_in);

@@ -185,9 +185,13 @@ hipError_t launch_fold_group_stage2(const FoldGroup& g, hipStream_t s);
 hipError_t launch_fold_pupil(const FoldPupil& p, const double* inv_wl, int nb, int n, bool split,
                              uint8_t* out, long stride, hipStream_t s);
 
-// True where forming the pupil in the loader beats writing it first: the fast
-// loader takes an amplitude or OPD plane and no phase; each 128-column tile
-// forms the pupil again.
-bool fold_pupil_in_loader(const FoldPupil& p, int m);
+// True where forming the pupil in the loader beats writing it first.  Each
+// 128-column tile forms the pupil again.  With a phase plane, or no plane, the
+// loader tests for every plane: up to two of 64 columns that costs less than a launch
+// that writes the pupil where it loads whole runs (16 wavelengths of 512^2 -> 128^2
+// 31.7 against 40.1 us split, 41.9 against 47.7 float32; 4 of 1024^2 -> 512^2 72.0
+// against 55.3), single values only on small pupils (5 of 300^2 -> 101^2 26.2 against
+// 27.2; 11 of 401^2 -> 173^2 38.1 against 35.2).
+bool fold_pupil_in_loader(const FoldPupil& p, int n, int m);
 
 }  // namespace dlx

@@ -226,7 +226,9 @@ struct PupilLoad {
   bool has_opd, has_amp, has_phase;
   double inv_wl, tx, tyY, dx, x0, co;   // co: 1 if there is an OPD, else 0
   float ca, cb;                     // amplitude = ca * value + cb, signed; zero outside the rows
-  struct Raw { float4 op, om, ap, am; };   // plus runs (k ascending), minus runs (descending)
+  struct Runs { float4 op, om, ap, am; };   // plus runs (k ascending), minus runs (descending)
+  struct AnyRuns : Runs { float4 pp, pm; };
+  using Raw = std::conditional_t<ANY, AnyRuns, Runs>;
 
   __device__ __forceinline__ void init(const FoldPupil& p, int n_, int py, int beta, int quad_,
                                        double inv) {
@@ -264,11 +266,21 @@ struct PupilLoad {
     const int p = s * kStageK + quad * 4;
     if (!ANY || has_opd) { r.op = run_up(opd, p); r.om = run_down(opd, p); }
     if (!ANY || has_amp) { r.ap = run_up(amp, p); r.am = run_down(amp, p); }
+    if constexpr (ANY)
+      if (has_phase) { r.pp = run_up(phase, p); r.pm = run_down(phase, p); }
   }
   __device__ __forceinline__ void part(int s, int beta, const Raw& r, FoldPart& o) const {
     const int p = s * kStageK + quad * 4;
     const float vo[2][4] = {{r.op.x, r.op.y, r.op.z, r.op.w}, {r.om.w, r.om.z, r.om.y, r.om.x}};
     const float va[2][4] = {{r.ap.x, r.ap.y, r.ap.z, r.ap.w}, {r.am.w, r.am.z, r.am.y, r.am.x}};
+    float vt[2][4];
+    if constexpr (ANY) {
+      const float x[2][4] = {{r.pp.x, r.pp.y, r.pp.z, r.pp.w}, {r.pm.w, r.pm.z, r.pm.y, r.pm.x}};
+#pragma unroll
+      for (int d = 0; d < 2; ++d)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) vt[d][e] = x[d][e];
+    }
     float2 v[2][4];
     // VEC: the run is whole or absent
     const float ra = !VEC || p < kh ? ca : 0.f, rb = !VEC || p < kh ? cb : 0.f;
@@ -283,7 +295,8 @@ struct PupilLoad {
           const int pc = p + e < kh ? p + e : kh - 1;
           const int x = d ? n - 1 - x0i - pc : x0i + pc;
           if (ANY && !has_opd) path = 0.0;
-          if (ANY && has_phase) t = (double)phase[x] * 0.15915494309189535;   // 1 / (2 pi)
+          if constexpr (ANY)
+            if (has_phase) t = (double)vt[d][e] * 0.15915494309189535;   // 1 / (2 pi)
           if (ANY && !has_amp) a = p + e < kh ? rb : 0.f;
           path = fma(path, co, fma(tx, pupil_coord(x, dx, x0), tyY));   // pupil_path's bits
         }
@@ -663,7 +676,7 @@ fold_stage1_small_kernel(FoldStage1 a) {
   const uint8_t* tab = a.table + (long)b * a.table_stride + table_block(wave >> 1, mhp, kp, q0 / 32);
   const int py = threadIdx.x >> 4, beta = threadIdx.x & 1, quad = (threadIdx.x >> 1) & 3;
   const int run = (threadIdx.x >> 3) & 1;
-  std::conditional_t<LOAD == FOLD_FIELD, FieldLoad<VEC>, PupilLoad<VEC, LOAD == kPupilTilt, false>> ld;
+  std::conditional_t<LOAD == FOLD_FIELD, FieldLoad<VEC>, PupilLoad<VEC, LOAD == kPupilTilt, LOAD == kPupilAny>> ld;
   FoldPhase ph{};
   bool phased = false;
   if constexpr (LOAD != FOLD_FIELD) {
@@ -1459,11 +1472,12 @@ fold_group_table_kernel(const FoldTableJob* __restrict__ jobs) {
   table_entry<true>(blockIdx.y * blockDim.x + threadIdx.x, j.step, j.n, j.m, j.out);
 }
 
-constexpr int kPupilWl = 16;   // wavelengths per thread: the planes are read once for them
+// Most wavelengths per thread: the planes are read once for them.
+constexpr int kPupilWl = 16;
 
 template <bool BF, bool VEC>
 __global__ void __launch_bounds__(256)
-fold_pupil_kernel(FoldPupil pup, FoldSteps wl, int nb, int n,
+fold_pupil_kernel(FoldPupil pup, FoldSteps wl, int nb, int per, int n,
                   uint8_t* __restrict__ out, long stride) {
   const int kh = fold_half(n);
   const long rb = fold_row_bytes(n);
@@ -1473,7 +1487,7 @@ fold_pupil_kernel(FoldPupil pup, FoldSteps wl, int nb, int n,
   pl.init(pup, n, py, beta, quad, 0.0);
   typename PupilLoad<VEC, true, true>::Raw raw{};
   pl.raw(s, raw);
-  const int b0 = blockIdx.z * kPupilWl, b1 = b0 + kPupilWl < nb ? b0 + kPupilWl : nb;
+  const int b0 = blockIdx.z * per, b1 = b0 + per < nb ? b0 + per : nb;
   for (int b = b0; b < b1; ++b) {
     pl.inv_wl = wl.step[b];
     FoldPart o;
@@ -1489,6 +1503,10 @@ fold_pupil_kernel(FoldPupil pup, FoldSteps wl, int nb, int n,
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+// The pupil's rows can be read in whole runs of four (a missing plane is aligned).
+bool pupil_vec(const FoldPupil& p, int n) {
+  return n % 8 == 0 && aligned16(p.opd) && aligned16(p.amp) && aligned16(p.phase);
+}
 
 template <bool BF, int LOAD, bool VEC, int BNQ>
 void stage1_go(const FoldStage1& a, long tiles, hipStream_t s) {
@@ -1539,12 +1557,11 @@ hipError_t stage1_load(const FoldStage1& a, FoldLoad load, hipStream_t s) {
   if (load == FOLD_MEM) return stage1_width<BF, FOLD_MEM, true>(a, s);
   if (load == FOLD_PUPIL && (a.pupil.phase || (!a.pupil.opd && !a.pupil.amp))) {
     // callers write such pupils to memory first where they have the room
-    const long tiles = (long)((fold_half(a.m) + 31) / 32) * ((fold_half(a.n) + 31) / 32) * a.batch;
-    stage1_go<BF, kPupilAny, false, 32>(a, tiles, s);
-    return hipGetLastError();
+    return pupil_vec(a.pupil, a.n) ? stage1_width<BF, kPupilAny, true>(a, s)
+                                   : stage1_width<BF, kPupilAny, false>(a, s);
   }
   if (load == FOLD_PUPIL) {
-    const bool vec = a.n % 8 == 0 && aligned16(a.pupil.opd) && aligned16(a.pupil.amp);
+    const bool vec = pupil_vec(a.pupil, a.n);
     if (a.pupil.tx != 0.0 || a.pupil.ty != 0.0)
       return vec ? stage1_width<BF, kPupilTilt, true>(a, s) : stage1_width<BF, kPupilTilt, false>(a, s);
     return vec ? stage1_width<BF, FOLD_PUPIL, true>(a, s) : stage1_width<BF, FOLD_PUPIL, false>(a, s);
@@ -1619,18 +1636,23 @@ hipError_t launch_fold_stage2(const FoldStage2& a, FoldEpilogue epi, bool split,
 
 hipError_t launch_fold_pupil(const FoldPupil& p, const double* inv_wl, int nb, int n, bool split,
                              uint8_t* out, long stride, hipStream_t s) {
-  const bool vec = n % 8 == 0 && aligned16(p.opd) && aligned16(p.amp);
+  const bool vec = pupil_vec(p, n);
   for (int b0 = 0; b0 < nb; b0 += FoldSteps::kMax) {
     const int k = nb - b0 < FoldSteps::kMax ? nb - b0 : FoldSteps::kMax;
     FoldSteps wl;
     for (int i = 0; i < k; ++i) wl.step[i] = inv_wl[b0 + i];
-    const dim3 grid((fold_half(n) + 31) / 32, fold_pad(fold_half(n)) / kStageK,
-                    (k + kPupilWl - 1) / kPupilWl);
+    // a thread forms its wavelengths one after another: fewer each while the launch
+    // has less than a workgroup per compute unit (4 of 512^2
+    // with a phase plane onto 256^2: 128 at 16 each; the PSF 37.5 -> 33.9 us)
+    const int px = (fold_half(n) + 31) / 32, py = fold_pad(fold_half(n)) / kStageK;
+    int per = kPupilWl;
+    while (per > 1 && px * py * ((k + per - 1) / per) < 256) per >>= 1;
+    const dim3 grid(px, py, (k + per - 1) / per);
     uint8_t* o = out + (long)b0 * stride;
-    if (split && vec) hipLaunchKernelGGL((fold_pupil_kernel<true, true>), grid, dim3(256), 0, s, p, wl, k, n, o, stride);
-    else if (split) hipLaunchKernelGGL((fold_pupil_kernel<true, false>), grid, dim3(256), 0, s, p, wl, k, n, o, stride);
-    else if (vec) hipLaunchKernelGGL((fold_pupil_kernel<false, true>), grid, dim3(256), 0, s, p, wl, k, n, o, stride);
-    else hipLaunchKernelGGL((fold_pupil_kernel<false, false>), grid, dim3(256), 0, s, p, wl, k, n, o, stride);
+    if (split && vec) hipLaunchKernelGGL((fold_pupil_kernel<true, true>), grid, dim3(256), 0, s, p, wl, k, per, n, o, stride);
+    else if (split) hipLaunchKernelGGL((fold_pupil_kernel<true, false>), grid, dim3(256), 0, s, p, wl, k, per, n, o, stride);
+    else if (vec) hipLaunchKernelGGL((fold_pupil_kernel<false, true>), grid, dim3(256), 0, s, p, wl, k, per, n, o, stride);
+    else hipLaunchKernelGGL((fold_pupil_kernel<false, false>), grid, dim3(256), 0, s, p, wl, k, per, n, o, stride);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
@@ -1684,8 +1706,10 @@ hipError_t launch_fold_group_stage2(const FoldGroup& g, hipStream_t s) {
   return hipGetLastError();
 }
 
-bool fold_pupil_in_loader(const FoldPupil& p, int m) {
-  return !p.phase && (p.opd || p.amp) && fold_half(m) <= 256;
+bool fold_pupil_in_loader(const FoldPupil& p, int n, int m) {
+  const int mh = fold_half(m);
+  if (!p.phase && (p.opd || p.amp)) return mh <= 256;
+  return n <= 256 ? mh <= 256 : pupil_vec(p, n) && mh <= 128;
 }
 
 }  // namespace dlx

@@ -105,6 +105,29 @@ def test_psf_loaders(rt, planes, n, offset, tilt, prec):
     assert _err(out, exact) < 12 * _sigma(n, prec)
 
 
+# n, m, wavelengths, offset of the planes in floats
+PHASE = [(64, 40, 3, 0), (61, 40, 3, 0), (64, 40, 3, 1),   # loader, 16 x 32: runs and single values
+         (400, 60, 64, 0), (136, 100, 64, 0), (130, 100, 66, 0),   # 32 x 32, 32 x 64
+         (200, 150, 40, 0), (202, 131, 40, 0),                     # 32 x 128
+         (300, 101, 5, 0), (512, 128, 2, 1), (264, 280, 2, 0)]     # folded pupil in memory
+
+
+@pytest.mark.parametrize("prec", ["fp32", "bf16x3"])
+@pytest.mark.parametrize("planes", ["amp opd phase", "phase", "none"])
+@pytest.mark.parametrize("n,m,nwl,offset", PHASE)
+def test_phase_and_missing_planes(rt, n, m, nwl, offset, planes, prec):
+    """Pupils outside the fast loader, at every width and written first."""
+    print(f"[fold-phase] {planes} n={n} m={m} nwl={nwl} offset={offset} {prec}", flush=True)
+    dev, ref = _planes(n, planes, n + m, offset)
+    wls, w = np.linspace(0.8e-6, 1.2e-6, nwl), np.linspace(0.5, 1.5, nwl)
+    tilt = (3e-7, -2e-7) if nwl % 2 else (0.0, 0.0)
+    out = rt.psf_poly(n, m, wls, w, 1.0 / n, P_OUT, scale=1.0 / n ** 2, tilt=tilt, precision=prec,
+                      **dev)
+    exact = sum(wi * np.abs(orc.mft(_pupil(n, ref, wl, tilt), wl, 1.0 / n, m, P_OUT)) ** 2
+                for wl, wi in zip(wls, w))
+    assert _err(out, exact) < 12 * _sigma(n, prec)
+
+
 @pytest.mark.parametrize("prec", ["fp32", "bf16x3"])
 @pytest.mark.parametrize("shifted", [False, True])
 @pytest.mark.parametrize("n,m,b", [(1, 2, 1), (5, 3, 2), (33, 31, 2), (72, 45, 3), (130, 100, 66),

@@ -1,9 +1,9 @@
-"""Stage 1 of the split-BF16x3 PSF with the pupil generated in its loader
-(cgemm_pupil_kernel): no pupil array is written, the loader forms the same
-split4 phasors as the pupil kernel (one shared definition), so the PSF must
-be bit-identical to the two-kernel path (DLUX_AMD_PUPIL_PROLOGUE=0) for both
-tile widths, with and without amplitude / OPD, with and without tilt, and equal to the
-FP64 oracle within 1e-5 of the peak.
+"""Stage 1 of the PSF with the pupil formed in its loader: no pupil array is
+written, the loader forms the same parity parts as the pupil kernel (one shared
+definition), so the PSF must be bit-identical to the two-kernel path
+(DLUX_AMD_PUPIL_PROLOGUE=0) in both forms, at every tile width, with and without
+amplitude / OPD / phase, with and without tilt, and equal to the FP64 oracle
+within 1e-5 of the peak.
 """
 
 import numpy as np
@@ -33,19 +33,19 @@ def _pupil(n, seed):
     return mask, opd
 
 
-# (n_in, n_out, wavelengths): 128 x 128 tiles (512 -> 256, 1024 -> 256), 128 x 64
-# tiles (512 -> 128), and shapes the kernel does not cover (too few tiles, or
-# more than two tile columns), where the pupil kernel runs
+# (n_in, n_out, wavelengths): 32 x 128 tiles, 32 x 64, and the 16-row kernel; in each
+# the workspace has room for the folded pupil, so that the switch takes effect
 SHAPES = [(512, 256, 64), (1024, 256, 32), (512, 128, 64), (1024, 256, 16), (256, 256, 64),
-          (256, 128, 16)]
+          (256, 128, 16), (401, 173, 30), (512, 100, 16), (256, 128, 2), (255, 101, 3)]
 
 
 # with a tilt the loader forms tx X + ty Y + OPD in FP64; with none it takes the
 # OPD as the path, which must give the same bits as the pupil kernel's sum
+@pytest.mark.parametrize("prec", ["fp32", "bf16x3"])
 @pytest.mark.parametrize("tilted", [True, False])
 @pytest.mark.parametrize("n_in,n_out,nwl", SHAPES)
-def test_prologue_bit_identical_to_pupil_kernel(rt, monkeypatch, n_in, n_out, nwl, tilted):
-    print(f"[pupil prologue] {n_in}->{n_out} x{nwl} tilted={tilted}", flush=True)
+def test_prologue_bit_identical_to_pupil_kernel(rt, monkeypatch, n_in, n_out, nwl, tilted, prec):
+    print(f"[pupil prologue] {n_in}->{n_out} x{nwl} tilted={tilted} {prec}", flush=True)
     mask, opd = _pupil(n_in, n_in + nwl)
     p_out = 2.5e-7 * 512 / n_in
     wls = np.linspace(0.8e-6, 1.2e-6, nwl)
@@ -53,11 +53,13 @@ def test_prologue_bit_identical_to_pupil_kernel(rt, monkeypatch, n_in, n_out, nw
     scale = 1.0 / np.sqrt(np.sum(mask ** 2))
     cases = [dict(amp=mask.astype(np.float32), opd=opd.astype(np.float32)),
              dict(amp=None, opd=opd.astype(np.float32)),
-             dict(amp=mask.astype(np.float32), opd=None)]
+             dict(amp=mask.astype(np.float32), opd=None),
+             dict(amp=mask.astype(np.float32), opd=opd.astype(np.float32),
+                  phase=(opd * 3e6).astype(np.float32))]
     for i, kw in enumerate(cases):
         args = (n_in, n_out, wls, w, 1.0 / n_in, p_out)
         tilt = (1.3 * p_out, -0.6 * p_out) if tilted else (0.0, 0.0)
-        common = dict(scale=scale, tilt=tilt, precision="bf16x3", **kw)
+        common = dict(scale=scale, tilt=tilt, precision=prec, **kw)
         monkeypatch.delenv("DLUX_AMD_PUPIL_PROLOGUE", raising=False)
         fused = rt.psf_poly(*args, **common)
         monkeypatch.setenv("DLUX_AMD_PUPIL_PROLOGUE", "0")
