@@ -583,10 +583,14 @@ fold_stage1_kernel(FoldStage1 a) {
       }
     }
   };
+  // whether a field has a phase is asked outside the loop; by the split form's
+  // 128-column tiles inside it, as a second loop spills (64 fields 512^2 -> 256^2,
+  // shifted: 73.4 us against 71.1; float32 without a shift 126.7 against 138.0)
+  constexpr bool kAsk = LOAD == FOLD_FIELD && BF && BNQ == 128;
   auto convert = [&](auto PH, int s, const typename decltype(ld)::Raw& r) __attribute__((always_inline)) {
     FoldPart o;
     if constexpr (LOAD != FOLD_FIELD) ld.part(s, beta, r, o);
-    else ld.part(s, beta, r, decltype(PH)::value, win[s & 1], o);
+    else ld.part(s, beta, r, kAsk ? phased : decltype(PH)::value, win[s & 1], o);
     uint8_t* buf = lds + (s & 1) * kBuf;
     const int pr = part_row(py, beta), fl = part_slot(py, beta);
 #pragma unroll
@@ -631,11 +635,12 @@ fold_stage1_kernel(FoldStage1 a) {
       lds_barrier();
     }
     convert(PH, 0, raw[0]);
-    // whole pairs: no path of the loop skips a load or a part, and the choice of a
-    // field's phase is made outside it (16 fields 512^2 -> 256^2, float32: 48.0 ->
-    // 46.4 us).  At 128 columns a field's parts stay in a block of their own:
-    // merged with the products they spilled 567 registers
-    using Whole = std::bool_constant<LOAD != FOLD_FIELD || BNQ < 128>;
+    // whole pairs: no path of the loop skips a load or a part (16 fields 512^2 ->
+    // 256^2, float32: 48.0 -> 46.4 us).  At 128 columns only the aligned loader
+    // without a tilt has the registers: elsewhere the parts stay in a block of their
+    // own (48 pupils of 511^2 -> 257^2, split: 42 spilled registers and 121 us
+    // merged, 4 and 97 apart; 512^2 tilted 64.5 and 61.9)
+    using Whole = std::bool_constant<(LOAD == FOLD_PUPIL && VEC) || BNQ < 128>;
     int s = 0;
     for (; s + 2 < nst; s += 2) {
       step(IC<0>{}, Whole{}, PH, s);
@@ -644,8 +649,8 @@ fold_stage1_kernel(FoldStage1 a) {
     step(IC<0>{}, std::false_type{}, PH, s);
     if (s + 1 < nst) step(IC<1>{}, std::false_type{}, PH, s + 1);
   };
-  if (LOAD == FOLD_FIELD && phased) run(std::bool_constant<LOAD == FOLD_FIELD>{});
-  else run(std::false_type{});
+  if (kAsk || (LOAD == FOLD_FIELD && phased)) run(std::bool_constant<LOAD == FOLD_FIELD>{});
+  else if constexpr (!kAsk) run(std::false_type{});
   lds_barrier();
   if constexpr (LOAD == FOLD_FIELD)
     if (phased) y_phase<BNQ>(lds, acc, ph.c2, ph.cy, a.n, py0);
