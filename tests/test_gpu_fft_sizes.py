@@ -1,5 +1,6 @@
 """Every transform length of the LDS FFT (2 to 8192: one to four stages, radices
-2 to 16, one to four rows per workgroup, padded rows skipped or not) against
+2 to 16, one to eight rows per workgroup, padded rows skipped or, as in unpadded
+fields and those whose half is no multiple of the row count, not) against
 complex128 transforms.
 
 Bound: a Cooley-Tukey transform of M points in unit roundoff u = 2^-24 has a
@@ -46,8 +47,9 @@ def _rel(x, ref):
 
 
 SIZES = [(2, 2), (2, 4), (4, 8), (6, 16), (20, 32), (64, 64), (96, 128), (130, 256),
-         (254, 256), (256, 256), (256, 512), (300, 512), (512, 1024), (1000, 1024),
-         (1024, 2048), (600, 2048), (2048, 4096), (130, 8192)]
+         (254, 256), (256, 256), (256, 512), (300, 512), (512, 512), (512, 1024),
+         (1000, 1024), (1024, 1024), (1024, 2048), (600, 2048), (1002, 2048), (2048, 2048),
+         (2048, 4096), (130, 8192)]
 
 
 @pytest.mark.parametrize("inverse", [False, True])

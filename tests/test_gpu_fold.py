@@ -74,7 +74,8 @@ PSF = [(1, 1, 1), (2, 3, 1), (3, 2, 2), (16, 33, 1), (31, 64, 3), (33, 17, 2), (
        (130, 100, 66), (136, 100, 64),          # 32 x 64 (and a second chunk of two)
        (200, 150, 40), (202, 131, 40),          # 32 x 128, 64 rows
        (130, 270, 40),                          # 32 x 64 (float32) or 32 x 128 (split)
-       (40, 600, 2), (130, 600, 14), (200, 600, 16)]   # folded pupil in memory, 32 / 64 / 128
+       (128, 600, 2), (130, 600, 14), (200, 600, 16),   # folded pupil in memory, 32 / 64 / 128
+       (40, 600, 2)]                            # in the loader: no room for the folded pupil
 
 
 @pytest.mark.parametrize("prec", ["fp32", "bf16x3"])

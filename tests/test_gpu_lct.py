@@ -5,7 +5,7 @@ lenses, mirrors and the conjugate plane; the conjugate plane as the MFT; the
 FFT form as the Collins sum on the FFT grid).  abcdLux, where the reference
 keeps these transforms, is absent: parity with it is unpinned.
 
-Bounds (peak-normalised max error of the complex field): FP32 GEMM form 2e-5,
+Bounds (peak-normalised max error of the complex field): FP32 form 2e-5,
 split-BF16x3 form 5e-5; FFT form 2e-5.
 """
 
@@ -60,6 +60,37 @@ def test_lct_vs_oracle(rt, case, prec):
                       _MATS[case])
         err = _peak(got[b], ref)
         print(f"  wl {wls[b]:.2e} err {err:.2e}")
+        assert err < tol
+
+
+# n_in, n_out, fields: the 16-row kernel on odd sides; tiles of 64 columns with a
+# second chunk of two fields, of 32, and of 128, each with whole runs or single values
+SIZES = [(33, 31, 2), (131, 100, 66), (400, 60, 64), (200, 150, 40), (203, 131, 40)]
+
+
+@pytest.mark.parametrize("prec", ["fp32", "bf16x3"])
+@pytest.mark.parametrize("case", ["lens_free", "free_back"])
+@pytest.mark.parametrize("n,m,b", SIZES)
+def test_lct_sizes(rt, n, m, b, case, prec):
+    """The chirps in the field loader, in the y factor and in the epilogue at every
+    tile, on off-centre grids, for both signs of B, in the 2-norm.  Per contraction
+    the split form is off by at most 3 2^-18 of a term, the sums of n terms by
+    2^-24 sqrt(n); four phases of 1.3e-7 each."""
+    print(f"[lct size] n={n} m={m} b={b} {case} {prec}", flush=True)
+    rng = np.random.default_rng(n + m)
+    dx, dxo, c_in, c_out = 2e-3 / n, 1.9e-3 / m, 1.3e-5, -3.1e-5
+    wls = np.linspace(0.8e-6, 1.2e-6, b)
+    u = ((rng.standard_normal((b, n, n)) + 1j * rng.standard_normal((b, n, n))) / n).astype(
+        np.complex64)
+    got = rt.lct(torch.as_tensor(u).cuda(), wls, _MATS[case], dx, c_in, m, dxo, c_out,
+                 precision=prec).cpu().numpy()
+    tol = np.sqrt(2) * ((3 * 2.0 ** -18 if prec == "bf16x3" else 0.0) + 2.0 ** -24 * np.sqrt(n)) \
+        + 4 * 1.3e-7
+    for i in sorted({0, b // 2, b - 1}):
+        ref = orc.lct(u[i], wls[i], orc.spec_xs(n, dx, c_in), orc.spec_xs(m, dxo, c_out),
+                      _MATS[case])
+        err = np.linalg.norm(got[i] - ref) / np.linalg.norm(ref)
+        print(f"  {err:.2e} / {tol:.2e}")
         assert err < tol
 
 
