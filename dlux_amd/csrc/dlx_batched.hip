@@ -19,7 +19,6 @@
 #include <cstdlib>
 #include <map>
 #include <mutex>
-#include <numeric>
 #include <unordered_map>
 #include <vector>
 
@@ -657,8 +656,7 @@ int dlx_mft_batched_psf(int32_t n, const dlx_mft_instance* instances, int32_t n_
 
   // the launches, as a replayed graph when this shape was seen before
   bool eager = true;
-  if (cs == hipStreamCaptureStatusNone)
-    if (int st = launch_plan_graph(Q, ws, fresh, s, &eager)) return st;
+  if (int st = launch_plan_graph(Q, ws, fresh, s, &eager)) return st;
   if (eager)
     if (int st = launch_plan(Q, ws, fresh, s)) return st;
   if (fresh)

@@ -4,8 +4,8 @@
 // steps -- not on the field, the shifts or the weights -- so repeated
 // propagations (phase-retrieval iterations, a serving loop over the same
 // wavelength grid) reuse them instead of generating them per call.  An entry
-// holds the tables of one call's wavelengths, in both directions, or the plan
-// and tables of one uneven batch.
+// holds the tables of one call's wavelengths -- in both directions where a
+// gradient may follow -- or of one uneven batch.
 //
 // Stream safety: an entry records an event after its generation; a user on any
 // stream waits on it (hipStreamWaitEvent) before the tables are read.  Each

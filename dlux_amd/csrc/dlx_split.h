@@ -27,12 +27,4 @@ __device__ __forceinline__ void split2_bf16(float x0, float x1, uint32_t& hi, ui
   lo = bf16x2_rne(x0 - __uint_as_float(hi << 16), x1 - __uint_as_float(hi & 0xFFFF0000u));
 }
 
-// The value of lane q ^ M of the quad (DPP quad permutation); all four lanes active.
-template <int M>
-__device__ __forceinline__ uint32_t quad_xor(uint32_t v) {
-  // quad_perm [q ^ M for q in 0..3]
-  constexpr int ctrl = M == 1 ? 0xB1 : (M == 2 ? 0x4E : 0x1B);
-  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xF, 0xF, true);
-}
-
 }  // namespace dlx

@@ -197,15 +197,21 @@ class Server:
         keep.append(h)
         return h.to(self.dev, non_blocking=True)
 
-    # Device-time estimates used to place work: the contractions at ~300 TFLOP/s
-    # (8 (N_out N_in^2 + N_out^2 N_in) FLOPs per wavelength, four contractions'
-    # worth for a gradient) and the angular spectrum's three FFT launches (each
-    # reading and writing the padded array) at ~2.3 TB/s.
+    # Device-time estimates used to place work, from single requests of every size of
+    # the mix in the split form (within 20 % of most of their times, 35 us to 0.9 ms,
+    # and of 45 % of all; one rate was off by up to 2.6 one way and 100 the other): launches, the contractions by the plain
+    # complex products' count (8 (N_out N_in^2 + N_out^2 N_in) a wavelength, four
+    # times that for a gradient), and the fields, folded fields and gradient planes
+    # at 5 TB/s; the angular spectrum's three launches each read and write the padded
+    # array.
     def cost(self, r: Request) -> float:
         if r.kind == "asm":
-            return 3 * 16.0 * r.n_out ** 2 / 2.3e12
-        f = 8.0 * (r.n_out * r.n_in ** 2 + r.n_out ** 2 * r.n_in) * len(r.wavelengths)
-        return (4.0 if r.kind == "grad" else 1.0) * f / 300e12
+            return 3 * 16.0 * r.n_out ** 2 / 3.9e12
+        nwl = len(r.wavelengths)
+        f = 8.0 * (r.n_out * r.n_in ** 2 + r.n_out ** 2 * r.n_in) * nwl
+        if r.kind == "grad":
+            return 60e-6 + 4.0 * f / 1300e12 + 22.0 * r.n_in ** 2 * nwl / 5e12
+        return 35e-6 + f / 900e12 + 18.0 * r.n_in ** 2 * nwl / 5e12
 
     def _ws(self, nbytes: int) -> torch.Tensor:
         """The current stream's workspace arena, grown (x1.5) when too small."""
