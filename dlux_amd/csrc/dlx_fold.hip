@@ -1540,12 +1540,13 @@ hipError_t stage1_width(const FoldStage1& a, hipStream_t s) {
   //        128      18.9 / 26.0 / 42.9          12.8 / 14.3 / 20.4
   //        256      30.0 / 28.2 / 44.9          18.8 / 17.2 / 22.9
   //       1024      90.7 / 85.6 / 89.0          56.9 / 44.5 / 40.3
-  // An odd count of 64-column tiles leaves half of a 128-column one empty.  float32,
-  // bound by its products, takes 64 then (24 fields 511^2 -> 257^2, both stages:
-  // 145.3 us at 128 columns, 123.8 at 64; 126.3 and 138.0 at 64 of 512^2 -> 256^2),
-  // the split form, bound by forming the parts, does not (62.9 and 68.3).
-  const int c64 = (mh + 63) / 64;
-  const bool whole = BF || c64 % 2 == 0 || c64 > 9;
+  // (measured at this geometry; other sides enter by their tile counts).  Three
+  // 64-column tiles leave a quarter of two 128-column ones empty: float32, bound by
+  // its products, takes 64 then (24 fields 511^2 -> 257^2, both stages: 145.3 us at
+  // 128 columns, 123.8 at 64; 126.3 and 138.0 at 64 of 512^2 -> 256^2; five tiles, 8 of
+  // 512^2 -> 620^2, 94.1 and 98.5, eleven, 4 of 512^2 -> 1300^2, 133.9 and 138.6), the
+  // split form, bound by forming the parts, does not (62.9 and 68.3).
+  const bool whole = BF || (mh + 63) / 64 != 3;
   if (mh > 64 && whole && tiles(64) > 256) stage1_go<BF, LOAD, VEC, 128>(a, tiles(128), s);
   else if (mh > 32 && tiles(64) >= 192) stage1_go<BF, LOAD, VEC, 64>(a, tiles(64), s);
   else if (LOAD != FOLD_MEM && tiles(32) < 384) {
