@@ -36,10 +36,10 @@ ERR_BOUND = 1e-5
 # known size (profiles/mft_poly_512to256_64wl_hbm_traffic.md).  The counters cannot
 # be read from inside this process.
 # Keyed by (form, pupil generated in stage 1's loader).
-TRAFFIC_BYTES = {("bf16x3", True): 113.9e6}
+TRAFFIC_BYTES = {("bf16x3", True): 115.3e6}
 # MFMA busy fraction of the stage-1 kernel from rocprofv3 SQ_VALU_MFMA_BUSY_CYCLES /
 # (GRBM_GUI_ACTIVE / 8 x 1024 SIMDs) (profiles/mft_poly_512to256_64wl_mfma_counters.md).
-MFMA_BUSY_PMC = {("bf16x3", True): 0.261}
+MFMA_BUSY_PMC = {("bf16x3", True): 0.330}
 
 
 def _stage1_kernel(head, prologue):
@@ -696,7 +696,7 @@ def main():
     avg2 = t2_ms / max(c2, 1)
     achieved = n1 / (avg1 * 1e-3) / 1e12
     pair = cfg.mft_flops / ((avg1 + avg2) * 1e-3) / 1e12
-    terms = 3.0 if head == "bf16x3" else 1.0
+    terms = 4.0 if head == "bf16x3" else 1.0
     line = {
         "metric": METRIC,
         "value": 1e3 / ms,

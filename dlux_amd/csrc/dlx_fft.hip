@@ -337,7 +337,7 @@ struct RowFft {
 // What bounds a launch: LDS and vector work per element beside 16 bytes of HBM
 // traffic.  2048^2 angular spectrum of a 1024^2 field, us per launch (first /
 // mid / last), radix-8 stages with every stage and both ends through LDS: 15.8 /
-// 39.1 / 25.0; this form: 11.8 / 24.2 / 15.6.
+// 39.1 / 25.0; this form: 12.3 / 24.5 / 16.2.
 template <int LOG2M, int LOG2R, int PASS, bool INV>
 __global__ void __launch_bounds__(fft_threads(LOG2M, LOG2R), 4)
 fft_rows_kernel(const float2* __restrict__ in, float2* __restrict__ out, FftParams P) {

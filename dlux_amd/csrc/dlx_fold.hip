@@ -445,11 +445,11 @@ __device__ __forceinline__ void get_block(const uint8_t* x, f32x16_t& v) {
 // A workgroup takes 32 rows py of all eight (alpha, beta, c) parts -- the four
 // mirrored pixels of a loaded quad feed both alphas -- and BNQ outputs qx: at
 // 128 the field is formed once per 128-column tile (256 outputs), each wave
-// holds eight 32 x 32 blocks (eight fragment reads from LDS per 24 MFMAs of a
+// holds eight 32 x 32 blocks (eight fragment reads from LDS per 32 MFMAs of a
 // split stage), and two workgroups share a CU.  Launches with fewer tiles take
-// 64 or 32 columns.  Issue bounds the loop: 24 MFMAs and 180 vector instructions
+// 64 or 32 columns.  Issue bounds the loop: 32 MFMAs and 180 vector instructions
 // (phasors, folds, split) per wave and split stage.  64 wavelengths of 512^2 ->
-// 256^2: 38 us split, 88 float32, where the complex contractions took 101 and 332.
+// 256^2: 40-43 us split, 82-90 float32, where the complex contractions took 101 and 332.
 // ---------------------------------------------------------------------------
 struct Stage1Prob {
   const uint8_t* src;
@@ -930,7 +930,7 @@ fold_stage1_mem_kernel(FoldStage1 a) {
 // signs of y at its sign of x.  BQ = 32, for launches that leave compute units
 // idle: wave (beta, alpha) holds both components of one part, and two trades
 // leave it the outputs of one sign of x (alpha) and one of y (beta).  Reading U
-// and the products take similar times: 23.5 us split, 50 float32 at 64 wavelengths
+// and the products take similar times: 24-26 us split, 46-50 float32 at 64 wavelengths
 // of 512^2 -> 256^2 (64 MB of U; the complex contraction took 50 and 176).
 // ---------------------------------------------------------------------------
 struct Stage2Prob {
@@ -1198,9 +1198,9 @@ __device__ __forceinline__ int group_tile(const FoldGroup& l) {
 // instance's x shift rotates the even and odd parts (e' = e cos f + i o sin f,
 // o' = o cos f + i e sin f; cos and sin of the stage's k from a window in LDS),
 // the parts are split, and the tile's products run; the y shift is applied to
-// the results.  768 instances of 256^2 to 1024^2 take 182 + 141 + 96 us in the
-// three widths and 172 in stage 2 (the complex contractions 1360 in all); issue
-// bounds it as the stage above.
+// the results.  768 instances of 256^2 to 1024^2 take 228 + 164 + 119 us in the
+// three widths and 184 in stage 2 traced one by one, 610 in a row (the complex
+// contractions 1360 in all); issue bounds it as the stage above.
 template <int BNQ>
 __global__ void __launch_bounds__(kThreads, 2)
 fold_group_stage1_kernel(FoldGroup g) {
@@ -1531,15 +1531,15 @@ hipError_t stage1_width(const FoldStage1& a, hipStream_t s) {
   // compute units idle.  Measured per launch, us, at 16 / 32 / 64 / 128 columns
   // (16: the 16-row kernel at 32), 512^2 -> 256^2 pupils:
   //   tiles of 64   float32                     split
-  //        128      24.7 / 25.0 / 31.1 / 47.2   16.7 / 17.9 / 21.6 / 22.1
-  //        192      33.5 / 39.8 / 33.2 / 49.0   21.2 / 24.8 / 21.4 / 24.0
-  //        256      41.0 / 40.6 / 34.7 / 49.3   26.4 / 25.2 / 22.0 / 24.8
-  //        320      49.4 / 52.3 / 56.3 / 49.1   30.4 / 32.4 / 29.4 / 25.2
-  //       1024       122 /  113 /  102 / 82.9   78.6 / 71.6 / 52.6 / 39.2
+  //        128      20.0 / 21.4 / 28.1 / 42.7   14.1 / 15.8 / 18.0 / 21.2
+  //        192      27.2 / 31.4 / 28.4 / 43.9   18.5 / 22.3 / 19.7 / 22.6
+  //        256      33.5 / 32.3 / 29.1 / 44.5   22.2 / 22.9 / 20.8 / 24.0
+  //        320      43.4 / 44.2 / 46.6 / 44.7   25.6 / 28.2 / 26.5 / 24.7
+  //       1024       115 /  109 / 94.2 / 81.8   68.0 / 67.4 / 51.4 / 40.3
   // and for a folded field in memory, at 32 / 64 / 128:
-  //        128      18.9 / 26.0 / 42.9          12.8 / 14.3 / 20.4
-  //        256      30.0 / 28.2 / 44.9          18.8 / 17.2 / 22.9
-  //       1024      90.7 / 85.6 / 89.0          56.9 / 44.5 / 40.3
+  //        128      16.6 / 23.7 / 39.1          11.0 / 13.2 / 20.2
+  //        256      26.6 / 25.6 / 42.1          17.2 / 16.4 / 22.9
+  //       1024      90.6 / 88.7 / 85.9          65.9 / 49.2 / 46.8
   // (measured at this geometry; other sides enter by their tile counts).  Three
   // 64-column tiles leave a quarter of two 128-column ones empty: float32, bound by
   // its products, takes 64 then (24 fields 511^2 -> 257^2, both stages: 145.3 us at
@@ -1582,9 +1582,9 @@ hipError_t stage2_size(const FoldStage2& a, hipStream_t s) {
   auto tiles = [&](int q) { return (long)tx * ((mh + q - 1) / q) * a.batch; };
   // 32 rows a workgroup where 64 leave half of the compute units idle (or half of
   // the waves, at mh <= 32).  us at 32 / 64 rows, 512^2 -> 256^2, by tiles of 64:
-  // 64: 16.8 / 24.8 float32, 10.8 / 13.1 split; 160: 29.4 / 25.4 float32;
-  // 256: 30.2 / 26.8 float32, 18.9 / 15.7 split; one wavelength of 256^2 -> 128^2
-  // (4 tiles) 11.2 / 15.0 float32
+  // 64: 13.8 / 21.9 float32, 8.5 / 11.2 split; 128: 14.4 / 22.2, 9.7 / 12.0; 160:
+  // 26.4 / 22.5, 14.6 / 12.5; 512: 50.8 / 45.9, 31.1 / 24.2; one wavelength of 256^2 ->
+  // 128^2 (4 tiles) 11.2 / 15.0 float32
   if (mh <= 32 || tiles(64) <= 128)
     hipLaunchKernelGGL((fold_stage2_kernel<BF, EPI, 32, 4>), dim3((unsigned)tiles(32)),
                        dim3(kThreads), 0, s, a);

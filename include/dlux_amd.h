@@ -149,12 +149,14 @@ int dlx_intensity(int64_t npix, int32_t batch, const void* field,
  *   E_l = sqrt(w_l) * c_l * Y_l^T P_l X_l
  * and psf = sum_l |E_l|^2 (float32 N_out x N_out).  amp/opd/phase as in
  * dlx_pupil_field (NULL allowed); `scale` is the lambda-independent pupil
- * scale s (initial 1/N^2 times any power normalisation).  In the split-BF16x3
- * form with no phase, the pupil is generated inside the first contraction
- * from amp and opd where its tiles fill the GPU and amp / opd are 16-byte
- * aligned (no pupil array is written); the result is the
- * same bits either way (environment DLUX_AMD_PUPIL_PROLOGUE=0 forces the
- * two-kernel form).
+ * scale s (initial 1/N^2 times any power normalisation).  The pupil is formed
+ * inside the first contraction, in either precision and for any side and
+ * alignment, up to N_out = 512 -- with a phase plane or no plane, up to N_in =
+ * 256, or N_out = 256 where N_in is a multiple of 8 and the planes are 16-byte
+ * aligned -- and written to the workspace first otherwise, where that has room
+ * for it (on grids below about 200 it may not: then it is formed inside).  The
+ * result is the same bits either way; environment DLUX_AMD_PUPIL_PROLOGUE=0 has
+ * it written first wherever there is room (not in dlx_psf_poly_vjp).
  * Replaces the reference chain OpticalSystem.propagate -> propagate_mono ->
  * layers -> to_focus -> MFT -> psf.sum(0): optical_systems.py:147-223,
  * :391-425, :560-594, :659-680.
